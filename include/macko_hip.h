@@ -133,11 +133,26 @@ MACKO_API int macko_compress_f16_fill(const void *dense, int32_t rows, int32_t c
 
 /*
  * Y[b, :] = M X[b, :] for b < batch.  X is [batch, ldx] and Y [batch, ldy], row-major fp16 with
- * ldx >= cols and ldy >= rows (elements).  The matrix is streamed once per group of up to eight
- * vectors (as many as fit next to each other in LDS), the rest like macko_spmv_f16.  No
- * counterpart in the upstream package, whose LLM runner maps the single-vector operator over
- * the batch dimension (python_scripts/util_run_pruned_llm.py:112-118).
+ * ldx >= cols and ldy >= rows (elements).  From a few vectors on the product runs on the matrix
+ * cores, with the matrix decoded once for up to 128 vectors.  No counterpart in the upstream
+ * package, whose LLM runner maps the single-vector operator over the batch dimension
+ * (python_scripts/util_run_pruned_llm.py:112-118).
+ *
+ *   macko_spmv_f16_batched_workspace  *bytes = scratch memory that makes the product with these vectors
+ *                                     faster (0: none wanted).  X is then brought into the matrix cores' operand order
+ *                                     once instead of being gathered by every workgroup.
+ *   macko_spmv_f16_batched_ws         the product with `workspace` (device memory, 16-byte aligned, held
+ *                                     for this call until the stream has passed it; contents irrelevant
+ *                                     before and after).  NULL, misaligned or too small: not used.
+ *   macko_spmv_f16_batched            the same without workspace.
  */
+MACKO_API int macko_spmv_f16_batched_workspace(const void *x, int32_t rows, int32_t cols,
+                                     int64_t padded_entries, int32_t batch, int64_t ldx,
+                                     int64_t *bytes);
+MACKO_API int macko_spmv_f16_batched_ws(const void *values, const void *deltas, const int32_t *row_ptr,
+                              const void *x, void *y, int32_t rows, int32_t cols,
+                              int64_t padded_entries, int32_t batch, int64_t ldx, int64_t ldy,
+                              void *workspace, int64_t workspace_bytes, void *stream);
 MACKO_API int macko_spmv_f16_batched(const void *values, const void *deltas, const int32_t *row_ptr,
                            const void *x, void *y, int32_t rows, int32_t cols,
                            int64_t padded_entries, int32_t batch, int64_t ldx, int64_t ldy,

@@ -46,7 +46,7 @@ __device__ __forceinline__ void ring_issue(u32 vo, u32 dof, const u32x4 &bv, con
 }
 template <int D, int J, int N> __device__ __forceinline__ void ring_take(u32x4 &v, u32 &d) { Tracked::ring_take<D, J, N>(v, d); }
 
-// NB = vectors multiplied per launch (1, 2, 4 or 8).  With NB > 1 the NB copies of x are interleaved in
+// NB = vectors multiplied per launch (1, 2 or 4).  With NB > 1 the NB copies of x are interleaved in
 // LDS (element c of vector b at half-word c * NB + b), so one LDS read per stored entry fetches the
 // operand of every vector, and a row ends with NB sums.  NB > 1 exists for fp16 values, x in LDS,
 // plain product only.
@@ -66,14 +66,14 @@ template <int BLOCK, int D, bool X_LDS, bool AXPBY, int VB, int NB, int XF, bool
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_num_vgpr(kCompilerVgprs)))
 spmv_stream_kernel(const SpmvArgs a)
 {
-    static_assert(NB == 1 || (NB <= 8 && X_LDS && !AXPBY && VB == 2), "batched variant: fp16, x in LDS, plain product");
+    static_assert(NB == 1 || (NB <= 4 && X_LDS && !AXPBY && VB == 2), "batched variant: fp16, x in LDS, plain product");
     static_assert(XF == 0 || (NB == 1 && X_LDS && VB == 2), "fused staging: fp16, one vector, x in LDS");
     static_assert(!ROWS || (X_LDS && NB == 1 && XF == 0), "all rows of a tile in one pass: one vector, x in LDS");
     static_assert(!PLAN || (X_LDS && NB == 1 && XF == 0), "prepared cuts: one vector, x in LDS");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     MACKO_RESERVE_FIXED_REGISTERS(MACKO_STREAM_FIXED_REGISTERS);
     constexpr int WAVES = BLOCK / kWave;
-    constexpr int kBatchShift = NB == 8 ? 3 : (NB == 4 ? 2 : (NB == 2 ? 1 : 0));
+    constexpr int kBatchShift = NB == 4 ? 2 : (NB == 2 ? 1 : 0);
     constexpr int kTileLoads = 2 * D;  // tracked loads per full ring
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -381,7 +381,6 @@ spmv_stream_kernel(const SpmvArgs a)
     typedef __attribute__((address_space(3))) const uint16_t *lds_u16_ptr;
     typedef __attribute__((address_space(3))) const u32 *lds_u32_ptr;
     typedef __attribute__((address_space(3))) const u32x2 *lds_u32x2_ptr;
-    typedef __attribute__((address_space(3))) const u32x4 *lds_u32x4_ptr;
     // LDS byte address of x[0] (x sits kLdsFront bytes, times NB, into this kernel's dynamic LDS)
     const u32 x_addr = (u32)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds + kLdsFront * NB;
     // row_addr: LDS byte address the next entry of the current row would read if its nibble were 0,
@@ -411,14 +410,10 @@ spmv_stream_kernel(const SpmvArgs a)
                 u32 xs[NB / 2 > 0 ? NB / 2 : 1];  // the NB operands, two per word
                 if (NB == 2) {
                     xs[0] = *reinterpret_cast<lds_u32_ptr>(at);
-                } else if (NB == 4) {
+                } else {
                     const u32x2 t = *reinterpret_cast<lds_u32x2_ptr>(at);
                     xs[0] = t.x;
                     xs[1 % (NB / 2)] = t.y;
-                } else {
-                    const u32x4 t = *reinterpret_cast<lds_u32x4_ptr>(at);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) xs[q % (NB / 2)] = t[q];
                 }
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
@@ -967,8 +962,8 @@ int plan_waves(int rows, int cols, long long padded, long long *n_waves)
     return 0;
 }
 
-// LDS the split kernel keeps behind x at most (16 waves, up to 8 vectors and a flag each)
-constexpr size_t kSplitPieceBytes = 16 * 4 * 9 + 4;
+// LDS the split kernel keeps behind x at most (16 waves, up to 4 vectors and a flag each)
+constexpr size_t kSplitPieceBytes = 16 * 4 * 5 + 4;
 
 int check_spmv_args(const void *values, const void *deltas, const int32_t *row_ptr, const void *x, void *y,
                     int32_t rows, int32_t cols, int64_t padded, int value_bytes = 2)
@@ -1148,18 +1143,51 @@ extern "C" int macko_spmv_i8f16_axpby(const void *values, const void *deltas, co
     return spmv_dispatch<true, 1>(a, as_stream(stream));
 }
 
+namespace macko {
+namespace {
+
+// Vectors of the next gather launch: 4, 2 or 1, as many as are left and fit in LDS next to each other.
+int gather_step(int left, int cols, long long padded, const DeviceInfo &info)
+{
+    const size_t per_vector = (size_t)kLdsFront + 2 * (size_t)cols + kLdsBack;
+    for (int step = 4; step > 1; step /= 2)
+        if (padded > 0 && left >= step && step * per_vector + kSplitPieceBytes <= (size_t)info.max_lds_bytes) return step;
+    return 1;
+}
+
+bool batched_on_tiles(int rows, int cols, long long padded, int batch, long long ldx, const DeviceInfo &info)
+{
+    return spmv_tile_takes(rows, cols, padded, batch, ldx, gather_step(batch, cols, padded, info) == batch ? 1 : 2);
+}
+
+}  // namespace
+}  // namespace macko
+
 // Y[b, :] = M X[b, :] for `batch` vectors: X is [batch, ldx] and Y [batch, ldy] row-major fp16
-// (ldx >= cols, ldy >= rows).  The matrix is streamed once per group of up to eight vectors (as
-// many as fit in LDS next to each other), so the cost per vector drops accordingly.  The upstream
-// package has no batched entry: its LLM runner maps the single-vector operator over the batch
-// dimension (python_scripts/util_run_pruned_llm.py:112-118).
-extern "C" int macko_spmv_f16_batched(const void *values, const void *deltas, const int32_t *row_ptr,
-                                      const void *x, void *y, int32_t rows, int32_t cols,
-                                      int64_t padded_entries, int32_t batch, int64_t ldx, int64_t ldy,
-                                      void *stream)
+// (ldx >= cols, ldy >= rows).  Two or four vectors go through the gather kernels in one launch; from
+// there on the matrix cores do it (macko_spmv_tile.hip), decoding the matrix once for 64 or 128
+// vectors.  The upstream package has no batched entry: its LLM runner maps the single-vector operator
+// over the batch dimension (python_scripts/util_run_pruned_llm.py:112-118).
+extern "C" int macko_spmv_f16_batched_workspace(const void *x, int32_t rows, int32_t cols, int64_t padded_entries,
+                                                int32_t batch, int64_t ldx, int64_t *bytes)
 {
     using namespace macko;
-    if (batch < 0 || ldx < cols || ldy < rows || ldx >= (1ll << 31) || ldy >= (1ll << 31))
+    if (bytes == nullptr || rows < 0 || cols < 0 || padded_entries < 0 || batch < 0 || ldx < cols) return MACKO_E_INVALID_ARGUMENT;
+    *bytes = 0;
+    if (batch == 0) return 0;
+    DeviceInfo info;
+    const int rc = device_info(&info);
+    if (rc != 0) return rc;
+    if (batched_on_tiles(rows, cols, padded_entries, batch, ldx, info)) *bytes = (int64_t)spmv_tile_workspace(cols, batch, x, ldx);
+    return 0;
+}
+
+extern "C" int macko_spmv_f16_batched_ws(const void *values, const void *deltas, const int32_t *row_ptr, const void *x,
+                                         void *y, int32_t rows, int32_t cols, int64_t padded_entries, int32_t batch,
+                                         int64_t ldx, int64_t ldy, void *workspace, int64_t workspace_bytes, void *stream)
+{
+    using namespace macko;
+    if (batch < 0 || ldx < cols || ldy < rows || ldx >= (1ll << 31) || ldy >= (1ll << 31) || workspace_bytes < 0)
         return MACKO_E_INVALID_ARGUMENT;
     if (batch == 0) return 0;
     int rc = check_spmv_args(values, deltas, row_ptr, x, y, rows, cols, padded_entries);
@@ -1167,31 +1195,33 @@ extern "C" int macko_spmv_f16_batched(const void *values, const void *deltas, co
     DeviceInfo info;
     rc = device_info(&info);
     if (rc != 0) return rc;
-    const size_t per_vector = (size_t)kLdsFront + 2 * (size_t)cols + kLdsBack;
-    int done = 0;
-    while (done < batch) {
-        const int left = batch - done;
-        SpmvArgs a{(const u32 *)values, (const u32 *)deltas, row_ptr,
-                   (const uint16_t *)x + (size_t)done * (size_t)ldx, (uint16_t *)y + (size_t)done * (size_t)ldy,
-                   rows, cols, padded_entries, 1.0f, 0.0f, 0, 0, 0, 0, 0, (int)ldx, (int)ldy};
-        int step;
-        if (padded_entries > 0 && left >= 8 && 8 * per_vector + kSplitPieceBytes <= (size_t)info.max_lds_bytes) {
-            step = 8;
-            rc = spmv_dispatch<false, 2, 8>(a, as_stream(stream));
-        } else if (padded_entries > 0 && left >= 4 && 4 * per_vector + kSplitPieceBytes <= (size_t)info.max_lds_bytes) {
-            step = 4;
-            rc = spmv_dispatch<false, 2, 4>(a, as_stream(stream));
-        } else if (padded_entries > 0 && left >= 2 && 2 * per_vector + kSplitPieceBytes <= (size_t)info.max_lds_bytes) {
-            step = 2;
-            rc = spmv_dispatch<false, 2, 2>(a, as_stream(stream));
-        } else {
-            step = 1;
-            rc = spmv_dispatch<false>(a, as_stream(stream));
+    auto args_from = [&](int first) {
+        return SpmvArgs{(const u32 *)values, (const u32 *)deltas, row_ptr,
+                        (const uint16_t *)x + (size_t)first * (size_t)ldx, (uint16_t *)y + (size_t)first * (size_t)ldy,
+                        rows, cols, padded_entries, 1.0f, 0.0f, 0, 0, 0, 0, 0, (int)ldx, (int)ldy};
+    };
+    if (batched_on_tiles(rows, cols, padded_entries, batch, ldx, info))
+        return spmv_tile_launch(args_from(0), batch, workspace, (size_t)workspace_bytes, as_stream(stream));
+    for (int done = 0; done < batch;) {
+        const SpmvArgs a = args_from(done);
+        const int step = gather_step(batch - done, cols, padded_entries, info);
+        switch (step) {
+        case 4: rc = spmv_dispatch<false, 2, 4>(a, as_stream(stream)); break;
+        case 2: rc = spmv_dispatch<false, 2, 2>(a, as_stream(stream)); break;
+        default: rc = spmv_dispatch<false>(a, as_stream(stream)); break;
         }
         if (rc != 0) return rc;
         done += step;
     }
     return 0;
+}
+
+extern "C" int macko_spmv_f16_batched(const void *values, const void *deltas, const int32_t *row_ptr, const void *x,
+                                      void *y, int32_t rows, int32_t cols, int64_t padded_entries, int32_t batch,
+                                      int64_t ldx, int64_t ldy, void *stream)
+{
+    return macko_spmv_f16_batched_ws(values, deltas, row_ptr, x, y, rows, cols, padded_entries, batch, ldx, ldy, nullptr, 0,
+                                     stream);
 }
 
 namespace macko {

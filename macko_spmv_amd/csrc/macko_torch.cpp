@@ -142,9 +142,18 @@ at::Tensor multiply_batched_hip(const at::Tensor &M_values, const at::Tensor &M_
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(M_values.device());
     at::Tensor Y = at::empty({X.size(0), M_rows}, M_values.options());
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
-    check_rc(macko_spmv_f16_batched(M_values.data_ptr(), M_deltas.data_ptr(), M_row_indices.data_ptr<int>(),
-                                    X.data_ptr(), Y.data_ptr(), (int32_t)M_rows, (int32_t)M_cols, M_values.numel(),
-                                    (int32_t)X.size(0), X.size(1), M_rows, (void *)stream),
+    TORCH_CHECK(X.size(0) < (1ll << 31), "batch too large");
+    int64_t scratch_bytes = 0;
+    check_rc(macko_spmv_f16_batched_workspace(X.data_ptr(), (int32_t)M_rows, (int32_t)M_cols, M_values.numel(),
+                                              (int32_t)X.size(0), X.size(1), &scratch_bytes),
+             "multiply_batched");
+    // from torch's pool: used on this stream only, so it may go back to the pool when the call returns
+    at::Tensor scratch;
+    if (scratch_bytes > 0) scratch = at::empty({scratch_bytes}, M_deltas.options());
+    check_rc(macko_spmv_f16_batched_ws(M_values.data_ptr(), M_deltas.data_ptr(), M_row_indices.data_ptr<int>(),
+                                       X.data_ptr(), Y.data_ptr(), (int32_t)M_rows, (int32_t)M_cols, M_values.numel(),
+                                       (int32_t)X.size(0), X.size(1), M_rows,
+                                       scratch_bytes > 0 ? scratch.data_ptr() : nullptr, scratch_bytes, (void *)stream),
              "multiply_batched");
     return Y;
 }
