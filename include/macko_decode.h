@@ -55,6 +55,21 @@ MACKO_API int macko_decode_rope_attention_f16(const void *q, const void *k, cons
                                     void *out, int32_t n_heads, int32_t head_dim, int32_t max_len,
                                     float scale, void *stream);
 
+/*
+ * The same up to the last step: the context of every head is worked in MACKO_ATTENTION_PARTS pieces by
+ * workgroups of their own, and their results are left as they are, to be merged by the product that
+ * consumes them (macko_spmv_f16_attention_axpby).  head_dim 64 or 128, all pointers 16-byte aligned.
+ *   parts  fp32 [n_heads][MACKO_ATTENTION_PARTS][head_dim], the sums of v weighted by exp(score - m_p),
+ *          then [n_heads][MACKO_ATTENTION_PARTS][2], the pieces' (m_p, sum of the weights);
+ *          out = sum_p exp(m_p - max m) parts_p / sum_p exp(m_p - max m) sum_p.
+ */
+#define MACKO_ATTENTION_PARTS 4
+MACKO_API int macko_decode_rope_attention_parts_f16(const void *q, const void *k, const void *v,
+                                          const float *cos_table, const float *sin_table,
+                                          const int64_t *position, void *k_cache, void *v_cache,
+                                          float *parts, int32_t n_heads, int32_t head_dim,
+                                          int32_t max_len, float scale, void *stream);
+
 /* out[i] = silu(gate[i]) * up[i], i < n. */
 MACKO_API int macko_decode_silu_mul_f16(const void *gate, const void *up, void *out, int32_t n,
                               void *stream);

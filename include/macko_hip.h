@@ -168,6 +168,9 @@ MACKO_API int macko_spmv_f16_batched(const void *values, const void *deltas, con
  * macko_spmv_f16_rmsnorm:        y = M n,  n[i] = fp16(x[i] * rsqrt(mean(x^2) + eps) * norm_weight[i])
  * macko_spmv_f16_silu_mul_axpby: y = alpha * M g + beta * y,  g[i] = fp16(silu(gate[i]) * up[i]);
  *                                with alpha == 1 and beta == 0, y is not read.
+ * macko_spmv_f16_attention_axpby: y = alpha * M a + beta * y,  a = the attention output that
+ *                                macko_decode_rope_attention_parts_f16 (macko_decode.h) left in pieces,
+ *                                cols = n_heads * head_dim, head_dim 64 or 128; parts 16-byte aligned.
  */
 MACKO_API int macko_spmv_f16_rmsnorm(const void *values, const void *deltas, const int32_t *row_ptr,
                            const void *x, const void *norm_weight, float eps, void *y,
@@ -176,6 +179,11 @@ MACKO_API int macko_spmv_f16_silu_mul_axpby(const void *values, const void *delt
                                   const void *gate, const void *up, void *y, int32_t rows,
                                   int32_t cols, int64_t padded_entries, float alpha, float beta,
                                   void *stream);
+
+MACKO_API int macko_spmv_f16_attention_axpby(const void *values, const void *deltas,
+                                   const int32_t *row_ptr, const float *parts, int32_t head_dim,
+                                   void *y, int32_t rows, int32_t cols, int64_t padded_entries,
+                                   float alpha, float beta, void *stream);
 
 /*
  * int8 values variant.  Same arrays, except that `values` holds int8 [P] (8-byte aligned) and

@@ -85,6 +85,20 @@ def _decode_rope_attention_fake(q, k, v, cos_table, sin_table, position, k_cache
     return torch.empty_like(q)
 
 
+_ATTENTION_PARTS = 4  # MACKO_ATTENTION_PARTS, include/macko_decode.h
+
+
+@torch.library.register_fake("macko_spmv::decode_rope_attention_parts")
+def _decode_rope_attention_parts_fake(q, k, v, cos_table, sin_table, position, k_cache, v_cache, scale):
+    n_heads, _, head_dim = k_cache.shape
+    return torch.empty((n_heads * _ATTENTION_PARTS * (head_dim + 2),), device=q.device, dtype=torch.float32)
+
+
+@torch.library.register_fake("macko_spmv::multiply_attention_axpby")
+def _multiply_attention_axpby_fake(M_values, M_deltas, M_row_indices, M_rows, M_cols, parts, head_dim, C, alpha, beta):
+    return None
+
+
 @torch.library.register_fake("macko_spmv::decode_rmsnorm")
 def _decode_rmsnorm_fake(x, weight, eps):
     return torch.empty_like(x)
@@ -254,6 +268,15 @@ def multiply_silu_mul_axpby(compressed_M, gate, up, C, alpha=1.0, beta=0.0):
     applied while the down projection stages its input.  Same limits as multiply_rmsnorm."""
     assert compressed_M[0].is_cuda and gate.is_cuda and up.is_cuda and C.is_cuda
     torch.ops.macko_spmv.multiply_silu_mul_axpby.default(*compressed_M[:5], gate, up, C, float(alpha), float(beta))
+    return C
+
+
+def multiply_attention_axpby(compressed_M, parts, head_dim, C, alpha=1.0, beta=0.0):
+    """In place C = alpha * M @ attention + beta * C, the attention output in the pieces that
+    torch.ops.macko_spmv.decode_rope_attention_parts leaves, merged while the product stages its input.
+    head_dim 64 or 128; same limits as multiply_rmsnorm."""
+    assert compressed_M[0].is_cuda and parts.is_cuda and C.is_cuda
+    torch.ops.macko_spmv.multiply_attention_axpby.default(*compressed_M[:5], parts, head_dim, C, float(alpha), float(beta))
     return C
 
 

@@ -29,10 +29,12 @@ namespace {
 using namespace spmv_detail;
 
 // The hand-tracked loads (macko_spmv_tracked.h) with this kernel's register map: the compiler keeps
-// below v78; v78,v79 row_ptr probes; v80..v87 two 16-byte pieces of x; v88.. the ring (up to four
-// slots: v88..v103 values, v104..v107 delta words at depth 4).
+// below v78; v78,v79 row_ptr probes; v80..v87 two 16-byte pieces of x; v88.. the ring (two slots:
+// v88..v95 values, v96,v97 delta words); v98..v121 operands of a function applied while staging (XF).
 constexpr int kCompilerVgprs = 78;
+constexpr int kOperandRegs = 98;
 #define MACKO_STREAM_FIXED_REGISTERS "v78", "v79", "v80", "v81", "v82", "v83", "v84", "v85", "v86", "v87", "v88", "v89", "v90", "v91", "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107"
+#define MACKO_STREAM_OPERAND_REGISTERS "v108", "v109", "v110", "v111", "v112", "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121"
 typedef TrackedLoads<kCompilerVgprs> Tracked;
 template <int K> __device__ __forceinline__ void probe_issue(u32 o, const u32x4 &b) { Tracked::probe_issue<K>(o, b); }
 template <int K, int N> __device__ __forceinline__ int probe_take() { return Tracked::probe_take<K, N>(); }
@@ -41,10 +43,74 @@ template <int J, int N> __device__ __forceinline__ void xpiece_to_lds(u32 a) { T
 template <int D, int J, int VB>
 __device__ __forceinline__ void ring_issue(u32 vo, u32 dof, const u32x4 &bv, const u32x4 &bd, bool stream)
 {
-    static_assert(D == 1 || D == 2 || (D == 4 && VB == 2), "ring depth");
+    static_assert(D == 1 || D == 2, "ring depth");
     Tracked::ring_issue<D, J, VB>(vo, dof, bv, bd, stream);
 }
 template <int D, int J, int N> __device__ __forceinline__ void ring_take(u32x4 &v, u32 &d) { Tracked::ring_take<D, J, N>(v, d); }
+
+// The input of XF != 0 from operands that have landed in the fixed registers; what lies beyond the first
+// two pieces per thread (XF == 3: four columns per thread) goes through ordinary loads.  Same arithmetic
+// in the same order as stage_x_untracked.
+constexpr int kStreamThreads = 1024;
+template <int XF>
+__device__ __forceinline__ void stage_function(unsigned char *lds, const SpmvArgs &a, index_constant<XF>, int tid, int lane, int wave)
+{
+    constexpr int BLOCK = kStreamThreads, WAVES = BLOCK / kWave;
+    uint16_t *dst = reinterpret_cast<uint16_t *>(lds + kLdsFront);
+    u32x4 *d4 = reinterpret_cast<u32x4 *>(dst);
+    const int nvec = a.cols >> 3;
+    if constexpr (XF == 3) {
+        float4 o[kAttentionParts];
+        float ml[2 * kAttentionParts];
+        static_for<kAttentionParts>([&](auto p) {
+            constexpr int P = decltype(p)::value;
+            o[P] = __builtin_bit_cast(float4, Tracked::piece_copy<kOperandRegs + 4 * P>());
+        });
+        static_for<kAttentionParts / 2>([&](auto p) {
+            constexpr int P = decltype(p)::value;
+            const float4 four = __builtin_bit_cast(float4, Tracked::piece_copy<kOperandRegs + 4 * (kAttentionParts + P)>());
+            ml[4 * P] = four.x;
+            ml[4 * P + 1] = four.y;
+            ml[4 * P + 2] = four.z;
+            ml[4 * P + 3] = four.w;
+        });
+        if (tid < a.cols >> 2) *reinterpret_cast<u32x2 *>(dst + 4 * tid) = merged_columns(o, ml);
+        for (int i = tid + BLOCK; i < a.cols >> 2; i += BLOCK) stage_merged(a, dst, i);
+    } else {
+        const u32x4 x0 = Tracked::piece_copy<kCompilerVgprs + 2>(), x1 = Tracked::piece_copy<kCompilerVgprs + 6>();
+        if constexpr (XF == 1) {
+            float ss = 0.f;
+            if (tid < nvec) ss = sum_of_squares(x0, ss);
+            if (tid + BLOCK < nvec) ss = sum_of_squares(x1, ss);
+            for (int i = tid + 2 * BLOCK; i < nvec; i += BLOCK) {
+                const u32x4 v = reinterpret_cast<const u32x4 *>(a.x)[i];
+                d4[i] = v;
+                ss = sum_of_squares(v, ss);
+            }
+            float *red = reinterpret_cast<float *>(lds + kLdsFront + 2 * (size_t)a.cols + kLdsBack);
+            const float ws = wave_sum(ss);
+            if (lane == 0) red[wave] = ws;
+            __syncthreads();
+            float total = 0.f;
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) total += red[w];
+            const float inv = rsqrtf(total / (float)a.cols + a.eps);
+            const u32x4 g0 = Tracked::piece_copy<kOperandRegs>(), g1 = Tracked::piece_copy<kOperandRegs + 4>();
+            if (tid < nvec) d4[tid] = scaled_piece(x0, inv, g0);
+            if (tid + BLOCK < nvec) d4[tid + BLOCK] = scaled_piece(x1, inv, g1);
+            for (int i = tid + 2 * BLOCK; i < nvec; i += BLOCK)
+                d4[i] = scaled_piece(d4[i], inv, reinterpret_cast<const u32x4 *>(a.x2)[i]);
+        } else {
+            const u32x4 g0 = Tracked::piece_copy<kOperandRegs>(), g1 = Tracked::piece_copy<kOperandRegs + 4>();
+            if (tid < nvec) d4[tid] = gated_piece(x0, g0);
+            if (tid + BLOCK < nvec) d4[tid + BLOCK] = gated_piece(x1, g1);
+            for (int i = tid + 2 * BLOCK; i < nvec; i += BLOCK)
+                d4[i] = gated_piece(reinterpret_cast<const u32x4 *>(a.x)[i], reinterpret_cast<const u32x4 *>(a.x2)[i]);
+        }
+    }
+    if (tid < kLdsFront / 4) reinterpret_cast<u32 *>(lds)[tid] = 0;
+    if (tid < kLdsBack / 2) dst[a.cols + tid] = 0;
+}
 
 // NB = vectors multiplied per launch (1, 2 or 4).  With NB > 1 the NB copies of x are interleaved in
 // LDS (element c of vector b at half-word c * NB + b), so one LDS read per stored entry fetches the
@@ -54,6 +120,13 @@ template <int D, int J, int N> __device__ __forceinline__ void ring_take(u32x4 &
 // launch of its own: 0 = none (x as given), 1 = RMS norm (x * rsqrt(mean(x^2) + eps) * x2, x2 the
 // norm weight), 2 = SiLU gate (silu(x) * x2).  The staged vector is rounded to fp16 exactly as a
 // separate kernel writing it to memory would.  XF != 0 needs cols % 8 == 0 and 16-byte aligned x, x2.
+// 3 = the pieces of an attention output, merged (a.parts; the attention kernel leaves them to its
+// consumer, which saves it waiting for its own workgroups).  In long streams (D == 2) the operands of
+// these functions travel through tracked loads like x itself: a wave's first tiles are requested right
+// behind them, and the function is computed while those are in flight (at density 0.5, 12288 x 4096 with
+// the norm 14.65 us with the tiles requested behind the staging, 14.25 now, 22016 x 4096 25.05 and 24.7,
+// 4096 x 11008 with the gate 14.9 and 14.5).  Short ones stage first: with one tile per wave the same
+// order costs 0.2 to 0.4 us (4096 x 4096 at 0.1: 4.5 against 4.9).
 // ROWS = with the pass that works all the rows of a tile at once (rows_pass below), for matrices of
 // short rows.  A variant of its own: compiled into the kernel, that pass costs the row loop of
 // every matrix 0.3 to 0.7 us per launch (measured on 4096 x 4096 and 11008 x 4096 at density 0.1),
@@ -72,6 +145,8 @@ spmv_stream_kernel(const SpmvArgs a)
     static_assert(!PLAN || (X_LDS && NB == 1 && XF == 0), "prepared cuts: one vector, x in LDS");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     MACKO_RESERVE_FIXED_REGISTERS(MACKO_STREAM_FIXED_REGISTERS);
+    if constexpr (XF == 3) MACKO_RESERVE_FIXED_REGISTERS(MACKO_STREAM_OPERAND_REGISTERS);
+    static_assert(BLOCK == kStreamThreads, "stage_function");
     constexpr int WAVES = BLOCK / kWave;
     constexpr int kBatchShift = NB == 4 ? 2 : (NB == 2 ? 1 : 0);
     constexpr int kTileLoads = 2 * D;  // tracked loads per full ring
@@ -128,9 +203,28 @@ spmv_stream_kernel(const SpmvArgs a)
         probe_issue<1>((u32)i1 * 4, buf_rows);
     }
     const u32x4 buf_x = make_buffer(a.x, (u32)x_nvec * 16);  // past the end reads as zero
-    if (X_LDS && NB == 1 && XF == 0) {
+    constexpr bool kTrackedOperands = XF != 0 && D == 2;
+    if (X_LDS && NB == 1 && (XF == 0 || (kTrackedOperands && XF < 3))) {
         xpiece_issue<0>((u32)tid * 16, buf_x);
         xpiece_issue<1>((u32)(tid + BLOCK) * 16, buf_x);
+    }
+    if constexpr (kTrackedOperands && XF < 3) {  // the second operand's pieces
+        const u32x4 buf_x2 = make_buffer(a.x2, (u32)a.cols * 2);
+        Tracked::piece_issue<kOperandRegs>((u32)tid * 16, buf_x2);
+        Tracked::piece_issue<kOperandRegs + 4>((u32)(tid + BLOCK) * 16, buf_x2);
+    }
+    if constexpr (kTrackedOperands && XF == 3) {  // four columns per thread: their pieces and the pieces' (maximum, sum) pairs
+        const u32 floats = (u32)a.cols * kAttentionParts + ((u32)a.cols >> a.head_shift) * 2 * kAttentionParts;
+        const u32x4 buf_parts = make_buffer(a.parts, floats * 4);
+        static_for<kAttentionParts>([&](auto p) {
+            constexpr int P = decltype(p)::value;
+            Tracked::piece_issue<kOperandRegs + 4 * P>(tid < a.cols >> 2 ? part_offset(a, tid, P) * 4 : kNoTileDeltas, buf_parts);
+        });
+        static_for<kAttentionParts / 2>([&](auto p) {
+            constexpr int P = decltype(p)::value;
+            Tracked::piece_issue<kOperandRegs + 4 * (kAttentionParts + P)>(
+                tid < a.cols >> 2 ? pair_offset(a, tid) * 4 + 16 * P : kNoTileDeltas, buf_parts);
+        });
     }
     if constexpr (PLAN) {  // the window of row starts from my first row on, behind the x pieces
         base[0] = (int)((u32)cut_row[0] < (u32)a.rows ? (u32)cut_row[0] : (u32)a.rows);
@@ -157,11 +251,11 @@ spmv_stream_kernel(const SpmvArgs a)
     // ---- 2. x: everything beyond the two register pieces per thread, and unaligned or odd-length
     //         x, goes to LDS through ordinary loads (rare: more than 16384 columns, or an x that is
     //         not 16-byte aligned) ------------------------------------------------------------------
-    stage_x_untracked<BLOCK, X_LDS, NB, XF>(lds, a, tid, lane, wave, x_vec, x_nvec);
+    if constexpr (!kTrackedOperands) stage_x_untracked<BLOCK, X_LDS, NB, XF>(lds, a, tid, lane, wave, x_vec, x_nvec);
     MACKO_STAMP(1);
 
     // ---- 3. which rows are mine -----------------------------------------------------------------------
-    constexpr int kXLoads = X_LDS && NB == 1 && XF == 0 ? kXRegs : 0;
+    constexpr int kXLoads = !X_LDS || NB > 1 || (XF != 0 && !kTrackedOperands) ? 0 : XF == 0 ? kXRegs : XF == 3 ? kAttentionParts + kAttentionParts / 2 : 2 * kXRegs;
     int window[2] = {0, 0};
     if constexpr (!PLAN) {
         window[0] = probe_take<0, kXLoads + 1>();
@@ -332,7 +426,12 @@ spmv_stream_kernel(const SpmvArgs a)
     }
 
     // ---- 5. x pieces into LDS (older than the ring loads just issued, if any) ---------------------------
-    if (NB > 1 || XF != 0) {
+    if (NB > 1 || (XF != 0 && !kTrackedOperands)) {
+        __syncthreads();
+    } else if constexpr (XF != 0) {
+        // the operands are older than the ring loads just issued, if any
+        if (__builtin_expect(have_work, 1)) Tracked::wait<kTileLoads>(); else Tracked::wait<0>();
+        stage_function(lds, a, index_constant<XF>{}, tid, lane, wave);
         __syncthreads();
     } else if (X_LDS) {
         const u32 lds_x = (u32)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds + kLdsFront;
@@ -1241,6 +1340,34 @@ int check_fused_args(const void *x, const void *x2, int32_t cols, int64_t padded
 }  // namespace
 }  // namespace macko
 
+namespace macko {
+namespace {
+// What the fused products have in common: operands and checks.
+int fused_args(SpmvArgs *out, const void *values, const void *deltas, const int32_t *row_ptr, const void *x, const void *x2,
+               void *y, int32_t rows, int32_t cols, int64_t padded, float alpha, float beta)
+{
+    int rc = check_spmv_args(values, deltas, row_ptr, x, y, rows, cols, padded);
+    if (rc != 0) return rc;
+    rc = check_fused_args(x, x2, cols, padded);
+    if (rc != 0) return rc;
+    SpmvArgs a{};
+    a.values = (const u32 *)values;
+    a.deltas = (const u32 *)deltas;
+    a.row_ptr = row_ptr;
+    a.x = (const uint16_t *)x;
+    a.x2 = (const uint16_t *)x2;
+    a.y = (uint16_t *)y;
+    a.rows = rows;
+    a.cols = cols;
+    a.padded = padded;
+    a.alpha = alpha;
+    a.beta = beta;
+    *out = a;
+    return 0;
+}
+}  // namespace
+}  // namespace macko
+
 // y = M * rmsnorm(x), rmsnorm(x)[i] = fp16(x[i] * rsqrt(mean(x^2) + eps) * norm_weight[i]): the
 // normalisation in front of a projection, folded into the product's own staging of its input.
 // No upstream counterpart: the upstream harness runs the stock module for the norm
@@ -1250,12 +1377,10 @@ extern "C" int macko_spmv_f16_rmsnorm(const void *values, const void *deltas, co
                                       int64_t padded_entries, void *stream)
 {
     using namespace macko;
-    int rc = check_spmv_args(values, deltas, row_ptr, x, y, rows, cols, padded_entries);
+    SpmvArgs a;
+    const int rc = fused_args(&a, values, deltas, row_ptr, x, norm_weight, y, rows, cols, padded_entries, 1.0f, 0.0f);
     if (rc != 0) return rc;
-    rc = check_fused_args(x, norm_weight, cols, padded_entries);
-    if (rc != 0) return rc;
-    SpmvArgs a{(const u32 *)values, (const u32 *)deltas, row_ptr, (const uint16_t *)x, (uint16_t *)y,
-               rows, cols, padded_entries, 1.0f, 0.0f, 0, 0, 0, 0, 0, 0, 0, (const uint16_t *)norm_weight, eps};
+    a.eps = eps;
     return spmv_dispatch<false, 2, 1, 1>(a, as_stream(stream));
 }
 
@@ -1267,12 +1392,25 @@ extern "C" int macko_spmv_f16_silu_mul_axpby(const void *values, const void *del
                                              int64_t padded_entries, float alpha, float beta, void *stream)
 {
     using namespace macko;
-    int rc = check_spmv_args(values, deltas, row_ptr, gate, y, rows, cols, padded_entries);
+    SpmvArgs a;
+    const int rc = fused_args(&a, values, deltas, row_ptr, gate, up, y, rows, cols, padded_entries, alpha, beta);
     if (rc != 0) return rc;
-    rc = check_fused_args(gate, up, cols, padded_entries);
-    if (rc != 0) return rc;
-    SpmvArgs a{(const u32 *)values, (const u32 *)deltas, row_ptr, (const uint16_t *)gate, (uint16_t *)y,
-               rows, cols, padded_entries, alpha, beta, 0, 0, 0, 0, 0, 0, 0, (const uint16_t *)up, 0.0f};
     if (beta == 0.0f && alpha == 1.0f) return spmv_dispatch<false, 2, 1, 2>(a, as_stream(stream));
     return spmv_dispatch<true, 2, 1, 2>(a, as_stream(stream));
+}
+
+// y = alpha * M * attention + beta * y, the attention output being merged from the pieces that
+// macko_decode_rope_attention_parts_f16 leaves.  No upstream counterpart (see above).
+extern "C" int macko_spmv_f16_attention_axpby(const void *values, const void *deltas, const int32_t *row_ptr,
+                                              const float *parts, int32_t head_dim, void *y, int32_t rows, int32_t cols,
+                                              int64_t padded_entries, float alpha, float beta, void *stream)
+{
+    using namespace macko;
+    if ((head_dim != 64 && head_dim != 128) || cols % head_dim != 0) return MACKO_E_INVALID_ARGUMENT;
+    SpmvArgs a;
+    const int rc = fused_args(&a, values, deltas, row_ptr, parts, parts, y, rows, cols, padded_entries, alpha, beta);
+    if (rc != 0) return rc;
+    a.parts = parts;
+    a.head_shift = head_dim == 128 ? 7 : 6;
+    return spmv_dispatch<true, 2, 1, 3>(a, as_stream(stream));
 }

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "macko_common.h"
+#include "macko_decode.h"
 
 namespace macko {
 namespace spmv_detail {
@@ -12,6 +13,7 @@ constexpr int kLdsFront = 16;   // zero bytes in front of x in LDS
 constexpr int kLdsBack = 64;    // zero bytes behind x
 constexpr int kTileShift = 9;   // log2(kTile)
 constexpr int kXRegs = 2;       // 16-byte pieces of x a thread fetches with tracked loads
+constexpr int kAttentionParts = MACKO_ATTENTION_PARTS;  // pieces of a head's context (macko_decode.h)
 constexpr int kLookBack = 2048; // entries covered by one 16-byte-per-lane load of deltas
 
 struct SpmvArgs {
@@ -41,6 +43,9 @@ struct SpmvArgs {
     // fused x staging (XF != 0): the second operand of the function that produces x, and its epsilon
     const uint16_t *x2;
     float eps;
+    // XF == 3: the pieces of an attention output (macko_decode.h) and log2 of its head dimension
+    const float *parts;
+    int head_shift;
     // Split kernel only.  log2 of the number of waves per workgroup that stream tiles (the others
     // only help to stage x).
     u32 active_shift;
@@ -304,7 +309,7 @@ __device__ __forceinline__ float pick_lane(const float (&c)[8], int idx, int L)
 
 // The kernel for matrices with few, long rows (macko_spmv_split.hip): workgroups own whole rows and
 // their waves share the workgroup's tiles evenly.  Variant selectors: axpby (y = alpha*Mx + beta*y),
-// value_bytes 2 (fp16) or 1 (int8), n_vectors 1/2/4, fused 0/1/2 (see SpmvArgs::x2), x_in_lds.
+// value_bytes 2 (fp16) or 1 (int8), n_vectors 1/2/4, fused 0/1/2/3 (see SpmvArgs::x2), x_in_lds.
 // lds_x = bytes of LDS that x takes (0 when x is gathered from memory).  Returns an ABI error code.
 int spmv_split_launch(const spmv_detail::SpmvArgs &a, bool axpby, int value_bytes, int n_vectors, int fused,
                       bool x_in_lds, int grid, size_t lds_x, hipStream_t stream);

@@ -76,6 +76,7 @@ __device__ __forceinline__ u32x4 look_take()
 // launch of its own: 0 = none (x as given), 1 = RMS norm (x * rsqrt(mean(x^2) + eps) * x2, x2 the
 // norm weight), 2 = SiLU gate (silu(x) * x2).  The staged vector is rounded to fp16 exactly as a
 // separate kernel writing it to memory would.  XF != 0 needs cols % 8 == 0 and 16-byte aligned x, x2.
+// 3 = the pieces of an attention output, merged (a.parts).
 template <int BLOCK, int D, bool X_LDS, bool AXPBY, int VB, int NB, int XF>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_num_vgpr(kCompilerVgprs)))
 spmv_split_kernel(const SpmvArgs a)
@@ -800,6 +801,7 @@ int spmv_split_launch(const spmv_detail::SpmvArgs &a, bool axpby, int value_byte
         if (axpby) return launch_split<2, true, true, 2, 1, 2>(a, grid, lds_x, stream);
         return launch_split<2, true, false, 2, 1, 2>(a, grid, lds_x, stream);
     }
+    if (fused == 3 && axpby && x_in_lds) return launch_split<2, true, true, 2, 1, 3>(a, grid, lds_x, stream);
     if (fused != 0) return MACKO_E_INVALID_ARGUMENT;
     if (n_vectors > 1) {
         if (axpby || value_bytes != 2 || !x_in_lds) return MACKO_E_INVALID_ARGUMENT;

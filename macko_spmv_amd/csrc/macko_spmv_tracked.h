@@ -61,6 +61,32 @@ struct TrackedLoads {
                      : "memory");
     }
 
+    // any 16-byte piece -> v[REG : REG+3] (a kernel's own registers behind the ring)
+    template <int REG>
+    static __device__ __forceinline__ void piece_issue(u32 byte_offset, const u32x4 &buffer)
+    {
+        static_assert(REG >= BASE, "fixed registers only");
+        asm volatile("buffer_load_dwordx4 v[%c2:%c3], %0, %1, 0 offen" ::"v"(byte_offset), "s"(buffer), "n"(REG), "n"(REG + 3)
+                     : "memory");
+    }
+    // copies a piece that has landed (the caller has waited for it)
+    template <int REG>
+    static __device__ __forceinline__ u32x4 piece_copy()
+    {
+        u32x4 v;
+        asm volatile("v_mov_b32 %0, v%c4\n\tv_mov_b32 %1, v%c5\n\tv_mov_b32 %2, v%c6\n\tv_mov_b32 %3, v%c7"
+                     : "=v"(v.x), "=v"(v.y), "=v"(v.z), "=v"(v.w)
+                     : "n"(REG), "n"(REG + 1), "n"(REG + 2), "n"(REG + 3)
+                     : "memory");
+        return v;
+    }
+    // waits until at most N loads are outstanding
+    template <int N>
+    static __device__ __forceinline__ void wait()
+    {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+    }
+
     // Ring slot J of a D-deep ring: issue both loads.  VB = bytes per stored value: 2 (fp16, 16 bytes
     // per lane and tile) or 1 (int8, 8 bytes per lane and tile, which land in the first two registers
     // of the slot).  `stream` (wave-uniform) adds the non-temporal hint: the matrix is read once per
@@ -107,11 +133,86 @@ struct TrackedLoads {
     }
 };
 
+// ---- functions applied to the input while it is staged (XF; SpmvArgs::x2, parts) --------------------
+__device__ __forceinline__ float low_half(u32 w) { return half_bits_to_float((uint16_t)(w & 0xffffu)); }
+__device__ __forceinline__ float high_half(u32 w) { return half_bits_to_float((uint16_t)(w >> 16)); }
+__device__ __forceinline__ u32 pack_halves(float l, float h)
+{
+    return (u32)float_to_half_bits(l) | ((u32)float_to_half_bits(h) << 16);
+}
+__device__ __forceinline__ float sum_of_squares(const u32x4 &v, float ss)
+{
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss += low_half(v[e]) * low_half(v[e]) + high_half(v[e]) * high_half(v[e]);
+    return ss;
+}
+// XF == 1: x * inv * g
+__device__ __forceinline__ u32x4 scaled_piece(const u32x4 &v, float inv, const u32x4 &g)
+{
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        o[e] = pack_halves(low_half(v[e]) * inv * low_half(g[e]), high_half(v[e]) * inv * high_half(g[e]));
+    return o;
+}
+// XF == 2: silu(g) * u
+__device__ __forceinline__ u32x4 gated_piece(const u32x4 &g, const u32x4 &u)
+{
+    auto gate = [](float gv, float uv) { return gv / (1.0f + __expf(-gv)) * uv; };
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        o[e] = pack_halves(gate(low_half(g[e]), low_half(u[e])), gate(high_half(g[e]), high_half(u[e])));
+    return o;
+}
+// XF == 3: four columns of an attention output from the kAttentionParts pieces of its head's context:
+// o[p] the weighted sum of v under piece p's own maximum, ml its (maximum, sum of weights) pairs
+__device__ __forceinline__ u32x2 merged_columns(const float4 (&o)[kAttentionParts], const float (&ml)[2 * kAttentionParts])
+{
+    float top = ml[0];
+#pragma unroll
+    for (int p = 1; p < kAttentionParts; ++p) top = fmaxf(top, ml[2 * p]);
+    float total = 0.f;
+    float4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int p = 0; p < kAttentionParts; ++p) {
+        const float w = __expf(ml[2 * p] - top);
+        total = __builtin_fmaf(w, ml[2 * p + 1], total);
+        sum.x = __builtin_fmaf(w, o[p].x, sum.x);
+        sum.y = __builtin_fmaf(w, o[p].y, sum.y);
+        sum.z = __builtin_fmaf(w, o[p].z, sum.z);
+        sum.w = __builtin_fmaf(w, o[p].w, sum.w);
+    }
+    const float inv = 1.0f / total;
+    return u32x2{pack_halves(sum.x * inv, sum.y * inv), pack_halves(sum.z * inv, sum.w * inv)};
+}
+// where columns 4 i .. 4 i + 3 of piece p stand, and their head's pairs (floats behind a.parts)
+__device__ __forceinline__ u32 part_offset(const SpmvArgs &a, int i, int p)
+{
+    const u32 c = 4u * (u32)i, head = c >> a.head_shift, d = c & ((1u << a.head_shift) - 1u);
+    return (((head * kAttentionParts + (u32)p) << a.head_shift) + d);
+}
+__device__ __forceinline__ u32 pair_offset(const SpmvArgs &a, int i)
+{
+    const u32 head = (4u * (u32)i) >> a.head_shift;
+    return (u32)a.cols * kAttentionParts + head * 2 * kAttentionParts;
+}
+__device__ __forceinline__ void stage_merged(const SpmvArgs &a, uint16_t *dst, int i)  // ordinary loads
+{
+    float4 o[kAttentionParts];
+    float ml[2 * kAttentionParts];
+#pragma unroll
+    for (int p = 0; p < kAttentionParts; ++p) o[p] = *reinterpret_cast<const float4 *>(a.parts + part_offset(a, i, p));
+#pragma unroll
+    for (int p = 0; p < 2 * kAttentionParts; ++p) ml[p] = a.parts[pair_offset(a, i) + p];
+    *reinterpret_cast<u32x2 *>(dst + 4 * i) = merged_columns(o, ml);
+}
+
 // What of x does not travel through the two tracked pieces per thread goes to LDS through ordinary
 // loads: everything with NB > 1 vectors (interleaved: element c of vector b at half-word c * NB + b)
-// or a function applied while staging (XF: 1 = RMS norm, 2 = SiLU gate; SpmvArgs::x2), else the
-// pieces beyond 2 * BLOCK (more than 16 * BLOCK columns) and an x that is not 16-byte aligned or of
-// odd length.  Also zeroes the bytes in front of and behind x.  The caller provides the barrier.
+// or a function applied while staging (XF: 1 = RMS norm, 2 = SiLU gate, 3 = attention pieces merged),
+// else the pieces beyond 2 * BLOCK (more than 16 * BLOCK columns) and an x that is not 16-byte aligned
+// or of odd length.  Also zeroes the bytes in front of and behind x.  The caller provides the barrier.
 template <int BLOCK, bool X_LDS, int NB, int XF>
 __device__ __forceinline__ void stage_x_untracked(unsigned char *lds, const SpmvArgs &a, int tid, int lane, int wave,
                                                   bool x_vec, int x_nvec)
@@ -154,9 +255,6 @@ __device__ __forceinline__ void stage_x_untracked(unsigned char *lds, const Spmv
         uint16_t *dst = reinterpret_cast<uint16_t *>(lds + kLdsFront);
         u32x4 *d4 = reinterpret_cast<u32x4 *>(dst);
         const int nvec = a.cols >> 3;
-        auto lo = [](u32 w) { return half_bits_to_float((uint16_t)(w & 0xffffu)); };
-        auto hi = [](u32 w) { return half_bits_to_float((uint16_t)(w >> 16)); };
-        auto pack = [](float l, float h) { return (u32)float_to_half_bits(l) | ((u32)float_to_half_bits(h) << 16); };
         if (XF == 1) {
             // pass 1: raw x into LDS and the sum of squares; pass 2: each thread scales the pieces
             // it wrote itself, so only the sum needs a barrier
@@ -164,8 +262,7 @@ __device__ __forceinline__ void stage_x_untracked(unsigned char *lds, const Spmv
             for (int i = tid; i < nvec; i += BLOCK) {
                 const u32x4 v = reinterpret_cast<const u32x4 *>(a.x)[i];
                 d4[i] = v;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) ss += lo(v[e]) * lo(v[e]) + hi(v[e]) * hi(v[e]);
+                ss = sum_of_squares(v, ss);
             }
             float *red = reinterpret_cast<float *>(lds + kLdsFront + 2 * (size_t)a.cols + kLdsBack);
             const float ws = wave_sum(ss);
@@ -175,24 +272,13 @@ __device__ __forceinline__ void stage_x_untracked(unsigned char *lds, const Spmv
 #pragma unroll
             for (int w = 0; w < WAVES; ++w) total += red[w];
             const float inv = rsqrtf(total / (float)a.cols + a.eps);
-            for (int i = tid; i < nvec; i += BLOCK) {
-                const u32x4 v = d4[i];
-                const u32x4 g = reinterpret_cast<const u32x4 *>(a.x2)[i];
-                u32x4 o;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = pack(lo(v[e]) * inv * lo(g[e]), hi(v[e]) * inv * hi(g[e]));
-                d4[i] = o;
-            }
+            for (int i = tid; i < nvec; i += BLOCK)
+                d4[i] = scaled_piece(d4[i], inv, reinterpret_cast<const u32x4 *>(a.x2)[i]);
+        } else if (XF == 2) {
+            for (int i = tid; i < nvec; i += BLOCK)
+                d4[i] = gated_piece(reinterpret_cast<const u32x4 *>(a.x)[i], reinterpret_cast<const u32x4 *>(a.x2)[i]);
         } else {
-            auto gate = [](float g, float u) { return g / (1.0f + __expf(-g)) * u; };
-            for (int i = tid; i < nvec; i += BLOCK) {
-                const u32x4 g = reinterpret_cast<const u32x4 *>(a.x)[i];
-                const u32x4 u = reinterpret_cast<const u32x4 *>(a.x2)[i];
-                u32x4 o;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = pack(gate(lo(g[e]), lo(u[e])), gate(hi(g[e]), hi(u[e])));
-                d4[i] = o;
-            }
+            for (int i = tid; i < a.cols >> 2; i += BLOCK) stage_merged(a, dst, i);
         }
         if (tid < kLdsFront / 4) reinterpret_cast<u32 *>(lds)[tid] = 0;
         if (tid < kLdsBack / 2) dst[a.cols + tid] = 0;

@@ -444,11 +444,10 @@ void multiply_silu_mul_axpby_hip(const at::Tensor &M_values, const at::Tensor &M
              "multiply_silu_mul_axpby");
 }
 
-// Rotary embedding, cache append and attention of one decode step in one launch; q, k, v are the
-// raw projections.  Returns the attention output [n_heads * head_dim].
-at::Tensor decode_rope_attention_hip(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
-                                     const at::Tensor &cos_table, const at::Tensor &sin_table,
-                                     const at::Tensor &position, at::Tensor k_cache, at::Tensor v_cache, double scale)
+// What the kernels that do rotary, cache append and attention in one launch check about their operands.
+void check_rope_attention(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v, const at::Tensor &cos_table,
+                          const at::Tensor &sin_table, const at::Tensor &position, const at::Tensor &k_cache,
+                          const at::Tensor &v_cache)
 {
     check_half_gpu(q, "q");
     check_half_gpu(k, "k");
@@ -464,15 +463,65 @@ at::Tensor decode_rope_attention_hip(const at::Tensor &q, const at::Tensor &k, c
                     sin_table.numel() == cos_table.numel(),
                 "cos/sin tables must be contiguous float32 GPU tensors [max_len, head_dim/2]");
     TORCH_CHECK(position.is_cuda() && position.dtype() == at::kLong && position.numel() == 1, "bad position");
+}
+
+// Rotary embedding, cache append and attention of one decode step in one launch; q, k, v are the
+// raw projections.  Returns the attention output [n_heads * head_dim].
+at::Tensor decode_rope_attention_hip(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
+                                     const at::Tensor &cos_table, const at::Tensor &sin_table,
+                                     const at::Tensor &position, at::Tensor k_cache, at::Tensor v_cache, double scale)
+{
+    check_rope_attention(q, k, v, cos_table, sin_table, position, k_cache, v_cache);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
     at::Tensor out = at::empty_like(q);
     check_rc(macko_decode_rope_attention_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos_table.data_ptr<float>(),
-                                             sin_table.data_ptr<float>(), position.data_ptr<int64_t>(),
-                                             k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), (int32_t)n_heads,
-                                             (int32_t)head_dim, (int32_t)max_len, (float)scale,
+                                             sin_table.data_ptr<float>(), position.data_ptr<int64_t>(), k_cache.data_ptr(),
+                                             v_cache.data_ptr(), out.data_ptr(), (int32_t)k_cache.size(0),
+                                             (int32_t)k_cache.size(2), (int32_t)k_cache.size(1), (float)scale,
                                              (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()),
              "decode_rope_attention");
     return out;
+}
+
+// The same with the output left in pieces for multiply_attention_axpby: float32, one row per head and
+// piece and one (maximum, sum) pair behind them all for each.
+at::Tensor decode_rope_attention_parts_hip(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
+                                           const at::Tensor &cos_table, const at::Tensor &sin_table,
+                                           const at::Tensor &position, at::Tensor k_cache, at::Tensor v_cache, double scale)
+{
+    check_rope_attention(q, k, v, cos_table, sin_table, position, k_cache, v_cache);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+    const int64_t n_heads = k_cache.size(0), head_dim = k_cache.size(2);
+    at::Tensor parts = at::empty({n_heads * MACKO_ATTENTION_PARTS * (head_dim + 2)}, cos_table.options());
+    check_rc(macko_decode_rope_attention_parts_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos_table.data_ptr<float>(),
+                                                   sin_table.data_ptr<float>(), position.data_ptr<int64_t>(),
+                                                   k_cache.data_ptr(), v_cache.data_ptr(), parts.data_ptr<float>(),
+                                                   (int32_t)n_heads, (int32_t)head_dim, (int32_t)k_cache.size(1),
+                                                   (float)scale,
+                                                   (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()),
+             "decode_rope_attention_parts");
+    return parts;
+}
+
+// C = alpha * M @ attention + beta * C, in place on C; the attention output in pieces, as
+// decode_rope_attention_parts left it.
+void multiply_attention_axpby_hip(const at::Tensor &M_values, const at::Tensor &M_deltas, const at::Tensor &M_row_indices,
+                                  int64_t M_rows, int64_t M_cols, const at::Tensor &parts, int64_t head_dim, at::Tensor C,
+                                  double alpha, double beta)
+{
+    check_macko_operands(M_values, M_deltas, M_row_indices, M_rows, M_cols);
+    check_half_gpu(C, "C");
+    TORCH_CHECK(head_dim == 64 || head_dim == 128, "head_dim must be 64 or 128");
+    TORCH_CHECK(parts.dtype() == at::kFloat && parts.is_cuda() && parts.is_contiguous() && M_cols % head_dim == 0 &&
+                    parts.numel() == M_cols / head_dim * MACKO_ATTENTION_PARTS * (head_dim + 2),
+                "parts must be what decode_rope_attention_parts returned for M_cols / head_dim heads");
+    TORCH_CHECK(C.numel() >= M_rows, "C must hold M_rows elements");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(M_values.device());
+    check_rc(macko_spmv_f16_attention_axpby(M_values.data_ptr(), M_deltas.data_ptr(), M_row_indices.data_ptr<int>(),
+                                            parts.data_ptr<float>(), (int32_t)head_dim, C.data_ptr(), (int32_t)M_rows,
+                                            (int32_t)M_cols, M_values.numel(), (float)alpha, (float)beta,
+                                            (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()),
+             "multiply_attention_axpby");
 }
 
 }  // namespace
@@ -507,6 +556,10 @@ TORCH_LIBRARY(macko_spmv, m)
           "Tensor gate, Tensor up, Tensor(a!) C, float alpha, float beta) -> ()");
     m.def("decode_rope_attention(Tensor q, Tensor k, Tensor v, Tensor cos_table, Tensor sin_table, Tensor position, "
           "Tensor(a!) k_cache, Tensor(b!) v_cache, float scale) -> Tensor");
+    m.def("decode_rope_attention_parts(Tensor q, Tensor k, Tensor v, Tensor cos_table, Tensor sin_table, "
+          "Tensor position, Tensor(a!) k_cache, Tensor(b!) v_cache, float scale) -> Tensor");
+    m.def("multiply_attention_axpby(Tensor M_values, Tensor M_deltas, Tensor M_row_indices, int M_rows, int M_cols, "
+          "Tensor parts, int head_dim, Tensor(a!) C, float alpha, float beta) -> ()");
     m.def("decompress(Tensor M_values, Tensor M_deltas, Tensor M_row_indices, int M_rows, int M_cols) -> Tensor");
 }
 
@@ -529,6 +582,8 @@ TORCH_LIBRARY_IMPL(macko_spmv, CUDA, m)
     m.impl("multiply_rmsnorm", &multiply_rmsnorm_hip);
     m.impl("multiply_silu_mul_axpby", &multiply_silu_mul_axpby_hip);
     m.impl("decode_rope_attention", &decode_rope_attention_hip);
+    m.impl("decode_rope_attention_parts", &decode_rope_attention_parts_hip);
+    m.impl("multiply_attention_axpby", &multiply_attention_axpby_hip);
     m.impl("decompress", &decompress_hip);
 }
 

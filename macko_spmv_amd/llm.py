@@ -392,14 +392,20 @@ class DecodeEngine:
                 qkv = macko_spmv.multiply_rmsnorm(L["qkv"], x, L["norm1"], self.eps)
             else:
                 qkv = self._matvec(L["qkv"], ops.decode_rmsnorm(x, L["norm1"], self.eps))
-            if self.fuse:
+            if sparse and self.head_dim in (64, 128):
+                parts = ops.decode_rope_attention_parts(qkv[:H], qkv[H:2 * H], qkv[2 * H:], self.cos, self.sin, position,
+                                                        L["k_cache"], L["v_cache"], self.scale)
+                macko_spmv.multiply_attention_axpby(L["o"], parts, self.head_dim, x, 1.0, 1.0)
+                a = None
+            elif self.fuse:
                 a = ops.decode_rope_attention(qkv[:H], qkv[H:2 * H], qkv[2 * H:], self.cos, self.sin, position,
                                               L["k_cache"], L["v_cache"], self.scale)
             else:
                 q = ops.decode_rope_append(qkv[:H], qkv[H:2 * H], qkv[2 * H:], self.cos, self.sin, position,
                                            L["k_cache"], L["v_cache"])
                 a = ops.decode_attention(q, L["k_cache"], L["v_cache"], position, self.scale)
-            self._matvec_add(L["o"], a, x)
+            if a is not None:
+                self._matvec_add(L["o"], a, x)
             if sparse:
                 gu = macko_spmv.multiply_rmsnorm(L["gate_up"], x, L["norm2"], self.eps)
                 macko_spmv.multiply_silu_mul_axpby(L["down"], gu[:I], gu[I:], x, 1.0, 1.0)
