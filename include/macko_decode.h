@@ -74,6 +74,34 @@ MACKO_API int macko_decode_rope_attention_parts_f16(const void *q, const void *k
 MACKO_API int macko_decode_silu_mul_f16(const void *gate, const void *up, void *out, int32_t n,
                               void *stream);
 
+/*
+ * The same parts for all tokens of a prompt at once.  Rows are contiguous, every pointer is 16-byte
+ * aligned, cols % 8 == 0; `packed` is written in the operand order of macko_spmv_f16_packed
+ * (macko_packed_bytes(cols, batch) bytes).
+ *   pack_rmsnorm   packed = rmsnorm(x[b, :]) * weight
+ *   pack_silu_mul  packed = silu(gate[b, :]) * up[b, :]
+ *   rope_append    q [batch, n_heads * head_dim] rotated in place, k rotated and v into the caches
+ *                  [n_heads, max_len, head_dim] at positions[b]; cos_rows / sin_rows fp16
+ *                  [batch, head_dim], both halves of a row alike; head_dim % 16 == 0
+ *   attention      packed = attention of token b over cache positions 0..positions[b]; q rotated,
+ *                  head_dim 64 or 128
+ */
+MACKO_API int macko_prefill_pack_rmsnorm_f16(const void *x, const void *weight, void *packed, int32_t cols,
+                                   int32_t batch, float eps, void *stream);
+/* y[b, :] = rmsnorm(x[b, :]) * weight as plain rows. */
+MACKO_API int macko_rmsnorm_rows_f16(const void *x, const void *weight, void *y, int32_t cols,
+                           int32_t batch, float eps, void *stream);
+MACKO_API int macko_prefill_pack_silu_mul_f16(const void *gate, const void *up, void *packed, int32_t cols,
+                                    int32_t batch, void *stream);
+MACKO_API int macko_prefill_rope_append_f16(void *q, const void *k, const void *v, const void *cos_rows,
+                                  const void *sin_rows, const int64_t *positions, void *k_cache,
+                                  void *v_cache, int32_t batch, int32_t n_heads, int32_t head_dim,
+                                  int32_t max_len, void *stream);
+MACKO_API int macko_prefill_attention_f16(const void *q, const void *k_cache, const void *v_cache,
+                                const int64_t *positions, void *packed, int32_t batch,
+                                int32_t n_heads, int32_t head_dim, int32_t max_len, float scale,
+                                void *stream);
+
 #ifdef __cplusplus
 }
 #endif

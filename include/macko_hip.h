@@ -159,6 +159,22 @@ MACKO_API int macko_spmv_f16_batched(const void *values, const void *deltas, con
                            void *stream);
 
 /*
+ * The product with several vectors in two steps, for vectors that several matrices multiply or that
+ * their producer writes in operand order itself (macko_decode.h).
+ *   macko_packed_bytes    size of `batch` vectors of `cols` >= 64 elements in operand order
+ *   macko_pack_f16        X [batch, ldx] into it (packed 16-byte aligned)
+ *   macko_spmv_f16_packed Y[b, :] = M X[b, :] (+ residual[b, :], laid out like Y, NULL: none; may be Y)
+ *                         with one rounding to fp16.
+ */
+MACKO_API int macko_packed_bytes(int32_t cols, int32_t batch, int64_t *bytes);
+MACKO_API int macko_pack_f16(const void *x, int32_t cols, int32_t batch, int64_t ldx, void *packed,
+                   void *stream);
+MACKO_API int macko_spmv_f16_packed(const void *values, const void *deltas, const int32_t *row_ptr,
+                          const void *packed, const void *residual, void *y, int32_t rows,
+                          int32_t cols, int64_t padded_entries, int32_t batch, int64_t ldy,
+                          void *stream);
+
+/*
  * Products whose input vector is produced on the fly while it is staged for the product, so a
  * decode step needs no launch for the producer.  No counterpart in the upstream package, whose
  * LLM runner leaves these parts to stock modules (python_scripts/util_run_pruned_llm.py:136-160).

@@ -99,6 +99,41 @@ def _multiply_attention_axpby_fake(M_values, M_deltas, M_row_indices, M_rows, M_
     return None
 
 
+def _packed_like(t, cols, batch):
+    # whole blocks of 64 columns and 16 vectors
+    return torch.empty(((cols + 63) // 64 * ((batch + 15) // 16) * 1024,), device=t.device, dtype=torch.float16)
+
+
+@torch.library.register_fake("macko_spmv::pack_rmsnorm")
+def _pack_rmsnorm_fake(x, weight, eps):
+    return _packed_like(x, x.shape[1], x.shape[0])
+
+
+@torch.library.register_fake("macko_spmv::rmsnorm_rows")
+def _rmsnorm_rows_fake(x, weight, eps):
+    return torch.empty_like(x)
+
+
+@torch.library.register_fake("macko_spmv::pack_silu_mul")
+def _pack_silu_mul_fake(gate, up):
+    return _packed_like(gate, gate.shape[1], gate.shape[0])
+
+
+@torch.library.register_fake("macko_spmv::multiply_packed")
+def _multiply_packed_fake(M_values, M_deltas, M_row_indices, M_rows, M_cols, packed, batch, residual):
+    return torch.empty((batch, M_rows), device=M_values.device, dtype=M_values.dtype)
+
+
+@torch.library.register_fake("macko_spmv::prefill_rope_append")
+def _prefill_rope_append_fake(q, k, v, cos_rows, sin_rows, positions, k_cache, v_cache):
+    return None
+
+
+@torch.library.register_fake("macko_spmv::prefill_attention")
+def _prefill_attention_fake(q, k_cache, v_cache, positions, scale):
+    return _packed_like(q, q.shape[1], q.shape[0])
+
+
 @torch.library.register_fake("macko_spmv::decode_rmsnorm")
 def _decode_rmsnorm_fake(x, weight, eps):
     return torch.empty_like(x)

@@ -27,7 +27,8 @@ TORCH_LIB = "libmacko_torch.so"
 BENCH_LIB = "libmacko_bench.so"  # kernels of bench.py only; the package never loads it
 ARCH = "gfx950"
 
-HIP_SOURCES = ["macko_spmv.hip", "macko_spmv_split.hip", "macko_spmv_tile.hip", "macko_compress.hip", "macko_runtime.hip", "macko_decode.hip"]
+HIP_SOURCES = ["macko_spmv.hip", "macko_spmv_split.hip", "macko_spmv_tile.hip", "macko_compress.hip", "macko_runtime.hip", "macko_decode.hip",
+               "macko_prefill.hip"]
 TORCH_SOURCES = ["macko_torch.cpp"]
 BENCH_SOURCES = ["macko_bench_kernels.hip"]
 

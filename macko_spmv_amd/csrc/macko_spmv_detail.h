@@ -319,6 +319,7 @@ int spmv_split_launch(const spmv_detail::SpmvArgs &a, bool axpby, int value_byte
 // without workspace it reads X as it is, more slowly).
 bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long ldx, int gather_launches);
 size_t spmv_tile_workspace(int cols, int batch, const void *x, long long ldx);
+int spmv_tile_pack(const uint16_t *x, int cols, int batch, long long ldx, void *packed, hipStream_t stream);
 int spmv_tile_launch(const spmv_detail::SpmvArgs &a, int batch, void *workspace, size_t workspace_bytes, hipStream_t stream);
 
 }  // namespace macko

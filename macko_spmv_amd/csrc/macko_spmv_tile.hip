@@ -29,6 +29,7 @@
 // sum that is not finite is computed again from its row's entries alone.
 #include <atomic>
 
+#include "macko_packed.h"
 #include "macko_spmv_detail.h"
 
 namespace macko {
@@ -71,6 +72,7 @@ struct TileArgs {
     const u32x4 *packed;  // X in operand order (pack_vectors_kernel), null: read X itself
     int packed_tiles;     // vector tiles in it
     int packed_steps;     // 64-column steps in it
+    const uint16_t *residual;  // added to Y before it is rounded (laid out like Y, may be Y), or null
 };
 
 __device__ __forceinline__ void lds_barrier()
@@ -89,26 +91,10 @@ __device__ __forceinline__ u32 clamp_between(u32 v, int lo, int hi)
     return r;
 }
 
-// The halves of a 16-byte piece from element `by` on, zeros behind them (by >= 8: all zero).
-__device__ __forceinline__ u32x4 shift_down(u32x4 v, int by)
-{
-    unsigned long long lo = v.x | ((unsigned long long)v.y << 32), hi = v.z | ((unsigned long long)v.w << 32);
-    if (by >= 4) {
-        lo = hi;
-        hi = 0;
-        by -= 4;
-    }
-    if (by >= 4) lo = 0, by = 0;
-    if (by > 0) {
-        const int s = 16 * by;
-        lo = (lo >> s) | (hi << (64 - s));
-        hi >>= s;
-    }
-    return u32x4{(u32)lo, (u32)(lo >> 32), (u32)hi, (u32)(hi >> 32)};
-}
-
-// sum of row [e0, e1)'s entries times one vector, by one wave; columns clamped to the vector
-__device__ __forceinline__ float exact_row_times_vector(const u32 *values, const u32 *deltas, u32 e0, u32 e1, const uint16_t *x, int cols)
+// sum of row [e0, e1)'s entries times one vector (x(c): its element c as bits), by one wave; columns
+// clamped to the vector
+template <typename X>
+__device__ __forceinline__ float exact_row_times_vector(const u32 *values, const u32 *deltas, u32 e0, u32 e1, X x, int cols)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const uint16_t *vals = reinterpret_cast<const uint16_t *>(values);
@@ -126,15 +112,13 @@ __device__ __forceinline__ float exact_row_times_vector(const u32 *values, const
         const int incl = wave_scan_inclusive(step);
         int c = column + incl;
         c = c < 0 ? 0 : (c >= cols ? cols - 1 : c);
-        if (j < e1) acc = __builtin_fmaf(v, half_bits_to_float(x[c]), acc);
+        if (j < e1) acc = __builtin_fmaf(v, half_bits_to_float(x(c)), acc);
         column += __builtin_amdgcn_readlane(incl, kWave - 1);
     }
     return wave_sum(acc);
 }
 
-// X in the order the waves of spmv_tile_kernel load it: per 64 columns and 16 vectors one block of
-// 2 x 64 pieces of 16 bytes, piece s * 64 + 16 q + n = columns 16 q + 8 s .. + 7 of vector n; zeros beyond
-// the columns and vectors there are.  A wave packs one block.
+// X in operand order (macko_packed.h).  A wave packs one block.
 __global__ void __launch_bounds__(256) pack_vectors_kernel(const uint16_t *__restrict__ x, u32x4 *__restrict__ packed,
                                                            int cols, int batch, u32 ldx, int tiles, int blocks)
 {
@@ -142,7 +126,7 @@ __global__ void __launch_bounds__(256) pack_vectors_kernel(const uint16_t *__res
     if (block >= blocks) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int k64 = block / tiles, tile = block - k64 * tiles;
-    const int piece = lane & 7, k = k64 * 64 + piece * 8;
+    const int piece = k64 * 8 + (lane & 7), k = piece * 8;
     const int last_piece = cols - 8;
     u32x4 v[2];
 #pragma unroll
@@ -157,7 +141,7 @@ __global__ void __launch_bounds__(256) pack_vectors_kernel(const uint16_t *__res
         v[0] = shift_down(v[0], by);
         v[1] = shift_down(v[1], by);
     }
-    u32x4 *dst = packed + (size_t)block * 128 + (piece & 1) * 64 + (piece >> 1) * 16 + (lane >> 3);
+    u32x4 *dst = packed + packed_piece(piece, tile * 16 + (lane >> 3), tiles);
     dst[0] = v[0];
     dst[8] = v[1];
 }
@@ -255,7 +239,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs 
                 for (int t = 0; t < NTW; ++t) {
                     int tile = (vector0 >> 4) + group * NTW + t;
                     tile = tile < a.packed_tiles ? tile : a.packed_tiles - 1;
-                    const u32x4 *block = a.packed + (size_t)(u32)(step * a.packed_tiles + tile) * 128;
+                    const u32x4 *block = a.packed + (size_t)(u32)(step * a.packed_tiles + tile) * kBlockPieces;
                     b[i][t][0] = block[lane];
                     b[i][t][1] = block[lane + 64];
                 }
@@ -434,12 +418,26 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs 
                 u32 e0 = (u32)uniform(a.row_ptr[bad_row]), e1 = (u32)uniform(a.row_ptr[bad_row + 1]);
                 e0 = e0 < a.padded ? e0 : a.padded;
                 e1 = e1 < a.padded ? e1 : a.padded;
-                const float exact = exact_row_times_vector(a.values, a.deltas, e0, e1, a.x + (size_t)bad_n * a.ldx, a.cols);
+                const float exact = exact_row_times_vector(
+                    a.values, a.deltas, e0, e1,
+                    [&](int c) {
+                        if constexpr (PACKED)
+                            return reinterpret_cast<const uint16_t *>(a.packed + packed_piece(c >> 3, bad_n, a.packed_tiles))[c & 7];
+                        else
+                            return a.x[(size_t)bad_n * a.ldx + (size_t)c];
+                    },
+                    a.cols);
                 sum[i] = lane == L ? exact : sum[i];
             }
         }
         if (n < a.batch) {
             uint16_t *dst = a.y + (size_t)n * a.ldy + row;
+            if (a.residual != nullptr) {
+                const uint16_t *add = a.residual + (size_t)n * a.ldy + row;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (row + i < row1) sum[i] += half_bits_to_float(add[i]);
+            }
             if (a.vector_store && row + 4 <= row1) {
                 const u32 lo = (u32)float_to_half_bits(sum[0]) | ((u32)float_to_half_bits(sum[1]) << 16);
                 const u32 hi = (u32)float_to_half_bits(sum[2]) | ((u32)float_to_half_bits(sum[3]) << 16);
@@ -509,15 +507,8 @@ int launch_tile_shape(TileArgs a, const TileShape &s, int max_lds, hipStream_t s
     a.vector_store = (a.ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 7) == 0) ? 1 : 0;
     const long long grid = s.row_blocks * a.vector_blocks;
     if (grid >= (1ll << 31)) return MACKO_E_INVALID_ARGUMENT;
-    if (a.packed != nullptr) {
-        a.packed_tiles = (a.batch + 15) / 16;
-        a.packed_steps = (a.cols + 63) / 64;
-        const int blocks = a.packed_tiles * a.packed_steps;
-        hipLaunchKernelGGL(pack_vectors_kernel, dim3((blocks + 3) / 4), dim3(256), 0, stream, a.x, (u32x4 *)a.packed, a.cols,
-                           a.batch, a.ldx, a.packed_tiles, blocks);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return (int)e;
-    }
+    a.packed_tiles = packed_tiles(a.batch);
+    a.packed_steps = packed_steps(a.cols);
 #define MACKO_TILE(RT_, NTW_, SC_)                                                                          \
     if (s.row_tiles == RT_ && s.wave_tiles == NTW_ && s.steps == SC_) {                                     \
         if (a.packed != nullptr) return launch_tile<RT_, NTW_, SC_, true>(a, (unsigned)grid, lds, stream);  \
@@ -616,14 +607,14 @@ bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long 
     if (rows == 0 || padded == 0 || cols < 64) return false;
     if (gather_launches < 2 && batch < 8) return false;
     // offsets into X and into its operand-order copy are 32-bit
-    return (long long)batch * ldx * 2 < (1ll << 32) && ((long long)batch + 15) * (cols + 63) * 2 < (1ll << 32);
+    return (long long)batch * ldx * 2 < (1ll << 32) && (long long)packed_bytes(cols, batch) < (1ll << 32);
 }
 
 size_t spmv_tile_workspace(int cols, int batch, const void *x, long long ldx)
 {
     const bool aligned = ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && (ldx & 7) == 0;
     if ((long long)batch * cols < (aligned || batch < 4 ? kPackFrom : kPackUnalignedFrom)) return 0;
-    return (size_t)((batch + 15) / 16) * (size_t)((cols + 63) / 64) * 2048;
+    return packed_bytes(cols, batch);
 }
 
 int spmv_tile_launch(const SpmvArgs &args, int batch, void *workspace, size_t workspace_bytes, hipStream_t stream)
@@ -644,11 +635,78 @@ int spmv_tile_launch(const SpmvArgs &args, int batch, void *workspace, size_t wo
     a.ldx = (u32)args.ldx;
     a.ldy = (u32)args.ldy;
     const size_t wanted = spmv_tile_workspace(args.cols, batch, args.x, args.ldx);
-    if (wanted > 0 && workspace != nullptr && workspace_bytes >= wanted && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0)
+    if (wanted > 0 && workspace != nullptr && workspace_bytes >= wanted && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
+        const int e = spmv_tile_pack(args.x, args.cols, batch, args.ldx, workspace, stream);
+        if (e != 0) return e;
         a.packed = (const u32x4 *)workspace;
+    }
     TileShape shape;
     if (!choose_tile_shape(&shape, a.rows, a.cols, args.padded, batch, a.packed != nullptr, info)) return MACKO_E_INVALID_ARGUMENT;
     return launch_tile_shape(a, shape, info.max_lds_bytes, stream);
 }
 
+int spmv_tile_pack(const uint16_t *x, int cols, int batch, long long ldx, void *packed, hipStream_t stream)
+{
+    const int tiles = packed_tiles(batch), blocks = tiles * packed_steps(cols);
+    hipLaunchKernelGGL(pack_vectors_kernel, dim3((blocks + 3) / 4), dim3(256), 0, stream, x, (u32x4 *)packed, cols, batch, (u32)ldx,
+                       tiles, blocks);
+    return (int)hipGetLastError();
+}
+
 }  // namespace macko
+
+// Products of vectors that are in operand order already: several matrices share one packing, and
+// what produces the vectors writes them that way (macko_prefill.hip).  No upstream counterpart.
+extern "C" int macko_packed_bytes(int32_t cols, int32_t batch, int64_t *bytes)
+{
+    using namespace macko;
+    if (bytes == nullptr || cols < 64 || batch < 1 || packed_bytes(cols, batch) >= (1ull << 32)) return MACKO_E_INVALID_ARGUMENT;
+    *bytes = (int64_t)packed_bytes(cols, batch);
+    return 0;
+}
+
+extern "C" int macko_pack_f16(const void *x, int32_t cols, int32_t batch, int64_t ldx, void *packed, void *stream)
+{
+    using namespace macko;
+    if (x == nullptr || packed == nullptr || cols < 64 || batch < 1 || ldx < cols || (reinterpret_cast<uintptr_t>(x) & 1) ||
+        (reinterpret_cast<uintptr_t>(packed) & 15) || packed_bytes(cols, batch) >= (1ull << 32) ||
+        (long long)batch * ldx * 2 >= (1ll << 32))
+        return MACKO_E_INVALID_ARGUMENT;
+    return spmv_tile_pack((const uint16_t *)x, cols, batch, ldx, packed, as_stream(stream));
+}
+
+extern "C" int macko_spmv_f16_packed(const void *values, const void *deltas, const int32_t *row_ptr, const void *packed,
+                                     const void *residual, void *y, int32_t rows, int32_t cols, int64_t padded_entries,
+                                     int32_t batch, int64_t ldy, void *stream)
+{
+    using namespace macko;
+    if (rows < 0 || cols < 64 || batch < 1 || padded_entries < 0 || padded_entries % kChunk != 0 ||
+        padded_entries >= (1ll << 31) - 8192 || ldy < rows || ldy >= (1ll << 31))
+        return MACKO_E_INVALID_ARGUMENT;
+    if (rows == 0) return 0;
+    if (row_ptr == nullptr || y == nullptr || packed == nullptr || (padded_entries > 0 && (values == nullptr || deltas == nullptr)) ||
+        packed_bytes(cols, batch) >= (1ull << 32))
+        return MACKO_E_INVALID_ARGUMENT;
+    if ((reinterpret_cast<uintptr_t>(values) & 15) || (reinterpret_cast<uintptr_t>(deltas) & 3) ||
+        (reinterpret_cast<uintptr_t>(row_ptr) & 3) || (reinterpret_cast<uintptr_t>(packed) & 15) ||
+        (reinterpret_cast<uintptr_t>(residual) & 1) || (reinterpret_cast<uintptr_t>(y) & 1))
+        return MACKO_E_INVALID_ARGUMENT;
+    DeviceInfo info;
+    const int rc = device_info(&info);
+    if (rc != 0) return rc;
+    TileArgs a{};
+    a.values = (const u32 *)values;
+    a.deltas = (const u32 *)deltas;
+    a.row_ptr = row_ptr;
+    a.y = (uint16_t *)y;
+    a.rows = rows;
+    a.cols = cols;
+    a.batch = batch;
+    a.padded = (u32)padded_entries;
+    a.ldy = (u32)ldy;
+    a.packed = (const u32x4 *)packed;
+    a.residual = (const uint16_t *)residual;
+    TileShape shape;
+    if (!choose_tile_shape(&shape, rows, cols, padded_entries, batch, true, info)) return MACKO_E_INVALID_ARGUMENT;
+    return launch_tile_shape(a, shape, info.max_lds_bytes, as_stream(stream));
+}

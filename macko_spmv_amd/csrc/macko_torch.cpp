@@ -15,6 +15,7 @@
 #include <torch/library.h>
 
 #include <chrono>
+#include <optional>
 #include <tuple>
 
 #include "macko_decode.h"
@@ -524,6 +525,130 @@ void multiply_attention_axpby_hip(const at::Tensor &M_values, const at::Tensor &
              "multiply_attention_axpby");
 }
 
+// ---- a prompt's tokens together (include/macko_decode.h) ----------------------------------------
+
+void *current_stream() { return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
+
+// Vectors [batch, cols] in operand order: a flat half tensor.
+at::Tensor packed_like(const at::Tensor &t, int64_t cols, int64_t batch)
+{
+    int64_t bytes = 0;
+    TORCH_CHECK(cols < (1ll << 31) && batch < (1ll << 31), "too many vectors");
+    check_rc(macko_packed_bytes((int32_t)cols, (int32_t)batch, &bytes), "pack");
+    return at::empty({bytes / 2}, t.options());
+}
+
+at::Tensor pack_rmsnorm_hip(const at::Tensor &x, const at::Tensor &weight, double eps)
+{
+    check_half_gpu(x, "x");
+    check_half_gpu(weight, "weight");
+    TORCH_CHECK(x.dim() == 2 && weight.numel() == x.size(1), "x must be [batch, cols], weight [cols]");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    at::Tensor packed = packed_like(x, x.size(1), x.size(0));
+    check_rc(macko_prefill_pack_rmsnorm_f16(x.data_ptr(), weight.data_ptr(), packed.data_ptr(), (int32_t)x.size(1),
+                                            (int32_t)x.size(0), (float)eps, current_stream()),
+             "pack_rmsnorm");
+    return packed;
+}
+
+// rmsnorm(x) * weight over the last dimension.
+at::Tensor rmsnorm_rows_hip(const at::Tensor &x, const at::Tensor &weight, double eps)
+{
+    check_half_gpu(x, "x");
+    check_half_gpu(weight, "weight");
+    TORCH_CHECK(x.dim() >= 1 && weight.numel() == x.size(-1), "weight must hold one element per column of x");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    at::Tensor y = at::empty_like(x);
+    if (x.numel() == 0) return y;
+    TORCH_CHECK(x.numel() / x.size(-1) < (1ll << 31), "too many rows");
+    check_rc(macko_rmsnorm_rows_f16(x.data_ptr(), weight.data_ptr(), y.data_ptr(), (int32_t)x.size(-1),
+                                    (int32_t)(x.numel() / x.size(-1)), (float)eps, current_stream()),
+             "rmsnorm_rows");
+    return y;
+}
+
+at::Tensor pack_silu_mul_hip(const at::Tensor &gate, const at::Tensor &up)
+{
+    check_half_gpu(gate, "gate");
+    check_half_gpu(up, "up");
+    TORCH_CHECK(gate.dim() == 2 && gate.sizes() == up.sizes(), "gate and up must be [batch, cols]");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(gate.device());
+    at::Tensor packed = packed_like(gate, gate.size(1), gate.size(0));
+    check_rc(macko_prefill_pack_silu_mul_f16(gate.data_ptr(), up.data_ptr(), packed.data_ptr(), (int32_t)gate.size(1),
+                                             (int32_t)gate.size(0), current_stream()),
+             "pack_silu_mul");
+    return packed;
+}
+
+// Y[b] = M @ X[b] (+ residual[b]) for `batch` vectors in operand order -> [batch, M_rows].
+at::Tensor multiply_packed_hip(const at::Tensor &M_values, const at::Tensor &M_deltas, const at::Tensor &M_row_indices,
+                               int64_t M_rows, int64_t M_cols, const at::Tensor &packed, int64_t batch,
+                               const std::optional<at::Tensor> &residual)
+{
+    check_macko_operands(M_values, M_deltas, M_row_indices, M_rows, M_cols);
+    check_half_gpu(packed, "packed");
+    int64_t bytes = 0;
+    TORCH_CHECK(batch >= 1 && batch < (1ll << 31), "bad batch");
+    check_rc(macko_packed_bytes((int32_t)M_cols, (int32_t)batch, &bytes), "multiply_packed");
+    TORCH_CHECK(packed.numel() * 2 == bytes, "packed must hold `batch` vectors of M_cols elements");
+    if (residual.has_value()) {
+        check_half_gpu(*residual, "residual");
+        TORCH_CHECK(residual->dim() == 2 && residual->size(0) == batch && residual->size(1) == M_rows, "residual must be [batch, M_rows]");
+    }
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(M_values.device());
+    at::Tensor Y = at::empty({batch, M_rows}, M_values.options());
+    check_rc(macko_spmv_f16_packed(M_values.data_ptr(), M_deltas.data_ptr(), M_row_indices.data_ptr<int>(), packed.data_ptr(),
+                                   residual.has_value() ? residual->data_ptr() : nullptr, Y.data_ptr(), (int32_t)M_rows,
+                                   (int32_t)M_cols, M_values.numel(), (int32_t)batch, M_rows, current_stream()),
+             "multiply_packed");
+    return Y;
+}
+
+void check_caches(const at::Tensor &k_cache, const at::Tensor &v_cache, const at::Tensor &positions, int64_t batch, int64_t width)
+{
+    check_half_gpu(k_cache, "k_cache");
+    check_half_gpu(v_cache, "v_cache");
+    TORCH_CHECK(k_cache.dim() == 3 && v_cache.sizes() == k_cache.sizes() && width == k_cache.size(0) * k_cache.size(2),
+                "caches must be [heads, max_len, head_dim]");
+    TORCH_CHECK(positions.is_cuda() && positions.dtype() == at::kLong && positions.is_contiguous() && positions.numel() == batch,
+                "bad positions");
+}
+
+void prefill_rope_append_hip(at::Tensor q, const at::Tensor &k, const at::Tensor &v, const at::Tensor &cos_rows,
+                             const at::Tensor &sin_rows, const at::Tensor &positions, at::Tensor k_cache, at::Tensor v_cache)
+{
+    check_half_gpu(q, "q");
+    check_half_gpu(k, "k");
+    check_half_gpu(v, "v");
+    check_half_gpu(cos_rows, "cos_rows");
+    check_half_gpu(sin_rows, "sin_rows");
+    TORCH_CHECK(q.dim() == 2 && q.sizes() == k.sizes() && q.sizes() == v.sizes(), "q, k, v must be [batch, heads * head_dim]");
+    check_caches(k_cache, v_cache, positions, q.size(0), q.size(1));
+    TORCH_CHECK(cos_rows.numel() == q.size(0) * k_cache.size(2) && sin_rows.numel() == cos_rows.numel(),
+                "cos / sin must be [batch, head_dim]");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+    check_rc(macko_prefill_rope_append_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos_rows.data_ptr(), sin_rows.data_ptr(),
+                                           positions.data_ptr<int64_t>(), k_cache.data_ptr(), v_cache.data_ptr(),
+                                           (int32_t)q.size(0), (int32_t)k_cache.size(0), (int32_t)k_cache.size(2),
+                                           (int32_t)k_cache.size(1), current_stream()),
+             "prefill_rope_append");
+}
+
+at::Tensor prefill_attention_hip(const at::Tensor &q, const at::Tensor &k_cache, const at::Tensor &v_cache,
+                                 const at::Tensor &positions, double scale)
+{
+    check_half_gpu(q, "q");
+    TORCH_CHECK(q.dim() == 2, "q must be [batch, heads * head_dim]");
+    check_caches(k_cache, v_cache, positions, q.size(0), q.size(1));
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+    at::Tensor packed = packed_like(q, q.size(1), q.size(0));
+    check_rc(macko_prefill_attention_f16(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr<int64_t>(),
+                                         packed.data_ptr(), (int32_t)q.size(0), (int32_t)k_cache.size(0), (int32_t)k_cache.size(2),
+                                         (int32_t)k_cache.size(1), (float)scale, current_stream()),
+             "prefill_attention");
+    return packed;
+}
+
 }  // namespace
 
 TORCH_LIBRARY(macko_spmv, m)
@@ -560,6 +685,14 @@ TORCH_LIBRARY(macko_spmv, m)
           "Tensor position, Tensor(a!) k_cache, Tensor(b!) v_cache, float scale) -> Tensor");
     m.def("multiply_attention_axpby(Tensor M_values, Tensor M_deltas, Tensor M_row_indices, int M_rows, int M_cols, "
           "Tensor parts, int head_dim, Tensor(a!) C, float alpha, float beta) -> ()");
+    m.def("pack_rmsnorm(Tensor x, Tensor weight, float eps) -> Tensor");
+    m.def("rmsnorm_rows(Tensor x, Tensor weight, float eps) -> Tensor");
+    m.def("pack_silu_mul(Tensor gate, Tensor up) -> Tensor");
+    m.def("multiply_packed(Tensor M_values, Tensor M_deltas, Tensor M_row_indices, int M_rows, int M_cols, "
+          "Tensor packed, int batch, Tensor? residual) -> Tensor");
+    m.def("prefill_rope_append(Tensor(a!) q, Tensor k, Tensor v, Tensor cos_rows, Tensor sin_rows, Tensor positions, "
+          "Tensor(b!) k_cache, Tensor(c!) v_cache) -> ()");
+    m.def("prefill_attention(Tensor q, Tensor k_cache, Tensor v_cache, Tensor positions, float scale) -> Tensor");
     m.def("decompress(Tensor M_values, Tensor M_deltas, Tensor M_row_indices, int M_rows, int M_cols) -> Tensor");
 }
 
@@ -584,6 +717,12 @@ TORCH_LIBRARY_IMPL(macko_spmv, CUDA, m)
     m.impl("decode_rope_attention", &decode_rope_attention_hip);
     m.impl("decode_rope_attention_parts", &decode_rope_attention_parts_hip);
     m.impl("multiply_attention_axpby", &multiply_attention_axpby_hip);
+    m.impl("pack_rmsnorm", &pack_rmsnorm_hip);
+    m.impl("rmsnorm_rows", &rmsnorm_rows_hip);
+    m.impl("pack_silu_mul", &pack_silu_mul_hip);
+    m.impl("multiply_packed", &multiply_packed_hip);
+    m.impl("prefill_rope_append", &prefill_rope_append_hip);
+    m.impl("prefill_attention", &prefill_attention_hip);
     m.impl("decompress", &decompress_hip);
 }
 

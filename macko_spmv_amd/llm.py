@@ -119,6 +119,13 @@ def load_compressed_linears(model, compressed_sd):
 
 # ---- a minimal Llama-architecture decoder (batch 1) ------------------------------------------------
 
+def _inference_half(*tensors):
+    """fp16 tensors on the GPU through which no gradient has to flow: what the hand-written kernels between
+    the projections take."""
+    grad = torch.is_grad_enabled()
+    return all(t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad) for t in tensors)
+
+
 class RMSNorm(nn.Module):
     def __init__(self, dim, eps=1e-5):
         super().__init__()
@@ -126,6 +133,8 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x):
+        if _inference_half(x, self.weight) and x.is_contiguous() and x.shape[-1] % 8 == 0 and x.numel() > 0:
+            return torch.ops.macko_spmv.rmsnorm_rows(x, self.weight, self.eps)
         v = x.float()
         v = v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + self.eps)
         return (v * self.weight.float()).to(x.dtype)
@@ -156,6 +165,11 @@ class Attention(nn.Module):
         return self.o_proj(out)
 
 
+def _causal_mask(max_len, positions, dtype):
+    key_pos = torch.arange(max_len, device=positions.device)
+    return torch.where(key_pos[None, :] <= positions[:, None], 0.0, float("-inf")).to(dtype)[None, None]
+
+
 def _rope(x, cos, sin):
     x1, x2 = x[..., : x.shape[-1] // 2], x[..., x.shape[-1] // 2:]
     return x * cos + torch.cat((-x2, x1), dim=-1) * sin
@@ -180,7 +194,46 @@ class Block(nn.Module):
         self.input_layernorm = RMSNorm(dim)
         self.post_attention_layernorm = RMSNorm(dim)
 
+    def takes_fused(self, x):
+        """Whether several tokens go through the layer by way of forward_fused: inference in fp16 on the
+        GPU, all seven projections compressed, nothing hooked to the modules that would be passed over."""
+        att, mlp = self.self_attn, self.mlp
+        projections = (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
+        norms = (self.input_layernorm, self.post_attention_layernorm)
+        return (x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
+                and all(type(p) is MackoLinear for p in projections)
+                and att.n_heads * att.head_dim == x.shape[2] and projections[4].c_3 % 8 == 0 and projections[4].c_3 >= 64
+                and all(type(n) is RMSNorm for n in norms)
+                and not any(m._forward_hooks or m._forward_pre_hooks for m in (att, mlp, *projections, *norms))
+                and att.k_cache.is_contiguous() and att.v_cache.is_contiguous()
+                and _inference_half(x, *(n.weight for n in norms), att.k_cache, att.v_cache))
+
+    def forward_fused(self, x, cos, sin, positions):
+        """The layer for several tokens with one kernel for each part between the projections; what a
+        projection consumes is written in its operand order, and the residuals are added where the
+        o and down projections round their results."""
+        ops, att, mlp = torch.ops.macko_spmv, self.self_attn, self.mlp
+        t = x.shape[1]
+        rows = x.reshape(t, -1).contiguous()
+
+        def product(linear, packed, residual=None):
+            return ops.multiply_packed(linear.c_0, linear.c_1, linear.c_2, linear.c_3, linear.c_4, packed, t, residual)
+
+        normed = ops.pack_rmsnorm(rows, self.input_layernorm.weight, self.input_layernorm.eps)
+        q, k, v = product(att.q_proj, normed), product(att.k_proj, normed), product(att.v_proj, normed)
+        k_cache, v_cache = att.k_cache[0], att.v_cache[0]
+        ops.prefill_rope_append(q, k, v, cos.reshape(t, -1), sin.reshape(t, -1), positions, k_cache, v_cache)
+        attended = ops.prefill_attention(q, k_cache, v_cache, positions, 1.0 / math.sqrt(att.head_dim))
+        rows = product(att.o_proj, attended, rows)
+        normed = ops.pack_rmsnorm(rows, self.post_attention_layernorm.weight, self.post_attention_layernorm.eps)
+        gated = ops.pack_silu_mul(product(mlp.gate_proj, normed), product(mlp.up_proj, normed))
+        return product(mlp.down_proj, gated, rows).view(1, t, -1)
+
     def forward(self, x, cos, sin, positions, mask):
+        if self.takes_fused(x):
+            return self.forward_fused(x, cos, sin, positions)
+        if mask is None:  # no layer was expected to need it
+            mask = _causal_mask(self.self_attn.max_len, positions, x.dtype)
         x = x + self.self_attn(self.input_layernorm(x), cos, sin, positions, mask)
         return x + self.mlp(self.post_attention_layernorm(x))
 
@@ -213,8 +266,9 @@ class LlamaDecoder(nn.Module):
         x = self.model.embed_tokens(tokens)
         cos = self.cos[positions].to(x.dtype)[None, None]
         sin = self.sin[positions].to(x.dtype)[None, None]
-        key_pos = torch.arange(self.max_len, device=tokens.device)
-        mask = torch.where(key_pos[None, :] <= positions[:, None], 0.0, float("-inf")).to(x.dtype)[None, None]
+        # a layer that works all its tokens in hand-written kernels needs no mask
+        mask = None if all(layer.takes_fused(x) for layer in self.model.layers) else \
+            _causal_mask(self.max_len, positions, x.dtype)
         for layer in self.model.layers:
             x = layer(x, cos, sin, positions, mask)
         return self.lm_head(self.model.norm(x))

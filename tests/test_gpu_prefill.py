@@ -1,0 +1,147 @@
+"""The kernels that work all tokens of a prompt between the projections, against plain torch in float64 at the
+edges of their tiles (16 tokens, 32 cache positions, 64 columns), and the layer built from them against the
+module path."""
+import numpy as np
+import pytest
+import torch
+
+import macko_spmv_amd as mk
+from macko_spmv_amd import llm
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+ops = torch.ops.macko_spmv
+
+
+def _unpack(packed, cols, batch):
+    """Operand order back to [batch, cols], and what lies beyond them."""
+    steps, tiles = (cols + 63) // 64, (batch + 15) // 16
+    # [step, tile, s, q, n, 8] -> [tile, n, step, q, s, 8]
+    full = packed.view(steps, tiles, 2, 4, 16, 8).permute(1, 4, 0, 3, 2, 5).reshape(tiles * 16, steps * 64)
+    rest = full.clone()
+    rest[:batch, :cols] = 0
+    return full[:batch, :cols], rest
+
+
+@pytest.mark.parametrize("batch,cols", [(1, 64), (2, 72), (15, 4096), (16, 512), (17, 1376), (33, 16392), (128, 4096)])
+def test_norm_and_gate_in_operand_order(batch, cols):
+    g = torch.Generator(device="cuda").manual_seed(cols + batch)
+    x, up = (torch.randn(batch, cols, device="cuda", generator=g).half() for _ in range(2))
+    w = (1 + 0.1 * torch.randn(cols, device="cuda", generator=g)).half()
+    xd = x.double()
+    want = xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    got, rest = _unpack(ops.pack_rmsnorm(x, w, 1e-5), cols, batch)
+    # one rounding to fp16 of a value with a few fp32 roundings in it
+    assert torch.allclose(got.double(), want, rtol=2.0 ** -10, atol=2.0 ** -24) and not rest.any()
+    assert torch.equal(ops.rmsnorm_rows(x, w, 1e-5), got)
+    want = xd / (1 + torch.exp(-xd)) * up.double()
+    got, rest = _unpack(ops.pack_silu_mul(x, up), cols, batch)
+    assert torch.allclose(got.double(), want, rtol=2.0 ** -10, atol=2.0 ** -24) and not rest.any()
+
+
+@pytest.mark.parametrize("batch,n_heads,head_dim,max_len,start", [(1, 1, 64, 1, 0), (2, 3, 128, 40, 0), (16, 2, 64, 16, 0), (17, 4, 128, 33, 0),
+                                                                  (31, 2, 64, 200, 7), (128, 32, 128, 512, 0), (100, 2, 128, 900, 640)])
+def test_rope_append_and_attention(batch, n_heads, head_dim, max_len, start):
+    g = torch.Generator(device="cuda").manual_seed(batch + max_len)
+    width = n_heads * head_dim
+    q, k, v = (torch.randn(batch, width, device="cuda", generator=g).half() for _ in range(3))
+    inv = 1.0 / (10000.0 ** (torch.arange(0, head_dim, 2, device="cuda").float() / head_dim))
+    ang = torch.outer(torch.arange(max_len, device="cuda").float(), inv)
+    ang = torch.cat((ang, ang), dim=-1)
+    positions = start + torch.arange(batch, device="cuda")
+    if batch == 31:
+        positions = positions.flip(0).contiguous()   # any order
+    cos, sin = ang.cos().half()[positions], ang.sin().half()[positions]
+    kc, vc = (torch.randn(n_heads, max_len, head_dim, device="cuda", generator=g).half() for _ in range(2))
+    top = int(positions.max())
+    kc[:, top + 1:] = float("nan")   # what lies behind the context is not used
+    vc[:, top + 1:] = float("nan")
+    kc0, vc0 = kc.clone(), vc.clone()
+
+    def rope(t):
+        t = t.double().view(batch, n_heads, head_dim)
+        rot = torch.cat((-t[..., head_dim // 2:], t[..., :head_dim // 2]), dim=-1)
+        return t * cos.double()[:, None] + rot * sin.double()[:, None]
+
+    q_in = q.clone()
+    ops.prefill_rope_append(q, k, v, cos, sin, positions, kc, vc)
+    assert torch.allclose(q.double().view(batch, n_heads, head_dim), rope(q_in), rtol=2.0 ** -10, atol=2.0 ** -20)
+    assert torch.allclose(kc[:, positions].double().transpose(0, 1), rope(k), rtol=2.0 ** -10, atol=2.0 ** -20)
+    assert torch.equal(vc[:, positions].transpose(0, 1).reshape(batch, width), v)
+    keep = torch.ones(max_len, dtype=torch.bool, device="cuda")
+    keep[positions] = False
+    assert torch.equal(kc[:, keep].view(torch.int16), kc0[:, keep].view(torch.int16))
+    assert torch.equal(vc[:, keep].view(torch.int16), vc0[:, keep].view(torch.int16))
+
+    scale = head_dim ** -0.5
+    got, rest = _unpack(ops.prefill_attention(q, kc, vc, positions, scale), width, batch)
+    assert not rest.any()
+    qd, kd, vd = q.float().view(batch, n_heads, head_dim), kc.float()[:, :top + 1], vc.float()[:, :top + 1]
+    for h in range(n_heads):
+        s = (qd[:, h] @ kd[h].t()) * scale
+        s = s.masked_fill(torch.arange(top + 1, device="cuda")[None, :] > positions[:, None], float("-inf"))
+        p = torch.softmax(s, dim=-1)
+        want = p @ vd[h]
+        # weights rounded to fp16 (2^-11 each) and one rounding of the result
+        bound = 2.0 ** -10 * want.abs() + 2.0 ** -10 * (p @ vd[h].abs()) + 2.0 ** -20
+        assert ((got[:, h * head_dim:(h + 1) * head_dim].float() - want).abs() <= bound).all(), h
+
+
+@pytest.mark.parametrize("batch,rows,cols", [(1, 7, 64), (5, 100, 200), (40, 333, 1000), (130, 4100, 512)])
+def test_product_of_packed_vectors_with_residual(batch, rows, cols):
+    rng = np.random.default_rng(rows)
+    dense = helpers.random_sparse(rng, rows, cols, 0.4)
+    c = mk.compress(torch.from_numpy(dense).cuda())
+    x = rng.standard_normal((batch, cols)).astype(np.float16)
+    up = np.full((batch, cols), 30.0, dtype=np.float16)
+    gate = torch.from_numpy(x).cuda()
+    packed = ops.pack_silu_mul(gate, torch.from_numpy(up).cuda())
+    staged = _unpack(packed, cols, batch)[0].cpu().numpy().astype(np.float64)
+    r = rng.standard_normal((batch, rows)).astype(np.float16)
+    d64 = dense.astype(np.float64)
+    for residual in (None, torch.from_numpy(r).cuda()):
+        y = ops.multiply_packed(*c, packed, batch, residual).cpu().double().numpy()
+        want = staged @ d64.T + (r.astype(np.float64) if residual is not None else 0.0)
+        bound = 2.0 ** -11 * np.abs(want) + 2.0 ** -25 + (cols + 3) * 2.0 ** -24 * (np.abs(staged) @ np.abs(d64).T + np.abs(want))
+        assert (np.abs(y - want) <= bound).all()
+
+
+def test_operators_have_fake_implementations():
+    M = torch.randn((128, 128), dtype=torch.float16, device="cuda")
+    c = mk.compress(M)
+    x, w = torch.randn(5, 128, device="cuda").half(), torch.ones(128, device="cuda").half()
+    packed = ops.pack_rmsnorm(x, w, 1e-5)
+    torch.library.opcheck(ops.pack_rmsnorm, (x, w, 1e-5))
+    torch.library.opcheck(ops.rmsnorm_rows, (x, w, 1e-5))
+    torch.library.opcheck(ops.pack_silu_mul, (x, x.clone()))
+    torch.library.opcheck(ops.multiply_packed, (*c, packed, 5, x))
+    kc, vc = torch.zeros(2, 30, 64, device="cuda").half(), torch.zeros(2, 30, 64, device="cuda").half()
+    pos, cs = torch.arange(5, device="cuda"), torch.ones(5, 64, device="cuda").half()
+    torch.library.opcheck(ops.prefill_rope_append, (x.clone(), x.clone(), x.clone(), cs, cs, pos, kc, vc))
+    torch.library.opcheck(ops.prefill_attention, (x, kc, vc, pos, 0.125))
+
+
+@pytest.mark.parametrize("dim,hidden,heads,t", [(256, 688, 4, 2), (256, 704, 2, 19), (512, 1376, 8, 64)])
+def test_fused_layers_against_the_module_path(dim, hidden, heads, t):
+    torch.set_grad_enabled(False)
+    cfg = dict(n_layers=2, dim=dim, hidden=hidden, n_heads=heads, vocab=1000, max_len=80)
+    model, _ = llm.build_model(0.4, sparse=True, **cfg)
+    prompt, pos = torch.randint(0, 1000, (1, t), device="cuda"), torch.arange(t, device="cuda")
+    x = model.model.embed_tokens(prompt)
+    assert all(layer.takes_fused(x) for layer in model.model.layers)
+    fused = model(prompt, pos).float()
+    caches = [layer.self_attn.k_cache.clone() for layer in model.model.layers]
+    # a hook on one projection sends its layer (only) through the modules
+    calls = []
+    handle = model.model.layers[1].mlp.up_proj.register_forward_hook(lambda *a: calls.append(1))
+    mixed = model(prompt, pos).float()
+    assert calls and not model.model.layers[1].takes_fused(x) and model.model.layers[0].takes_fused(x)
+    handle.remove()
+    for layer in model.model.layers:
+        layer.mlp.register_forward_pre_hook(lambda *a: None)
+    plain = model(prompt, pos).float()
+    assert not any(layer.takes_fused(x) for layer in model.model.layers)
+    # fp16 activations between the parts, rounded in other places
+    assert torch.allclose(fused, plain, rtol=2e-2, atol=2e-2) and torch.allclose(mixed, plain, rtol=2e-2, atol=2e-2)
+    for kept, layer in zip(caches, model.model.layers):
+        assert torch.allclose(kept.float(), layer.self_attn.k_cache.float(), rtol=2e-2, atol=2e-2)
