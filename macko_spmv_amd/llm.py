@@ -215,6 +215,7 @@ class Block(nn.Module):
         ops, att, mlp = torch.ops.macko_spmv, self.self_attn, self.mlp
         t = x.shape[1]
         rows = x.reshape(t, -1).contiguous()
+        positions = positions.contiguous()
 
         def product(linear, packed, residual=None):
             return ops.multiply_packed(linear.c_0, linear.c_1, linear.c_2, linear.c_3, linear.c_4, packed, t, residual)
@@ -230,9 +231,9 @@ class Block(nn.Module):
         return product(mlp.down_proj, gated, rows).view(1, t, -1)
 
     def forward(self, x, cos, sin, positions, mask):
-        if self.takes_fused(x):
-            return self.forward_fused(x, cos, sin, positions)
-        if mask is None:  # no layer was expected to need it
+        if mask is None:  # causal; any other mask is the general path's
+            if self.takes_fused(x):
+                return self.forward_fused(x, cos, sin, positions)
             mask = _causal_mask(self.self_attn.max_len, positions, x.dtype)
         x = x + self.self_attn(self.input_layernorm(x), cos, sin, positions, mask)
         return x + self.mlp(self.post_attention_layernorm(x))
@@ -267,10 +268,10 @@ class LlamaDecoder(nn.Module):
         cos = self.cos[positions].to(x.dtype)[None, None]
         sin = self.sin[positions].to(x.dtype)[None, None]
         # a layer that works all its tokens in hand-written kernels needs no mask
-        mask = None if all(layer.takes_fused(x) for layer in self.model.layers) else \
-            _causal_mask(self.max_len, positions, x.dtype)
-        for layer in self.model.layers:
-            x = layer(x, cos, sin, positions, mask)
+        fused = [layer.takes_fused(x) for layer in self.model.layers]
+        mask = None if all(fused) else _causal_mask(self.max_len, positions, x.dtype)
+        for layer, without_mask in zip(self.model.layers, fused):
+            x = layer(x, cos, sin, positions, None if without_mask else mask)
         return self.lm_head(self.model.norm(x))
 
 

@@ -145,3 +145,24 @@ def test_fused_layers_against_the_module_path(dim, hidden, heads, t):
     assert torch.allclose(fused, plain, rtol=2e-2, atol=2e-2) and torch.allclose(mixed, plain, rtol=2e-2, atol=2e-2)
     for kept, layer in zip(caches, model.model.layers):
         assert torch.allclose(kept.float(), layer.self_attn.k_cache.float(), rtol=2e-2, atol=2e-2)
+
+
+def test_layer_keeps_a_given_mask_and_strided_positions():
+    torch.set_grad_enabled(False)
+    model, _ = llm.build_model(0.4, sparse=True, n_layers=1, dim=256, hidden=704, n_heads=2, vocab=1000, max_len=48)
+    layer, t = model.model.layers[0], 20
+    pos = torch.arange(t, device="cuda")
+    x = model.model.embed_tokens(torch.randint(0, 1000, (1, t), device="cuda"))
+    cos, sin = (table[pos].half()[None, None] for table in (model.cos, model.sin))
+    assert layer.takes_fused(x)
+    causal = layer(x, cos, sin, pos, None)
+    spread = torch.stack((pos, pos), 1)[:, 0]
+    assert not spread.is_contiguous() and torch.equal(layer(x, cos, sin, spread, None), causal)
+    # a mask that lets a token see only itself is not the causal one
+    own = torch.full((1, 1, t, 48), float("-inf"), device="cuda", dtype=torch.float16)
+    own[0, 0, pos, pos] = 0
+    masked = layer(x, cos, sin, pos, own)
+    handle = layer.mlp.register_forward_pre_hook(lambda *a: None)   # through the modules
+    want = layer(x, cos, sin, pos, own)
+    handle.remove()
+    assert torch.equal(masked, want) and not torch.allclose(masked, causal, rtol=2e-2, atol=2e-2)
