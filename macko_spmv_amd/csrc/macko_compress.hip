@@ -17,7 +17,7 @@
 // writes values and nibbles.  One wave owns one row in both passes; lanes take 8 consecutive
 // columns and learn the previous non-zero's column from a DPP running maximum.
 
-#include "macko_common.h"
+#include "macko_packed.h"
 
 namespace macko {
 namespace {
@@ -27,95 +27,143 @@ constexpr int kBlock = kRowsPerBlock * kWave;
 constexpr int kNoColumn = (int)0x80000000;
 constexpr int kAhead = 4;                     // tiles of its row a wave keeps in flight
 
-// The two element formats.  A chunk is the 8 consecutive elements a lane handles per tile.
+// The two element formats.  A chunk is the 8 consecutive elements a lane handles per tile; a half of it
+// (4 elements, kHalfWords words) is what one look-up in the table of byte selectors packs together.
 struct Fp16Format {
     typedef uint16_t Elem;
     typedef u32x4 Chunk;                          // 8 halves
+    typedef Chunk __attribute__((aligned(2))) AnyChunk;  // where a row starts at any element
     static constexpr bool kKeepTrailing = false;  // padding entries behind the last non-zero are dropped
+    static constexpr int kHalfWords = 2;
+    static __device__ __forceinline__ Chunk shift(const Chunk &v, int by) { return shift_down(v, by); }  // by >= 0 elements
     static __device__ __forceinline__ u32 at(const Chunk &v, int i) { return (v[i >> 1] >> (16 * (i & 1))) & 0xffffu; }
     static __device__ __forceinline__ void put(Chunk &v, int i, u32 bits) { v[i >> 1] |= bits << (16 * (i & 1)); }
     // non-zero as a float: -0.0 is a zero, NaN is not
     static __device__ __forceinline__ bool nonzero(u32 bits) { return (bits & 0x7fffu) != 0; }
+    // bit i set when element i is non-zero
+    static __device__ __forceinline__ u32 nonzero_bits(const Chunk &v)
+    {
+        u32 m = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) m |= min1(v[w] & 0x7fff7fffu) << (2 * w);
+        return (m | (m >> 15)) & 0xffu;
+    }
     // what is stored: the element itself, a NaN as 0x7fff
     static __device__ __forceinline__ u32 stored(u32 bits) { return (bits & 0x7fffu) > 0x7c00u ? 0x7fffu : bits; }
-    // the 8 values of a full group from their stage words (value in the low half of each)
-    static __device__ __forceinline__ Chunk pack(const u32 (&e)[8])
-    {
-        Chunk v;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = __builtin_amdgcn_perm(e[2 * k + 1], e[2 * k], 0x05040100u);
-        return v;
-    }
-    // a half is a NaN when its low 15 bits exceed 0x7c00: adding 0x03ff then carries into bit 15
+    // a half is a NaN when its low 15 bits exceed 0x7c00
     static __device__ __forceinline__ bool any_nan(const Chunk &v)
     {
-        u32 hit = 0;
+        const Halves a = __builtin_elementwise_max(magnitude(v[0]), magnitude(v[1]));
+        const Halves b = __builtin_elementwise_max(magnitude(v[2]), magnitude(v[3]));
+        const Halves top = __builtin_elementwise_max(__builtin_elementwise_max(a, b), Halves{0x7c00, 0x7c00});
+        return __builtin_bit_cast(u32, top) != 0x7c007c00u;
+    }
+    // byte selectors that bring the elements of a half whose bits are set in m to its front, word `w` of it
+    static __device__ __forceinline__ u32 selectors(u32 m, int w)
+    {
+        u32 sel = 0;
+        int n = -2 * w;
+        for (u32 i = 0; i < 4; ++i)
+            if ((m >> i) & 1u) {
+                if (n == 0 || n == 1) sel |= ((2 * i) | (2 * i + 1) << 8) << (16 * n);
+                ++n;
+            }
+        return sel;
+    }
+    static __device__ __forceinline__ void pack(const Chunk &v, int half, const u32 *sel, u32 (&out)[4])
+    {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) hit |= ((v[w] & 0x7fff7fffu) + 0x03ff03ffu) & 0x80008000u;
-        return hit != 0;
+        for (int w = 0; w < 2; ++w) {
+            const u32 both = __builtin_amdgcn_perm(v[2 * half + 1], v[2 * half], sel[w]);
+            out[2 * w] = both;
+            out[2 * w + 1] = both >> 16;
+        }
+    }
+
+private:
+    typedef unsigned short Halves __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ Halves magnitude(u32 w) { return __builtin_bit_cast(Halves, w & 0x7fff7fffu); }
+    static __device__ __forceinline__ u32 min1(u32 w)
+    {
+        return __builtin_bit_cast(u32, __builtin_elementwise_min(__builtin_bit_cast(Halves, w), Halves{1, 1}));
     }
 };
 struct Int8Format {
     typedef unsigned char Elem;
     typedef u32x2 Chunk;                         // 8 bytes
+    typedef Chunk __attribute__((aligned(1))) AnyChunk;
     static constexpr bool kKeepTrailing = true;  // cpu_compressor.cuh:75-117 has no withdrawal step
+    static constexpr int kHalfWords = 1;
+    static __device__ __forceinline__ Chunk shift(const Chunk &v, int by)
+    {
+        return by < 8 ? __builtin_bit_cast(Chunk, __builtin_bit_cast(unsigned long long, v) >> (8 * by)) : Chunk{};
+    }
     static __device__ __forceinline__ u32 at(const Chunk &v, int i) { return (v[i >> 2] >> (8 * (i & 3))) & 0xffu; }
     static __device__ __forceinline__ void put(Chunk &v, int i, u32 bits) { v[i >> 2] |= bits << (8 * (i & 3)); }
     static __device__ __forceinline__ bool nonzero(u32 bits) { return bits != 0; }
+    static __device__ __forceinline__ u32 nonzero_bits(const Chunk &v)
+    {
+        // bit 7 of a byte: whether it is non-zero
+        auto high = [](u32 w) { return (w | ((w & 0x7f7f7f7fu) + 0x7f7f7f7fu)) & 0x80808080u; };
+        const u32 m = (high(v[0]) >> 7) | (high(v[1]) >> 3);  // bits 0, 8, 16, 24 and 4, 12, 20, 28
+        return (m | (m >> 7) | (m >> 14) | (m >> 21)) & 0xffu;
+    }
     static __device__ __forceinline__ u32 stored(u32 bits) { return bits; }
     static __device__ __forceinline__ bool any_nan(const Chunk &) { return false; }
-    static __device__ __forceinline__ Chunk pack(const u32 (&e)[8])
+    static __device__ __forceinline__ u32 selectors(u32 m, int)
     {
-        Chunk v;
+        u32 sel = 0;
+        int n = 0;
+        for (u32 i = 0; i < 4; ++i)
+            if ((m >> i) & 1u) sel |= i << (8 * n++);
+        return sel;
+    }
+    static __device__ __forceinline__ void pack(const Chunk &v, int half, const u32 *sel, u32 (&out)[4])
+    {
+        const u32 all = __builtin_amdgcn_perm(0u, v[half], sel[0]);
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const u32 lo = __builtin_amdgcn_perm(e[4 * k + 1], e[4 * k], 0x0c0c0400u);
-            const u32 hi = __builtin_amdgcn_perm(e[4 * k + 3], e[4 * k + 2], 0x0c0c0400u);
-            v[k] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-        }
-        return v;
+        for (int i = 0; i < 4; ++i) out[i] = all >> (8 * i);
     }
 };
 
-// 8 consecutive elements of a row, zero beyond `cols`.  STREAM: the dense matrix will not be read
-// again soon (non-temporal hint).
+// 8 consecutive elements of a row, whatever its alignment (a 16-byte load that starts at any element costs
+// at most one cache line more per wave; element by element, as this was where rows are not 16-byte aligned,
+// it took eight loads).  The row's last elements come from a load that ends with the row and are moved to
+// their place when they are used (cut8), so that no lane has a path of its own.  STREAM: the dense matrix
+// will not be read again soon (non-temporal hint).
 template <typename F, bool STREAM>
-__device__ __forceinline__ typename F::Chunk load8(const typename F::Elem *__restrict__ row, int col, int cols,
-                                                   bool vector_ok)
+__device__ __forceinline__ typename F::Chunk load8(const typename F::Elem *__restrict__ row, int col, int cols)
 {
     typename F::Chunk v = {};
-    if (col + 8 <= cols && vector_ok) {
-        const typename F::Chunk *p = reinterpret_cast<const typename F::Chunk *>(row + col);
+    if (cols >= 8) {
+        const typename F::AnyChunk *p = reinterpret_cast<const typename F::AnyChunk *>(row + (col < cols - 8 ? col : cols - 8));
         v = STREAM ? __builtin_nontemporal_load(p) : *p;
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const u32 h = (col + i < cols) ? (u32)row[col + i] : 0u;
-            F::put(v, i, h);
-        }
+        for (int i = 0; i < 8; ++i) F::put(v, i, col + i < cols ? (u32)row[col + i] : 0u);
     }
     return v;
 }
 
-// bit i set when element i is non-zero
+// what load8 gave for columns [col, col + 8) of the tile that starts at `first`: zero beyond `cols`
 template <typename F>
-__device__ __forceinline__ u32 nonzero_bits(const typename F::Chunk &v)
+__device__ __forceinline__ typename F::Chunk cut8(typename F::Chunk v, int first, int col, int cols)
 {
-    u32 m = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) m |= (F::nonzero(F::at(v, i)) ? 1u : 0u) << i;
-    return m;
+    if (first + kTile > cols && cols >= 8) {  // wave-uniform
+        const int by = col - (cols - 8);
+        v = F::shift(v, by > 0 ? by : 0);
+    }
+    return v;
 }
 
 // Column of the last non-zero strictly before this lane's chunk, given the lane's own last
 // non-zero column (kNoColumn if none) and the carry from earlier passes.  Also returns the
 // last non-zero column of the whole pass through `pass_last`.
-__device__ __forceinline__ int previous_nonzero(int own_last, int carry, int lane, int &pass_last)
+__device__ __forceinline__ int previous_nonzero(int own_last, int carry, int &pass_last)
 {
     const int incl = wave_scan_max_inclusive(own_last);
     pass_last = __builtin_amdgcn_readlane(incl, kWave - 1);
-    int before = __shfl_up(incl, 1);
-    before = lane == 0 ? kNoColumn : before;
+    const int before = __builtin_amdgcn_update_dpp(kNoColumn, incl, 0x138, 0xF, 0xF, false);  // wave_shr:1
     return before > carry ? before : carry;
 }
 
@@ -134,7 +182,6 @@ __global__ void __launch_bounds__(kBlock) count_rows_kernel(const typename F::El
     const int row = blockIdx.x * kRowsPerBlock + uniform(threadIdx.x >> 6);
     if (row >= rows) return;
     const Elem *src = dense + (size_t)row * (size_t)cols;
-    const bool vector_ok = (reinterpret_cast<uintptr_t>(src) & (sizeof(Chunk) - 1)) == 0;
     int carry = -1;  // column of the last non-zero seen in earlier passes
     int mine = 0;
     // kAhead tiles of the row are in flight at any time: a wave walks its row alone, so what hides
@@ -143,20 +190,20 @@ __global__ void __launch_bounds__(kBlock) count_rows_kernel(const typename F::El
 #pragma unroll
     for (int k = 0; k < kAhead; ++k) {
         const int col = k * kTile + lane * kChunk;
-        ahead[k] = load8<F, STREAM>(src, col, cols, vector_ok && col < cols);
+        ahead[k] = load8<F, STREAM>(src, col, cols);
     }
     for (int c0 = 0; c0 < cols; c0 += kAhead * kTile) {
 #pragma unroll
         for (int k = 0; k < kAhead; ++k) {
             const int col = c0 + k * kTile + lane * kChunk;
             if (c0 + k * kTile >= cols) break;  // wave-uniform
-            const Chunk v = ahead[k];
+            const Chunk v = cut8<F>(ahead[k], c0 + k * kTile, col, cols);
             const int ncol = col + kAhead * kTile;
-            if (c0 + (k + kAhead) * kTile < cols) ahead[k] = load8<F, STREAM>(src, ncol, cols, vector_ok && ncol < cols);
-            const u32 nz = nonzero_bits<F>(v);
+            if (c0 + (k + kAhead) * kTile < cols) ahead[k] = load8<F, STREAM>(src, ncol, cols);
+            const u32 nz = F::nonzero_bits(v);
             const int own_last = nz ? col + 31 - __builtin_clz(nz) : kNoColumn;
             int pass_last;
-            const int p = previous_nonzero(own_last, carry, lane, pass_last);
+            const int p = previous_nonzero(own_last, carry, pass_last);
             // every non-zero is an entry; padding entries can only stand in front of the first
             // non-zero of my 8 columns (the others follow their predecessor within 8 columns)
             if (nz) mine += __builtin_popcount(nz) + ((col + __builtin_ctz(nz) - p - 1) >> 4);
@@ -229,21 +276,6 @@ __global__ void __launch_bounds__(1024) scan_rows_kernel(int *__restrict__ row_p
     }
 }
 
-// Packs the nibbles of 8 staged entries (bits 16..19 of each word, bits 20..23 zero) into one delta
-// word: byte 2 of four words at a time into one register, neighbouring bytes folded into one byte.
-__device__ __forceinline__ u32 pack_nibbles(const u32 (&e)[8])
-{
-    u32 folded[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const u32 a = __builtin_amdgcn_perm(e[4 * h + 1], e[4 * h], 0x0c0c0602u);      // n0 | n1 << 8
-        const u32 b = __builtin_amdgcn_perm(e[4 * h + 3], e[4 * h + 2], 0x0c0c0602u);  // n2 | n3 << 8
-        const u32 four = __builtin_amdgcn_perm(b, a, 0x05040100u);                     // n0, n1, n2, n3 in bytes
-        folded[h] = four | (four >> 4);  // byte 0 = n0 | n1 << 4, byte 2 = n2 | n3 << 4
-    }
-    return __builtin_amdgcn_perm(folded[1], folded[0], 0x06040200u);
-}
-
 // Orders this wave's LDS writes before its later LDS reads by other lanes.  The staging area is
 // private to the wave and a wave's LDS operations are carried out in the order issued, so this is
 // a matter of instruction order only: fences of wavefront scope, which wait for nothing (a wider
@@ -257,7 +289,21 @@ __device__ __forceinline__ void wave_lds_fence()
 
 // Pass 2.  The wave stages the entries of its row in LDS at the offset they have inside their
 // 8-entry group of the output, so that every complete group leaves as one 16-byte store of
-// values and one 4-byte store of nibbles.  Groups cut by a row boundary are shared with the
+// values and one 4-byte store of nibbles.
+//
+// Values: a lane packs each half of its 8 columns with byte permutes (selectors by the half's mask) and
+// stores the 4 elements one by one, wanted or not, the last ones first.  What a half stores behind its own
+// entries lands where a later half has an entry of a lower number, which is stored after it; a wave's LDS
+// operations are carried out in the order issued.  So no element needs an address or a test of its own.
+// A half without entries stores to a spare place (it would share its place with the half behind it).
+// Nibbles: 256-entry table by the lane's entry mask, packed; one or two OR operations on words that are
+// zero beforehand.
+// What bounds it is memory: 11008 x 4096 fp16 at density 0.5 reads 90 MB and writes 56 in 34.4 us (4.3 TB/s).
+// With a 4-byte LDS store per column behind a select, and the groups packed from those words again, it took
+// 39.7, half of them vector instructions.  Waiting for a row's loads all at once, so that no tile's wait
+// for its load is also one for the stores of the tile before, with 8 tiles in flight: 36.4.
+//
+// Groups cut by a row boundary are shared with the
 // neighbouring row's wave: their values go out as 2-byte stores and their nibbles as bytes.  A
 // byte holds two nibbles; where a row ends on an odd entry its last nibble shares a byte with the
 // first nibble of the next non-empty row.  That byte is written by the earlier row's wave, which
@@ -273,36 +319,49 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
 {
     typedef typename F::Elem Elem;
     typedef typename F::Chunk Chunk;
-    constexpr int kStage = kTile + 8;  // a tile's entries plus the carried part of a group
-    __shared__ __attribute__((aligned(16))) u32 stage_all[kRowsPerBlock][kStage + kWave];  // + a spare word per lane
-    // gap_table[m]: the 8 nibbles of a lane whose non-zero columns are the set bits of m, as far as
-    // they can be told from m alone: 15 where there is no non-zero, the distance to the previous
-    // set bit less one for a non-zero, and 0 for the first non-zero, whose distance reaches back
-    // into earlier lanes and is put in by the lane itself
+    // the carried part of a group, a tile's entries, and what the last half stores behind its own
+    constexpr int kStage = 8 + kTile + 8;
+    constexpr int kNibbleWords = kTile / 8 + 2;
+    __shared__ __attribute__((aligned(16))) Elem stage_all[kRowsPerBlock][kStage + 4 * kWave];  // + 4 spare places per lane
+    __shared__ u32 nibbles_all[kRowsPerBlock][kNibbleWords];
+    // gap_table[m]: the nibbles of a lane whose entries are the set bits of m, packed, lowest first: the
+    // distance to the previous set bit less one, and 0 for the first, whose distance reaches back into
+    // earlier lanes and is put in by the lane itself
     __shared__ u32 gap_table[256];
+    __shared__ __attribute__((aligned(8))) u32 pack_table[16][F::kHalfWords];
     static_assert(kBlock == 256, "one table entry per thread");
-    {
-        const u32 m = threadIdx.x;
-        u32 word = 0;
-        int previous = -1;
-        for (int i = 0; i < 8; ++i) {
-            u32 nib = 15u;
-            if ((m >> i) & 1u) {
-                nib = previous < 0 ? 0u : (u32)(i - previous - 1);
-                previous = i;
-            }
-            word |= nib << (4 * i);
-        }
-        gap_table[m] = word;
-    }
-    __syncthreads();
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = uniform(threadIdx.x >> 6);
     const int row = blockIdx.x * kRowsPerBlock + wave;
+    const Elem *src = dense + (size_t)row * (size_t)cols;
+
+    // kAhead tiles of the row in flight
+    Chunk ahead[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+        const int col = k * kTile + lane * kChunk;
+        ahead[k] = row < rows && k * kTile < cols ? load8<F, STREAM>(src, col, cols) : Chunk{};
+    }
+    {
+        const u32 m = threadIdx.x;
+        u32 word = 0;
+        int previous = -1, n = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if ((m >> i) & 1u) {
+                if (previous >= 0) word |= (u32)(i - previous - 1) << (4 * n);
+                previous = i;
+                ++n;
+            }
+        gap_table[m] = word;
+        if (m < 16 * F::kHalfWords) pack_table[m / F::kHalfWords][m % F::kHalfWords] = F::selectors(m / F::kHalfWords, m % F::kHalfWords);
+    }
+    __syncthreads();
     if (row >= rows) return;
     const int e0 = row_ptr[row];
     const int e1 = row_ptr[row + 1];
-    u32 *stage = stage_all[wave];
+    Elem *stage = stage_all[wave];
+    u32 *nibbles = nibbles_all[wave];
     Chunk *value_groups = reinterpret_cast<Chunk *>(values);
     unsigned char *delta_bytes = reinterpret_cast<unsigned char *>(delta_words);
 
@@ -337,67 +396,59 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
         return m ? (u32)__builtin_ctzll(m) : 15u;
     };
 
-    const Elem *src = dense + (size_t)row * (size_t)cols;
-    const bool vector_ok = (reinterpret_cast<uintptr_t>(src) & (sizeof(Chunk) - 1)) == 0;
-
-    // stage[i] holds output entry base + i; [lo, hi) is staged and not yet written out
+    // entry base + i is stage[i] and nibble i of `nibbles`; [lo, hi) is staged and not yet written out;
+    // nibbles that are not staged are zero
     int base = e0 & ~7;
     int lo = e0 - base;
     int hi = lo;
     int carry = -1;
+    nibbles[lane] = 0;
+    if (lane < kNibbleWords - kWave) nibbles[kWave + lane] = 0;
+    wave_lds_fence();
 
     // writes out groups [0, n_groups) of the stage; group g holds entries [a, b) with
     // a = lo for group 0 and b = hi - 8g for a last, incomplete group (which ends the row)
     auto flush = [&](int n_groups, u32 nibble_behind) {
         for (int g = lane; g < n_groups; g += kWave) {
-            u32 e[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) e[i] = stage[8 * g + i];
+            const Chunk v = *reinterpret_cast<const Chunk *>(stage + 8 * g);
+            const u32 word = nibbles[g];
             const int a = g == 0 ? lo : 0;
             const int b = hi - 8 * g < 8 ? hi - 8 * g : 8;
             const int out = (base >> 3) + g;
             if (a == 0 && b == 8) {
-                value_groups[out] = F::pack(e);
-                delta_words[out] = pack_nibbles(e);
+                value_groups[out] = v;
+                delta_words[out] = word;
             } else {
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-                    if (i >= a && i < b) values[8 * (size_t)out + i] = (Elem)e[i];
+                    if (i >= a && i < b) values[8 * (size_t)out + i] = (Elem)F::at(v, i);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const bool low_mine = 2 * j >= a && 2 * j < b;
                     const bool high_mine = 2 * j + 1 >= a && 2 * j + 1 < b;
                     // low nibble mine: my byte, whoever the high nibble belongs to
                     if (low_mine) {
-                        const u32 low = (e[2 * j] >> 16) & 15u;
-                        const u32 high = high_mine ? (e[2 * j + 1] >> 16) & 15u : nibble_behind;
-                        delta_bytes[4 * (size_t)out + j] = (unsigned char)(low | (high << 4));
+                        const u32 both = (word >> (8 * j)) & 0xffu;
+                        delta_bytes[4 * (size_t)out + j] = (unsigned char)(high_mine ? both : (both & 15u) | (nibble_behind << 4));
                     }
                 }
             }
         }
     };
 
-    // kAhead tiles of the row in flight, as in pass 1
-    Chunk ahead[kAhead];
-#pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-        const int col = k * kTile + lane * kChunk;
-        ahead[k] = load8<F, STREAM>(src, col, cols, vector_ok && col < cols);
-    }
     bool row_done = false;
     for (int c0 = 0; c0 < cols && !row_done; c0 += kAhead * kTile) {
 #pragma unroll
         for (int k = 0; k < kAhead; ++k) {
             if (row_done || c0 + k * kTile >= cols) break;  // wave-uniform
             const int col = c0 + k * kTile + lane * kChunk;
-            const Chunk v = ahead[k];
+            Chunk v = cut8<F>(ahead[k], c0 + k * kTile, col, cols);
             const int ncol = col + kAhead * kTile;
-            if (c0 + (k + kAhead) * kTile < cols) ahead[k] = load8<F, STREAM>(src, ncol, cols, vector_ok && ncol < cols);
-            const u32 nz = nonzero_bits<F>(v);
+            if (c0 + (k + kAhead) * kTile < cols) ahead[k] = load8<F, STREAM>(src, ncol, cols);
+            const u32 nz = F::nonzero_bits(v);
             const int own_last = nz ? col + 31 - __builtin_clz(nz) : kNoColumn;
             int pass_last;
-            int p = previous_nonzero(own_last, carry, lane, pass_last);
+            const int p = previous_nonzero(own_last, carry, pass_last);
             carry = pass_last > carry ? pass_last : carry;
             // Non-zeros are entries.  A padding entry stands at p + 16, p + 32, ...: among my 8
             // columns at most one, and only in front of my first non-zero (behind it the previous
@@ -406,8 +457,8 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
             const int first_nz = nz ? __builtin_ctz(nz) : 8;
             const bool has_pad = pad_at < first_nz && col + pad_at < cols;
             const u32 entry_bits = nz | (has_pad ? 1u << pad_at : 0u);
-            u32 nibbles = gap_table[nz];
-            if (nz) nibbles |= ((u32)(col + first_nz - p - 1) & 15u) << (4 * first_nz);
+            // a padding entry is 16 columns or a multiple of that behind p: 15, too
+            const u32 first = has_pad ? 15u : (u32)(col + first_nz - p - 1) & 15u;
             const int mine = __builtin_popcount(entry_bits);
             const int incl = wave_scan_inclusive(mine);
             const int produced = __builtin_amdgcn_readlane(incl, kWave - 1);
@@ -419,21 +470,36 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
             // in front of it.  So a lane keeps all of its entries or none.
             const int slot = incl - mine;
             const u32 kept = slot < n_new ? entry_bits : 0u;
-            Chunk vs = v;
             if (__builtin_expect(__ballot(F::any_nan(v)) != 0ull, 0)) {  // NaNs are stored in one form
-                vs = Chunk{};
+                Chunk vs = Chunk{};
 #pragma unroll
                 for (int i = 0; i < 8; ++i) F::put(vs, i, F::stored(F::at(v, i)));
+                v = vs;
             }
-            // every lane writes all 8 of its columns, no branches: what is not kept goes to a word
-            // of the lane's own behind the stage
-            const int first_index = hi + slot;
+            const int index = hi + slot;
+            u32 packed[2][4];
+            Elem *place[2];
+            const u32 half_mask[2] = {kept & 15u, kept >> 4};
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const bool take = ((kept >> i) & 1u) != 0;
-                const int rank = __builtin_popcount(kept & ((1u << i) - 1u));
-                const u32 word = F::at(vs, i) | (((nibbles >> (4 * i)) & 15u) << 16);
-                stage[take ? first_index + rank : kStage + lane] = word;
+            for (int h = 0; h < 2; ++h) {
+                u32 sel[F::kHalfWords];
+#pragma unroll
+                for (int w = 0; w < F::kHalfWords; ++w) sel[w] = pack_table[half_mask[h]][w];
+                F::pack(v, h, sel, packed[h]);
+                place[h] = stage + (half_mask[h] ? index + (h ? __builtin_popcount(half_mask[0]) : 0) : kStage + 4 * lane);
+            }
+#pragma unroll
+            for (int j = 3; j >= 0; --j) {
+                place[0][j] = (Elem)packed[0][j];
+                place[1][j] = (Elem)packed[1][j];
+                wave_lds_fence();
+            }
+            if (kept) {
+                const u32 word = gap_table[kept] | first;
+                const int shift = 4 * (index & 7);
+                const u32 behind = (word >> 1) >> (31 - shift);
+                __hip_atomic_fetch_or(nibbles + (index >> 3), word << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                if (behind) __hip_atomic_fetch_or(nibbles + (index >> 3) + 1, behind, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             }
             hi += n_new;
             wave_lds_fence();
@@ -442,13 +508,16 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
             flush(n_groups, row_done && shares_last_byte ? first_nibble_behind() : 0u);
             if (row_done) break;
             if (n_groups > 0) {  // carry the incomplete group to the front of the stage
-                const int rest = hi & 7;
-                const u32 moved = lane < rest ? stage[8 * n_groups + lane] : 0u;
+                const Chunk moved = *reinterpret_cast<const Chunk *>(stage + 8 * n_groups);
+                const u32 moved_nibbles = nibbles[n_groups];
                 wave_lds_fence();
-                if (lane < rest) stage[lane] = moved;
+                if (lane == 0) *reinterpret_cast<Chunk *>(stage) = moved;
+                nibbles[lane] = lane == 0 ? moved_nibbles : 0u;
+                if (lane < kNibbleWords - kWave) nibbles[kWave + lane] = 0;
+                wave_lds_fence();
                 base += 8 * n_groups;
                 lo = 0;
-                hi = rest;
+                hi &= 7;
             }
         }
     }

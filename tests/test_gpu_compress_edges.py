@@ -1,0 +1,36 @@
+"""The compressor at the edges of its lanes (8 columns), tiles (512) and rounds (2048), on rows that start at
+any element: bit for bit what the checker gives."""
+import numpy as np
+import pytest
+import torch
+
+import macko_spmv_amd as mk
+from oracle import macko_oracle as mo
+
+pytestmark = pytest.mark.gpu
+COLS = (1, 3, 7, 8, 9, 15, 17, 63, 505, 511, 512, 513, 1000, 2041, 2048, 2055, 4096, 4099)
+
+
+@pytest.mark.parametrize("int8", (False, True))
+@pytest.mark.parametrize("density", (0.0, 0.02, 0.3, 0.97, 1.0))
+@pytest.mark.parametrize("offset", (0, 1))
+def test_compress_at_edges(int8, density, offset):
+    rng = np.random.default_rng(int(density * 100) + offset)
+    for cols in COLS:
+        rows = int(rng.integers(1, 12))
+        flat = rng.standard_normal(rows * cols + offset)
+        flat = np.clip(np.rint(flat * 60), -128, 127).astype(np.int8) if int8 else flat.astype(np.float16)
+        flat[rng.random(flat.size) >= density] = 0
+        dense = flat[offset:].reshape(rows, cols)
+        if rows > 3:
+            dense[2] = 0
+        if not int8 and density == 0.3:
+            dense[0, cols // 2:] = -0.0
+            dense[rows - 1, cols // 2] = np.nan
+        M = torch.from_numpy(flat).cuda()[offset:].view(rows, cols)
+        got = (mk.compress_int8 if int8 else mk.compress)(M)
+        values, deltas, row_ptr, n = (mo.compress_int8 if int8 else mo.compress)(dense)
+        v = got[0].cpu().numpy()
+        assert np.array_equal(v if int8 else v.view(np.uint16), values), (cols, rows)
+        assert np.array_equal(got[1].cpu().numpy(), deltas), (cols, rows)
+        assert np.array_equal(got[2].cpu().numpy(), row_ptr), (cols, rows)
