@@ -23,6 +23,7 @@ from collections import OrderedDict
 
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 import macko_spmv_amd as macko_spmv
 
@@ -120,10 +121,14 @@ def load_compressed_linears(model, compressed_sd):
 # ---- a minimal Llama-architecture decoder (batch 1) ------------------------------------------------
 
 def _inference_half(*tensors):
-    """fp16 tensors on the GPU through which no gradient has to flow: what the hand-written kernels between
-    the projections take."""
+    """fp16 tensors on the GPU, 16-byte aligned, through which no gradient, tangent or batching rule has to
+    flow: what the hand-written kernels between the projections take."""
+    if not torch.compiler.is_compiling() and (torch.autograd.forward_ad._current_level >= 0
+                                              or torch._C._functorch.peek_interpreter_stack() is not None):
+        return False
     grad = torch.is_grad_enabled()
-    return all(t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad) for t in tensors)
+    return all(t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad)
+               and t.storage_offset() % 8 == 0 for t in tensors)
 
 
 class RMSNorm(nn.Module):
@@ -133,7 +138,8 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x):
-        if _inference_half(x, self.weight) and x.is_contiguous() and x.shape[-1] % 8 == 0 and x.numel() > 0:
+        if (_inference_half(x, self.weight) and x.is_contiguous() and x.shape[-1] % 8 == 0 and x.numel() > 0
+                and self.weight.is_contiguous() and self.weight.shape == x.shape[-1:]):
             return torch.ops.macko_spmv.rmsnorm_rows(x, self.weight, self.eps)
         v = x.float()
         v = v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + self.eps)
@@ -163,6 +169,9 @@ class Attention(nn.Module):
         att = torch.softmax((att + mask).float(), dim=-1).to(x.dtype)
         out = torch.matmul(att, self.v_cache).transpose(1, 2).reshape(1, t, -1)
         return self.o_proj(out)
+
+
+_FUSED_CAUSAL = "causal"  # in the place of a mask: the layer goes through Block.forward_fused
 
 
 def _causal_mask(max_len, positions, dtype):
@@ -196,15 +205,17 @@ class Block(nn.Module):
 
     def takes_fused(self, x):
         """Whether several tokens go through the layer by way of forward_fused: inference in fp16 on the
-        GPU, all seven projections compressed, nothing hooked to the modules that would be passed over."""
+        GPU, all seven projections compressed, nothing hooked to the layer or the modules passed over."""
         att, mlp = self.self_attn, self.mlp
         projections = (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
         norms = (self.input_layernorm, self.post_attention_layernorm)
         return (x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
                 and all(type(p) is MackoLinear for p in projections)
                 and att.n_heads * att.head_dim == x.shape[2] and projections[4].c_3 % 8 == 0 and projections[4].c_3 >= 64
-                and all(type(n) is RMSNorm for n in norms)
-                and not any(m._forward_hooks or m._forward_pre_hooks for m in (att, mlp, *projections, *norms))
+                and all(type(n) is RMSNorm for n in norms) and type(att) is Attention and type(mlp) is MLP
+                and not _has_any_global_hook()
+                and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m)
+                            for m in (self, att, mlp, *projections, *norms))
                 and att.k_cache.is_contiguous() and att.v_cache.is_contiguous()
                 and _inference_half(x, *(n.weight for n in norms), att.k_cache, att.v_cache))
 
@@ -231,10 +242,8 @@ class Block(nn.Module):
         return product(mlp.down_proj, gated, rows).view(1, t, -1)
 
     def forward(self, x, cos, sin, positions, mask):
-        if mask is None:  # causal; any other mask is the general path's
-            if self.takes_fused(x):
-                return self.forward_fused(x, cos, sin, positions)
-            mask = _causal_mask(self.self_attn.max_len, positions, x.dtype)
+        if isinstance(mask, str) and mask == _FUSED_CAUSAL:  # LlamaDecoder's own, where takes_fused; a mask is the general path's
+            return self.forward_fused(x, cos, sin, positions)
         x = x + self.self_attn(self.input_layernorm(x), cos, sin, positions, mask)
         return x + self.mlp(self.post_attention_layernorm(x))
 
@@ -267,11 +276,14 @@ class LlamaDecoder(nn.Module):
         x = self.model.embed_tokens(tokens)
         cos = self.cos[positions].to(x.dtype)[None, None]
         sin = self.sin[positions].to(x.dtype)[None, None]
-        # a layer that works all its tokens in hand-written kernels needs no mask
-        fused = [layer.takes_fused(x) for layer in self.model.layers]
-        mask = None if all(fused) else _causal_mask(self.max_len, positions, x.dtype)
-        for layer, without_mask in zip(self.model.layers, fused):
-            x = layer(x, cos, sin, positions, None if without_mask else mask)
+        mask = None  # only made for a layer that needs one
+        for layer in self.model.layers:
+            if type(layer) is Block and layer.takes_fused(x):
+                x = layer(x, cos, sin, positions, _FUSED_CAUSAL)
+                continue
+            if mask is None:
+                mask = _causal_mask(self.max_len, positions, x.dtype)
+            x = layer(x, cos, sin, positions, mask)
         return self.lm_head(self.model.norm(x))
 
 

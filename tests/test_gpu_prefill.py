@@ -155,9 +155,11 @@ def test_layer_keeps_a_given_mask_and_strided_positions():
     x = model.model.embed_tokens(torch.randint(0, 1000, (1, t), device="cuda"))
     cos, sin = (table[pos].half()[None, None] for table in (model.cos, model.sin))
     assert layer.takes_fused(x)
-    causal = layer(x, cos, sin, pos, None)
+    causal = layer(x, cos, sin, pos, llm._FUSED_CAUSAL)
     spread = torch.stack((pos, pos), 1)[:, 0]
-    assert not spread.is_contiguous() and torch.equal(layer(x, cos, sin, spread, None), causal)
+    assert not spread.is_contiguous() and torch.equal(layer(x, cos, sin, spread, llm._FUSED_CAUSAL), causal)
+    with pytest.raises(TypeError):   # no mask is no call of the layer
+        layer(x, cos, sin, pos, None)
     # a mask that lets a token see only itself is not the causal one
     own = torch.full((1, 1, t, 48), float("-inf"), device="cuda", dtype=torch.float16)
     own[0, 0, pos, pos] = 0
@@ -166,3 +168,20 @@ def test_layer_keeps_a_given_mask_and_strided_positions():
     want = layer(x, cos, sin, pos, own)
     handle.remove()
     assert torch.equal(masked, want) and not torch.allclose(masked, causal, rtol=2e-2, atol=2e-2)
+
+
+def test_norm_goes_the_general_way_where_the_kernel_cannot():
+    """Unaligned tokens, forward-mode derivatives, vmap: as torch's own operators take them."""
+    norm = llm.RMSNorm(64).cuda().half().requires_grad_(False)
+    flat = torch.randn(5 * 64 + 8, device="cuda").half()
+    x = flat[:320].view(5, 64)
+    want = norm(x.float()).double()   # fp32: through torch
+    unaligned = flat[1:321].view(5, 64)
+    unaligned.copy_(x.clone())
+    got = norm(unaligned)
+    assert torch.allclose(got.double(), want, rtol=2.0 ** -10, atol=2.0 ** -24)
+    x = unaligned.clone()
+    assert torch.equal(torch.func.vmap(norm)(x), norm(unaligned))
+    y, tangent = torch.func.jvp(norm, (x,), (x,))
+    # the norm does not change with its input's length, up to eps and the rounding of x times the weight
+    assert torch.equal(y, norm(unaligned)) and tangent.abs().max() < 1e-2
