@@ -529,6 +529,14 @@ void multiply_attention_axpby_hip(const at::Tensor &M_values, const at::Tensor &
 
 void *current_stream() { return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
 
+// The prompt's kernels move 16 bytes at a time.  A tensor that starts elsewhere (a view into a larger buffer, memory
+// of another library) goes through a copy of its own; one that is written is copied back.
+at::Tensor aligned16(const at::Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) ? t.clone() : t; }
+void copy_back(at::Tensor &to, const at::Tensor &from)
+{
+    if (!from.is_same(to)) to.copy_(from);
+}
+
 // Vectors [batch, cols] in operand order: a flat half tensor.
 at::Tensor packed_like(const at::Tensor &t, int64_t cols, int64_t batch)
 {
@@ -545,7 +553,8 @@ at::Tensor pack_rmsnorm_hip(const at::Tensor &x, const at::Tensor &weight, doubl
     TORCH_CHECK(x.dim() == 2 && weight.numel() == x.size(1), "x must be [batch, cols], weight [cols]");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     at::Tensor packed = packed_like(x, x.size(1), x.size(0));
-    check_rc(macko_prefill_pack_rmsnorm_f16(x.data_ptr(), weight.data_ptr(), packed.data_ptr(), (int32_t)x.size(1),
+    const at::Tensor rows = aligned16(x), scale = aligned16(weight);
+    check_rc(macko_prefill_pack_rmsnorm_f16(rows.data_ptr(), scale.data_ptr(), packed.data_ptr(), (int32_t)x.size(1),
                                             (int32_t)x.size(0), (float)eps, current_stream()),
              "pack_rmsnorm");
     return packed;
@@ -561,7 +570,8 @@ at::Tensor rmsnorm_rows_hip(const at::Tensor &x, const at::Tensor &weight, doubl
     at::Tensor y = at::empty_like(x);
     if (x.numel() == 0) return y;
     TORCH_CHECK(x.numel() / x.size(-1) < (1ll << 31), "too many rows");
-    check_rc(macko_rmsnorm_rows_f16(x.data_ptr(), weight.data_ptr(), y.data_ptr(), (int32_t)x.size(-1),
+    const at::Tensor rows = aligned16(x), scale = aligned16(weight);
+    check_rc(macko_rmsnorm_rows_f16(rows.data_ptr(), scale.data_ptr(), y.data_ptr(), (int32_t)x.size(-1),
                                     (int32_t)(x.numel() / x.size(-1)), (float)eps, current_stream()),
              "rmsnorm_rows");
     return y;
@@ -574,7 +584,8 @@ at::Tensor pack_silu_mul_hip(const at::Tensor &gate, const at::Tensor &up)
     TORCH_CHECK(gate.dim() == 2 && gate.sizes() == up.sizes(), "gate and up must be [batch, cols]");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(gate.device());
     at::Tensor packed = packed_like(gate, gate.size(1), gate.size(0));
-    check_rc(macko_prefill_pack_silu_mul_f16(gate.data_ptr(), up.data_ptr(), packed.data_ptr(), (int32_t)gate.size(1),
+    const at::Tensor g = aligned16(gate), u = aligned16(up);
+    check_rc(macko_prefill_pack_silu_mul_f16(g.data_ptr(), u.data_ptr(), packed.data_ptr(), (int32_t)gate.size(1),
                                              (int32_t)gate.size(0), current_stream()),
              "pack_silu_mul");
     return packed;
@@ -627,11 +638,16 @@ void prefill_rope_append_hip(at::Tensor q, const at::Tensor &k, const at::Tensor
     TORCH_CHECK(cos_rows.numel() == q.size(0) * k_cache.size(2) && sin_rows.numel() == cos_rows.numel(),
                 "cos / sin must be [batch, head_dim]");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-    check_rc(macko_prefill_rope_append_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos_rows.data_ptr(), sin_rows.data_ptr(),
-                                           positions.data_ptr<int64_t>(), k_cache.data_ptr(), v_cache.data_ptr(),
+    const at::Tensor q16 = aligned16(q), k16 = aligned16(k), v16 = aligned16(v), cos16 = aligned16(cos_rows), sin16 = aligned16(sin_rows);
+    const at::Tensor keys = aligned16(k_cache), cached = aligned16(v_cache);
+    check_rc(macko_prefill_rope_append_f16(q16.data_ptr(), k16.data_ptr(), v16.data_ptr(), cos16.data_ptr(), sin16.data_ptr(),
+                                           positions.data_ptr<int64_t>(), keys.data_ptr(), cached.data_ptr(),
                                            (int32_t)q.size(0), (int32_t)k_cache.size(0), (int32_t)k_cache.size(2),
                                            (int32_t)k_cache.size(1), current_stream()),
              "prefill_rope_append");
+    copy_back(q, q16);
+    copy_back(k_cache, keys);
+    copy_back(v_cache, cached);
 }
 
 at::Tensor prefill_attention_hip(const at::Tensor &q, const at::Tensor &k_cache, const at::Tensor &v_cache,
@@ -642,7 +658,8 @@ at::Tensor prefill_attention_hip(const at::Tensor &q, const at::Tensor &k_cache,
     check_caches(k_cache, v_cache, positions, q.size(0), q.size(1));
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
     at::Tensor packed = packed_like(q, q.size(1), q.size(0));
-    check_rc(macko_prefill_attention_f16(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr<int64_t>(),
+    const at::Tensor q16 = aligned16(q), keys = aligned16(k_cache), cached = aligned16(v_cache);
+    check_rc(macko_prefill_attention_f16(q16.data_ptr(), keys.data_ptr(), cached.data_ptr(), positions.data_ptr<int64_t>(),
                                          packed.data_ptr(), (int32_t)q.size(0), (int32_t)k_cache.size(0), (int32_t)k_cache.size(2),
                                          (int32_t)k_cache.size(1), (float)scale, current_stream()),
              "prefill_attention");

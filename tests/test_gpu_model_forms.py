@@ -1,0 +1,43 @@
+"""Forms of input that a layer of the decoder takes through its modules, and that it has to take as well where
+hand-written kernels stand between the projections: memory that is not 16-byte aligned, norm weights of any stride,
+projections that do not fit, infinite scores."""
+import pytest
+import torch
+
+from macko_spmv_amd import llm
+
+pytestmark = pytest.mark.gpu
+ops = torch.ops.macko_spmv
+
+
+def _elsewhere(t, by=1):
+    """A copy of t whose memory starts `by` elements behind an aligned address, as storage of its own (offset 0)."""
+    flat = torch.empty(t.numel() + by, device=t.device, dtype=t.dtype)
+    moved = torch.from_dlpack(flat[by:].view(t.shape).copy_(t))
+    assert moved.data_ptr() % 16 and moved.storage_offset() == 0
+    return moved
+
+
+def test_operators_between_the_projections_take_memory_of_any_alignment():
+    g = torch.Generator(device="cuda").manual_seed(3)
+    half = lambda *shape: torch.randn(shape, device="cuda", generator=g).half()
+    x, up, w = half(19, 128), half(19, 128), half(128)
+    assert torch.equal(ops.rmsnorm_rows(_elsewhere(x), _elsewhere(w), 1e-5), ops.rmsnorm_rows(x, w, 1e-5))
+    assert torch.equal(ops.pack_rmsnorm(_elsewhere(x), _elsewhere(w), 1e-5), ops.pack_rmsnorm(x, w, 1e-5))
+    assert torch.equal(ops.pack_silu_mul(_elsewhere(x), _elsewhere(up)), ops.pack_silu_mul(x, up))
+    k, v, cos, sin, kc, vc = half(19, 128), half(19, 128), half(19, 64), half(19, 64), half(2, 30, 64), half(2, 30, 64)
+    pos = torch.arange(19, device="cuda")
+    q1, k1, v1 = x.clone(), kc.clone(), vc.clone()
+    ops.prefill_rope_append(q1, k, v, cos, sin, pos, k1, v1)
+    q2, k2, v2 = _elsewhere(x), _elsewhere(kc), _elsewhere(vc)
+    ops.prefill_rope_append(q2, _elsewhere(k), _elsewhere(v), _elsewhere(cos), _elsewhere(sin), pos, k2, v2)
+    assert torch.equal(q1, q2) and torch.equal(k1, k2) and torch.equal(v1, v2)
+    assert torch.equal(ops.prefill_attention(q2, k2, v2, pos, 0.125), ops.prefill_attention(q1, k1, v1, pos, 0.125))
+
+
+def test_norm_takes_memory_of_any_alignment():
+    norm = llm.RMSNorm(64).cuda().half().requires_grad_(False)
+    x = torch.randn(5, 64, device="cuda").half()
+    want = norm(x.float()).double()   # fp32: through torch
+    # one rounding to fp16 of a value with a few fp32 roundings in it
+    assert torch.allclose(norm(_elsewhere(x)).double(), want, rtol=2.0 ** -10, atol=2.0 ** -24)
