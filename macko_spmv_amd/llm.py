@@ -121,14 +121,16 @@ def load_compressed_linears(model, compressed_sd):
 # ---- a minimal Llama-architecture decoder (batch 1) ------------------------------------------------
 
 def _inference_half(*tensors):
-    """fp16 tensors on the GPU, 16-byte aligned, through which no gradient, tangent or batching rule has to
-    flow: what the hand-written kernels between the projections take."""
-    if not torch.compiler.is_compiling() and (torch.autograd.forward_ad._current_level >= 0
-                                              or torch._C._functorch.peek_interpreter_stack() is not None):
+    """fp16 tensors on the GPU through which no gradient, tangent or batching rule has to flow: what the
+    hand-written kernels between the projections take.  The operators copy what is not 16-byte aligned; eagerly
+    such views keep to torch's operators (Dynamo cannot trace storage_offset(); and what it makes of the
+    interpreter stack is never None, but has the right type)."""
+    transformed = isinstance(torch._C._functorch.peek_interpreter_stack(), torch._C._functorch.CInterpreter)
+    if transformed or torch.autograd.forward_ad._current_level >= 0:
         return False
-    grad = torch.is_grad_enabled()
+    grad, tracing = torch.is_grad_enabled(), torch.compiler.is_compiling()
     return all(t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad)
-               and t.storage_offset() % 8 == 0 for t in tensors)
+               and (tracing or t.storage_offset() % 8 == 0) for t in tensors)
 
 
 class RMSNorm(nn.Module):

@@ -41,3 +41,18 @@ def test_norm_takes_memory_of_any_alignment():
     want = norm(x.float()).double()   # fp32: through torch
     # one rounding to fp16 of a value with a few fp32 roundings in it
     assert torch.allclose(norm(_elsewhere(x)).double(), want, rtol=2.0 ** -10, atol=2.0 ** -24)
+
+
+@pytest.mark.parametrize("tokens", [1, 19])
+def test_compiled_decoder_gives_what_the_eager_one_gives(tokens):
+    with torch.no_grad():
+        model, _ = llm.build_model(0.4, sparse=True, n_layers=2, dim=256, hidden=704, n_heads=2, vocab=1000, max_len=48)
+        prompt, pos = torch.randint(0, 1000, (1, tokens), device="cuda"), torch.arange(tokens, device="cuda")
+        want = model(prompt, pos)
+        caches = [layer.self_attn.k_cache.clone() for layer in model.model.layers]
+        for layer in model.model.layers:
+            layer.self_attn.k_cache.zero_()
+        torch._dynamo.reset()
+        got = torch.compile(model, fullgraph=True, backend="aot_eager")(prompt, pos)
+        assert torch.equal(got, want)
+        assert all(torch.equal(layer.self_attn.k_cache, kept) for layer, kept in zip(model.model.layers, caches))

@@ -1,0 +1,60 @@
+"""The decoder under the tools that trace it, which must take it whole: what it decides about the route of a layer in
+Python may not break a graph, and a traced graph computes what the modules compute."""
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+from macko_spmv_amd import llm
+
+
+def _fake_model(mode, dim=256, hidden=704, heads=2):
+    """Half-precision decoder with compressed projections on a GPU that need not exist."""
+    with mode, torch.device("cuda"):
+        default = torch.get_default_dtype()
+        torch.set_default_dtype(torch.float16)
+        try:
+            model = llm.LlamaDecoder(100, dim, hidden, 2, heads, 48).requires_grad_(False)
+        finally:
+            torch.set_default_dtype(default)
+        for layer in model.model.layers:
+            for parent, name in llm.PROJECTIONS:
+                module = getattr(layer, parent)
+                rows, cols = getattr(module, name).weight.shape
+                n = rows * cols // 2
+                setattr(module, name, llm.MackoLinear(torch.empty(n, dtype=torch.float16), torch.empty(n // 2, dtype=torch.uint8),
+                                                      torch.empty(rows + 1, dtype=torch.int32), rows, cols))
+    return model
+
+
+def _operators(function, *args):
+    """Names of this package's operators in the one graph that Dynamo makes of a call."""
+    graphs = []
+
+    def backend(graph, example_inputs):
+        graphs.append(graph)
+        return graph.forward
+
+    torch._dynamo.reset()
+    torch.compile(function, fullgraph=True, backend=backend)(*args)
+    assert len(graphs) == 1
+    return [str(n.target).split(".")[1] for n in graphs[0].graph.nodes if str(n.target).startswith("macko_spmv.")]
+
+
+def test_decoder_compiles_as_one_graph():
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    model = _fake_model(mode)
+    with mode, torch.no_grad(), torch.device("cuda"):
+        for tokens in (1, 20):
+            found = _operators(model, torch.empty((1, tokens), dtype=torch.long), torch.empty((tokens,), dtype=torch.long))
+            per_layer = (["pack_rmsnorm"] + 3 * ["multiply_packed"] + ["prefill_rope_append", "prefill_attention", "multiply_packed",
+                         "pack_rmsnorm", "multiply_packed", "multiply_packed", "pack_silu_mul", "multiply_packed"])
+            if tokens == 1:
+                per_layer = ["rmsnorm_rows"] + 4 * ["multiply"] + ["rmsnorm_rows"] + 3 * ["multiply"]
+            assert found == 2 * per_layer + ["rmsnorm_rows"]
+        norm, x = model.model.norm, torch.empty((3, 256), dtype=torch.float16)
+        assert _operators(norm, x) == ["rmsnorm_rows"]
+        # a batching rule, a tangent or a gradient goes through torch's own operators
+        assert _operators(torch.func.vmap(norm), x) == []
+        assert _operators(lambda a: torch.func.jvp(norm, (a,), (a,)), x) == []
+    with mode, torch.enable_grad(), torch.device("cuda"):
+        assert _operators(norm, torch.empty((3, 256), dtype=torch.float16, requires_grad=True)) == []
