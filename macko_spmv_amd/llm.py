@@ -129,7 +129,8 @@ def _inference_half(*tensors):
     if transformed or torch.autograd.forward_ad._current_level >= 0:
         return False
     grad, tracing = torch.is_grad_enabled(), torch.compiler.is_compiling()
-    return all(t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad)
+    # (a torch.fx proxy is no tensor and has no answers)
+    return all(isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad)
                and (tracing or t.storage_offset() % 8 == 0) for t in tensors)
 
 
@@ -211,8 +212,8 @@ class Block(nn.Module):
         att, mlp = self.self_attn, self.mlp
         projections = (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
         norms = (self.input_layernorm, self.post_attention_layernorm)
-        return (x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
-                and all(type(p) is MackoLinear for p in projections)
+        return (all(type(p) is MackoLinear for p in projections)
+                and isinstance(x, torch.Tensor) and x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
                 and att.n_heads * att.head_dim == x.shape[2] and projections[4].c_3 % 8 == 0 and projections[4].c_3 >= 64
                 and all(type(n) is RMSNorm for n in norms) and type(att) is Attention and type(mlp) is MLP
                 and not _has_any_global_hook()

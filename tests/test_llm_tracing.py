@@ -58,3 +58,20 @@ def test_decoder_compiles_as_one_graph():
         assert _operators(lambda a: torch.func.jvp(norm, (a,), (a,)), x) == []
     with mode, torch.enable_grad(), torch.device("cuda"):
         assert _operators(norm, torch.empty((3, 256), dtype=torch.float16, requires_grad=True)) == []
+
+
+def _dense_model():
+    torch.manual_seed(0)
+    model = llm.LlamaDecoder(100, 64, 128, 2, 2, 32).requires_grad_(False)
+    return model, torch.randint(0, 100, (1, 7)), torch.arange(7)
+
+
+def test_symbolic_trace_of_norm_layer_and_decoder():
+    model, tokens, positions = _dense_model()
+    want = model(tokens, positions)
+    assert torch.equal(torch.fx.symbolic_trace(model)(tokens, positions), want)
+    x = torch.randn(1, 7, 64)
+    assert torch.equal(torch.fx.symbolic_trace(model.model.norm)(x), model.model.norm(x))
+    layer, cos = model.model.layers[0], torch.randn(1, 1, 7, 32)
+    mask = torch.zeros(1, 1, 7, 32)
+    assert torch.equal(torch.fx.symbolic_trace(layer)(x, cos, cos, positions, mask), layer(x, cos, cos, positions, mask))
