@@ -141,9 +141,10 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x):
-        if (_inference_half(x, self.weight) and x.is_contiguous() and x.shape[-1] % 8 == 0 and x.numel() > 0
-                and self.weight.is_contiguous() and self.weight.shape == x.shape[-1:]):
-            return torch.ops.macko_spmv.rmsnorm_rows(x, self.weight, self.eps)
+        if not torch.jit.is_scripting():
+            if (_inference_half(x, self.weight) and x.is_contiguous() and x.shape[-1] % 8 == 0 and x.numel() > 0
+                    and self.weight.is_contiguous() and self.weight.shape == x.shape[-1:]):
+                return torch.ops.macko_spmv.rmsnorm_rows(x, self.weight, self.eps)
         v = x.float()
         v = v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + self.eps)
         return (v * self.weight.float()).to(x.dtype)
@@ -177,7 +178,7 @@ class Attention(nn.Module):
 _FUSED_CAUSAL = "causal"  # in the place of a mask: the layer goes through Block.forward_fused
 
 
-def _causal_mask(max_len, positions, dtype):
+def _causal_mask(max_len: int, positions, dtype: torch.dtype):
     key_pos = torch.arange(max_len, device=positions.device)
     return torch.where(key_pos[None, :] <= positions[:, None], 0.0, float("-inf")).to(dtype)[None, None]
 
@@ -245,8 +246,9 @@ class Block(nn.Module):
         return product(mlp.down_proj, gated, rows).view(1, t, -1)
 
     def forward(self, x, cos, sin, positions, mask):
-        if isinstance(mask, str) and mask == _FUSED_CAUSAL:  # LlamaDecoder's own, where takes_fused; a mask is the general path's
-            return self.forward_fused(x, cos, sin, positions)
+        if not torch.jit.is_scripting():
+            if isinstance(mask, str) and mask == _FUSED_CAUSAL:  # LlamaDecoder's own, where takes_fused; a mask is the general path's
+                return self.forward_fused(x, cos, sin, positions)
         x = x + self.self_attn(self.input_layernorm(x), cos, sin, positions, mask)
         return x + self.mlp(self.post_attention_layernorm(x))
 
@@ -279,6 +281,16 @@ class LlamaDecoder(nn.Module):
         x = self.model.embed_tokens(tokens)
         cos = self.cos[positions].to(x.dtype)[None, None]
         sin = self.sin[positions].to(x.dtype)[None, None]
+        if torch.jit.is_scripting():
+            mask = _causal_mask(self.max_len, positions, x.dtype)
+            for layer in self.model.layers:
+                x = layer(x, cos, sin, positions, mask)
+        else:
+            x = self._run_layers(x, cos, sin, positions)
+        return self.lm_head(self.model.norm(x))
+
+    @torch.jit.unused
+    def _run_layers(self, x, cos, sin, positions):
         mask = None  # only made for a layer that needs one
         for layer in self.model.layers:
             if type(layer) is Block and layer.takes_fused(x):
@@ -287,7 +299,7 @@ class LlamaDecoder(nn.Module):
             if mask is None:
                 mask = _causal_mask(self.max_len, positions, x.dtype)
             x = layer(x, cos, sin, positions, mask)
-        return self.lm_head(self.model.norm(x))
+        return x
 
 
 def prune_rows_(weight, density):

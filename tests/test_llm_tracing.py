@@ -75,3 +75,15 @@ def test_symbolic_trace_of_norm_layer_and_decoder():
     layer, cos = model.model.layers[0], torch.randn(1, 1, 7, 32)
     mask = torch.zeros(1, 1, 7, 32)
     assert torch.equal(torch.fx.symbolic_trace(layer)(x, cos, cos, positions, mask), layer(x, cos, cos, positions, mask))
+
+
+def test_script_of_norm_layer_and_decoder():
+    model, tokens, positions = _dense_model()
+    want = model(tokens, positions)
+    x, cos, mask = torch.randn(1, 7, 64), torch.randn(1, 1, 7, 32), torch.zeros(1, 1, 7, 32)
+    normed, layered = model.model.norm(x), model.model.layers[0](x, cos, cos, positions, mask)
+    assert torch.equal(torch.jit.script(model.model.norm)(x), normed)
+    assert torch.equal(torch.jit.script(model.model.layers[0])(x, cos, cos, positions, mask), layered)
+    scripted = torch.jit.script(model)
+    for _ in range(3):   # the profiling executor specialises after the first calls
+        assert torch.allclose(scripted(tokens, positions), want, rtol=1e-5, atol=1e-6)
