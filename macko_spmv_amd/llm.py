@@ -211,12 +211,14 @@ class Block(nn.Module):
         """Whether several tokens go through the layer by way of forward_fused: inference in fp16 on the
         GPU, all seven projections compressed, nothing hooked to the layer or the modules passed over."""
         att, mlp = self.self_attn, self.mlp
+        if type(att) is not Attention or type(mlp) is not MLP:
+            return False
         projections = (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
         norms = (self.input_layernorm, self.post_attention_layernorm)
         return (all(type(p) is MackoLinear for p in projections)
                 and isinstance(x, torch.Tensor) and x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
                 and att.n_heads * att.head_dim == x.shape[2] and projections[4].c_3 % 8 == 0 and projections[4].c_3 >= 64
-                and all(type(n) is RMSNorm for n in norms) and type(att) is Attention and type(mlp) is MLP
+                and all(type(n) is RMSNorm for n in norms)
                 and not _has_any_global_hook()
                 and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m)
                             for m in (self, att, mlp, *projections, *norms))

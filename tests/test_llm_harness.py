@@ -294,3 +294,26 @@ def test_concat_compressed_against_the_oracle_on_the_host():
         assert a.dtype == b.dtype and a.shape == b.shape
         assert torch.equal(a.view(torch.int16) if a.dtype == torch.float16 else a,
                            b.view(torch.int16) if b.dtype == torch.float16 else b)
+
+
+def test_layer_with_other_modules_in_the_place_of_its_own():
+    # an attention or MLP of another class need not have projections of these names
+    torch.manual_seed(0)
+    with torch.no_grad():
+        model = llm.LlamaDecoder(100, 64, 128, 2, 2, 32)
+        tokens, positions = torch.randint(0, 100, (1, 7)), torch.arange(7)
+        want = model(tokens, positions)
+        layer = model.model.layers[0]
+
+        class Wrapped(torch.nn.Module):
+            def __init__(self, inner):
+                super().__init__()
+                self.inner = inner
+
+            def forward(self, *args):
+                return self.inner(*args)
+
+        layer.mlp = Wrapped(layer.mlp)
+        assert torch.equal(model(tokens, positions), want)
+        layer.self_attn = Wrapped(layer.self_attn)
+        assert torch.equal(model(tokens, positions), want)
