@@ -218,7 +218,7 @@ class Block(nn.Module):
         return (all(type(p) is MackoLinear for p in projections)
                 and isinstance(x, torch.Tensor) and x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
                 and att.n_heads * att.head_dim == x.shape[2] and projections[4].c_3 % 8 == 0 and projections[4].c_3 >= 64
-                and all(type(n) is RMSNorm for n in norms)
+                and all(type(n) is RMSNorm and n.weight.is_contiguous() and n.weight.shape == x.shape[2:] for n in norms)
                 and not _has_any_global_hook()
                 and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m)
                             for m in (self, att, mlp, *projections, *norms))

@@ -56,3 +56,21 @@ def test_compiled_decoder_gives_what_the_eager_one_gives(tokens):
         got = torch.compile(model, fullgraph=True, backend="aot_eager")(prompt, pos)
         assert torch.equal(got, want)
         assert all(torch.equal(layer.self_attn.k_cache, kept) for layer, kept in zip(model.model.layers, caches))
+
+
+def _small_model(**change):
+    return llm.build_model(0.4, sparse=True, **{**dict(n_layers=1, dim=256, hidden=704, n_heads=2, vocab=1000, max_len=48), **change})[0]
+
+
+@pytest.mark.parametrize("make", [lambda w: w[:1].expand(256), lambda w: w[::2]])
+def test_layer_takes_norm_weights_of_any_stride(make):
+    with torch.no_grad():
+        model = _small_model()
+        prompt, pos = torch.randint(0, 1000, (1, 19), device="cuda"), torch.arange(19, device="cuda")
+        norm = model.model.layers[0].post_attention_layernorm
+        weight = make(1 + 0.1 * torch.randn(512, device="cuda").half())
+        norm.weight = torch.nn.Parameter(weight.contiguous(), requires_grad=False)
+        want = model(prompt, pos).float()
+        norm.weight = torch.nn.Parameter(weight, requires_grad=False)
+        # the same weights, through the modules: fp16 activations rounded in other places
+        assert torch.allclose(model(prompt, pos).float(), want, rtol=2e-2, atol=2e-2)

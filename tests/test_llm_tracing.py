@@ -87,3 +87,23 @@ def test_script_of_norm_layer_and_decoder():
     scripted = torch.jit.script(model)
     for _ in range(3):   # the profiling executor specialises after the first calls
         assert torch.allclose(scripted(tokens, positions), want, rtol=1e-5, atol=1e-6)
+
+
+def _takes_fused(change):
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    layer = _fake_model(mode).model.layers[0]
+    with mode, torch.no_grad(), torch.device("cuda"):
+        change(layer)
+        return layer.takes_fused(torch.empty((1, 20, 256), dtype=torch.float16))
+
+
+def test_layer_with_norm_weights_of_any_stride_goes_through_its_modules():
+    def norm_weight(make):
+        def change(layer):
+            weight = make(torch.ones(512, dtype=torch.float16, device="cuda"))
+            layer.post_attention_layernorm.weight = torch.nn.Parameter(weight, requires_grad=False)
+        return change
+
+    assert _takes_fused(lambda layer: None) and _takes_fused(norm_weight(lambda w: w[:256]))
+    for make in (lambda w: w[:1].expand(256), lambda w: w[::2], lambda w: w[:1], lambda w: w[:256][None]):
+        assert not _takes_fused(norm_weight(make))
