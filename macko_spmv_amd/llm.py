@@ -215,9 +215,15 @@ class Block(nn.Module):
             return False
         projections = (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
         norms = (self.input_layernorm, self.post_attention_layernorm)
-        return (all(type(p) is MackoLinear for p in projections)
-                and isinstance(x, torch.Tensor) and x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
-                and att.n_heads * att.head_dim == x.shape[2] and projections[4].c_3 % 8 == 0 and projections[4].c_3 >= 64
+        if not all(type(p) is MackoLinear for p in projections) or not isinstance(x, torch.Tensor):
+            return False
+        # rows and cols of a projection that fit the layer; one that does not is the modules' to refuse (the packed
+        # vectors are whole 64-column blocks, whose size does not tell)
+        dim, hidden = x.shape[2], projections[4].c_3
+        fitting = [(dim, dim)] * 4 + [(hidden, dim)] * 2 + [(dim, hidden)]
+        return (x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
+                and att.n_heads * att.head_dim == dim and hidden % 8 == 0 and hidden >= 64
+                and all((p.c_3, p.c_4) == fit for p, fit in zip(projections, fitting))
                 and all(type(n) is RMSNorm and n.weight.is_contiguous() and n.weight.shape == x.shape[2:] for n in norms)
                 and not _has_any_global_hook()
                 and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m)

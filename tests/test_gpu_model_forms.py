@@ -4,6 +4,7 @@ projections that do not fit, infinite scores."""
 import pytest
 import torch
 
+import macko_spmv_amd as mk
 from macko_spmv_amd import llm
 
 pytestmark = pytest.mark.gpu
@@ -74,3 +75,13 @@ def test_layer_takes_norm_weights_of_any_stride(make):
         norm.weight = torch.nn.Parameter(weight, requires_grad=False)
         # the same weights, through the modules: fp16 activations rounded in other places
         assert torch.allclose(model(prompt, pos).float(), want, rtol=2e-2, atol=2e-2)
+
+
+def test_layer_refuses_a_projection_of_fewer_columns():
+    with torch.no_grad():
+        model = _small_model()
+        weight = torch.randn(256, 250, device="cuda").half()
+        model.model.layers[0].self_attn.q_proj = llm.MackoLinear(*mk.compress(weight))
+        prompt, pos = torch.randint(0, 1000, (1, 19), device="cuda"), torch.arange(19, device="cuda")
+        with pytest.raises(RuntimeError):
+            model(prompt, pos)

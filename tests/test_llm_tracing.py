@@ -107,3 +107,16 @@ def test_layer_with_norm_weights_of_any_stride_goes_through_its_modules():
     assert _takes_fused(lambda layer: None) and _takes_fused(norm_weight(lambda w: w[:256]))
     for make in (lambda w: w[:1].expand(256), lambda w: w[::2], lambda w: w[:1], lambda w: w[:256][None]):
         assert not _takes_fused(norm_weight(make))
+
+
+@pytest.mark.parametrize("parent,name,rows,cols", [("self_attn", "q_proj", 256, 250), ("self_attn", "k_proj", 128, 256),
+                                                   ("self_attn", "o_proj", 256, 251), ("mlp", "up_proj", 704, 255),
+                                                   ("mlp", "up_proj", 696, 256), ("mlp", "down_proj", 256, 700)])
+def test_layer_with_a_projection_that_does_not_fit_goes_through_its_modules(parent, name, rows, cols):
+    """... which refuse it: a matrix of fewer columns must not be multiplied with the first of them."""
+    def change(layer):
+        n = rows * cols // 16 * 8
+        setattr(getattr(layer, parent), name, llm.MackoLinear(
+            torch.empty(n, dtype=torch.float16), torch.empty(n // 2, dtype=torch.uint8), torch.empty(rows + 1, dtype=torch.int32), rows, cols))
+
+    assert not _takes_fused(change)
