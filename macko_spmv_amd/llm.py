@@ -482,7 +482,7 @@ class DecodeEngine:
                 qkv = macko_spmv.multiply_rmsnorm(L["qkv"], x, L["norm1"], self.eps)
             else:
                 qkv = self._matvec(L["qkv"], ops.decode_rmsnorm(x, L["norm1"], self.eps))
-            if sparse and self.head_dim in (64, 128):
+            if sparse and isinstance(L["o"], tuple) and self.head_dim in (64, 128):
                 parts = ops.decode_rope_attention_parts(qkv[:H], qkv[H:2 * H], qkv[2 * H:], self.cos, self.sin, position,
                                                         L["k_cache"], L["v_cache"], self.scale)
                 macko_spmv.multiply_attention_axpby(L["o"], parts, self.head_dim, x, 1.0, 1.0)

@@ -317,3 +317,22 @@ def test_layer_with_other_modules_in_the_place_of_its_own():
         assert torch.equal(model(tokens, positions), want)
         layer.self_attn = Wrapped(layer.self_attn)
         assert torch.equal(model(tokens, positions), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_engine_with_a_dense_o_projection_among_compressed_ones(head_dim):
+    with torch.no_grad():
+        cfg = dict(n_layers=2, dim=4 * head_dim, hidden=688, n_heads=4, vocab=1000, max_len=40)
+        sparse, _ = llm.build_model(0.4, sparse=True, **cfg)
+        dense, _ = llm.build_model(0.4, sparse=False, **cfg)   # the same weights
+        for layer, other in zip(sparse.model.layers, dense.model.layers):
+            layer.self_attn.o_proj = other.self_attn.o_proj
+        engine = llm.DecodeEngine(sparse)
+        assert not isinstance(engine.layers[0]["o"], tuple) and isinstance(engine.layers[0]["qkv"], tuple)
+        tokens = torch.randint(0, 1000, (1, 9), device="cuda")
+        for i in range(9):
+            got = engine.step(tokens[0, i:i + 1], torch.tensor([i], device="cuda")).float()
+            want = dense(tokens[:, i:i + 1], torch.tensor([i], device="cuda"))[0, 0].float()
+            # as the engine's other tests: fp16 activations rounded in other places
+            assert torch.allclose(got, want, rtol=2e-2, atol=2e-2), i
