@@ -60,6 +60,26 @@ def test_decoder_compiles_as_one_graph():
         assert _operators(norm, torch.empty((3, 256), dtype=torch.float16, requires_grad=True)) == []
 
 
+def test_one_graph_takes_prompts_of_any_length():
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    model, graphs = _fake_model(mode), []
+
+    def backend(graph, example_inputs):
+        graphs.append(graph)
+        return graph.forward
+
+    torch._dynamo.reset()
+    with mode, torch.no_grad(), torch.device("cuda"):
+        tokens, positions = torch.empty((1, 20), dtype=torch.long), torch.empty((20,), dtype=torch.long)
+        torch._dynamo.mark_dynamic(tokens, 1)   # an error if the length becomes part of the graph
+        torch._dynamo.mark_dynamic(positions, 0)
+        compiled = torch.compile(model, fullgraph=True, backend=backend)
+        compiled(tokens, positions)
+        for length in (2, 16, 33):
+            assert compiled(torch.empty((1, length), dtype=torch.long), torch.empty((length,), dtype=torch.long)).shape == (1, length, 100)
+    assert len(graphs) == 1
+
+
 def _dense_model():
     torch.manual_seed(0)
     model = llm.LlamaDecoder(100, 64, 128, 2, 2, 32).requires_grad_(False)
