@@ -120,13 +120,21 @@ def load_compressed_linears(model, compressed_sd):
 
 # ---- a minimal Llama-architecture decoder (batch 1) ------------------------------------------------
 
+def _recording():
+    """Whether the call is being recorded into a graph to keep (torch.jit.trace, make_fx, torch.export): that graph
+    may be given gradients, another device or another type, so it gets torch's operators."""
+    if torch.jit.is_tracing() or torch.compiler._is_exporting_flag:  # is_exporting() is True in every compiled call
+        return True
+    return not torch.compiler.is_compiling() and torch._C._get_dispatch_mode(torch._C._TorchDispatchModeKey.PROXY) is not None
+
+
 def _inference_half(*tensors):
     """fp16 tensors on the GPU through which no gradient, tangent or batching rule has to flow: what the
     hand-written kernels between the projections take.  The operators copy what is not 16-byte aligned; eagerly
     such views keep to torch's operators (Dynamo cannot trace storage_offset(); and what it makes of the
     interpreter stack is never None, but has the right type)."""
     transformed = isinstance(torch._C._functorch.peek_interpreter_stack(), torch._C._functorch.CInterpreter)
-    if transformed or torch.autograd.forward_ad._current_level >= 0:
+    if transformed or torch.autograd.forward_ad._current_level >= 0 or _recording():
         return False
     grad, tracing = torch.is_grad_enabled(), torch.compiler.is_compiling()
     # (a torch.fx proxy is no tensor and has no answers)

@@ -109,6 +109,27 @@ def test_script_of_norm_layer_and_decoder():
         assert torch.allclose(scripted(tokens, positions), want, rtol=1e-5, atol=1e-6)
 
 
+def test_recorded_graphs_get_torchs_operators():
+    """... which have a gradient and run on any device, whatever the call that was recorded ran on."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    model = _fake_model(mode)
+    norm = model.model.norm
+    with mode, torch.no_grad(), torch.device("cuda"):
+        x = torch.empty((3, 256), dtype=torch.float16)
+        exported = torch.export.export(norm, (x,), strict=True).graph
+    with torch.no_grad():
+        recorded = make_fx(norm)(x).graph
+    for graph in (exported, recorded):
+        assert not [n for n in graph.nodes if "macko_spmv" in str(n.target)]
+    chosen = []
+    with torch.no_grad():
+        torch.jit.trace(lambda a: (chosen.append(llm._inference_half(x)), a + 1)[1], torch.zeros(1), check_trace=False)
+        chosen.append(llm._inference_half(x))
+    assert chosen == [False, True]
+
+
 def _takes_fused(change):
     mode = FakeTensorMode(allow_non_fake_inputs=True)
     layer = _fake_model(mode).model.layers[0]
