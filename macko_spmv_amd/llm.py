@@ -23,6 +23,7 @@ from collections import OrderedDict
 
 import torch
 from torch import nn
+from torch._subclasses.fake_tensor import FakeTensor
 from torch.nn.modules.module import _has_any_global_hook
 
 import macko_spmv_amd as macko_spmv
@@ -120,6 +121,9 @@ def load_compressed_linears(model, compressed_sd):
 
 # ---- a minimal Llama-architecture decoder (batch 1) ------------------------------------------------
 
+_PLAIN_TENSORS = (torch.Tensor, nn.Parameter, FakeTensor)
+
+
 def _recording():
     """Whether the call is being recorded into a graph to keep (torch.jit.trace, make_fx, torch.export): that graph
     may be given gradients, another device or another type, so it gets torch's operators."""
@@ -137,8 +141,9 @@ def _inference_half(*tensors):
     if transformed or torch.autograd.forward_ad._current_level >= 0 or _recording():
         return False
     grad, tracing = torch.is_grad_enabled(), torch.compiler.is_compiling()
-    # (a torch.fx proxy is no tensor and has no answers)
-    return all(isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad)
+    # a torch.fx proxy is no tensor and has no answers; a subclass (DTensor, ...) has its own idea of torch's operators
+    # and none of these
+    return all(type(t) in _PLAIN_TENSORS and t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad)
                and (tracing or t.storage_offset() % 8 == 0) for t in tensors)
 
 

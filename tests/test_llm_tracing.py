@@ -130,6 +130,27 @@ def test_recorded_graphs_get_torchs_operators():
     assert chosen == [False, True]
 
 
+class _Recorder(torch.Tensor):
+    """A subclass with a meaning of its own for torch's operators, as a distributed or a quantised tensor has."""
+    seen = []
+
+    @staticmethod
+    def __new__(cls):
+        return torch.Tensor._make_wrapper_subclass(cls, (3, 256), dtype=torch.float16, device="cuda")
+
+    @classmethod
+    def __torch_dispatch__(cls, function, types, args, kwargs=None):
+        cls.seen.append(str(function).split(".")[0])
+        return cls()
+
+
+def test_norm_of_a_tensor_subclass_goes_through_torchs_operators():
+    norm = _fake_model(FakeTensorMode(allow_non_fake_inputs=True)).model.norm
+    with torch.no_grad():
+        norm(_Recorder())
+    assert _Recorder.seen and set(_Recorder.seen) == {"aten"}
+
+
 def _takes_fused(change):
     mode = FakeTensorMode(allow_non_fake_inputs=True)
     layer = _fake_model(mode).model.layers[0]
