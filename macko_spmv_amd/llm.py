@@ -133,7 +133,7 @@ def _recording():
 
 
 def _inference_half(*tensors):
-    """fp16 tensors on the GPU through which no gradient, tangent or batching rule has to flow: what the
+    """fp16 tensors on one GPU through which no gradient, tangent or batching rule has to flow: what the
     hand-written kernels between the projections take.  The operators copy what is not 16-byte aligned; eagerly
     such views keep to torch's operators (Dynamo cannot trace storage_offset(); and what it makes of the
     interpreter stack is never None, but has the right type)."""
@@ -143,8 +143,8 @@ def _inference_half(*tensors):
     grad, tracing = torch.is_grad_enabled(), torch.compiler.is_compiling()
     # a torch.fx proxy is no tensor and has no answers; a subclass (DTensor, ...) has its own idea of torch's operators
     # and none of these
-    return all(type(t) in _PLAIN_TENSORS and t.is_cuda and t.dtype == torch.float16 and not (grad and t.requires_grad)
-               and (tracing or t.storage_offset() % 8 == 0) for t in tensors)
+    return all(type(t) in _PLAIN_TENSORS and t.is_cuda and t.device == tensors[0].device
+               and t.dtype == torch.float16 and not (grad and t.requires_grad) and (tracing or t.storage_offset() % 8 == 0) for t in tensors)
 
 
 class RMSNorm(nn.Module):

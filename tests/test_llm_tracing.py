@@ -151,6 +151,14 @@ def test_norm_of_a_tensor_subclass_goes_through_torchs_operators():
     assert _Recorder.seen and set(_Recorder.seen) == {"aten"}
 
 
+def test_operands_of_several_gpus_are_refused():
+    """... by torch's operators; a kernel would read the other GPU's memory."""
+    norm = _fake_model(FakeTensorMode(allow_non_fake_inputs=True)).model.norm
+    with norm.weight.fake_mode, torch.no_grad():
+        with pytest.raises(RuntimeError):
+            norm(torch.empty((3, 256), dtype=torch.float16, device="cuda:1"))
+
+
 def _takes_fused(change):
     mode = FakeTensorMode(allow_non_fake_inputs=True)
     layer = _fake_model(mode).model.layers[0]
