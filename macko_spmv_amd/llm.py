@@ -228,7 +228,7 @@ class Block(nn.Module):
             return False
         projections = (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
         norms = (self.input_layernorm, self.post_attention_layernorm)
-        if not all(type(p) is MackoLinear for p in projections) or not isinstance(x, torch.Tensor):
+        if not all(type(p) is MackoLinear for p in projections) or not isinstance(x, torch.Tensor) or x.dim() != 3:
             return False
         # rows and cols of a projection that fit the layer; one that does not is the modules' to refuse (the packed
         # vectors are whole 64-column blocks, whose size does not tell)
@@ -241,6 +241,7 @@ class Block(nn.Module):
                 and not _has_any_global_hook()
                 and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m)
                             for m in (self, att, mlp, *projections, *norms))
+                and att.k_cache.shape == att.v_cache.shape == (1, att.n_heads, att.max_len, att.head_dim)
                 and att.k_cache.is_contiguous() and att.v_cache.is_contiguous()
                 and _inference_half(x, *(n.weight for n in norms), att.k_cache, att.v_cache))
 
@@ -314,7 +315,10 @@ class LlamaDecoder(nn.Module):
     def _run_layers(self, x, cos, sin, positions):
         mask = None  # only made for a layer that needs one
         for layer in self.model.layers:
-            if type(layer) is Block and layer.takes_fused(x):
+            # positions that do not fit the tokens or a cache that does not fit the mask are the modules' to refuse
+            if (type(layer) is Block and layer.takes_fused(x) and layer.self_attn.max_len == self.max_len
+                    and positions.shape == x.shape[1:2] and positions.dtype == torch.int64
+                    and positions.device == cos.device == x.device):
                 x = layer(x, cos, sin, positions, _FUSED_CAUSAL)
                 continue
             if mask is None:

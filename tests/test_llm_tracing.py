@@ -130,6 +130,26 @@ def test_recorded_graphs_get_torchs_operators():
     assert chosen == [False, True]
 
 
+@pytest.mark.parametrize("tokens,positions", [((1, 20), (1, 20)), ((1, 20), (40,)), ((20,), (20,)), ((1, 20), (5, 4))])
+def test_positions_that_do_not_fit_the_tokens_are_refused(tokens, positions):
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    model = _fake_model(mode)
+    with mode, torch.no_grad(), torch.device("cuda"):
+        with pytest.raises(RuntimeError):
+            model(torch.empty(tokens, dtype=torch.long), torch.empty(positions, dtype=torch.long))
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 48, 128), (1, 2, 64, 128), (1, 4, 48, 64)])
+def test_caches_that_do_not_fit_are_refused(shape):
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    model = _fake_model(mode)
+    with mode, torch.no_grad(), torch.device("cuda"):
+        attention = model.model.layers[1].self_attn
+        attention.k_cache, attention.v_cache = torch.empty(shape, dtype=torch.float16), torch.empty(shape, dtype=torch.float16)
+        with pytest.raises(RuntimeError):
+            model(torch.empty((1, 20), dtype=torch.long), torch.empty((20,), dtype=torch.long))
+
+
 class _Recorder(torch.Tensor):
     """A subclass with a meaning of its own for torch's operators, as a distributed or a quantised tensor has."""
     seen = []
