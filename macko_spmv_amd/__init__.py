@@ -266,9 +266,10 @@ def multiply(compressed_M, V):
 
 
 def multiply_batched(compressed_M, X):
-    """Y[b] = M @ X[b] for X of shape (batch, cols) -> (batch, rows).  The matrix is decoded once per
-    64 or 128 vectors and multiplied on the matrix cores.  Upstream has only the single-vector operator and maps it over
-    the batch dimension (python_scripts/util_run_pruned_llm.py:112-118)."""
+    """Y[b] = M @ X[b] for X of shape (batch, cols) -> (batch, rows).  From a few vectors on mostly on the
+    matrix cores, with the matrix decoded once per 64 or 128 vectors.  Upstream has only the
+    single-vector operator and maps it over the batch dimension
+    (python_scripts/util_run_pruned_llm.py:112-118)."""
     assert compressed_M[0].is_cuda and X.is_cuda
     assert X.dim() == 2 and X.is_contiguous()
     return torch.ops.macko_spmv.multiply_batched.default(*compressed_M[:5], X)

@@ -112,7 +112,7 @@ __device__ __forceinline__ void stage_function(unsigned char *lds, const SpmvArg
     if (tid < kLdsBack / 2) dst[a.cols + tid] = 0;
 }
 
-// NB = vectors multiplied per launch (1, 2 or 4).  With NB > 1 the NB copies of x are interleaved in
+// NB = vectors multiplied per launch (1, 2, 4 or 8).  With NB > 1 the NB copies of x are interleaved in
 // LDS (element c of vector b at half-word c * NB + b), so one LDS read per stored entry fetches the
 // operand of every vector, and a row ends with NB sums.  NB > 1 exists for fp16 values, x in LDS,
 // plain product only.
@@ -139,7 +139,7 @@ template <int BLOCK, int D, bool X_LDS, bool AXPBY, int VB, int NB, int XF, bool
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_num_vgpr(kCompilerVgprs)))
 spmv_stream_kernel(const SpmvArgs a)
 {
-    static_assert(NB == 1 || (NB <= 4 && X_LDS && !AXPBY && VB == 2), "batched variant: fp16, x in LDS, plain product");
+    static_assert(NB == 1 || (NB <= 8 && X_LDS && !AXPBY && VB == 2), "batched variant: fp16, x in LDS, plain product");
     static_assert(XF == 0 || (NB == 1 && X_LDS && VB == 2), "fused staging: fp16, one vector, x in LDS");
     static_assert(!ROWS || (X_LDS && NB == 1 && XF == 0), "all rows of a tile in one pass: one vector, x in LDS");
     static_assert(!PLAN || (X_LDS && NB == 1 && XF == 0), "prepared cuts: one vector, x in LDS");
@@ -148,7 +148,7 @@ spmv_stream_kernel(const SpmvArgs a)
     if constexpr (XF == 3) MACKO_RESERVE_FIXED_REGISTERS(MACKO_STREAM_OPERAND_REGISTERS);
     static_assert(BLOCK == kStreamThreads, "stage_function");
     constexpr int WAVES = BLOCK / kWave;
-    constexpr int kBatchShift = NB == 4 ? 2 : (NB == 2 ? 1 : 0);
+    constexpr int kBatchShift = NB == 8 ? 3 : (NB == 4 ? 2 : (NB == 2 ? 1 : 0));
     constexpr int kTileLoads = 2 * D;  // tracked loads per full ring
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -480,6 +480,7 @@ spmv_stream_kernel(const SpmvArgs a)
     typedef __attribute__((address_space(3))) const uint16_t *lds_u16_ptr;
     typedef __attribute__((address_space(3))) const u32 *lds_u32_ptr;
     typedef __attribute__((address_space(3))) const u32x2 *lds_u32x2_ptr;
+    typedef __attribute__((address_space(3))) const u32x4 *lds_u32x4_ptr;
     // LDS byte address of x[0] (x sits kLdsFront bytes, times NB, into this kernel's dynamic LDS)
     const u32 x_addr = (u32)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds + kLdsFront * NB;
     // row_addr: LDS byte address the next entry of the current row would read if its nibble were 0,
@@ -509,10 +510,14 @@ spmv_stream_kernel(const SpmvArgs a)
                 u32 xs[NB / 2 > 0 ? NB / 2 : 1];  // the NB operands, two per word
                 if (NB == 2) {
                     xs[0] = *reinterpret_cast<lds_u32_ptr>(at);
-                } else {
+                } else if (NB == 4) {
                     const u32x2 t = *reinterpret_cast<lds_u32x2_ptr>(at);
                     xs[0] = t.x;
                     xs[1 % (NB / 2)] = t.y;
+                } else {
+                    const u32x4 t = *reinterpret_cast<lds_u32x4_ptr>(at);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) xs[q % (NB / 2)] = t[q];
                 }
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
@@ -1061,8 +1066,8 @@ int plan_waves(int rows, int cols, long long padded, long long *n_waves)
     return 0;
 }
 
-// LDS the split kernel keeps behind x at most (16 waves, up to 4 vectors and a flag each)
-constexpr size_t kSplitPieceBytes = 16 * 4 * 5 + 4;
+// LDS the split kernel keeps behind the vectors at most (16 waves, their sums and a flag each)
+constexpr size_t split_piece_bytes(int vectors) { return 16 * 4 * (size_t)(vectors + 1) + 4; }
 
 int check_spmv_args(const void *values, const void *deltas, const int32_t *row_ptr, const void *x, void *y,
                     int32_t rows, int32_t cols, int64_t padded, int value_bytes = 2)
@@ -1245,28 +1250,69 @@ extern "C" int macko_spmv_i8f16_axpby(const void *values, const void *deltas, co
 namespace macko {
 namespace {
 
-// Vectors of the next gather launch: 4, 2 or 1, as many as are left and fit in LDS next to each other.
+// Vectors of the next gather launch: 8, 4, 2 or 1, as many as are left and fit in LDS next to each other.
 int gather_step(int left, int cols, long long padded, const DeviceInfo &info)
 {
     const size_t per_vector = (size_t)kLdsFront + 2 * (size_t)cols + kLdsBack;
-    for (int step = 4; step > 1; step /= 2)
-        if (padded > 0 && left >= step && step * per_vector + kSplitPieceBytes <= (size_t)info.max_lds_bytes) return step;
+    for (int step = 8; step > 1; step /= 2)
+        if (padded > 0 && left >= step && step * per_vector + split_piece_bytes(step) <= (size_t)info.max_lds_bytes) return step;
     return 1;
 }
 
-bool batched_on_tiles(int rows, int cols, long long padded, int batch, long long ldx, const DeviceInfo &info)
+// Estimated us of one gather launch for `n` vectors: start, staging of X (slower where it is not 16-byte aligned),
+// tiles and row ends of a wave, at least the time to read the matrix.  Fitted to the measurements below, for the
+// route chosen more than for the time itself (standard deviation about 9 % from 1024 rows on).
+double gather_us(int n, int rows, int cols, long long padded, bool aligned, const DeviceInfo &info)
 {
-    return spmv_tile_takes(rows, cols, padded, batch, ldx, gather_step(batch, cols, padded, info) == batch ? 1 : 2);
+    const double waves = 16.0 * info.compute_units, tiles = (double)padded / kTile;
+    const bool split = launch_shape(rows, padded, info).split;
+    double per_wave = tiles / waves > 1.0 ? tiles / waves : 1.0;
+    if (!split && tiles / rows > per_wave) per_wave = tiles / rows;  // a row is one wave's
+    const double us = 2.87 + (aligned ? 0.37e-4 : 1.3e-4) * n * cols + (0.54 + 0.067 * n) * per_wave + (0.63 + 0.227 * n) * rows / waves +
+                      (split ? 1.3 + 0.5 * n : 0.0);
+    const double memory = 2.5 + 2.5e-6 * (double)padded / 6.75;
+    return us > memory ? us : memory;
+}
+
+// Which products of several vectors go to the matrix cores.  The kernel there pays for the dense area and for X
+// in every block of 48 rows, the gather kernels for stored entries and again for the next few vectors, so the
+// gather kernels win where there are many rows, few entries and few vectors: the two estimates decide.  Measured
+// (us, gather / matrix cores; 8 vectors are one gather launch, 3 are two): 4096 x 4096 density 0.1, 8 vectors 7.9 / 6.6;
+// 11008 x 4096, 8 vectors, 0.05 13.4 / 15.1, 0.2 16.2 / 15.7, 0.5 21.8 / 16.5; 28672 x 4096, 8 vectors, 0.05 25.8 / 40.7,
+// 0.2 32.6 / 40.6, 0.5 47.0 / 45.8; 28672 x 8192, 0.1, 8 vectors 36.5 / 60.7, 12 61.4 / 64.3, 15 98.0 / 60.1; 8192 x 28672,
+// 3 vectors, 0.1 33.8 / 47.8, 0.3 69.6 / 54.0.  Over 30 shapes of 512 to 49152 rows, densities 0.03 to 0.6 and 3 to 32 vectors
+// (1659 products) the route taken is on average 0.2 % behind the better one, 3 % or more in 40 (at most 22 %).
+// 2 and 4 vectors in one gather launch stay there.  Rows of less than 100 entries do not: their ends are a serial
+// chain in the gather kernels (20000 x 300 at 0.1, 8 vectors: 19.2 / 9.6).
+int batched_on_tiles(bool *tiles, const void *x, int rows, int cols, long long padded, int batch, long long ldx, bool packed,
+                     const DeviceInfo &info)
+{
+    *tiles = false;
+    if (!spmv_tile_takes(rows, cols, padded, batch, ldx)) return 0;
+    if (batch < 8 && gather_step(batch, cols, padded, info) == batch) return 0;
+    *tiles = true;
+    if (padded < 100ll * rows) return 0;
+    const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (ldx & 7) == 0;
+    double tile_us = 0.0, us = 0.0;
+    const int rc = spmv_tile_estimate(rows, cols, padded, batch, packed, &tile_us);
+    if (rc != 0) return rc;
+    for (int left = batch; left > 0 && us < tile_us;) {
+        const int step = gather_step(left, cols, padded, info);
+        us += gather_us(step, rows, cols, padded, aligned, info);
+        left -= step;
+    }
+    *tiles = us >= tile_us;
+    return 0;
 }
 
 }  // namespace
 }  // namespace macko
 
 // Y[b, :] = M X[b, :] for `batch` vectors: X is [batch, ldx] and Y [batch, ldy] row-major fp16
-// (ldx >= cols, ldy >= rows).  Two or four vectors go through the gather kernels in one launch; from
-// there on the matrix cores do it (macko_spmv_tile.hip), decoding the matrix once for 64 or 128
-// vectors.  The upstream package has no batched entry: its LLM runner maps the single-vector operator
-// over the batch dimension (python_scripts/util_run_pruned_llm.py:112-118).
+// (ldx >= cols, ldy >= rows).  Through the gather kernels in launches of up to eight vectors, or on the
+// matrix cores (macko_spmv_tile.hip), which decode the matrix once for 64 or 128.  The upstream
+// package has no batched entry: its LLM runner maps the single-vector operator over the batch
+// dimension (python_scripts/util_run_pruned_llm.py:112-118).
 extern "C" int macko_spmv_f16_batched_workspace(const void *x, int32_t rows, int32_t cols, int64_t padded_entries,
                                                 int32_t batch, int64_t ldx, int64_t *bytes)
 {
@@ -1275,10 +1321,13 @@ extern "C" int macko_spmv_f16_batched_workspace(const void *x, int32_t rows, int
     *bytes = 0;
     if (batch == 0) return 0;
     DeviceInfo info;
-    const int rc = device_info(&info);
+    int rc = device_info(&info);
     if (rc != 0) return rc;
-    if (batched_on_tiles(rows, cols, padded_entries, batch, ldx, info)) *bytes = (int64_t)spmv_tile_workspace(cols, batch, x, ldx);
-    return 0;
+    const size_t wanted = spmv_tile_workspace(cols, batch, x, ldx);
+    bool tiles = false;
+    if (wanted > 0) rc = batched_on_tiles(&tiles, x, rows, cols, padded_entries, batch, ldx, true, info);
+    if (tiles) *bytes = (int64_t)wanted;
+    return rc;
 }
 
 extern "C" int macko_spmv_f16_batched_ws(const void *values, const void *deltas, const int32_t *row_ptr, const void *x,
@@ -1299,12 +1348,18 @@ extern "C" int macko_spmv_f16_batched_ws(const void *values, const void *deltas,
                         (const uint16_t *)x + (size_t)first * (size_t)ldx, (uint16_t *)y + (size_t)first * (size_t)ldy,
                         rows, cols, padded_entries, 1.0f, 0.0f, 0, 0, 0, 0, 0, (int)ldx, (int)ldy};
     };
-    if (batched_on_tiles(rows, cols, padded_entries, batch, ldx, info))
+    const size_t wanted = spmv_tile_workspace(cols, batch, x, ldx);
+    const bool packed = wanted > 0 && workspace != nullptr && (size_t)workspace_bytes >= wanted && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
+    bool tiles = false;
+    rc = batched_on_tiles(&tiles, x, rows, cols, padded_entries, batch, ldx, packed, info);
+    if (rc != 0) return rc;
+    if (tiles)
         return spmv_tile_launch(args_from(0), batch, workspace, (size_t)workspace_bytes, as_stream(stream));
     for (int done = 0; done < batch;) {
         const SpmvArgs a = args_from(done);
         const int step = gather_step(batch - done, cols, padded_entries, info);
         switch (step) {
+        case 8: rc = spmv_dispatch<false, 2, 8>(a, as_stream(stream)); break;
         case 4: rc = spmv_dispatch<false, 2, 4>(a, as_stream(stream)); break;
         case 2: rc = spmv_dispatch<false, 2, 2>(a, as_stream(stream)); break;
         default: rc = spmv_dispatch<false>(a, as_stream(stream)); break;
@@ -1334,7 +1389,7 @@ int check_fused_args(const void *x, const void *x2, int32_t cols, int64_t padded
     DeviceInfo info;
     int rc = device_info(&info);
     if (rc != 0) return rc;
-    if ((size_t)kLdsFront + 2 * (size_t)cols + kLdsBack + 64 + kSplitPieceBytes > (size_t)info.max_lds_bytes) return MACKO_E_INVALID_ARGUMENT;
+    if ((size_t)kLdsFront + 2 * (size_t)cols + kLdsBack + 64 + split_piece_bytes(1) > (size_t)info.max_lds_bytes) return MACKO_E_INVALID_ARGUMENT;
     return 0;
 }
 }  // namespace

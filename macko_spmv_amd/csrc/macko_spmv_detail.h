@@ -309,15 +309,16 @@ __device__ __forceinline__ float pick_lane(const float (&c)[8], int idx, int L)
 
 // The kernel for matrices with few, long rows (macko_spmv_split.hip): workgroups own whole rows and
 // their waves share the workgroup's tiles evenly.  Variant selectors: axpby (y = alpha*Mx + beta*y),
-// value_bytes 2 (fp16) or 1 (int8), n_vectors 1/2/4, fused 0/1/2/3 (see SpmvArgs::x2), x_in_lds.
+// value_bytes 2 (fp16) or 1 (int8), n_vectors 1/2/4/8, fused 0/1/2/3 (see SpmvArgs::x2), x_in_lds.
 // lds_x = bytes of LDS that x takes (0 when x is gathered from memory).  Returns an ABI error code.
 int spmv_split_launch(const spmv_detail::SpmvArgs &a, bool axpby, int value_bytes, int n_vectors, int fused,
                       bool x_in_lds, int grid, size_t lds_x, hipStream_t stream);
 
-// The kernel for several vectors on the matrix cores (macko_spmv_tile.hip): whether a product is its
-// kind, the scratch memory it wants for these vectors (0: none), and the launch (a.ldx, a.ldy set;
-// without workspace it reads X as it is, more slowly).
-bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long ldx, int gather_launches);
+// The kernel for several vectors on the matrix cores (macko_spmv_tile.hip): whether it can do a product,
+// its estimated time in us (`packed`: with X in operand order), the scratch memory it wants for these
+// vectors (0: none), and the launch (a.ldx, a.ldy set; without workspace it reads X as it is, more slowly).
+bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long ldx);
+int spmv_tile_estimate(int rows, int cols, long long padded, int batch, bool packed, double *us);
 size_t spmv_tile_workspace(int cols, int batch, const void *x, long long ldx);
 int spmv_tile_pack(const uint16_t *x, int cols, int batch, long long ldx, void *packed, hipStream_t stream);
 int spmv_tile_launch(const spmv_detail::SpmvArgs &a, int batch, void *workspace, size_t workspace_bytes, hipStream_t stream);

@@ -68,7 +68,7 @@ __device__ __forceinline__ u32x4 look_take()
 }
 
 
-// NB = vectors multiplied per launch (1, 2 or 4).  With NB > 1 the NB copies of x are interleaved in
+// NB = vectors multiplied per launch (1, 2, 4 or 8).  With NB > 1 the NB copies of x are interleaved in
 // LDS (element c of vector b at half-word c * NB + b), so one LDS read per stored entry fetches the
 // operand of every vector, and a row ends with NB sums.  NB > 1 exists for fp16 values, x in LDS,
 // plain product only.
@@ -81,12 +81,12 @@ template <int BLOCK, int D, bool X_LDS, bool AXPBY, int VB, int NB, int XF>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_num_vgpr(kCompilerVgprs)))
 spmv_split_kernel(const SpmvArgs a)
 {
-    static_assert(NB == 1 || (NB <= 4 && X_LDS && !AXPBY && VB == 2), "batched variant: fp16, x in LDS, plain product");
+    static_assert(NB == 1 || (NB <= 8 && X_LDS && !AXPBY && VB == 2), "batched variant: fp16, x in LDS, plain product");
     static_assert(XF == 0 || (NB == 1 && X_LDS && VB == 2), "fused staging: fp16, one vector, x in LDS");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     MACKO_RESERVE_FIXED_REGISTERS(MACKO_SPLIT_FIXED_REGISTERS);
     constexpr int WAVES = BLOCK / kWave;
-    constexpr int kBatchShift = NB == 4 ? 2 : (NB == 2 ? 1 : 0);
+    constexpr int kBatchShift = NB == 8 ? 3 : (NB == 4 ? 2 : (NB == 2 ? 1 : 0));
     constexpr int kTileLoads = 2 * D;  // tracked loads per full ring
     constexpr int kPre = 1;  // ring slots filled before the workgroup's barrier
     constexpr int kNone = 0x7fffffff;
@@ -405,6 +405,7 @@ spmv_split_kernel(const SpmvArgs a)
     typedef __attribute__((address_space(3))) const uint16_t *lds_u16_ptr;
     typedef __attribute__((address_space(3))) const u32 *lds_u32_ptr;
     typedef __attribute__((address_space(3))) const u32x2 *lds_u32x2_ptr;
+    typedef __attribute__((address_space(3))) const u32x4 *lds_u32x4_ptr;
     // LDS byte address of x[0] (x sits kLdsFront bytes, times NB, into this kernel's dynamic LDS)
     const u32 x_addr = (u32)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds + kLdsFront * NB;
     // row_addr: LDS byte address the next entry of the current row would read if its nibble were 0,
@@ -518,10 +519,14 @@ spmv_split_kernel(const SpmvArgs a)
                 u32 xs[NB / 2 > 0 ? NB / 2 : 1];  // the NB operands, two per word
                 if (NB == 2) {
                     xs[0] = *reinterpret_cast<lds_u32_ptr>(at);
-                } else {
+                } else if (NB == 4) {
                     const u32x2 t = *reinterpret_cast<lds_u32x2_ptr>(at);
                     xs[0] = t.x;
                     xs[1 % (NB / 2)] = t.y;
+                } else {
+                    const u32x4 t = *reinterpret_cast<lds_u32x4_ptr>(at);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) xs[q % (NB / 2)] = t[q];
                 }
                 const bool valid = !CHECKED || (k >= kmin && k < kmax);
 #pragma unroll
@@ -805,6 +810,7 @@ int spmv_split_launch(const spmv_detail::SpmvArgs &a, bool axpby, int value_byte
     if (fused != 0) return MACKO_E_INVALID_ARGUMENT;
     if (n_vectors > 1) {
         if (axpby || value_bytes != 2 || !x_in_lds) return MACKO_E_INVALID_ARGUMENT;
+        if (n_vectors == 8) return launch_split<2, true, false, 2, 8, 0>(a, grid, lds_x, stream);
         if (n_vectors == 4) return launch_split<2, true, false, 2, 4, 0>(a, grid, lds_x, stream);
         if (n_vectors == 2) return launch_split<2, true, false, 2, 2, 0>(a, grid, lds_x, stream);
         return MACKO_E_INVALID_ARGUMENT;

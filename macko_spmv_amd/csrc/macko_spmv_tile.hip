@@ -525,8 +525,8 @@ int launch_tile_shape(TileArgs a, const TileShape &s, int max_lds, hipStream_t s
 
 // Estimated cycles of a launch: what one workgroup's chunk asks of the vector units (about 60
 // instructions per row and 512 entries), of the path from L2 (X: 48 bytes a cycle from operand order,
-// 14 from X itself), of LDS and of the matrix cores overlaps to about 0.6 of the sum (measured: 0.58
-// to 0.63 over the shapes below), behind a start and an end of about 9000 cycles.
+// 14 from X itself with 16 vectors, and with one vector half the time: fewer cache lines a load), of LDS
+// and of the matrix cores overlaps to about 0.6 of the sum, behind a start and an end of about 9000 cycles.
 double tile_cost(const TileShape &s, long long units, int cols, double density, int batch, bool packed, int compute_units)
 {
     const int groups = 1 << s.group_shift;
@@ -537,7 +537,7 @@ double tile_cost(const TileShape &s, long long units, int cols, double density, 
     const double passes = density * s.chunk / 504.0 > 1.0 ? density * s.chunk / 504.0 : 1.0;
     const double chunk = s.chunk;
     const double valu = rows * passes * 60.0;
-    const double x = vectors * chunk * 2.0 / (packed ? 48.0 : 14.0);
+    const double x = vectors * chunk * 2.0 * (packed ? 1.0 / 48.0 : (0.5 + (batch < 16 ? batch / 32.0 : 0.5)) / 14.0);
     const double lds = rows * passes * 53.0 + rows * chunk / 64.0 + groups * 16.0 * s.row_tiles * chunk / 64.0;
     const double mfma = s.row_tiles * (vectors / 16) * chunk / 8.0;
     const int n_chunks = (cols + s.chunk - 1) / s.chunk;
@@ -549,7 +549,8 @@ double tile_cost(const TileShape &s, long long units, int cols, double density, 
 // decode a row once instead of twice, blocks of 64 read half as much of X per workgroup, which wins
 // where there are few rows per compute unit (4096 x 4096, density 0.5, 128 vectors: 18.3 us against
 // 20.4; 11008 x 4096: 39.4 against 28.4).
-bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info)
+bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info,
+                       double *cycles = nullptr)
 {
     const long long units = ((long long)rows + kRowUnit - 1) / kRowUnit;
     const double density = (double)padded / ((double)rows * (double)cols);
@@ -592,22 +593,32 @@ bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, in
             if (s.row_tiles == 1) break;  // smaller blocks only read X more often
         }
     }
+    if (cycles != nullptr) *cycles = least;
     return found;
 }
 
 }  // namespace
 
-// Which products of several vectors this kernel does: those for which the gather kernels would need
-// more than one launch (`gather_launches`), and from 8 vectors on all.  Measured against the gather kernels
-// (us, gather / here): 4096 x 4096 density 0.5, 2 vectors 6.7 / 9.1, 3: 12.5 / 8.8, 4: 7.4 / 9.1, 6: 13.7 / 8.9,
-// 8: 10.8 / 8.9, 32: 42.3 / 11.5; density 0.1, 4: 5.2 / 6.1, 8: 7.7 / 6.5; 11008 x 4096 density 0.1, the least
-// favourable of all, 4: 9.7 / 15.4, 8: 13.7 / 15.6, 12: 23.1 / 15.6.
-bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long ldx, int gather_launches)
+// Whether this kernel can do a product of several vectors (which it should do: batched_on_tiles, macko_spmv.hip).
+bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long ldx)
 {
     if (rows == 0 || padded == 0 || cols < 64) return false;
-    if (gather_launches < 2 && batch < 8) return false;
     // offsets into X and into its operand-order copy are 32-bit
     return (long long)batch * ldx * 2 < (1ll << 32) && (long long)packed_bytes(cols, batch) < (1ll << 32);
+}
+
+// The time by the cost above, at 2.4 GHz, and the packing launch.  Right to about 10 % on either side where it
+// decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1: 24.4, 21).
+int spmv_tile_estimate(int rows, int cols, long long padded, int batch, bool packed, double *us)
+{
+    DeviceInfo info;
+    const int rc = device_info(&info);
+    if (rc != 0) return rc;
+    TileShape shape;
+    double cycles = 0.0;
+    if (!choose_tile_shape(&shape, rows, cols, padded, batch, packed, info, &cycles)) return MACKO_E_INVALID_ARGUMENT;
+    *us = cycles * (1.06 / 2400.0) + (packed ? 2.9 : 0.0);
+    return 0;
 }
 
 size_t spmv_tile_workspace(int cols, int batch, const void *x, long long ldx)
