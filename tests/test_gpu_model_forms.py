@@ -85,3 +85,55 @@ def test_layer_refuses_a_projection_of_fewer_columns():
         prompt, pos = torch.randint(0, 1000, (1, 19), device="cuda"), torch.arange(19, device="cuda")
         with pytest.raises(RuntimeError):
             model(prompt, pos)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_attention_of_infinite_and_nan_operands(head_dim):
+    """As a softmax in torch has it: scores of -inf weigh nothing, and everything where nothing else is left; +inf, NaN
+    and what a weight of zero meets in the values become NaN."""
+    heads, tokens, max_len = 5, 40, 64
+    g = torch.Generator(device="cuda").manual_seed(head_dim)
+    q, kc, vc = (torch.randn(shape, device="cuda", generator=g).half().abs_() for shape in
+                 ((tokens, heads * head_dim), (heads, max_len, head_dim), (heads, max_len, head_dim)))
+    inf = float("inf")
+    kc[0, 0], kc[1, :3], kc[2, 5, 7], kc[3, 33, 0] = -inf, -inf, inf, float("nan")
+    vc[4, 20, 3], vc[0, 0, 1], vc[0, tokens:], kc[0, tokens:] = inf, inf, float("nan"), float("nan")
+    pos = torch.arange(tokens, device="cuda")
+    scale = head_dim ** -0.5
+
+    def reference(q, last, h):
+        scores = (q.double()[None] @ kc[h, :last + 1].double().t().contiguous())[0] * scale
+        weights = torch.softmax(scores, -1)
+        return (weights[:, None] * vc[h, :last + 1].double()).sum(0)
+
+    packed = ops.prefill_attention(q, kc, vc, pos, scale)
+    steps, tiles = heads * head_dim // 64, (tokens + 15) // 16
+    rows = packed.view(steps, tiles, 2, 4, 16, 8).permute(1, 4, 0, 3, 2, 5).reshape(tiles * 16, -1)
+    assert not rows[tokens:].any()
+    seen = 0
+    for h in range(heads):
+        for t in range(tokens):
+            want, got = reference(q[t, h * head_dim:(h + 1) * head_dim], t, h), rows[t, h * head_dim:(h + 1) * head_dim].double()
+            # a value of a later token of the same 16 may be met by a weight of zero; torch's masked softmax meets all of them
+            if h == 4 and t < 20:
+                want = torch.where(torch.isinf(vc[4, 20].double()) & torch.isnan(got), got, want)
+            assert torch.equal(want.isnan(), got.isnan()) and torch.equal(want.isinf(), got.isinf()), (h, t)
+            seen += int(want.isnan().any())
+            ok = want.isfinite()
+            # weights and result rounded to fp16
+            assert torch.allclose(got[ok], want[ok], rtol=2.0 ** -9, atol=2.0 ** -20), (h, t)
+    assert seen > 50
+    # one token, in pieces
+    cos, sin = torch.ones(max_len, head_dim // 2, device="cuda"), torch.zeros(max_len, head_dim // 2, device="cuda")
+    for last in (0, 2, 6, 39):
+        k, v = kc[:, last].reshape(-1).contiguous(), vc[:, last].reshape(-1).contiguous()
+        parts = ops.decode_rope_attention_parts(q[last].contiguous(), k, v, cos, sin, pos[last:last + 1], kc.clone(), vc.clone(), scale)
+        whole = ops.decode_rope_attention(q[last].contiguous(), k, v, cos, sin, pos[last:last + 1], kc.clone(), vc.clone(), scale)
+        sums = parts[:heads * 4 * head_dim].view(heads, 4, head_dim)
+        pairs = parts[heads * 4 * head_dim:].view(heads, 4, 2)
+        weight = torch.exp(pairs[..., 0] - pairs[..., 0].max(1, keepdim=True).values)
+        merged = (weight[..., None] * sums).sum(1) / (weight * pairs[..., 1]).sum(1)[:, None]
+        got, want = merged.double(), whole.view(heads, head_dim).double()
+        assert torch.equal(want.isnan(), got.isnan()) and torch.equal(want.isinf(), got.isinf()), last
+        ok = want.isfinite()
+        assert torch.allclose(got[ok], want[ok], rtol=2.0 ** -9, atol=2.0 ** -20), last
