@@ -45,7 +45,6 @@ def test_edges_of_tiles_and_chunks(rows, cols, density, batch):
     rng = np.random.default_rng(rows * 7 + cols + batch)
     dense, X = _case(rng, rows, cols, density, batch)
     c = macko_spmv.compress(torch.from_numpy(dense).cuda())
-    print("case", rows, cols, density, batch, flush=True)
     Y = macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda())
     _check(Y.cpu().numpy(), dense, X, f"{rows}x{cols} d={density} b={batch}")
     # the same again, bit for bit: no sum depends on the order in which waves run

@@ -122,8 +122,8 @@ def test_operators_have_fake_implementations():
 
 
 @pytest.mark.parametrize("dim,hidden,heads,t", [(256, 688, 4, 2), (256, 704, 2, 19), (512, 1376, 8, 64)])
+@torch.no_grad()
 def test_fused_layers_against_the_module_path(dim, hidden, heads, t):
-    torch.set_grad_enabled(False)
     cfg = dict(n_layers=2, dim=dim, hidden=hidden, n_heads=heads, vocab=1000, max_len=80)
     model, _ = llm.build_model(0.4, sparse=True, **cfg)
     prompt, pos = torch.randint(0, 1000, (1, t), device="cuda"), torch.arange(t, device="cuda")
@@ -147,8 +147,84 @@ def test_fused_layers_against_the_module_path(dim, hidden, heads, t):
         assert torch.allclose(kept.float(), layer.self_attn.k_cache.float(), rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("part", ["attention", "mlp", "both"])
+@pytest.mark.parametrize("dim,hidden,heads,t", [(256, 688, 4, 2), (256, 704, 2, 19), (512, 1376, 8, 64)])
+@torch.no_grad()
+def test_what_a_fused_layer_adds(dim, hidden, heads, t, part):
+    """The increment of the layer's two halves, each alone (the other's last projection is zero) and together, against
+    float64; weights large enough for the scores to matter."""
+    g = torch.Generator(device="cuda").manual_seed(dim + t)
+    layer, max_len, hd = llm.Block(dim, hidden, heads, 80).half().cuda(), 80, dim // heads
+    dense = {}
+    for parent, name in llm.PROJECTIONS:
+        rows, cols = getattr(getattr(layer, parent), name).weight.shape
+        w = torch.randn(rows, cols, device="cuda", generator=g).mul_(0.1).half()
+        llm.prune_rows_(w, 0.4)
+        if (part, name) in (("attention", "down_proj"), ("mlp", "o_proj")):
+            w.zero_()
+        dense[name] = w.double()
+        setattr(getattr(layer, parent), name, llm.MackoLinear(*mk.compress(w)))
+    for norm in (layer.input_layernorm, layer.post_attention_layernorm):
+        norm.weight.copy_(1 + 0.3 * torch.randn(dim, device="cuda", generator=g))
+    x = torch.randn(1, t, dim, device="cuda", generator=g).half()
+    pos = torch.arange(t, device="cuda")
+    ang = torch.outer(pos.float(), 1.0 / (10000.0 ** (torch.arange(0, hd, 2, device="cuda").float() / hd)))
+    ang = torch.cat((ang, ang), -1)
+    cos, sin = ang.cos().half(), ang.sin().half()
+    assert layer.takes_fused(x)
+    got = layer(x, cos[None, None], sin[None, None], pos, llm._FUSED_CAUSAL)
+
+    def normed(v, norm):
+        return v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + norm.eps) * norm.weight.double()
+
+    def rope(v):
+        return v * cos.double() + torch.cat((-v[..., hd // 2:], v[..., :hd // 2]), -1) * sin.double()
+
+    x64 = x[0].double()
+    n = normed(x64, layer.input_layernorm)
+    q, k, v = ((n @ dense[name].t().contiguous()).view(t, heads, hd).transpose(0, 1) for name in ("q_proj", "k_proj", "v_proj"))
+    q, k = rope(q), rope(k)
+    out = torch.empty(t, heads, hd, device="cuda", dtype=torch.float64)
+    for h in range(heads):
+        scores = (q[h] @ k[h].t().contiguous()) * hd ** -0.5
+        out[:, h] = scores.masked_fill(pos[None] > pos[:, None], float("-inf")).softmax(-1) @ v[h]
+    after = x64 + out.reshape(t, -1) @ dense["o_proj"].t().contiguous()
+    n = normed(after, layer.post_attention_layernorm)
+    gate, up = n @ dense["gate_proj"].t().contiguous(), n @ dense["up_proj"].t().contiguous()
+    after = after + (gate * torch.sigmoid(gate) * up) @ dense["down_proj"].t().contiguous()
+    # about ten roundings to fp16 on the way (2^-11 at most, 2^-12.8 in the mean, each), those of q and k times
+    # scores of a few units: 2^-8
+    off = lambda a, b: float((a.double() - b).norm() / b.norm())
+    assert off(got[0].double() - x64, after - x64) < 2.0 ** -8
+    assert off(layer.self_attn.k_cache[0, :, :t], k) < 2.0 ** -9 and off(layer.self_attn.v_cache[0, :, :t], v) < 2.0 ** -9
+    assert not layer.self_attn.k_cache[:, :, t:].any() and not layer.self_attn.v_cache[:, :, t:].any()
+
+
+def test_gradients_take_the_modules():
+    layer = llm.Block(256, 704, 2, 48).half().cuda().requires_grad_(False)
+    for parent, name in llm.PROJECTIONS:
+        module = getattr(layer, parent)
+        setattr(module, name, llm.MackoLinear(*mk.compress(getattr(module, name).weight.detach())))
+    x = torch.randn(1, 19, 256, device="cuda").half()
+    norm = layer.input_layernorm
+    with torch.enable_grad():
+        assert layer.takes_fused(x)
+        assert not layer.takes_fused(x.clone().requires_grad_())
+        norm.weight.requires_grad_()
+        assert not layer.takes_fused(x)
+        leaf = x.clone().requires_grad_()
+        norm(leaf).float().pow(2).sum().backward()
+        want = x.double().requires_grad_()
+        (want * torch.rsqrt(want.pow(2).mean(-1, keepdim=True) + norm.eps)).pow(2).sum().backward()
+        assert norm.weight.grad is not None and leaf.grad.shape == x.shape
+        # the squared norm does not depend on x but for eps: what is left is rounding
+        assert leaf.grad.abs().max() < 0.05 and want.grad.abs().max() < 1e-3
+    with torch.no_grad():
+        assert layer.takes_fused(x)
+
+
+@torch.no_grad()
 def test_layer_keeps_a_given_mask_and_strided_positions():
-    torch.set_grad_enabled(False)
     model, _ = llm.build_model(0.4, sparse=True, n_layers=1, dim=256, hidden=704, n_heads=2, vocab=1000, max_len=48)
     layer, t = model.model.layers[0], 20
     pos = torch.arange(t, device="cuda")
