@@ -61,6 +61,7 @@ def _run(cmd, verbose):
         raise RuntimeError("build step failed:\n" + " ".join(cmd) + "\n" + proc.stdout)
     if verbose and proc.stdout.strip():
         print(proc.stdout, flush=True)
+    return proc.stdout
 
 
 _DEVICE_FLAGS = [
@@ -151,20 +152,49 @@ def verify_fixed_registers(verbose=False, extra_flags=()):
     return checked
 
 
+# A kernel whose registers do not suffice spills to scratch memory, and a call that is not inlined takes its stack
+# there: silently, at a multiple of the time (the largest variants of the tile kernel use 127 of 128 registers).
+RESOURCE_REMARKS = "-Rpass-analysis=kernel-resource-usage"
+# keeps a row of k and eight pieces of v per thread in flight and spills 31 registers of them; measured as it is
+KNOWN_TO_SPILL = ("attention_kernelILb1ELi128E",)
+
+
+def check_kernel_resources(remarks):
+    """`remarks`: what the compiler prints with RESOURCE_REMARKS.  Returns the number of kernels; raises if
+    one of them uses scratch memory, spills vector registers or has a dynamic stack (scalar registers spill to
+    lanes of a vector register)."""
+    kernel, checked = None, 0
+    for line in remarks.splitlines():
+        m = re.search(r"remark:\s+([\w ]+?)(?: \[[^\]]*\])?: (\S+)", line)
+        if not m:
+            continue
+        name, value = m.groups()
+        if name == "Function Name":
+            kernel = value
+            checked += 1
+        elif name in ("ScratchSize", "VGPRs Spill") and int(value) != 0 or name == "Dynamic Stack" and value != "False":
+            if any(known in kernel for known in KNOWN_TO_SPILL):
+                continue
+            raise RuntimeError(f"{name}: {value} in {kernel}")
+    if checked == 0:
+        raise RuntimeError("the compiler names no kernels; the resource check is stale")
+    return checked
+
+
 def build_hip(verbose=False):
     """Builds libmacko_hip.so.  The library only reaches its final path once the generated code
-    has passed the fixed-register check: an unchecked library must never be the one that loads."""
+    has passed the fixed-register and the resource check: an unchecked library must never be the one that loads."""
     out, _ = lib_paths()
     verify_fixed_registers(verbose)
     staging = out + ".building"
     cmd = [
         # only what include/*.h declare is exported
-        _hipcc(), *_DEVICE_FLAGS, "-fvisibility=hidden", "-fPIC", "-shared",
+        _hipcc(), *_DEVICE_FLAGS, RESOURCE_REMARKS, "-fvisibility=hidden", "-fPIC", "-shared",
         *[os.path.join(_CSRC, s) for s in HIP_SOURCES],
         "-o", staging,
     ]
     try:
-        _run(cmd, verbose)
+        check_kernel_resources(_run(cmd, False))
         os.replace(staging, out)
     finally:
         if os.path.exists(staging):

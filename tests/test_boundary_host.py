@@ -198,3 +198,17 @@ def test_build_directory_variable_redirects_every_artefact(tmp_path, monkeypatch
     monkeypatch.delenv("MACKO_SPMV_BUILD_DIRECTORY")
     assert os.path.dirname(_build.lib_paths()[0]) == in_tree
     assert _build.is_current()
+
+
+def test_kernel_resource_check_refuses_scratch_and_stacks():
+    from macko_spmv_amd import _build
+
+    def remarks(scratch=0, spilled=0, stack="False"):
+        lines = ["Function Name: _Z6kernelv", "TotalSGPRs: 34", f"ScratchSize [bytes/lane]: {scratch}", f"Dynamic Stack: {stack}",
+                 "Occupancy [waves/SIMD]: 8", "SGPRs Spill: 2", f"VGPRs Spill: {spilled}"]
+        return "\n".join(f"k.hip:84:1: remark:     {line} [-Rpass-analysis=kernel-resource-usage]\n   84 | {{" for line in lines)
+
+    assert _build.check_kernel_resources(remarks() + "\n" + remarks()) == 2
+    for bad in (remarks(scratch=16), remarks(spilled=3), remarks(stack="True"), ""):
+        with pytest.raises(RuntimeError):
+            _build.check_kernel_resources(bad)
