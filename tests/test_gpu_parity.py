@@ -250,8 +250,8 @@ def test_multiply_row_lengths_sorted():
                                                (33, 90000, 0.1), (512, 512, 0.0)])
 def test_multiply_batched(rows, cols, density):
     # every vector of the batch against the dense float64 product and against the single-vector path;
-    # batch sizes cover the 8-, 4-, 2- and 1-vector launches and their combinations, and LDS limits
-    # (20000 columns: four vectors per launch; 70000: two; 90000: one)
+    # batch sizes around both routes: one launch of 2 or 4 vectors, combinations of them and the matrix cores, and
+    # the limits of LDS (20000 columns: four vectors side by side; 70000: two; 90000: one)
     rng = np.random.default_rng(rows + cols)
     dense = helpers.random_sparse(rng, rows, cols, density, scale=0.05)
     if rows > 40:

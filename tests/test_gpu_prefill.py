@@ -1,6 +1,8 @@
 """The kernels that work all tokens of a prompt between the projections, against plain torch in float64 at the
 edges of their tiles (16 tokens, 32 cache positions, 64 columns), and the layer built from them against the
 module path."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -104,6 +106,38 @@ def test_product_of_packed_vectors_with_residual(batch, rows, cols):
         want = staged @ d64.T + (r.astype(np.float64) if residual is not None else 0.0)
         bound = 2.0 ** -11 * np.abs(want) + 2.0 ** -25 + (cols + 3) * 2.0 ** -24 * (np.abs(staged) @ np.abs(d64).T + np.abs(want))
         assert (np.abs(y - want) <= bound).all()
+
+
+@pytest.mark.parametrize("batch,rows,cols,offset,ldx", [(1, 40, 64, 0, 64), (17, 333, 200, 3, 211), (40, 100, 71, 1, 72)])
+def test_packing_and_residual_in_place_through_the_c_abi(batch, rows, cols, offset, ldx):
+    vp, i32, i64 = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64
+    lib = ctypes.CDLL(mk.HIP_LIBRARY_PATH)
+    lib.macko_packed_bytes.argtypes = [i32, i32, ctypes.POINTER(i64)]
+    lib.macko_pack_f16.argtypes = [vp, i32, i32, i64, vp, vp]
+    lib.macko_spmv_f16_packed.argtypes = [vp, vp, vp, vp, vp, vp, i32, i32, i64, i32, i64, vp]
+    rng = np.random.default_rng(rows)
+    dense = helpers.random_sparse(rng, rows, cols, 0.4)
+    c = mk.compress(torch.from_numpy(dense).cuda())
+    flat = torch.from_numpy(rng.standard_normal(offset + batch * ldx).astype(np.float16)).cuda()
+    x = flat[offset:].view(batch, ldx)[:, :cols]
+    size = i64(-1)
+    assert lib.macko_packed_bytes(cols, batch, ctypes.byref(size)) == 0
+    packed = torch.full((size.value // 2,), 7.0, dtype=torch.float16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.macko_pack_f16(x.data_ptr(), cols, batch, ldx, packed.data_ptr(), stream) == 0
+    got, rest = _unpack(packed, cols, batch)
+    assert torch.equal(got, x) and not rest.any()
+    r = rng.standard_normal((batch, rows)).astype(np.float16)
+    y = torch.from_numpy(r).cuda()   # the residual is where the result goes
+    assert lib.macko_spmv_f16_packed(c[0].data_ptr(), c[1].data_ptr(), c[2].data_ptr(), packed.data_ptr(), y.data_ptr(), y.data_ptr(),
+                                     rows, cols, c[0].numel(), batch, rows, stream) == 0
+    x64, d64 = x.cpu().double().numpy(), dense.astype(np.float64)
+    want = x64 @ d64.T + r.astype(np.float64)
+    bound = 2.0 ** -11 * np.abs(want) + 2.0 ** -25 + (cols + 3) * 2.0 ** -24 * (np.abs(x64) @ np.abs(d64).T + np.abs(want))
+    assert (np.abs(y.cpu().double().numpy() - want) <= bound).all()
+    # refused before any launch
+    assert lib.macko_pack_f16(x.data_ptr(), 63, batch, ldx, packed.data_ptr(), stream) == -1
+    assert lib.macko_pack_f16(x.data_ptr(), cols, batch, cols - 1, packed.data_ptr(), stream) == -1
 
 
 def test_operators_have_fake_implementations():

@@ -91,10 +91,11 @@ def test_short_rows_other_entry_points():
     want8 = q.astype(np.float64) @ x.astype(np.float64)
     assert np.all(np.abs(y8 - want8) <= 1e-3 + 1e-2 * np.abs(want8) + 2 ** -11 * np.abs(want8))
     # several vectors per pass
-    X = rng.standard_normal((3, cols)).astype(np.float16)
-    Y = macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda()).cpu().numpy()
-    for b in range(3):
-        helpers.assert_close_fp16(Y[b], helpers.dense_reference(dense, X[b]))
+    X = rng.standard_normal((4, cols)).astype(np.float16)
+    for batch in (2, 3, 4):   # 2 and 4 in one launch of the gather kernel
+        Y = macko_spmv.multiply_batched(c, torch.from_numpy(X[:batch]).cuda()).cpu().numpy()
+        for b in range(batch):
+            helpers.assert_close_fp16(Y[b], helpers.dense_reference(dense, X[b]))
 
 
 def test_short_rows_keep_inf_and_nan_to_the_rows_that_read_them():

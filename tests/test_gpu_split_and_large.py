@@ -84,11 +84,12 @@ def test_rows_split_between_waves_other_entry_points():
     C = torch.from_numpy(y0.copy()).cuda()
     macko_spmv.multiply_axpby(c, xg, C, alpha=0.5, beta=-2.0)
     helpers.assert_close_fp16(C.cpu().numpy(), 0.5 * want - 2.0 * y0.astype(np.float64), rel=1e-2, abs_=4e-3)
-    # several vectors per pass (16384 columns: four vectors per launch, then two, then one)
+    # several vectors: 2 and 4 in one launch of these kernels, 7 on the matrix cores
     X = rng.standard_normal((7, cols)).astype(np.float16)
-    Y = macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda()).cpu().numpy()
-    for b in range(7):
-        helpers.assert_close_fp16(Y[b], helpers.dense_reference(dense, X[b]))
+    for batch in (2, 4, 7):
+        Y = macko_spmv.multiply_batched(c, torch.from_numpy(X[:batch]).cuda()).cpu().numpy()
+        for b in range(batch):
+            helpers.assert_close_fp16(Y[b], helpers.dense_reference(dense, X[b]))
     # int8 values
     q = np.clip(np.round(dense.astype(np.float32) * 400), -127, 127).astype(np.int8)
     c8 = macko_spmv.compress_int8(torch.from_numpy(q).cuda())
@@ -162,11 +163,13 @@ def test_row_ends_next_to_inf_and_nan(rows, cols):
     assert np.isfinite(got).all()
     helpers.assert_close_fp16(got, 2.0 * helpers.dense_reference(dense, finite_x) + y0.astype(np.float64),
                               rel=1e-2, abs_=4e-3)
-    X = np.stack([x, x[::-1].copy(), x])
+    X = np.stack([x, x[::-1].copy(), x, x])
     X[1] = rng.standard_normal(cols).astype(np.float16)
-    Y = macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda()).cpu().numpy().astype(np.float32)
-    assert np.isfinite(Y).all()
-    assert np.allclose(Y[0], want_oracle, rtol=1e-2, atol=1e-3) and np.allclose(Y[2], want_oracle, rtol=1e-2, atol=1e-3)
+    for batch in (2, 3, 4):   # one launch of two, two launches or the matrix cores, one launch of four where they fit
+        Y = macko_spmv.multiply_batched(c, torch.from_numpy(X[:batch]).cuda()).cpu().numpy().astype(np.float32)
+        assert np.isfinite(Y).all()
+        for b in [0, 2, 3][:batch - 1]:
+            assert np.allclose(Y[b], want_oracle, rtol=1e-2, atol=1e-3)
     q = np.clip(np.round(dense.astype(np.float32) * 200), -127, 127).astype(np.int8)
     q[(q == 0) & (dense != 0)] = 1
     c8 = macko_spmv.compress_int8(torch.from_numpy(q).cuda())
