@@ -282,12 +282,15 @@ __global__ void __launch_bounds__(kAttnWaves *kWave) prefill_attention_kernel(co
         weight[w] = __expf(m_lds[w][sub] - top);
         total += weight[w] * l_lds[w][sub];
     }
-    const float inv = 1.0f / total;  // no weights at all (every score -inf) are 0 / 0, as in a softmax
+    // No weights at all (every score -inf) are 0 / 0, as in a softmax; vectors that do not exist are 0 * 0.  Chosen in
+    // front of the product, which then is rounded to fp16 once, together with the conversion.
+    const float inv = pos >= 0 ? 1.0f / total : 0.f;
     for (int d = wave; d < DTILES; d += kAttnWaves) {
         float4v sum = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < kAttnWaves; ++w) sum += weight[w] * o_lds[w][d][lane];
-        sum = pos >= 0 ? sum * inv : float4v{0.f, 0.f, 0.f, 0.f};  // vectors that do not exist are zero
+        sum = pos >= 0 ? sum : float4v{0.f, 0.f, 0.f, 0.f};
+        sum *= inv;
         const int c = head * HD + d * 16 + quarter * 4;  // four columns of vector n
         packed[packed_piece(c >> 3, n, tiles) * 2 + ((c >> 2) & 1)] = u32x2{pack2(sum[0], sum[1]), pack2(sum[2], sum[3])};
     }

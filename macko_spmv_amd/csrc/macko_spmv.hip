@@ -1284,18 +1284,18 @@ double gather_us(int n, int rows, int cols, long long padded, bool aligned, cons
 // (1659 products) the route taken is on average 0.2 % behind the better one, 3 % or more in 40 (at most 22 %).
 // 2 and 4 vectors in one gather launch stay there.  Rows of less than 100 entries do not: their ends are a serial
 // chain in the gather kernels (20000 x 300 at 0.1, 8 vectors: 19.2 / 9.6).
-int batched_on_tiles(bool *tiles, const void *x, int rows, int cols, long long padded, int batch, long long ldx, bool packed,
-                     const DeviceInfo &info)
+int batched_on_tiles(bool *tiles, TileShape *shape, const void *x, int rows, int cols, long long padded, int batch, long long ldx,
+                     bool packed, const DeviceInfo &info)
 {
     *tiles = false;
     if (!spmv_tile_takes(rows, cols, padded, batch, ldx)) return 0;
     if (batch < 8 && gather_step(batch, cols, padded, info) == batch) return 0;
-    *tiles = true;
-    if (padded < 100ll * rows) return 0;
     const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (ldx & 7) == 0;
     double tile_us = 0.0, us = 0.0;
-    const int rc = spmv_tile_estimate(rows, cols, padded, batch, packed, &tile_us);
+    const int rc = spmv_tile_estimate(rows, cols, padded, batch, packed, info, shape, &tile_us);
     if (rc != 0) return rc;
+    *tiles = true;
+    if (padded < 100ll * rows) return 0;
     for (int left = batch; left > 0 && us < tile_us;) {
         const int step = gather_step(left, cols, padded, info);
         us += gather_us(step, rows, cols, padded, aligned, info);
@@ -1325,7 +1325,8 @@ extern "C" int macko_spmv_f16_batched_workspace(const void *x, int32_t rows, int
     if (rc != 0) return rc;
     const size_t wanted = spmv_tile_workspace(cols, batch, x, ldx);
     bool tiles = false;
-    if (wanted > 0) rc = batched_on_tiles(&tiles, x, rows, cols, padded_entries, batch, ldx, true, info);
+    TileShape shape;
+    if (wanted > 0) rc = batched_on_tiles(&tiles, &shape, x, rows, cols, padded_entries, batch, ldx, true, info);
     if (tiles) *bytes = (int64_t)wanted;
     return rc;
 }
@@ -1351,10 +1352,11 @@ extern "C" int macko_spmv_f16_batched_ws(const void *values, const void *deltas,
     const size_t wanted = spmv_tile_workspace(cols, batch, x, ldx);
     const bool packed = wanted > 0 && workspace != nullptr && (size_t)workspace_bytes >= wanted && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
     bool tiles = false;
-    rc = batched_on_tiles(&tiles, x, rows, cols, padded_entries, batch, ldx, packed, info);
+    TileShape shape;
+    rc = batched_on_tiles(&tiles, &shape, x, rows, cols, padded_entries, batch, ldx, packed, info);
     if (rc != 0) return rc;
     if (tiles)
-        return spmv_tile_launch(args_from(0), batch, workspace, (size_t)workspace_bytes, as_stream(stream));
+        return spmv_tile_launch(args_from(0), batch, shape, packed ? workspace : nullptr, info, as_stream(stream));
     for (int done = 0; done < batch;) {
         const SpmvArgs a = args_from(done);
         const int step = gather_step(batch - done, cols, padded_entries, info);

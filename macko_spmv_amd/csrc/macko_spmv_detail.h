@@ -314,13 +314,24 @@ __device__ __forceinline__ float pick_lane(const float (&c)[8], int idx, int L)
 int spmv_split_launch(const spmv_detail::SpmvArgs &a, bool axpby, int value_bytes, int n_vectors, int fused,
                       bool x_in_lds, int grid, size_t lds_x, hipStream_t stream);
 
+// How spmv_tile_kernel cuts a product up for a launch.
+struct TileShape {
+    int row_tiles;     // RT: a workgroup's rows / 16, rounded up
+    int wave_tiles;    // NTW: vector tiles (16 vectors) per wave
+    int steps;         // SC: 64-column steps of X a wave keeps in registers per chunk
+    int group_shift;   // log2 of the vector groups of a workgroup
+    long long row_blocks;
+    int chunk;         // columns per chunk
+};
+
 // The kernel for several vectors on the matrix cores (macko_spmv_tile.hip): whether it can do a product,
-// its estimated time in us (`packed`: with X in operand order), the scratch memory it wants for these
-// vectors (0: none), and the launch (a.ldx, a.ldy set; without workspace it reads X as it is, more slowly).
+// the shape it would take and its estimated time in us (`packed`: with X in operand order), the scratch memory
+// it wants for these vectors (0: none), and the launch (a.ldx, a.ldy set; `workspace`: that scratch memory, or
+// null: it reads X as it is, more slowly).
 bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long ldx);
-int spmv_tile_estimate(int rows, int cols, long long padded, int batch, bool packed, double *us);
+int spmv_tile_estimate(int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, TileShape *shape, double *us);
 size_t spmv_tile_workspace(int cols, int batch, const void *x, long long ldx);
 int spmv_tile_pack(const uint16_t *x, int cols, int batch, long long ldx, void *packed, hipStream_t stream);
-int spmv_tile_launch(const spmv_detail::SpmvArgs &a, int batch, void *workspace, size_t workspace_bytes, hipStream_t stream);
+int spmv_tile_launch(const spmv_detail::SpmvArgs &a, int batch, const TileShape &shape, void *workspace, const DeviceInfo &info, hipStream_t stream);
 
 }  // namespace macko

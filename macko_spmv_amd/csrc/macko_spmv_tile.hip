@@ -46,7 +46,7 @@ constexpr int kRowUnit = 4;      // row blocks start at multiples of 4 rows (8-b
 constexpr int kTilePad = 8;      // spare columns behind every row of the dense chunk, 16 bytes
 constexpr int kTileFront = 16;   // the same in front of the first row
 // Elements of X (batch * cols) from which on it is brought into operand order first.  Packing is a
-// launch of its own, about 2 us; read as it is, a wave's load touches 16 cache lines instead of 8
+// launch of its own, about 3 us back to back (4.9 in a kernel trace, which counts the dispatch); read as it is, a wave's load touches 16 cache lines instead of 8
 // whole ones and L2 delivers 14 instead of 48 bytes a cycle to a compute unit (4096 x 4096 at density
 // 0.5: 16 vectors 9.7 us as they are and 10.8 packed, 24 vectors 12.0 and 11.4, 128 vectors 26 and 18).
 // Vectors that are not 16-byte aligned cost a second line per lane: packed from 4 vectors on (777 x 3333,
@@ -67,7 +67,7 @@ struct TileArgs {
     int n_chunks;
     u32 units_q, units_rem;  // 4-row units per row block (even_split)
     int vector_blocks;
-    int group_shift;      // log2 of the number of vector groups of a workgroup (1, 2, 4, 8)
+    int group_shift;      // log2 of the number of vector groups of a workgroup (1, 2, 4)
     int vector_store;     // 8-byte stores of Y are aligned
     const u32x4 *packed;  // X in operand order (pack_vectors_kernel), null: read X itself
     int packed_tiles;     // vector tiles in it
@@ -451,16 +451,6 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs 
     }
 }
 
-// How a product is cut up for a launch.
-struct TileShape {
-    int row_tiles;     // RT: a workgroup's rows / 16, rounded up
-    int wave_tiles;    // NTW: vector tiles (16 vectors) per wave
-    int steps;         // SC: 64-column steps of X a wave keeps in registers per chunk
-    int group_shift;   // log2 of the vector groups of a workgroup
-    long long row_blocks;
-    int chunk;         // columns per chunk
-};
-
 template <int RT, int NTW, int SC, bool PACKED>
 int launch_tile(const TileArgs &a, unsigned grid, size_t lds_bytes, hipStream_t stream)
 {
@@ -609,14 +599,10 @@ bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long 
 
 // The time by the cost above, at 2.4 GHz, and the packing launch.  Right to about 10 % on either side where it
 // decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1: 24.4, 21).
-int spmv_tile_estimate(int rows, int cols, long long padded, int batch, bool packed, double *us)
+int spmv_tile_estimate(int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, TileShape *shape, double *us)
 {
-    DeviceInfo info;
-    const int rc = device_info(&info);
-    if (rc != 0) return rc;
-    TileShape shape;
     double cycles = 0.0;
-    if (!choose_tile_shape(&shape, rows, cols, padded, batch, packed, info, &cycles)) return MACKO_E_INVALID_ARGUMENT;
+    if (!choose_tile_shape(shape, rows, cols, padded, batch, packed, info, &cycles)) return MACKO_E_INVALID_ARGUMENT;
     *us = cycles * (1.06 / 2400.0) + (packed ? 2.9 : 0.0);
     return 0;
 }
@@ -628,11 +614,8 @@ size_t spmv_tile_workspace(int cols, int batch, const void *x, long long ldx)
     return packed_bytes(cols, batch);
 }
 
-int spmv_tile_launch(const SpmvArgs &args, int batch, void *workspace, size_t workspace_bytes, hipStream_t stream)
+int spmv_tile_launch(const SpmvArgs &args, int batch, const TileShape &shape, void *workspace, const DeviceInfo &info, hipStream_t stream)
 {
-    DeviceInfo info;
-    const int rc = device_info(&info);
-    if (rc != 0) return rc;
     TileArgs a{};
     a.values = args.values;
     a.deltas = args.deltas;
@@ -645,14 +628,11 @@ int spmv_tile_launch(const SpmvArgs &args, int batch, void *workspace, size_t wo
     a.padded = (u32)args.padded;
     a.ldx = (u32)args.ldx;
     a.ldy = (u32)args.ldy;
-    const size_t wanted = spmv_tile_workspace(args.cols, batch, args.x, args.ldx);
-    if (wanted > 0 && workspace != nullptr && workspace_bytes >= wanted && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
+    if (workspace != nullptr) {
         const int e = spmv_tile_pack(args.x, args.cols, batch, args.ldx, workspace, stream);
         if (e != 0) return e;
         a.packed = (const u32x4 *)workspace;
     }
-    TileShape shape;
-    if (!choose_tile_shape(&shape, a.rows, a.cols, args.padded, batch, a.packed != nullptr, info)) return MACKO_E_INVALID_ARGUMENT;
     return launch_tile_shape(a, shape, info.max_lds_bytes, stream);
 }
 
