@@ -122,29 +122,39 @@ def load_compressed_linears(model, compressed_sd):
 # ---- a minimal Llama-architecture decoder (batch 1) ------------------------------------------------
 
 _PLAIN_TENSORS = (torch.Tensor, nn.Parameter, FakeTensor)
+_PROXY_MODE = torch._C._TorchDispatchModeKey.PROXY
 
 
-def _recording():
-    """Whether the call is being recorded into a graph to keep (torch.jit.trace, make_fx, torch.export): that graph
-    may be given gradients, another device or another type, so it gets torch's operators."""
-    if torch.jit.is_tracing() or torch.compiler._is_exporting_flag:  # is_exporting() is True in every compiled call
-        return True
-    return not torch.compiler.is_compiling() and torch._C._get_dispatch_mode(torch._C._TorchDispatchModeKey.PROXY) is not None
+def _observed():
+    """Whether something else than the call itself looks at its operators: a batching rule, a tangent, or a recording
+    into a graph to keep (torch.jit.trace, make_fx, torch.export), which may be given gradients, another device or
+    another type later."""
+    if torch.compiler.is_compiling():
+        # what Dynamo makes of the interpreter stack is never None, but has the right type; is_exporting() is True there always
+        return (torch.compiler._is_exporting_flag or torch.autograd.forward_ad._current_level >= 0
+                or isinstance(torch._C._functorch.peek_interpreter_stack(), torch._C._functorch.CInterpreter))
+    return (torch._C._is_tracing() or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_dispatch_mode(_PROXY_MODE) is not None
+            or torch._C._functorch.peek_interpreter_stack() is not None)
 
 
 def _inference_half(*tensors):
-    """fp16 tensors on one GPU through which no gradient, tangent or batching rule has to flow: what the
-    hand-written kernels between the projections take.  The operators copy what is not 16-byte aligned; eagerly
-    such views keep to torch's operators (Dynamo cannot trace storage_offset(); and what it makes of the
-    interpreter stack is never None, but has the right type)."""
-    transformed = isinstance(torch._C._functorch.peek_interpreter_stack(), torch._C._functorch.CInterpreter)
-    if transformed or torch.autograd.forward_ad._current_level >= 0 or _recording():
+    """fp16 tensors on one GPU through which no gradient has to flow, unobserved: what the hand-written kernels
+    between the projections take.  The operators copy what is not 16-byte aligned; eagerly such views keep to
+    torch's operators (Dynamo cannot trace storage_offset())."""
+    if _observed():
         return False
-    grad, tracing = torch.is_grad_enabled(), torch.compiler.is_compiling()
-    # a torch.fx proxy is no tensor and has no answers; a subclass (DTensor, ...) has its own idea of torch's operators
-    # and none of these
-    return all(type(t) in _PLAIN_TENSORS and t.is_cuda and t.device == tensors[0].device
-               and t.dtype == torch.float16 and not (grad and t.requires_grad) and (tracing or t.storage_offset() % 8 == 0) for t in tensors)
+    grad, tracing, device = torch.is_grad_enabled(), torch.compiler.is_compiling(), None
+    for t in tensors:
+        # a torch.fx proxy is no tensor and has no answers; a subclass (DTensor, ...) has its own idea of torch's operators
+        # and none of these
+        if (type(t) not in _PLAIN_TENSORS or not t.is_cuda or t.dtype != torch.float16 or (grad and t.requires_grad)
+                or not tracing and t.storage_offset() % 8 != 0):
+            return False
+        if device is None:
+            device = t.get_device()
+        elif t.get_device() != device:
+            return False
+    return True
 
 
 class RMSNorm(nn.Module):
@@ -224,26 +234,37 @@ class Block(nn.Module):
         """Whether several tokens go through the layer by way of forward_fused: inference in fp16 on the
         GPU, all seven projections compressed, nothing hooked to the layer or the modules passed over."""
         att, mlp = self.self_attn, self.mlp
-        if type(att) is not Attention or type(mlp) is not MLP:
+        if type(att) is not Attention or type(mlp) is not MLP or not isinstance(x, torch.Tensor) or x.dim() != 3:
             return False
         projections = (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
         norms = (self.input_layernorm, self.post_attention_layernorm)
-        if not all(type(p) is MackoLinear for p in projections) or not isinstance(x, torch.Tensor) or x.dim() != 3:
-            return False
+        for module in projections:
+            if type(module) is not MackoLinear:
+                return False
+        for module in norms:
+            if type(module) is not RMSNorm:
+                return False
         # rows and cols of a projection that fit the layer; one that does not is the modules' to refuse (the packed
         # vectors are whole 64-column blocks, whose size does not tell)
-        dim, hidden = x.shape[2], projections[4].c_3
-        fitting = [(dim, dim)] * 4 + [(hidden, dim)] * 2 + [(dim, hidden)]
-        return (x.shape[0] == 1 and x.shape[1] > 1 and att.head_dim in (64, 128)
-                and att.n_heads * att.head_dim == dim and hidden % 8 == 0 and hidden >= 64
-                and all((p.c_3, p.c_4) == fit for p, fit in zip(projections, fitting))
-                and all(type(n) is RMSNorm and n.weight.is_contiguous() and n.weight.shape == x.shape[2:] for n in norms)
-                and not _has_any_global_hook()
-                and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m)
-                            for m in (self, att, mlp, *projections, *norms))
-                and att.k_cache.shape == att.v_cache.shape == (1, att.n_heads, att.max_len, att.head_dim)
-                and att.k_cache.is_contiguous() and att.v_cache.is_contiguous()
-                and _inference_half(x, *(n.weight for n in norms), att.k_cache, att.v_cache))
+        one, tokens, dim = x.shape
+        hidden = projections[4].c_3
+        if (one != 1 or tokens <= 1 or att.head_dim not in (64, 128) or att.n_heads * att.head_dim != dim or hidden % 8 != 0 or hidden < 64):
+            return False
+        for module in projections[:4]:
+            if module.c_3 != dim or module.c_4 != dim:
+                return False
+        gate, up, down = projections[4:]
+        if gate.c_4 != dim or up.c_3 != hidden or up.c_4 != dim or down.c_3 != dim or down.c_4 != hidden:
+            return False
+        for module in (self, att, mlp, *projections, *norms):
+            if module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__:
+                return False
+        weights = (norms[0].weight, norms[1].weight)
+        k_cache, v_cache = att.k_cache, att.v_cache
+        return (all(w.shape == (dim,) and w.is_contiguous() for w in weights)
+                and k_cache.shape == v_cache.shape == (1, att.n_heads, att.max_len, att.head_dim)
+                and k_cache.is_contiguous() and v_cache.is_contiguous() and not _has_any_global_hook()
+                and _inference_half(x, *weights, k_cache, v_cache))
 
     def forward_fused(self, x, cos, sin, positions):
         """The layer for several tokens with one kernel for each part between the projections; what a
@@ -313,12 +334,17 @@ class LlamaDecoder(nn.Module):
 
     @torch.jit.unused
     def _run_layers(self, x, cos, sin, positions):
-        mask = None  # only made for a layer that needs one
+        mask = fits = None  # only made where a layer needs it
         for layer in self.model.layers:
-            # positions that do not fit the tokens or a cache that does not fit the mask are the modules' to refuse
-            if (type(layer) is Block and layer.takes_fused(x) and layer.self_attn.max_len == self.max_len
-                    and positions.shape == x.shape[1:2] and positions.dtype == torch.int64
-                    and positions.device == cos.device == x.device):
+            if type(layer) is Block and layer.takes_fused(x):
+                # positions that do not fit the tokens or a cache that does not fit the mask are the modules' to refuse
+                if fits is None:
+                    fits = (positions.shape == x.shape[1:2] and positions.dtype == torch.int64
+                            and positions.device == cos.device == x.device)
+                fused = fits and layer.self_attn.max_len == self.max_len
+            else:
+                fused = False
+            if fused:
                 x = layer(x, cos, sin, positions, _FUSED_CAUSAL)
                 continue
             if mask is None:
