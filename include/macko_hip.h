@@ -133,8 +133,9 @@ MACKO_API int macko_compress_f16_fill(const void *dense, int32_t rows, int32_t c
 
 /*
  * Y[b, :] = M X[b, :] for b < batch.  X is [batch, ldx] and Y [batch, ldy], row-major fp16 with
- * ldx >= cols and ldy >= rows (elements).  From a few vectors on the product runs on the matrix
- * cores, with the matrix decoded once for up to 128 vectors.  No counterpart in the upstream
+ * ldx >= cols and ldy >= rows (elements).  From a few vectors on the product mostly runs on the matrix
+ * cores, with the matrix decoded once for up to 128 vectors; with many rows, few entries and few
+ * vectors in launches of up to eight vectors without them.  No counterpart in the upstream
  * package, whose LLM runner maps the single-vector operator over the batch dimension
  * (python_scripts/util_run_pruned_llm.py:112-118).
  *

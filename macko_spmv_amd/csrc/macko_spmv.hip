@@ -1298,8 +1298,8 @@ int batched_on_tiles(bool *tiles, TileShape *shape, const void *x, int rows, int
     if (padded < 100ll * rows) return 0;
     for (int left = batch; left > 0 && us < tile_us;) {
         const int step = gather_step(left, cols, padded, info);
-        us += gather_us(step, rows, cols, padded, aligned, info);
-        left -= step;
+        us += (left / step) * gather_us(step, rows, cols, padded, aligned, info);
+        left %= step;
     }
     *tiles = us >= tile_us;
     return 0;

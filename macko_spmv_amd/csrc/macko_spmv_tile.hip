@@ -20,9 +20,9 @@
 // of X per row block; the gather kernels read LDS once per entry for a few vectors and stream the
 // matrix again for the next few.  Measured on 11008 x 4096 at density 0.5, 128 vectors: 341 us through the
 // gather kernels in groups of eight (17 TFLOP/s), 27.4 here (211 TFLOP/s of stored entries, twice that
-// on the matrix cores).  What bounds it now: no unit alone.  Of a launch's 55000 cycles per compute unit
-// the vector units are busy 25000 (decoding), LDS 28000 (scatter 14000, operands 12000), the matrix
-// cores 12000, and the megabyte of X takes 17000 to come out of L2; the rest is waiting for one another.
+// on the matrix cores).  What bounds it now: no unit alone.  Of the 54500 cycles a wave of that launch lives
+// the vector units are busy 25000 (decoding), LDS 28300 (12400 of them bank conflicts) and the matrix cores
+// 12300, by the counters; waves wait for 40 % of their cycles, for one another and for X out of L2.
 //
 // A zero of the dense chunk times an Inf or NaN of X is a NaN that the sparse product does not have
 // (it never reads columns without an entry).  Such a product can only make a sum non-finite, so every
@@ -47,7 +47,7 @@ constexpr int kTilePad = 8;      // spare columns behind every row of the dense 
 constexpr int kTileFront = 16;   // the same in front of the first row
 // Elements of X (batch * cols) from which on it is brought into operand order first.  Packing is a
 // launch of its own, about 3 us back to back (4.9 in a kernel trace, which counts the dispatch); read as it is, a wave's load touches 16 cache lines instead of 8
-// whole ones and L2 delivers 14 instead of 48 bytes a cycle to a compute unit (4096 x 4096 at density
+// whole ones and L2 delivers about 14 instead of 48 bytes a cycle to a compute unit, by the launches' times (4096 x 4096 at density
 // 0.5: 16 vectors 9.7 us as they are and 10.8 packed, 24 vectors 12.0 and 11.4, 128 vectors 26 and 18).
 // Vectors that are not 16-byte aligned cost a second line per lane: packed from 4 vectors on (777 x 3333,
 // 4 vectors: 8.8 us as they are, 7.5 packed).

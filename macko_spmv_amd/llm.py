@@ -165,8 +165,8 @@ class RMSNorm(nn.Module):
 
     def forward(self, x):
         if not torch.jit.is_scripting():
-            if (_inference_half(x, self.weight) and x.is_contiguous() and x.shape[-1] % 8 == 0 and x.numel() > 0
-                    and self.weight.is_contiguous() and self.weight.shape == x.shape[-1:]):
+            if (_inference_half(x, self.weight) and x.is_contiguous() and self.weight.shape == x.shape[-1:] and x.numel() > 0
+                    and x.shape[-1] % 8 == 0 and self.weight.is_contiguous()):
                 return torch.ops.macko_spmv.rmsnorm_rows(x, self.weight, self.eps)
         v = x.float()
         v = v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + self.eps)
