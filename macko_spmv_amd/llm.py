@@ -236,6 +236,9 @@ class Block(nn.Module):
         att, mlp = self.self_attn, self.mlp
         if type(att) is not Attention or type(mlp) is not MLP or not isinstance(x, torch.Tensor) or x.dim() != 3:
             return False
+        for kind, forward in _PASSED_OVER:
+            if kind.forward is not forward:
+                return False
         projections = (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
         norms = (self.input_layernorm, self.post_attention_layernorm)
         for module in projections:
@@ -294,6 +297,10 @@ class Block(nn.Module):
                 return self.forward_fused(x, cos, sin, positions)
         x = x + self.self_attn(self.input_layernorm(x), cos, sin, positions, mask)
         return x + self.mlp(self.post_attention_layernorm(x))
+
+
+# the classes whose forward a fused layer stands for; one that was replaced is called (with a mask)
+_PASSED_OVER = tuple((kind, kind.forward) for kind in (Block, Attention, MLP, RMSNorm, MackoLinear))
 
 
 class _Body(nn.Module):

@@ -199,6 +199,15 @@ def test_layer_with_norm_weights_of_any_stride_goes_through_its_modules():
         assert not _takes_fused(norm_weight(make))
 
 
+@pytest.mark.parametrize("kind", [llm.Block, llm.Attention, llm.MLP, llm.RMSNorm, llm.MackoLinear])
+def test_layer_calls_a_forward_that_was_replaced_in_its_class(kind, monkeypatch):
+    kept = kind.forward
+    monkeypatch.setattr(kind, "forward", lambda self, *args: kept(self, *args))
+    assert not _takes_fused(lambda layer: None)
+    monkeypatch.undo()
+    assert _takes_fused(lambda layer: None)
+
+
 @pytest.mark.parametrize("parent,name,rows,cols", [("self_attn", "q_proj", 256, 250), ("self_attn", "k_proj", 128, 256),
                                                    ("self_attn", "o_proj", 256, 251), ("mlp", "up_proj", 704, 255),
                                                    ("mlp", "up_proj", 696, 256), ("mlp", "down_proj", 256, 700)])
