@@ -166,7 +166,19 @@ MACKO_API int macko_spmv_f16_batched(const void *values, const void *deltas, con
  *   macko_pack_f16        X [batch, ldx] into it (packed 16-byte aligned)
  *   macko_spmv_f16_packed Y[b, :] = M X[b, :] (+ residual[b, :], laid out like Y, NULL: none; may be Y)
  *                         with one rounding to fp16.
+ *   macko_spmv_f16_packed_several  the same (without a residual) for up to MACKO_PACKED_MATRICES matrices of
+ *                         the same columns in one launch; in front of another matrix, rows % 4 == 0
  */
+#define MACKO_PACKED_MATRICES 3
+typedef struct macko_packed_matrix {
+    const void *values;
+    const void *deltas;
+    const int32_t *row_ptr;
+    void *y;
+    int32_t rows;
+    int64_t padded_entries;
+    int64_t ldy;
+} macko_packed_matrix;
 MACKO_API int macko_packed_bytes(int32_t cols, int32_t batch, int64_t *bytes);
 MACKO_API int macko_pack_f16(const void *x, int32_t cols, int32_t batch, int64_t ldx, void *packed,
                    void *stream);
@@ -174,6 +186,8 @@ MACKO_API int macko_spmv_f16_packed(const void *values, const void *deltas, cons
                           const void *packed, const void *residual, void *y, int32_t rows,
                           int32_t cols, int64_t padded_entries, int32_t batch, int64_t ldy,
                           void *stream);
+MACKO_API int macko_spmv_f16_packed_several(const macko_packed_matrix *matrices, int32_t n_matrices,
+                          const void *packed, int32_t cols, int32_t batch, void *stream);
 
 /*
  * Products whose input vector is produced on the fly while it is staged for the product, so a

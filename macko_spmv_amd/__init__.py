@@ -124,6 +124,11 @@ def _multiply_packed_fake(M_values, M_deltas, M_row_indices, M_rows, M_cols, pac
     return torch.empty((batch, M_rows), device=M_values.device, dtype=M_values.dtype)
 
 
+@torch.library.register_fake("macko_spmv::multiply_packed_several")
+def _multiply_packed_several_fake(M_values, M_deltas, M_row_indices, M_rows, M_cols, packed, batch):
+    return [torch.empty((batch, rows), device=values.device, dtype=values.dtype) for values, rows in zip(M_values, M_rows)]
+
+
 @torch.library.register_fake("macko_spmv::prefill_rope_append")
 def _prefill_rope_append_fake(q, k, v, cos_rows, sin_rows, positions, k_cache, v_cache):
     return None

@@ -54,15 +54,25 @@ constexpr int kTileFront = 16;   // the same in front of the first row
 constexpr long long kPackFrom = 100000;
 constexpr long long kPackUnalignedFrom = 12000;
 
-struct TileArgs {
+// One of the matrices of a launch.  Several with the same columns and vectors stand below each other; their rows
+// are numbered on, and where there is more than one, every one but the last ends on a whole unit of four rows.
+struct TileSource {
     const u32 *values;
     const u32 *deltas;
     const int *row_ptr;
-    const uint16_t *x;
     uint16_t *y;
-    int rows, cols, batch;
+    int first;   // its first row; behind the last matrix: no row
     u32 padded;
-    u32 ldx, ldy;
+    u32 ldy;
+};
+constexpr int kMaxSources = MACKO_PACKED_MATRICES;
+
+// What a launch of one matrix and one of several have in common, and the launch's arguments: with one matrix a wave
+// fetches no more of them than it needs (4096 x 4096, 8 vectors: 0.15 us a launch).
+struct TileCommon {
+    const uint16_t *x;
+    int rows, cols, batch;   // rows of all matrices
+    u32 ldx;
     int chunk;            // columns per chunk, a multiple of 64
     int n_chunks;
     u32 units_q, units_rem;  // 4-row units per row block (even_split)
@@ -73,6 +83,10 @@ struct TileArgs {
     int packed_tiles;     // vector tiles in it
     int packed_steps;     // 64-column steps in it
     const uint16_t *residual;  // added to Y before it is rounded (laid out like Y, may be Y), or null
+};
+template <int SOURCES>
+struct TileArgs : TileCommon {
+    TileSource source[SOURCES];
 };
 
 __device__ __forceinline__ void lds_barrier()
@@ -146,8 +160,9 @@ __global__ void __launch_bounds__(256) pack_vectors_kernel(const uint16_t *__res
     dst[8] = v[1];
 }
 
-template <int RT, int NTW, int SC, bool PACKED>
-__global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs a)
+// SEVERAL: more than one matrix, which a wave looks up for each of its rows.
+template <int RT, int NTW, int SC, bool PACKED, bool SEVERAL>
+__global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs<SEVERAL ? kMaxSources : 1> a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     typedef __attribute__((address_space(3))) u32x4 *lds_w32x4;
@@ -170,8 +185,18 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs 
     const int part = wave >> a.group_shift;
     const int parts = kTileWaves >> a.group_shift;
 
-    const __amdgpu_buffer_rsrc_t rs_values = __builtin_amdgcn_make_buffer_rsrc((void *)a.values, 0, (int)(a.padded * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rs_deltas = __builtin_amdgcn_make_buffer_rsrc((void *)a.deltas, 0, (int)(a.padded / 2), 0x00020000);
+    auto source_of = [&](int row) __attribute__((always_inline)) {
+        int m = 0;
+        if constexpr (SEVERAL)
+            for (int k = 1; k < kMaxSources; ++k) m += row >= a.source[k].first ? 1 : 0;
+        return m;
+    };
+    __amdgpu_buffer_rsrc_t rs_values[SEVERAL ? RT : 1], rs_deltas[SEVERAL ? RT : 1];
+    auto describe = [&](int slot, const TileSource &m) __attribute__((always_inline)) {
+        rs_values[slot] = __builtin_amdgcn_make_buffer_rsrc((void *)m.values, 0, (int)(m.padded * 2), 0x00020000);
+        rs_deltas[slot] = __builtin_amdgcn_make_buffer_rsrc((void *)m.deltas, 0, (int)(m.padded / 2), 0x00020000);
+    };
+    if constexpr (!SEVERAL) describe(0, a.source[0]);
 
     // ---- my rows: row j of mine is row (wave + 16 j) of the block.  pos: next entry (a multiple of 8),
     //      end: behind the row's last entry, col: column of the entry in front of pos ------------------
@@ -183,19 +208,22 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs 
         const bool any = pos[J] < end[J];
         const u32 vo = any ? (u32)pos[J] * 2 + (u32)lane * 16 : kNoTileValues;
         const u32 dof = any ? ((u32)pos[J] >> 1) + (u32)lane * 4 : kNoTileDeltas;
-        tile_v[J] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_values, (int)vo, 0, 0));
-        tile_d[J] = __builtin_amdgcn_raw_buffer_load_b32(rs_deltas, (int)dof, 0, 0);
+        tile_v[J] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_values[SEVERAL ? J : 0], (int)vo, 0, 0));
+        tile_d[J] = __builtin_amdgcn_raw_buffer_load_b32(rs_deltas[SEVERAL ? J : 0], (int)dof, 0, 0);
     };
     int begin[RT];  // the row's first entry: what stands in front of it in its group of 8 is the row before's
     static_for<RT>([&](auto slot) {
         constexpr int J = decltype(slot)::value;
         const int row = row0 + wave + 16 * J;
+        const TileSource &m = a.source[source_of(row)];
+        if constexpr (SEVERAL) describe(J, m);
         u32 e0 = 0, e1 = 0;
         if (row < row1) {
-            e0 = (u32)uniform(a.row_ptr[row]);
-            e1 = (u32)uniform(a.row_ptr[row + 1]);
-            e0 = e0 < a.padded ? e0 : a.padded;
-            e1 = e1 < a.padded ? e1 : a.padded;
+            const int *row_ptr = m.row_ptr + (SEVERAL ? row - m.first : row);
+            e0 = (u32)uniform(row_ptr[0]);
+            e1 = (u32)uniform(row_ptr[1]);
+            e0 = e0 < m.padded ? e0 : m.padded;
+            e1 = e1 < m.padded ? e1 : m.padded;
         }
         if (e1 < e0) e1 = e0;
         begin[J] = (int)e0;
@@ -415,11 +443,13 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs 
                 bad &= bad - 1;
                 const int bad_row = __builtin_amdgcn_readlane(row, L) + i;
                 const int bad_n = __builtin_amdgcn_readlane(n, L);
-                u32 e0 = (u32)uniform(a.row_ptr[bad_row]), e1 = (u32)uniform(a.row_ptr[bad_row + 1]);
-                e0 = e0 < a.padded ? e0 : a.padded;
-                e1 = e1 < a.padded ? e1 : a.padded;
+                const TileSource &m = a.source[source_of(bad_row)];
+                const int *row_ptr = m.row_ptr + (SEVERAL ? bad_row - m.first : bad_row);
+                u32 e0 = (u32)uniform(row_ptr[0]), e1 = (u32)uniform(row_ptr[1]);
+                e0 = e0 < m.padded ? e0 : m.padded;
+                e1 = e1 < m.padded ? e1 : m.padded;
                 const float exact = exact_row_times_vector(
-                    a.values, a.deltas, e0, e1,
+                    m.values, m.deltas, e0, e1,
                     [&](int c) {
                         if constexpr (PACKED)
                             return reinterpret_cast<const uint16_t *>(a.packed + packed_piece(c >> 3, bad_n, a.packed_tiles))[c & 7];
@@ -431,9 +461,21 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs 
             }
         }
         if (n < a.batch) {
-            uint16_t *dst = a.y + (size_t)n * a.ldy + row;
-            if (a.residual != nullptr) {
-                const uint16_t *add = a.residual + (size_t)n * a.ldy + row;
+            uint16_t *y = a.source[0].y;
+            u32 ldy = a.source[0].ldy;
+            int at = row;
+            if constexpr (SEVERAL) {  // my four rows are of one matrix
+#pragma unroll
+                for (int k = 1; k < kMaxSources; ++k)
+                    if (row >= a.source[k].first) {
+                        y = a.source[k].y;
+                        ldy = a.source[k].ldy;
+                        at = row - a.source[k].first;
+                    }
+            }
+            uint16_t *dst = y + (size_t)n * ldy + at;
+            if (!SEVERAL && a.residual != nullptr) {
+                const uint16_t *add = a.residual + (size_t)n * ldy + row;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     if (row + i < row1) sum[i] += half_bits_to_float(add[i]);
@@ -451,10 +493,13 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs 
     }
 }
 
-template <int RT, int NTW, int SC, bool PACKED>
-int launch_tile(const TileArgs &a, unsigned grid, size_t lds_bytes, hipStream_t stream)
+template <int RT, int NTW, int SC, bool PACKED, bool SEVERAL>
+int launch_tile(const TileArgs<kMaxSources> &all, unsigned grid, size_t lds_bytes, hipStream_t stream)
 {
-    auto kernel = spmv_tile_kernel<RT, NTW, SC, PACKED>;
+    TileArgs<SEVERAL ? kMaxSources : 1> a;
+    static_cast<TileCommon &>(a) = all;
+    for (int k = 0; k < (SEVERAL ? kMaxSources : 1); ++k) a.source[k] = all.source[k];
+    auto kernel = spmv_tile_kernel<RT, NTW, SC, PACKED, SEVERAL>;
     if (lds_bytes > 64 * 1024) {
         // one-time opt-in to more than 64 KiB of dynamic LDS, per device and kernel
         static std::atomic<bool> done[64];
@@ -472,6 +517,13 @@ int launch_tile(const TileArgs &a, unsigned grid, size_t lds_bytes, hipStream_t 
     return (int)hipGetLastError();
 }
 
+TileArgs<kMaxSources> no_matrices()
+{
+    TileArgs<kMaxSources> a{};
+    for (TileSource &m : a.source) m.first = 0x7fffffff;
+    return a;
+}
+
 size_t tile_lds_bytes(const TileShape &s)
 {
     const size_t dense = kTileFront + 2 * (size_t)(16 * s.row_tiles) * ((size_t)s.chunk * 2 + kTilePad * 2);
@@ -479,7 +531,7 @@ size_t tile_lds_bytes(const TileShape &s)
     return dense > sums ? dense : sums;
 }
 
-int launch_tile_shape(TileArgs a, const TileShape &s, int max_lds, hipStream_t stream)
+int launch_tile_shape(TileArgs<kMaxSources> a, const TileShape &s, int max_lds, hipStream_t stream)
 {
     const int groups = 1 << s.group_shift, parts = kTileWaves / groups;
     const size_t lds = tile_lds_bytes(s);
@@ -494,15 +546,19 @@ int launch_tile_shape(TileArgs a, const TileShape &s, int max_lds, hipStream_t s
     a.group_shift = s.group_shift;
     const int vectors = 16 * s.wave_tiles * groups;
     a.vector_blocks = (a.batch + vectors - 1) / vectors;
-    a.vector_store = (a.ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 7) == 0) ? 1 : 0;
+    const bool several = a.source[1].first < a.rows;
+    a.vector_store = 1;
+    for (const TileSource &m : a.source)
+        if (m.first < a.rows && (m.ldy % 4 != 0 || (reinterpret_cast<uintptr_t>(m.y) & 7) != 0)) a.vector_store = 0;
     const long long grid = s.row_blocks * a.vector_blocks;
     if (grid >= (1ll << 31)) return MACKO_E_INVALID_ARGUMENT;
     a.packed_tiles = packed_tiles(a.batch);
     a.packed_steps = packed_steps(a.cols);
-#define MACKO_TILE(RT_, NTW_, SC_)                                                                          \
-    if (s.row_tiles == RT_ && s.wave_tiles == NTW_ && s.steps == SC_) {                                     \
-        if (a.packed != nullptr) return launch_tile<RT_, NTW_, SC_, true>(a, (unsigned)grid, lds, stream);  \
-        return launch_tile<RT_, NTW_, SC_, false>(a, (unsigned)grid, lds, stream);                          \
+#define MACKO_TILE(RT_, NTW_, SC_)                                                                                 \
+    if (s.row_tiles == RT_ && s.wave_tiles == NTW_ && s.steps == SC_) {                                            \
+        if (several) return launch_tile<RT_, NTW_, SC_, true, true>(a, (unsigned)grid, lds, stream);               \
+        if (a.packed != nullptr) return launch_tile<RT_, NTW_, SC_, true, false>(a, (unsigned)grid, lds, stream);  \
+        return launch_tile<RT_, NTW_, SC_, false, false>(a, (unsigned)grid, lds, stream);                          \
     }
     MACKO_TILE(1, 1, 1) MACKO_TILE(2, 1, 1) MACKO_TILE(3, 1, 1)
     MACKO_TILE(1, 1, 2) MACKO_TILE(2, 1, 2) MACKO_TILE(3, 1, 2)
@@ -616,18 +672,13 @@ size_t spmv_tile_workspace(int cols, int batch, const void *x, long long ldx)
 
 int spmv_tile_launch(const SpmvArgs &args, int batch, const TileShape &shape, void *workspace, const DeviceInfo &info, hipStream_t stream)
 {
-    TileArgs a{};
-    a.values = args.values;
-    a.deltas = args.deltas;
-    a.row_ptr = args.row_ptr;
+    TileArgs<kMaxSources> a = no_matrices();
+    a.source[0] = TileSource{args.values, args.deltas, args.row_ptr, args.y, 0, (u32)args.padded, (u32)args.ldy};
     a.x = args.x;
-    a.y = args.y;
     a.rows = args.rows;
     a.cols = args.cols;
     a.batch = batch;
-    a.padded = (u32)args.padded;
     a.ldx = (u32)args.ldx;
-    a.ldy = (u32)args.ldy;
     if (workspace != nullptr) {
         const int e = spmv_tile_pack(args.x, args.cols, batch, args.ldx, workspace, stream);
         if (e != 0) return e;
@@ -644,6 +695,52 @@ int spmv_tile_pack(const uint16_t *x, int cols, int batch, long long ldx, void *
     return (int)hipGetLastError();
 }
 
+}  // namespace macko
+
+namespace macko {
+namespace {
+
+int packed_product(const macko_packed_matrix *matrices, int n, const void *packed, const void *residual, int cols, int batch, void *stream)
+{
+    if (matrices == nullptr || n < 1 || n > kMaxSources || cols < 64 || batch < 1 || (n > 1 && residual != nullptr)) return MACKO_E_INVALID_ARGUMENT;
+    TileArgs<kMaxSources> a = no_matrices();
+    long long rows = 0, padded = 0;
+    int used = 0;
+    for (int k = 0; k < n; ++k) {
+        const macko_packed_matrix &m = matrices[k];
+        if (m.rows < 0 || m.padded_entries < 0 || m.padded_entries % kChunk != 0 || m.padded_entries >= (1ll << 31) - 8192 ||
+            m.ldy < m.rows || m.ldy >= (1ll << 31))
+            return MACKO_E_INVALID_ARGUMENT;
+        if (m.rows == 0) continue;
+        if (m.row_ptr == nullptr || m.y == nullptr || packed == nullptr ||
+            (m.padded_entries > 0 && (m.values == nullptr || m.deltas == nullptr)) || packed_bytes(cols, batch) >= (1ull << 32))
+            return MACKO_E_INVALID_ARGUMENT;
+        if ((reinterpret_cast<uintptr_t>(m.values) & 15) || (reinterpret_cast<uintptr_t>(m.deltas) & 3) ||
+            (reinterpret_cast<uintptr_t>(m.row_ptr) & 3) || (reinterpret_cast<uintptr_t>(packed) & 15) ||
+            (reinterpret_cast<uintptr_t>(residual) & 1) || (reinterpret_cast<uintptr_t>(m.y) & 1))
+            return MACKO_E_INVALID_ARGUMENT;
+        if (rows % kRowUnit != 0) return MACKO_E_INVALID_ARGUMENT;  // the matrix in front does not end on a whole unit
+        a.source[used++] = TileSource{(const u32 *)m.values, (const u32 *)m.deltas, m.row_ptr, (uint16_t *)m.y, (int)rows,
+                                      (u32)m.padded_entries, (u32)m.ldy};
+        rows += m.rows;
+        padded += m.padded_entries;
+        if (used > 1 && rows >= (1ll << 31) - kRowUnit) return MACKO_E_INVALID_ARGUMENT;
+    }
+    if (rows == 0) return 0;
+    DeviceInfo info;
+    const int rc = device_info(&info);
+    if (rc != 0) return rc;
+    a.rows = (int)rows;
+    a.cols = cols;
+    a.batch = batch;
+    a.packed = (const u32x4 *)packed;
+    a.residual = (const uint16_t *)residual;
+    TileShape shape;
+    if (!choose_tile_shape(&shape, a.rows, cols, padded, batch, true, info)) return MACKO_E_INVALID_ARGUMENT;
+    return launch_tile_shape(a, shape, info.max_lds_bytes, as_stream(stream));
+}
+
+}  // namespace
 }  // namespace macko
 
 // Products of vectors that are in operand order already: several matrices share one packing, and
@@ -671,33 +768,12 @@ extern "C" int macko_spmv_f16_packed(const void *values, const void *deltas, con
                                      int32_t batch, int64_t ldy, void *stream)
 {
     using namespace macko;
-    if (rows < 0 || cols < 64 || batch < 1 || padded_entries < 0 || padded_entries % kChunk != 0 ||
-        padded_entries >= (1ll << 31) - 8192 || ldy < rows || ldy >= (1ll << 31))
-        return MACKO_E_INVALID_ARGUMENT;
-    if (rows == 0) return 0;
-    if (row_ptr == nullptr || y == nullptr || packed == nullptr || (padded_entries > 0 && (values == nullptr || deltas == nullptr)) ||
-        packed_bytes(cols, batch) >= (1ull << 32))
-        return MACKO_E_INVALID_ARGUMENT;
-    if ((reinterpret_cast<uintptr_t>(values) & 15) || (reinterpret_cast<uintptr_t>(deltas) & 3) ||
-        (reinterpret_cast<uintptr_t>(row_ptr) & 3) || (reinterpret_cast<uintptr_t>(packed) & 15) ||
-        (reinterpret_cast<uintptr_t>(residual) & 1) || (reinterpret_cast<uintptr_t>(y) & 1))
-        return MACKO_E_INVALID_ARGUMENT;
-    DeviceInfo info;
-    const int rc = device_info(&info);
-    if (rc != 0) return rc;
-    TileArgs a{};
-    a.values = (const u32 *)values;
-    a.deltas = (const u32 *)deltas;
-    a.row_ptr = row_ptr;
-    a.y = (uint16_t *)y;
-    a.rows = rows;
-    a.cols = cols;
-    a.batch = batch;
-    a.padded = (u32)padded_entries;
-    a.ldy = (u32)ldy;
-    a.packed = (const u32x4 *)packed;
-    a.residual = (const uint16_t *)residual;
-    TileShape shape;
-    if (!choose_tile_shape(&shape, rows, cols, padded_entries, batch, true, info)) return MACKO_E_INVALID_ARGUMENT;
-    return launch_tile_shape(a, shape, info.max_lds_bytes, as_stream(stream));
+    const macko_packed_matrix one = {values, deltas, row_ptr, y, rows, padded_entries, ldy};
+    return packed_product(&one, 1, packed, residual, cols, batch, stream);
+}
+
+extern "C" int macko_spmv_f16_packed_several(const macko_packed_matrix *matrices, int32_t n_matrices, const void *packed,
+                                             int32_t cols, int32_t batch, void *stream)
+{
+    return macko::packed_product(matrices, n_matrices, packed, nullptr, cols, batch, stream);
 }

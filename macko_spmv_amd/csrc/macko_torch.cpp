@@ -615,6 +615,37 @@ at::Tensor multiply_packed_hip(const at::Tensor &M_values, const at::Tensor &M_d
     return Y;
 }
 
+// The same for several matrices of M_cols columns in one launch -> one [batch, rows] per matrix.  All but the last
+// have a multiple of four rows.
+std::vector<at::Tensor> multiply_packed_several_hip(at::TensorList M_values, at::TensorList M_deltas, at::TensorList M_row_indices,
+                                                    at::IntArrayRef M_rows, int64_t M_cols, const at::Tensor &packed, int64_t batch)
+{
+    const size_t n = M_values.size();
+    TORCH_CHECK(n >= 1 && n <= MACKO_PACKED_MATRICES && M_deltas.size() == n && M_row_indices.size() == n && M_rows.size() == n,
+                "one to ", MACKO_PACKED_MATRICES, " matrices");
+    check_half_gpu(packed, "packed");
+    int64_t bytes = 0;
+    TORCH_CHECK(batch >= 1 && batch < (1ll << 31), "bad batch");
+    check_rc(macko_packed_bytes((int32_t)M_cols, (int32_t)batch, &bytes), "multiply_packed_several");
+    TORCH_CHECK(packed.numel() * 2 == bytes, "packed must hold `batch` vectors of M_cols elements");
+    for (size_t i = 0; i < n; ++i) {
+        check_macko_operands(M_values[i], M_deltas[i], M_row_indices[i], M_rows[i], M_cols);
+        TORCH_CHECK(M_values[i].device() == packed.device(), "the matrices and the vectors must live on one GPU");
+        TORCH_CHECK(i + 1 == n || M_rows[i] % 4 == 0, "all matrices but the last must have a multiple of four rows");
+    }
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(packed.device());
+    std::vector<at::Tensor> Y;
+    macko_packed_matrix matrices[MACKO_PACKED_MATRICES];
+    for (size_t i = 0; i < n; ++i) {
+        Y.push_back(at::empty({batch, M_rows[i]}, M_values[i].options()));
+        matrices[i] = {M_values[i].data_ptr(), M_deltas[i].data_ptr(), M_row_indices[i].data_ptr<int>(), Y[i].data_ptr(),
+                       (int32_t)M_rows[i], M_values[i].numel(), M_rows[i]};
+    }
+    check_rc(macko_spmv_f16_packed_several(matrices, (int32_t)n, packed.data_ptr(), (int32_t)M_cols, (int32_t)batch, current_stream()),
+             "multiply_packed_several");
+    return Y;
+}
+
 void check_caches(const at::Tensor &k_cache, const at::Tensor &v_cache, const at::Tensor &positions, int64_t batch, int64_t width)
 {
     check_half_gpu(k_cache, "k_cache");
@@ -707,6 +738,8 @@ TORCH_LIBRARY(macko_spmv, m)
     m.def("pack_silu_mul(Tensor gate, Tensor up) -> Tensor");
     m.def("multiply_packed(Tensor M_values, Tensor M_deltas, Tensor M_row_indices, int M_rows, int M_cols, "
           "Tensor packed, SymInt batch, Tensor? residual) -> Tensor");
+    m.def("multiply_packed_several(Tensor[] M_values, Tensor[] M_deltas, Tensor[] M_row_indices, int[] M_rows, int M_cols, "
+          "Tensor packed, SymInt batch) -> Tensor[]");
     m.def("prefill_rope_append(Tensor(a!) q, Tensor k, Tensor v, Tensor cos_rows, Tensor sin_rows, Tensor positions, "
           "Tensor(b!) k_cache, Tensor(c!) v_cache) -> ()");
     m.def("prefill_attention(Tensor q, Tensor k_cache, Tensor v_cache, Tensor positions, float scale) -> Tensor");
@@ -738,6 +771,7 @@ TORCH_LIBRARY_IMPL(macko_spmv, CUDA, m)
     m.impl("rmsnorm_rows", &rmsnorm_rows_hip);
     m.impl("pack_silu_mul", &pack_silu_mul_hip);
     m.impl("multiply_packed", &multiply_packed_hip);
+    m.impl("multiply_packed_several", &multiply_packed_several_hip);
     m.impl("prefill_rope_append", &prefill_rope_append_hip);
     m.impl("prefill_attention", &prefill_attention_hip);
     m.impl("decompress", &decompress_hip);

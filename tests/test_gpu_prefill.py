@@ -108,6 +108,32 @@ def test_product_of_packed_vectors_with_residual(batch, rows, cols):
         assert (np.abs(y - want) <= bound).all()
 
 
+@pytest.mark.parametrize("batch,rows,cols,density", [(2, (4, 0, 7), 64, 0.5), (17, (100, 52, 333), 200, 0.4), (128, (512, 512, 512), 1000, 0.1),
+                                                     (100, (1376, 1377), 512, 0.5), (33, (4096, 8, 4100), 640, 0.05), (130, (48, 4), 4104, 0.9),
+                                                     (64, (12400, 12400), 128, 0.3), (5, (21,), 72, 0.4)])
+def test_product_of_packed_vectors_with_several_matrices(batch, rows, cols, density):
+    rng = np.random.default_rng(sum(rows))
+    dense = [helpers.random_sparse(rng, r, cols, density) for r in rows]
+    c = [mk.compress(torch.from_numpy(d).cuda()) for d in dense]
+    x = rng.standard_normal((batch, cols)).astype(np.float16)
+    x[batch - 1, 3] = np.inf     # sums that are not finite are computed again, from their own matrix
+    up = torch.full((batch, cols), 30.0, device="cuda", dtype=torch.float16)
+    packed = ops.pack_silu_mul(torch.from_numpy(x).cuda(), up)
+    staged = _unpack(packed, cols, batch)[0].cpu().numpy().astype(np.float64)
+    got = ops.multiply_packed_several([m[0] for m in c], [m[1] for m in c], [m[2] for m in c], list(rows), cols, packed, batch)
+    assert [tuple(y.shape) for y in got] == [(batch, r) for r in rows]
+    for y, d in zip(got, dense):
+        y, d64 = y.cpu().double().numpy(), d.astype(np.float64)
+        used = d64[:, 3] != 0                    # rows that multiply the infinite element
+        finite = np.ones_like(y, dtype=bool)
+        finite[batch - 1, used] = False
+        assert not np.isfinite(y[~finite]).any() and np.isfinite(y[finite]).all()
+        x64 = np.where(np.isfinite(staged), staged, 0.0)
+        want = x64 @ d64.T
+        bound = 2.0 ** -11 * np.abs(want) + 2.0 ** -25 + (cols + 3) * 2.0 ** -24 * (np.abs(x64) @ np.abs(d64).T)
+        assert (np.abs(y - want) <= bound)[finite].all()
+
+
 @pytest.mark.parametrize("batch,rows,cols,offset,ldx", [(1, 40, 64, 0, 64), (17, 333, 200, 3, 211), (40, 100, 71, 1, 72)])
 def test_packing_and_residual_in_place_through_the_c_abi(batch, rows, cols, offset, ldx):
     vp, i32, i64 = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64
