@@ -322,6 +322,7 @@ struct TileShape {
     int group_shift;   // log2 of the vector groups of a workgroup
     long long row_blocks;
     int chunk;         // columns per chunk
+    int lane_entries;  // spmv_pipe_kernel: entries a lane takes at once; 0: spmv_tile_kernel
 };
 
 // The kernel for several vectors on the matrix cores (macko_spmv_tile.hip): whether it can do a product,

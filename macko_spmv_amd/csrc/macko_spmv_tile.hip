@@ -20,7 +20,7 @@
 // of X per row block; the gather kernels read LDS once per entry for a few vectors and stream the
 // matrix again for the next few.  Measured on 11008 x 4096 at density 0.5, 128 vectors: 341 us through the
 // gather kernels in groups of eight (17 TFLOP/s), 27.4 here (211 TFLOP/s of stored entries, twice that
-// on the matrix cores).  What bounds it now: no unit alone.  Of the 54500 cycles a wave of that launch lives
+// on the matrix cores; 25.2 by spmv_pipe_kernel below, which takes such products now).  What bounds it: no unit alone.  Of the 54500 cycles a wave of that launch lives
 // the vector units are busy 25000 (decoding), LDS 28300 (12400 of them bank conflicts) and the matrix cores
 // 12300, by the counters; waves wait for 40 % of their cycles, for one another and for X out of L2.
 //
@@ -28,6 +28,7 @@
 // (it never reads columns without an entry).  Such a product can only make a sum non-finite, so every
 // sum that is not finite is computed again from its row's entries alone.
 #include <atomic>
+#include <cmath>
 
 #include "macko_packed.h"
 #include "macko_spmv_detail.h"
@@ -132,6 +133,91 @@ __device__ __forceinline__ float exact_row_times_vector(const u32 *values, const
     return wave_sum(acc);
 }
 
+// The matrix a row of the launch belongs to.
+template <bool SEVERAL, int SOURCES>
+__device__ __forceinline__ int source_of(const TileArgs<SOURCES> &a, int row)
+{
+    int m = 0;
+    if constexpr (SEVERAL)
+        for (int k = 1; k < SOURCES; ++k) m += row >= a.source[k].first ? 1 : 0;
+    return m;
+}
+
+// The end of a launch: the partial sums of every tile of 16 rows and 16 vectors lie in LDS at `red`
+// ([row tile][vector tile][part], 1 KB each), are added in a fixed order and stored.
+template <bool PACKED, bool SEVERAL, int SOURCES>
+__device__ __forceinline__ void finish_tiles(const TileArgs<SOURCES> &a, u32 red, int n_tiles, int vector_tiles, int parts, int vector0,
+                                             int row0, int row1)
+{
+    typedef __attribute__((address_space(3))) u32x4 *lds_w32x4;
+    const int lane = threadIdx.x & (kWave - 1), wave = uniform(threadIdx.x >> 6), sub = lane & 15, quarter = lane >> 4;
+    for (int tile = wave; tile < n_tiles; tile += kTileWaves) {
+        float4v sum = float4v{0.f, 0.f, 0.f, 0.f};
+        for (int p = 0; p < parts; ++p)
+            sum += __builtin_bit_cast(float4v, *(lds_w32x4)(uintptr_t)(red + (u32)(tile * parts + p) * 1024 + (u32)lane * 16));
+        const int r = tile / vector_tiles;
+        const int n = vector0 + (tile - r * vector_tiles) * 16 + sub;
+        const int row = row0 + r * 16 + quarter * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float one = sum[i];
+            const u32 bits = __builtin_bit_cast(u32, one);
+            unsigned long long bad = __ballot(n < a.batch && row + i < row1 && (bits & 0x7f800000u) == 0x7f800000u);
+            while (__builtin_expect(bad != 0, 0)) {
+                const int L = __builtin_ctzll(bad);
+                bad &= bad - 1;
+                const int bad_row = __builtin_amdgcn_readlane(row, L) + i;
+                const int bad_n = __builtin_amdgcn_readlane(n, L);
+                const TileSource &m = a.source[source_of<SEVERAL>(a, bad_row)];
+                const int *row_ptr = m.row_ptr + (SEVERAL ? bad_row - m.first : bad_row);
+                u32 e0 = (u32)uniform(row_ptr[0]), e1 = (u32)uniform(row_ptr[1]);
+                e0 = e0 < m.padded ? e0 : m.padded;
+                e1 = e1 < m.padded ? e1 : m.padded;
+                const float exact = exact_row_times_vector(
+                    m.values, m.deltas, e0, e1,
+                    [&](int c) {
+                        if constexpr (PACKED)
+                            return reinterpret_cast<const uint16_t *>(a.packed + packed_piece(c >> 3, bad_n, a.packed_tiles))[c & 7];
+                        else
+                            return a.x[(size_t)bad_n * a.ldx + (size_t)c];
+                    },
+                    a.cols);
+                sum[i] = lane == L ? exact : sum[i];
+            }
+        }
+        if (n < a.batch) {
+            uint16_t *y = a.source[0].y;
+            u32 ldy = a.source[0].ldy;
+            int at = row;
+            if constexpr (SEVERAL) {  // my four rows are of one matrix
+#pragma unroll
+                for (int k = 1; k < kMaxSources; ++k)
+                    if (row >= a.source[k].first) {
+                        y = a.source[k].y;
+                        ldy = a.source[k].ldy;
+                        at = row - a.source[k].first;
+                    }
+            }
+            uint16_t *dst = y + (size_t)n * ldy + at;
+            if (!SEVERAL && a.residual != nullptr) {
+                const uint16_t *add = a.residual + (size_t)n * ldy + row;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (row + i < row1) sum[i] += half_bits_to_float(add[i]);
+            }
+            if (a.vector_store && row + 4 <= row1) {
+                const u32 lo = (u32)float_to_half_bits(sum[0]) | ((u32)float_to_half_bits(sum[1]) << 16);
+                const u32 hi = (u32)float_to_half_bits(sum[2]) | ((u32)float_to_half_bits(sum[3]) << 16);
+                *reinterpret_cast<u32x2 *>(dst) = u32x2{lo, hi};
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (row + i < row1) dst[i] = float_to_half_bits(sum[i]);
+            }
+        }
+    }
+}
+
 // X in operand order (macko_packed.h).  A wave packs one block.
 __global__ void __launch_bounds__(256) pack_vectors_kernel(const uint16_t *__restrict__ x, u32x4 *__restrict__ packed,
                                                            int cols, int batch, u32 ldx, int tiles, int blocks)
@@ -185,12 +271,6 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs<
     const int part = wave >> a.group_shift;
     const int parts = kTileWaves >> a.group_shift;
 
-    auto source_of = [&](int row) __attribute__((always_inline)) {
-        int m = 0;
-        if constexpr (SEVERAL)
-            for (int k = 1; k < kMaxSources; ++k) m += row >= a.source[k].first ? 1 : 0;
-        return m;
-    };
     __amdgpu_buffer_rsrc_t rs_values[SEVERAL ? RT : 1], rs_deltas[SEVERAL ? RT : 1];
     auto describe = [&](int slot, const TileSource &m) __attribute__((always_inline)) {
         rs_values[slot] = __builtin_amdgcn_make_buffer_rsrc((void *)m.values, 0, (int)(m.padded * 2), 0x00020000);
@@ -215,7 +295,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs<
     static_for<RT>([&](auto slot) {
         constexpr int J = decltype(slot)::value;
         const int row = row0 + wave + 16 * J;
-        const TileSource &m = a.source[source_of(row)];
+        const TileSource &m = a.source[source_of<SEVERAL>(a, row)];
         if constexpr (SEVERAL) describe(J, m);
         u32 e0 = 0, e1 = 0;
         if (row < row1) {
@@ -425,81 +505,270 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs<
             *(lds_w32x4)(uintptr_t)(red + slot * 1024 + (u32)lane * 16) = __builtin_bit_cast(u32x4, acc[r][t]);
         }
     lds_barrier();
-    const int n_tiles = RT * groups * NTW;
-    for (int tile = wave; tile < n_tiles; tile += kTileWaves) {
-        float4v sum = float4v{0.f, 0.f, 0.f, 0.f};
-        for (int p = 0; p < parts; ++p)
-            sum += __builtin_bit_cast(float4v, *(lds_w32x4)(uintptr_t)(red + (u32)(tile * parts + p) * 1024 + (u32)lane * 16));
-        const int r = tile / (groups * NTW);
-        const int n = vector0 + (tile - r * groups * NTW) * 16 + sub;
-        const int row = row0 + r * 16 + quarter * 4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float one = sum[i];
-            const u32 bits = __builtin_bit_cast(u32, one);
-            unsigned long long bad = __ballot(n < a.batch && row + i < row1 && (bits & 0x7f800000u) == 0x7f800000u);
-            while (__builtin_expect(bad != 0, 0)) {
-                const int L = __builtin_ctzll(bad);
-                bad &= bad - 1;
-                const int bad_row = __builtin_amdgcn_readlane(row, L) + i;
-                const int bad_n = __builtin_amdgcn_readlane(n, L);
-                const TileSource &m = a.source[source_of(bad_row)];
-                const int *row_ptr = m.row_ptr + (SEVERAL ? bad_row - m.first : bad_row);
-                u32 e0 = (u32)uniform(row_ptr[0]), e1 = (u32)uniform(row_ptr[1]);
-                e0 = e0 < m.padded ? e0 : m.padded;
-                e1 = e1 < m.padded ? e1 : m.padded;
-                const float exact = exact_row_times_vector(
-                    m.values, m.deltas, e0, e1,
-                    [&](int c) {
-                        if constexpr (PACKED)
-                            return reinterpret_cast<const uint16_t *>(a.packed + packed_piece(c >> 3, bad_n, a.packed_tiles))[c & 7];
-                        else
-                            return a.x[(size_t)bad_n * a.ldx + (size_t)c];
-                    },
-                    a.cols);
-                sum[i] = lane == L ? exact : sum[i];
-            }
-        }
-        if (n < a.batch) {
-            uint16_t *y = a.source[0].y;
-            u32 ldy = a.source[0].ldy;
-            int at = row;
-            if constexpr (SEVERAL) {  // my four rows are of one matrix
-#pragma unroll
-                for (int k = 1; k < kMaxSources; ++k)
-                    if (row >= a.source[k].first) {
-                        y = a.source[k].y;
-                        ldy = a.source[k].ldy;
-                        at = row - a.source[k].first;
-                    }
-            }
-            uint16_t *dst = y + (size_t)n * ldy + at;
-            if (!SEVERAL && a.residual != nullptr) {
-                const uint16_t *add = a.residual + (size_t)n * ldy + row;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (row + i < row1) sum[i] += half_bits_to_float(add[i]);
-            }
-            if (a.vector_store && row + 4 <= row1) {
-                const u32 lo = (u32)float_to_half_bits(sum[0]) | ((u32)float_to_half_bits(sum[1]) << 16);
-                const u32 hi = (u32)float_to_half_bits(sum[2]) | ((u32)float_to_half_bits(sum[3]) << 16);
-                *reinterpret_cast<u32x2 *>(dst) = u32x2{lo, hi};
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (row + i < row1) dst[i] = float_to_half_bits(sum[i]);
-            }
-        }
-    }
+    finish_tiles<PACKED, SEVERAL>(a, red, RT * groups * NTW, groups * NTW, parts, vector0, row0, row1);
 }
 
-template <int RT, int NTW, int SC, bool PACKED, bool SEVERAL>
-int launch_tile(const TileArgs<kMaxSources> &all, unsigned grid, size_t lds_bytes, hipStream_t stream)
+// The same product with the waves in two roles: 12 of the 16 scatter (one unit of 4 rows each, 48 rows per
+// workgroup), one on every SIMD multiplies (two groups of 16 * NTW vectors, the columns of a group in two parts), and a
+// barrier per chunk hands a dense chunk over.  For enough rows to give every compute unit about 48 and more than 16
+// vectors, where spmv_tile_kernel, whose waves do both, holds a chunk's X, the sums and the entries in the same 128
+// registers and can afford neither long chunks nor more than one row per pass:
+//   - a pass works four rows at once, 16 lanes each, E consecutive entries a lane (16 * E per row and chunk; the prefix
+//     sum has four steps instead of six, and what a pass costs besides its entries is shared by four rows);
+//   - no column is clamped: rows stand 16 * E columns apart in LDS, which is as far as the entries of a lane that reaches
+//     beyond its chunk can go on either side;
+//   - entries are requested into one of two register sets as soon as it is known where the next chunk starts, in
+//     front of the stores of this one.
+// The multiplying waves run at a higher priority: a matrix instruction and a v_dot8 of another wave on the same SIMD
+// exclude each other (measured: a v_dot8 takes 18 cycles beside a stream of matrix instructions, a plain addition 10).
+// 11008 x 4096, vectors in operand order, three matrices in turn: 128 vectors at density 0.5 28.7 -> 25.2 us, 0.15
+// 28.5 -> 18.8, 0.05 27.3 -> 18.0; 64 vectors at 0.2 19.4 -> 16.9; 28672 x 1024, 64 vectors, 0.1: 23.7 -> 15.7.  What bounds it: 2.2 us
+// in front of the first product and 1.5 behind the last one (row_ptr, the first entries, the sums); between them X out of
+// L2 (128 vectors: 1 MB per compute unit, 7 us at 64 bytes a cycle) and vector and matrix instructions in turn.  Tried
+// and slower: 8 + 8 waves, both roles at one priority, a chunk's places worked out behind the stores of the one
+// before, the next unit's A requested between products, lines touched some chunks ahead.
+constexpr int kPipeProducers = 12;
+constexpr int kPipeRowTiles = 3;
+constexpr int kPipeParts = 2;          // of the columns, per group of vectors
+constexpr int kPipeGroups = 2;
+constexpr int kPipeDepth = 2;          // units of 32 columns of X a wave has in flight
+constexpr int kPipeLanes = 16;         // lanes per row of a pass
+constexpr int kPipeChunkStep = 32 * kPipeParts * kPipeDepth;  // chunks are multiples of this
+constexpr int pipe_pad(int entries) { return entries * 16 + 8; }  // columns between rows; 16-byte aligned, rows on other banks
+
+template <int NTW, int E, bool SEVERAL>
+__global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<SEVERAL ? kMaxSources : 1> a)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    typedef __attribute__((address_space(3))) u32x4 *lds_w32x4;
+    typedef __attribute__((address_space(3))) uint16_t *lds_w16;
+    constexpr int RT = kPipeRowTiles, L = kPipeLanes, W = E / 8;  // W: words of nibbles a lane has
+    static_assert(E == 8 || E == 16, "entries per lane");
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = uniform(threadIdx.x >> 6);
+
+    u32 id = blockIdx.x;  // XCD k takes the k-th contiguous eighth, as above
+    if ((gridDim.x & 7) == 0) id = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const u32 row_block = id / (u32)a.vector_blocks;
+    const int vector0 = (int)(id - row_block * (u32)a.vector_blocks) * (NTW * 16 * kPipeGroups);
+    const int row0 = (int)even_split(row_block, a.units_q, a.units_rem) * kRowUnit;
+    const int row_end_unclamped = (int)even_split(row_block + 1, a.units_q, a.units_rem) * kRowUnit;
+    const int row1 = row_end_unclamped < a.rows ? row_end_unclamped : a.rows;
+
+    const u32 stride = (u32)a.chunk * 2 + pipe_pad(E) * 2;   // bytes per row of the dense chunk
+    const u32 buffer_bytes = stride * (16 * RT);
+    const u32 red = (u32)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
+    const u32 lds0 = red + pipe_pad(E) * 2;
+    const int last = a.n_chunks - 1;
+
+    if (wave < kPipeProducers) {
+        const int l = lane & (L - 1), h = lane / L;   // lane of a row, row of the unit
+        const int unit_row = row0 + wave * kRowUnit, row = unit_row + h;
+        const TileSource &m = a.source[source_of<SEVERAL>(a, unit_row)];
+        const __amdgpu_buffer_rsrc_t rs_values = __builtin_amdgcn_make_buffer_rsrc((void *)m.values, 0, (int)(m.padded * 2), 0x00020000);
+        const __amdgpu_buffer_rsrc_t rs_deltas = __builtin_amdgcn_make_buffer_rsrc((void *)m.deltas, 0, (int)(m.padded / 2), 0x00020000);
+        u32x4 tile_v[2][W];
+        u32 tile_d[2][W];
+        int pos = 0, end = 0;   // my next entry (the row's next entry + l * E), behind the row's last entry
+        // 2 * (column behind the entry in front of the row's next) + where the row stands in the buffer
+        u32 at_column;
+        u32 front = ~0u;        // takes out the nibbles of the row before mine, in its first group of 8
+        const u32 my_row = (u32)(wave * kRowUnit + h) * stride;
+        {
+            u32 e0 = 0, e1 = 0;
+            if (row < row1) {
+                const int *row_ptr = m.row_ptr + (SEVERAL ? row - m.first : row);
+                e0 = (u32)row_ptr[0];
+                e1 = (u32)row_ptr[1];
+            }
+            e0 = e0 < m.padded ? e0 : m.padded;
+            e1 = e1 < m.padded ? e1 : m.padded;
+            pos = (int)(e0 & ~7u) + l * E;
+            end = e1 > e0 ? (int)e1 : 0;
+            at_column = my_row - 2u * (e0 & 7u);
+            if (l == 0) front = ~0u << (4 * (e0 & 7u));
+        }
+        auto request = [&](auto set) __attribute__((always_inline)) {
+            constexpr int S = decltype(set)::value;
+            const bool any = pos < end;
+            const u32 vo = any ? (u32)pos * 2 : kNoTileValues;
+            const u32 dof = any ? (u32)pos >> 1 : kNoTileDeltas;
+            if constexpr (W == 2) {  // checked word by word against the end of the array
+                const u32x2 both = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_deltas, (int)dof, 0, 0));
+                tile_d[S][0] = both.x;
+                tile_d[S][W - 1] = both.y;
+            } else {
+                tile_d[S][0] = __builtin_amdgcn_raw_buffer_load_b32(rs_deltas, (int)dof, 0, 0);
+            }
+#pragma unroll
+            for (int w = 0; w < W; ++w)
+                tile_v[S][w] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_values, (int)vo, 16 * w, 0));
+        };
+        u32 base = 0, buffer = 0, shift = 0;
+        // Where my entries of set S go in this chunk, and which of the row's lanes belong to later ones: pos and
+        // at_column move on.  True: a row has more entries in the chunk than a pass holds.
+        auto place = [&](auto set) __attribute__((always_inline)) -> bool {
+            constexpr int S = decltype(set)::value;
+            tile_d[S][0] &= front;
+            const int left = end - pos;
+            if (__builtin_expect(__ballot(left > 0 && left < E) != 0, 0)) {  // entries behind the row's end: zeros, at columns nothing else takes
+#pragma unroll
+                for (int w = 0; w < 4 * W; ++w) {
+                    const u32 keep = left >= 2 * w + 2 ? ~0u : (left == 2 * w + 1 ? 0xffffu : 0u);
+                    tile_v[S][w >> 2][w & 3] &= keep;
+                }
+            }
+            u32 step = 2u * E;
+#pragma unroll
+            for (int w = 0; w < W; ++w) step = __builtin_amdgcn_udot8(tile_d[S][w], 0x22222222u, step, false);
+            u32 incl = step;  // sum over the lanes of the row up to mine
+            incl += (u32)__builtin_amdgcn_update_dpp(0, (int)incl, 0x111, 0xF, 0xF, true);   // row_shr:1
+            incl += (u32)__builtin_amdgcn_update_dpp(0, (int)incl, 0x112, 0xF, 0xF, true);
+            incl += (u32)__builtin_amdgcn_update_dpp(0, (int)incl, 0x114, 0xF, 0xF, true);
+            incl += (u32)__builtin_amdgcn_update_dpp(0, (int)incl, 0x118, 0xF, 0xF, true);
+            const u32 origin = at_column + shift;
+            const int hi = (int)(my_row + (buffer + (u32)a.chunk * 2));
+            base = left > 0 ? origin + (incl - step) : 0x7ffffff0u;
+            // the last lane whose last entry still belongs to this chunk: what it adds to the column and its number grow together
+            int key = (int)(origin + incl) - 2 >= hi ? 0 : (int)(incl << 8 | (u32)(l + 1));
+            auto larger = [&](int o) { key = o > key ? o : key; };
+            larger(__builtin_amdgcn_update_dpp(0, key, 0xB1, 0xF, 0xF, true));    // quad_perm 1,0,3,2
+            larger(__builtin_amdgcn_update_dpp(0, key, 0x4E, 0xF, 0xF, true));    // quad_perm 2,3,0,1
+            larger(__builtin_amdgcn_update_dpp(0, key, 0x141, 0xF, 0xF, true));   // row_half_mirror
+            larger(__builtin_amdgcn_update_dpp(0, key, 0x140, 0xF, 0xF, true));   // row_mirror
+            const int done = key & 0xff;   // lanes
+            pos += done * E;
+            at_column += (u32)key >> 8;
+            front = done ? ~0u : front;
+            return __ballot(done == L && pos < end) != 0;
+        };
+        auto write = [&](auto set) __attribute__((always_inline)) {
+            constexpr int S = decltype(set)::value;
+            const int hi = (int)(my_row + (buffer + (u32)a.chunk * 2));
+            if ((int)base < hi) {  // lanes wholly behind the chunk write nothing
+                u32 at[E];
+                u32 from = base;
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) at[8 * w + k] = __builtin_amdgcn_udot8(tile_d[S][w], twos_upto(k), from, false);
+                    from = at[8 * w + 7];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < E; ++k) {
+                    const u32 w = tile_v[S][k >> 3][(k >> 1) & 3];
+                    *(lds_w16)(uintptr_t)(at[k] + 2u * k) = (uint16_t)((k & 1) ? w >> 16 : w);
+                }
+            }
+        };
+        request(index_constant<0>{});
+        const u32 my_rows = (u32)(wave * kRowUnit) * stride + (u32)lane * 16;
+        auto scatter = [&](auto set, int c) __attribute__((always_inline)) {
+            constexpr int S = decltype(set)::value;
+            constexpr index_constant<1 - S> other{};
+            buffer = lds0 + (S ? buffer_bytes : 0u);
+            shift = buffer - (u32)(c * a.chunk) * 2;
+            bool more = place(set);
+            request(other);
+            __builtin_amdgcn_sched_barrier(0);
+            u32 z = buffer + my_rows;   // my four rows and what is between them, zero
+            int left = (int)stride * kRowUnit - 1024;
+            for (; left >= 0; left -= 1024) {
+                *(lds_w32x4)(uintptr_t)z = u32x4{0u, 0u, 0u, 0u};
+                z += 1024;
+            }
+            if (lane * 16 < left + 1024) *(lds_w32x4)(uintptr_t)z = u32x4{0u, 0u, 0u, 0u};
+            write(set);
+            while (__builtin_expect(more, 0)) {
+                more = place(other);
+                write(other);
+                request(other);
+            }
+            lds_barrier();
+        };
+        for (int c = 0;; c += 2) {
+            scatter(index_constant<0>{}, c);
+            if (c >= last) break;
+            scatter(index_constant<1>{}, c + 1);
+            if (c + 1 >= last) break;
+        }
+        lds_barrier();
+    } else {
+        __builtin_amdgcn_s_setprio(1);
+        const int sub = lane & 15, quarter = lane >> 4;
+        const int group = wave & 1, part = (wave >> 1) & 1;
+        float4v acc[RT][NTW];
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int t = 0; t < NTW; ++t) acc[r][t] = float4v{0.f, 0.f, 0.f, 0.f};
+        // A unit is 32 columns: half (u & 1) of the 64-column block u >> 1 of the operand order.  Mine are every
+        // other one: the same half of every block.  Beyond the last block it is requested again, for columns
+        // that hold zeros.
+        u32x4 b[kPipeDepth][NTW];
+        const __amdgpu_buffer_rsrc_t rs_x =
+            __builtin_amdgcn_make_buffer_rsrc((void *)a.packed, 0, (int)((u32)(a.packed_tiles * a.packed_steps) * (kBlockPieces * 16)), 0x00020000);
+        int x_of[NTW];
+#pragma unroll
+        for (int t = 0; t < NTW; ++t) {
+            int tile = (vector0 >> 4) + group * NTW + t;
+            tile = tile < a.packed_tiles ? tile : a.packed_tiles - 1;
+            x_of[t] = (tile * kBlockPieces + part * 64 + lane) * 16;
+        }
+        const u32 x_step = (u32)a.packed_tiles * (kBlockPieces * 16), x_last = (u32)(a.packed_steps - 1) * x_step;
+        u32 x_at = 0;
+        auto request = [&](auto slot) __attribute__((always_inline)) {
+            constexpr int J = decltype(slot)::value;
+#pragma unroll
+            for (int t = 0; t < NTW; ++t)
+                b[J][t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_x, x_of[t], (int)x_at, 0));
+            x_at = x_at < x_last ? x_at + x_step : x_last;
+            __builtin_amdgcn_sched_barrier(0);  // the waits count on this order
+        };
+        static_for<kPipeDepth>([&](auto slot) { request(slot); });
+        lds_barrier();
+        const u32 mine = lds0 + (u32)sub * stride + (u32)quarter * 32 + (u32)part * 16;
+        for (int c = 0; c <= last; ++c) {
+            u32 at = mine + (c & 1 ? buffer_bytes : 0u);
+            for (int u = 0; u < a.chunk; u += kPipeChunkStep) {
+                static_for<kPipeDepth>([&](auto slot) {
+                    constexpr int J = decltype(slot)::value;
+                    u32x4 av[RT];
+#pragma unroll
+                    for (int r = 0; r < RT; ++r) av[r] = *(lds_w32x4)(uintptr_t)(at + (u32)(16 * r) * stride);
+                    at += 128;
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int r = 0; r < RT; ++r)
+#pragma unroll
+                        for (int t = 0; t < NTW; ++t)
+                            acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, av[r]),
+                                                                               __builtin_bit_cast(half8, b[J][t]), acc[r][t], 0, 0, 0);
+                    request(slot);
+                });
+            }
+            lds_barrier();
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int t = 0; t < NTW; ++t) {
+                const u32 slot = (u32)((r * kPipeGroups + group) * NTW + t) * (u32)kPipeParts + (u32)part;
+                *(lds_w32x4)(uintptr_t)(red + slot * 1024 + (u32)lane * 16) = __builtin_bit_cast(u32x4, acc[r][t]);
+            }
+        __builtin_amdgcn_s_setprio(0);
+    }
+    lds_barrier();
+    finish_tiles<true, SEVERAL>(a, red, RT * kPipeGroups * NTW, kPipeGroups * NTW, kPipeParts, vector0, row0, row1);
+}
+
+template <bool SEVERAL, auto KERNEL>
+int launch_with(const TileArgs<kMaxSources> &all, unsigned grid, size_t lds_bytes, hipStream_t stream)
 {
     TileArgs<SEVERAL ? kMaxSources : 1> a;
     static_cast<TileCommon &>(a) = all;
     for (int k = 0; k < (SEVERAL ? kMaxSources : 1); ++k) a.source[k] = all.source[k];
-    auto kernel = spmv_tile_kernel<RT, NTW, SC, PACKED, SEVERAL>;
     if (lds_bytes > 64 * 1024) {
         // one-time opt-in to more than 64 KiB of dynamic LDS, per device and kernel
         static std::atomic<bool> done[64];
@@ -507,14 +776,20 @@ int launch_tile(const TileArgs<kMaxSources> &all, unsigned grid, size_t lds_byte
         hipError_t e = hipGetDevice(&dev);
         if (e != hipSuccess) return (int)e;
         if (dev < 0 || dev >= 64 || !done[dev].load(std::memory_order_acquire)) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERNEL),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess) return (int)e;
             if (dev >= 0 && dev < 64) done[dev].store(true, std::memory_order_release);
         }
     }
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kTileThreads), lds_bytes, stream, a);
+    hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(kTileThreads), lds_bytes, stream, a);
     return (int)hipGetLastError();
+}
+
+template <int RT, int NTW, int SC, bool PACKED, bool SEVERAL>
+int launch_tile(const TileArgs<kMaxSources> &a, unsigned grid, size_t lds_bytes, hipStream_t stream)
+{
+    return launch_with<SEVERAL, spmv_tile_kernel<RT, NTW, SC, PACKED, SEVERAL>>(a, grid, lds_bytes, stream);
 }
 
 TileArgs<kMaxSources> no_matrices()
@@ -522,6 +797,14 @@ TileArgs<kMaxSources> no_matrices()
     TileArgs<kMaxSources> a{};
     for (TileSource &m : a.source) m.first = 0x7fffffff;
     return a;
+}
+
+size_t pipe_lds_bytes(const TileShape &s)
+{
+    const size_t pad = 2 * (size_t)pipe_pad(s.lane_entries);
+    const size_t dense = pad + 2 * (size_t)(16 * kPipeRowTiles) * (2 * (size_t)s.chunk + pad);
+    const size_t sums = (size_t)kPipeRowTiles * s.wave_tiles * kPipeGroups * kPipeParts * 1024;
+    return dense > sums ? dense : sums;
 }
 
 size_t tile_lds_bytes(const TileShape &s)
@@ -533,11 +816,13 @@ size_t tile_lds_bytes(const TileShape &s)
 
 int launch_tile_shape(TileArgs<kMaxSources> a, const TileShape &s, int max_lds, hipStream_t stream)
 {
-    const int groups = 1 << s.group_shift, parts = kTileWaves / groups;
-    const size_t lds = tile_lds_bytes(s);
+    const bool pipe = s.lane_entries > 0;
+    const int groups = pipe ? kPipeGroups : 1 << s.group_shift, parts = kTileWaves / groups;
+    const size_t lds = pipe ? pipe_lds_bytes(s) : tile_lds_bytes(s);
     const long long units = (a.rows + kRowUnit - 1) / kRowUnit;
-    if (lds > (size_t)max_lds || s.chunk % 64 != 0 || s.chunk <= 0 || s.chunk > 64 * parts * s.steps || s.row_blocks < 1 ||
-        (units + s.row_blocks - 1) / s.row_blocks > 4 * s.row_tiles)
+    if (lds > (size_t)max_lds || s.chunk <= 0 || s.row_blocks < 1 ||
+        (pipe ? s.chunk % kPipeChunkStep != 0 || a.packed == nullptr : s.chunk % 64 != 0 || s.chunk > 64 * parts * s.steps) ||
+        (units + s.row_blocks - 1) / s.row_blocks > 4 * (pipe ? kPipeRowTiles : s.row_tiles))
         return MACKO_E_INVALID_ARGUMENT;
     a.chunk = s.chunk;
     a.n_chunks = (a.cols + s.chunk - 1) / s.chunk;
@@ -554,8 +839,15 @@ int launch_tile_shape(TileArgs<kMaxSources> a, const TileShape &s, int max_lds, 
     if (grid >= (1ll << 31)) return MACKO_E_INVALID_ARGUMENT;
     a.packed_tiles = packed_tiles(a.batch);
     a.packed_steps = packed_steps(a.cols);
+#define MACKO_PIPE(NTW_, E_)                                                                                       \
+    if (pipe && s.wave_tiles == NTW_ && s.lane_entries == E_) {                                                    \
+        if (several) return launch_with<true, spmv_pipe_kernel<NTW_, E_, true>>(a, (unsigned)grid, lds, stream);   \
+        return launch_with<false, spmv_pipe_kernel<NTW_, E_, false>>(a, (unsigned)grid, lds, stream);              \
+    }
+    MACKO_PIPE(1, 8) MACKO_PIPE(2, 8) MACKO_PIPE(4, 8) MACKO_PIPE(1, 16) MACKO_PIPE(2, 16) MACKO_PIPE(4, 16)
+#undef MACKO_PIPE
 #define MACKO_TILE(RT_, NTW_, SC_)                                                                                 \
-    if (s.row_tiles == RT_ && s.wave_tiles == NTW_ && s.steps == SC_) {                                            \
+    if (!pipe && s.row_tiles == RT_ && s.wave_tiles == NTW_ && s.steps == SC_) {                                   \
         if (several) return launch_tile<RT_, NTW_, SC_, true, true>(a, (unsigned)grid, lds, stream);               \
         if (a.packed != nullptr) return launch_tile<RT_, NTW_, SC_, true, false>(a, (unsigned)grid, lds, stream);  \
         return launch_tile<RT_, NTW_, SC_, false, false>(a, (unsigned)grid, lds, stream);                          \
@@ -567,7 +859,6 @@ int launch_tile_shape(TileArgs<kMaxSources> a, const TileShape &s, int max_lds, 
 #undef MACKO_TILE
     return MACKO_E_INVALID_ARGUMENT;
 }
-
 
 // Estimated cycles of a launch: what one workgroup's chunk asks of the vector units (about 60
 // instructions per row and 512 entries), of the path from L2 (X: 48 bytes a cycle from operand order,
@@ -596,7 +887,7 @@ double tile_cost(const TileShape &s, long long units, int cols, double density, 
 // where there are few rows per compute unit (4096 x 4096, density 0.5, 128 vectors: 18.3 us against
 // 20.4; 11008 x 4096: 39.4 against 28.4).
 bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info,
-                       double *cycles = nullptr)
+                       double *cycles)
 {
     const long long units = ((long long)rows + kRowUnit - 1) / kRowUnit;
     const double density = (double)padded / ((double)rows * (double)cols);
@@ -604,7 +895,7 @@ bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, in
     double least = 0.0;
     bool found = false;
     for (int shift = tiles <= 1 ? 0 : (tiles <= 4 ? 1 : 2); shift >= (tiles > 4 ? 1 : (tiles <= 1 ? 0 : 1)); --shift) {
-        TileShape s;
+        TileShape s{};
         s.group_shift = shift;
         s.wave_tiles = tiles > 2 ? 2 : 1;
         const int vectors = (16 * s.wave_tiles) << shift;
@@ -639,8 +930,68 @@ bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, in
             if (s.row_tiles == 1) break;  // smaller blocks only read X more often
         }
     }
-    if (cycles != nullptr) *cycles = least;
+    *cycles = least;
     return found;
+}
+
+// The shape of a launch of spmv_pipe_kernel and its estimated time in us.  The terms were fitted to 27000 products of
+// packed vectors (1500 to 28000 rows, 256 to 11000 columns, densities 0.05 to 0.9, 17 to 256 vectors; 7 % off in the
+// median, 16 % for one in ten): per launch, per round of workgroups, per chunk (a pass of 16 entries a lane costs
+// more than one of 8), and per column and vector.
+bool choose_pipe_shape(TileShape *shape, int rows, int cols, long long padded, int batch, const DeviceInfo &info, double *us)
+{
+    if (batch <= 16 || rows < 1 || padded < 1) return false;
+    TileShape s{};
+    s.wave_tiles = batch > 64 ? 4 : batch > 32 ? 2 : 1;
+    const int vectors = 16 * kPipeGroups * s.wave_tiles;
+    const long long blocks = (batch + vectors - 1) / vectors;
+    const long long units = ((long long)rows + kRowUnit - 1) / kRowUnit, most = 4 * kPipeRowTiles;
+    // as many workgroups as compute units, or a whole number of times that, in blocks of at most 48 rows
+    const long long rounds = (units * blocks + most * info.compute_units - 1) / (most * info.compute_units);
+    s.row_blocks = info.compute_units * rounds / blocks;
+    if (s.row_blocks * most < units) s.row_blocks = (units + most - 1) / most;
+    if (s.row_blocks > units) return false;
+    const double density = (double)padded / ((double)rows * (double)cols);
+    const int whole = (cols + kPipeChunkStep - 1) / kPipeChunkStep * kPipeChunkStep;
+    for (int e = 8; e <= 16; e += 8) {
+        s.lane_entries = e;
+        // columns per chunk: what LDS holds twice, and what a pass holds of a row's entries (with a margin for the spread
+        // between rows, for the lane that is not done and for what stands in front of the first entry)
+        const int pad = pipe_pad(e);
+        int chunk = ((info.max_lds_bytes - 2 * pad) / (2 * 16 * kPipeRowTiles) - 2 * pad) / 2 / kPipeChunkStep * kPipeChunkStep;
+        chunk = chunk < whole ? chunk : whole;
+        auto fits = [&](int c) {
+            const double mean = c * density;
+            return mean + 3.0 * std::sqrt(mean * (density < 1.0 ? 1.0 - density : 0.0)) + e + 8 <= kPipeLanes * e;
+        };
+        while (chunk > 0 && !fits(chunk)) chunk -= kPipeChunkStep;
+        if (chunk < (e == 8 ? 512 : 384) && chunk < whole) continue;
+        const int n_chunks = (cols + chunk - 1) / chunk;
+        s.chunk = ((cols + n_chunks - 1) / n_chunks + kPipeChunkStep - 1) / kPipeChunkStep * kPipeChunkStep;
+        if (pipe_lds_bytes(s) > (size_t)info.max_lds_bytes) continue;
+        const double full = (double)((s.row_blocks * blocks + info.compute_units - 1) / info.compute_units);
+        *us = 0.93 + full * (3.25 + n_chunks * ((e == 8 ? 0.31 : 0.56) + s.chunk / 512.0 * (0.31 + 0.26 * s.wave_tiles)));
+        *shape = s;
+        return true;
+    }
+    return false;
+}
+
+// The kernel and the shape of a launch, and its estimated time in us (without packing; at 2.4 GHz).  Right to about 10 %
+// where it decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1:
+// 24.4, 21).  Of the 27000 products above, the pipe kernel is taken for half, which are 22 % faster in the mean (up to
+// twice; 7 in 10000 are more than 3 % slower).
+bool choose_shape(TileShape *shape, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, double *us)
+{
+    double cycles = 0.0, pipe_us = 0.0;
+    if (!choose_tile_shape(shape, rows, cols, padded, batch, packed, info, &cycles)) return false;
+    *us = cycles * (1.06 / 2400.0);
+    TileShape pipe;
+    if (packed && choose_pipe_shape(&pipe, rows, cols, padded, batch, info, &pipe_us) && pipe_us < 0.97 * *us) {
+        *shape = pipe;
+        *us = pipe_us;
+    }
+    return true;
 }
 
 }  // namespace
@@ -653,13 +1004,10 @@ bool spmv_tile_takes(int rows, int cols, long long padded, int batch, long long 
     return (long long)batch * ldx * 2 < (1ll << 32) && (long long)packed_bytes(cols, batch) < (1ll << 32);
 }
 
-// The time by the cost above, at 2.4 GHz, and the packing launch.  Right to about 10 % on either side where it
-// decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1: 24.4, 21).
 int spmv_tile_estimate(int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, TileShape *shape, double *us)
 {
-    double cycles = 0.0;
-    if (!choose_tile_shape(shape, rows, cols, padded, batch, packed, info, &cycles)) return MACKO_E_INVALID_ARGUMENT;
-    *us = cycles * (1.06 / 2400.0) + (packed ? 2.9 : 0.0);
+    if (!choose_shape(shape, rows, cols, padded, batch, packed, info, us)) return MACKO_E_INVALID_ARGUMENT;
+    *us += packed ? 2.9 : 0.0;
     return 0;
 }
 
@@ -736,7 +1084,8 @@ int packed_product(const macko_packed_matrix *matrices, int n, const void *packe
     a.packed = (const u32x4 *)packed;
     a.residual = (const uint16_t *)residual;
     TileShape shape;
-    if (!choose_tile_shape(&shape, a.rows, cols, padded, batch, true, info)) return MACKO_E_INVALID_ARGUMENT;
+    double us = 0.0;
+    if (!choose_shape(&shape, a.rows, cols, padded, batch, true, info, &us)) return MACKO_E_INVALID_ARGUMENT;
     return launch_tile_shape(a, shape, info.max_lds_bytes, as_stream(stream));
 }
 

@@ -51,6 +51,33 @@ def test_edges_of_tiles_and_chunks(rows, cols, density, batch):
     assert torch.equal(Y, macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda()))
 
 
+# many rows and more than 16 vectors: the kernel whose waves scatter or multiply (48 rows, units of 4; lanes of 8 or 16
+# entries, 16 lanes a row; chunks of a multiple of 128 columns; 32, 64 or 128 vectors)
+@pytest.mark.parametrize("rows,cols,density,batch", [
+    (12288, 300, 0.05, 17), (12285, 512, 0.1, 32), (12289, 513, 0.3, 33), (24575, 128, 0.5, 64), (12001, 1281, 0.2, 65), (11009, 767, 0.45, 128),
+    (11500, 1025, 0.08, 128), (24001, 250, 0.3, 129), (49000, 70, 0.4, 40), (12288, 2000, 0.03, 100)])
+def test_many_rows(rows, cols, density, batch):
+    rng = np.random.default_rng(rows + cols + batch)
+    dense, X = _case(rng, rows, cols, density, batch)
+    dense[5::97] = 0                                                      # rows without entries
+    full = np.arange(3, rows, 211)
+    dense[full] = rng.standard_normal((full.size, cols)).astype(np.float16)   # more entries in a chunk than a pass holds
+    dense[-1] = 0
+    dense[-1, -1] = 1.0                                                   # one entry behind padding entries
+    dense[::13, cols // 5:cols // 5 * 4] = 0                              # gaps wider than a lane's columns
+    X[batch // 2, 1] = np.inf
+    c = macko_spmv.compress(torch.from_numpy(dense).cuda())
+    Y = macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda())
+    got, finite = Y.cpu().numpy(), np.ones((batch, rows), dtype=bool)
+    finite[batch // 2] = dense[:, 1] == 0       # and a padding entry multiplies it too (zero times inf)
+    exact = np.where(np.isfinite(X), X, 0).astype(np.float16)
+    keep = np.isfinite(got[batch // 2])
+    assert not keep[~finite[batch // 2]].any()
+    got[batch // 2] = np.where(keep, got[batch // 2], (exact[batch // 2].astype(np.float64) @ dense.astype(np.float64).T).astype(np.float16))
+    _check(got, dense, exact, f"{rows}x{cols} d={density} b={batch}")
+    assert torch.equal(Y.view(torch.int16), macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda()).view(torch.int16))
+
+
 @pytest.mark.parametrize("batch", [5, 16, 17, 100])
 @pytest.mark.parametrize("offset,ldx,ldy", [(0, 1008, 304), (0, 1001, 301), (1, 1003, 300), (3, 1016, 303), (8, 1024, 302)])
 def test_strided_and_unaligned_with_and_without_workspace(batch, offset, ldx, ldy):
