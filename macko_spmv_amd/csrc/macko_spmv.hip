@@ -901,12 +901,17 @@ LaunchShape launch_shape(int rows, long long padded, const DeviceInfo &info)
 {
     constexpr int waves = 1024 / kWave;
     LaunchShape s;
-    // about one wave per tile at most, so tiny matrices get a small grid; but when rows are about
-    // a tile long, prefer one wave per row over a slightly smaller wave count that would leave
-    // some waves with two rows
+    // A wave per tile; with more rows than tiles a wave per row, up to three rows per wave of a full chip: a
+    // row's end is about 1.3 us of a wave's own chain, and waves that are not there save nothing (64 x 128 at density
+    // 0.25: 4 workgroups 3.4 us, 1 workgroup 6.2; 1024 x 512 at 0.05: 64 3.5, 12 7.6; 4096 x 512 at 0.05: 256 3.8,
+    // 45 7.9; 9178 x 398 at 0.3: 256 5.4-5.9; 13604 x 352 at 0.09: 256 6.4, 137 6.2, in one pass per tile).  With more
+    // rows than that two waves per tile, which then have enough rows each for that pass (kRowsPassRowsPerWave).
     s.n_tiles = (padded + kTile - 1) / kTile;
     long long waves_wanted = s.n_tiles;
-    if (rows > waves_wanted) waves_wanted = rows < 2 * s.n_tiles ? rows : 2 * s.n_tiles;
+    if (rows > waves_wanted) {
+        const bool spread = rows < 2 * s.n_tiles || rows <= 3ll * info.compute_units * waves;
+        waves_wanted = spread ? rows : 2 * s.n_tiles;
+    }
     s.grid = (waves_wanted + waves - 1) / waves;
     if (s.grid > (long long)info.compute_units) s.grid = (long long)info.compute_units;
     if (s.grid < 1) s.grid = 1;

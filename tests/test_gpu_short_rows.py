@@ -12,6 +12,7 @@ import pytest
 import torch
 
 import macko_spmv
+import macko_spmv_amd
 from oracle import macko_oracle as mo
 from tests import helpers
 
@@ -125,3 +126,26 @@ def test_short_rows_keep_inf_and_nan_to_the_rows_that_read_them():
     got = y[touched].astype(np.float64)
     assert np.array_equal(np.isnan(got), np.isnan(want[touched]))
     assert np.array_equal(got[~np.isnan(got)], want[touched][~np.isnan(want[touched])])  # the same infinities
+
+
+@pytest.mark.parametrize("rows,cols,density", [
+    (1, 8, 1.0), (16, 3, 0.5), (17, 200, 0.1), (63, 128, 0.3), (64, 128, 0.05), (1030, 100, 0.02),   # a wave per row, with one to 65 workgroups
+    (4095, 70, 0.2), (4097, 70, 0.2),         # one row per wave of a full chip of 256 compute units, and the first wave with two
+    (12288, 90, 0.1), (12289, 90, 0.1),       # the last shape with three rows per wave; the next has waves by tiles
+    (13000, 64, 0.5), (13000, 2000, 0.05),    # ... half a tile per wave; long gaps
+])
+@pytest.mark.parametrize("int8", [False, True])
+def test_a_wave_per_row(rows, cols, density, int8):
+    rng = np.random.default_rng(rows + cols)
+    dense = helpers.random_sparse(rng, rows, cols, density, scale=0.05)
+    x = rng.standard_normal(cols).astype(np.float16)
+    if not int8:
+        c = _check(dense, x, "a wave per row", oracle=rows * cols <= 6_000_000)
+        y = torch.from_numpy(rng.standard_normal(rows).astype(np.float16)).cuda()
+        want = helpers.dense_reference(dense, x) * 2.0 - 0.5 * y.cpu().numpy().astype(np.float64)
+        helpers.assert_close_fp16(macko_spmv_amd.multiply_axpby(c, torch.from_numpy(x).cuda(), y, 2.0, -0.5).cpu().numpy(), want)
+        return
+    q = np.clip(np.round(dense.astype(np.float64) * 600), -127, 127).astype(np.int8)
+    c = macko_spmv_amd.compress_int8(torch.from_numpy(q).cuda())
+    got = macko_spmv_amd.multiply_int8(c, torch.from_numpy(x).cuda()).cpu().numpy()
+    helpers.assert_close_fp16(got, q.astype(np.float64) @ x.astype(np.float64))
