@@ -13,10 +13,13 @@ run hand-written HIP kernels through the C ABI in include/macko_hip.h; there is 
 implementation, and importing this package fails if the native libraries cannot be loaded.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import types
 
 import torch
+from torch.compiler import is_compiling as _is_compiling
 
 from . import _build
 
@@ -33,15 +36,44 @@ def _load_native():
     try:
         hip = ctypes.CDLL(hip_path, mode=ctypes.RTLD_GLOBAL)
         torch.ops.load_library(torch_path)
-    except OSError as exc:  # no silent fallback: the HIP path is the only path
+        # the same library as a module: the operators' functions for eager calls
+        spec = importlib.util.spec_from_file_location(
+            "libmacko_torch", torch_path, loader=importlib.machinery.ExtensionFileLoader("libmacko_torch", torch_path))
+        eager = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(eager)
+    except (OSError, ImportError) as exc:  # no silent fallback: the HIP path is the only path
         raise ImportError(
             f"macko_spmv_amd: cannot load its native libraries ({hip_path}, {torch_path}): {exc}. "
             "Rebuild them with `python macko_spmv_amd/_build.py`."
         ) from exc
-    return hip, hip_path, torch_path
+    return hip, hip_path, torch_path, eager
 
 
-_hip_lib, HIP_LIBRARY_PATH, TORCH_LIBRARY_PATH = _load_native()
+_hip_lib, HIP_LIBRARY_PATH, TORCH_LIBRARY_PATH, _eager = _load_native()
+
+
+def _operator(name):
+    """An operator as a function: for plain tensors that nothing else looks at, straight to its kernel (csrc/macko_torch.cpp,
+    "eager calls": 2 us of a call's 6 less), else torch.ops.macko_spmv.<name>."""
+    eager, general = getattr(_eager, name), getattr(torch.ops.macko_spmv, name).default
+
+    def call(*args):
+        if not _is_compiling():
+            out = eager(*args)
+            if out is not NotImplemented:
+                return out
+        return general(*args)
+
+    call.__name__ = name
+    return call
+
+
+# the operators that the package calls itself, as such functions
+ops = types.SimpleNamespace(**{name: _operator(name) for name in (
+    "multiply_batched", "multiply_int8", "multiply_int8_axpby", "multiply_rmsnorm", "multiply_silu_mul_axpby",
+    "multiply_attention_axpby", "decode_rmsnorm", "decode_rope_append", "decode_attention", "decode_silu_mul",
+    "decode_rope_attention", "decode_rope_attention_parts", "pack_rmsnorm", "rmsnorm_rows", "pack_silu_mul", "multiply_packed",
+    "multiply_packed_several", "prefill_rope_append", "prefill_attention")})
 
 
 @torch.library.register_fake("macko_spmv::multiply")
@@ -252,6 +284,10 @@ def compress(M):
 def multiply(compressed_M, V):
     """y = M @ V for a compressed M; fp16 in, fp32 accumulation, fp16 out
     (src/macko_spmv/__init__.py:134-149)."""
+    if not _is_compiling():
+        y = _eager.multiply(compressed_M, V)
+        if y is not NotImplemented:
+            return y
     assert compressed_M[0].is_cuda
     assert compressed_M[1].is_cuda
     assert compressed_M[2].is_cuda
@@ -277,12 +313,16 @@ def multiply_batched(compressed_M, X):
     (python_scripts/util_run_pruned_llm.py:112-118)."""
     assert compressed_M[0].is_cuda and X.is_cuda
     assert X.dim() == 2 and X.is_contiguous()
-    return torch.ops.macko_spmv.multiply_batched.default(*compressed_M[:5], X)
+    return ops.multiply_batched(*compressed_M[:5], X)
 
 
 def multiply_axpby(compressed_M, V, C, alpha=1.0, beta=0.0):
     """In place C = alpha * (M @ V) + beta * C: the epilogue of the upstream kernel's
     reuse_value_from_c instantiation (src/macko_spmv/cuda/kernels.cuh:113-118)."""
+    if not _is_compiling():
+        result = _eager.multiply_axpby(compressed_M, V, C, alpha, beta)
+        if result is not NotImplemented:
+            return result
     assert compressed_M[0].is_cuda and V.is_cuda and C.is_cuda
     assert V.is_contiguous() and C.is_contiguous()
     plan = _plan_of(compressed_M)
@@ -301,14 +341,14 @@ def multiply_rmsnorm(compressed_M, V, norm_weight, eps):
     applied while the product stages its input (no launch, no round trip through memory for it).
     Needs cols % 8 == 0 and a vector that fits in LDS.  No upstream counterpart."""
     assert compressed_M[0].is_cuda and V.is_cuda and norm_weight.is_cuda
-    return torch.ops.macko_spmv.multiply_rmsnorm.default(*compressed_M[:5], V, norm_weight, float(eps))
+    return ops.multiply_rmsnorm(*compressed_M[:5], V, norm_weight, float(eps))
 
 
 def multiply_silu_mul_axpby(compressed_M, gate, up, C, alpha=1.0, beta=0.0):
     """In place C = alpha * M @ (silu(gate) * up) + beta * C: the gated activation of a Llama MLP
     applied while the down projection stages its input.  Same limits as multiply_rmsnorm."""
     assert compressed_M[0].is_cuda and gate.is_cuda and up.is_cuda and C.is_cuda
-    torch.ops.macko_spmv.multiply_silu_mul_axpby.default(*compressed_M[:5], gate, up, C, float(alpha), float(beta))
+    ops.multiply_silu_mul_axpby(*compressed_M[:5], gate, up, C, float(alpha), float(beta))
     return C
 
 
@@ -317,7 +357,7 @@ def multiply_attention_axpby(compressed_M, parts, head_dim, C, alpha=1.0, beta=0
     torch.ops.macko_spmv.decode_rope_attention_parts leaves, merged while the product stages its input.
     head_dim 64 or 128; same limits as multiply_rmsnorm."""
     assert compressed_M[0].is_cuda and parts.is_cuda and C.is_cuda
-    torch.ops.macko_spmv.multiply_attention_axpby.default(*compressed_M[:5], parts, head_dim, C, float(alpha), float(beta))
+    ops.multiply_attention_axpby(*compressed_M[:5], parts, head_dim, C, float(alpha), float(beta))
     return C
 
 
@@ -342,7 +382,7 @@ def multiply_int8(compressed_M, V):
     assert compressed_M[2].is_cuda
     assert V.is_cuda
     assert V.is_contiguous()
-    return torch.ops.macko_spmv.multiply_int8.default(*compressed_M[:5], V)
+    return ops.multiply_int8(*compressed_M[:5], V)
 
 
 def multiply_int8_axpby(compressed_M, V, C, alpha=1.0, beta=0.0):
@@ -350,7 +390,7 @@ def multiply_int8_axpby(compressed_M, V, C, alpha=1.0, beta=0.0):
     src/macko_spmv/cuda/kernels.cuh:208-211)."""
     assert compressed_M[0].is_cuda and V.is_cuda and C.is_cuda
     assert V.is_contiguous() and C.is_contiguous()
-    torch.ops.macko_spmv.multiply_int8_axpby.default(*compressed_M[:5], V, C, float(alpha), float(beta))
+    ops.multiply_int8_axpby(*compressed_M[:5], V, C, float(alpha), float(beta))
     return C
 
 

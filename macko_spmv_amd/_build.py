@@ -15,6 +15,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
@@ -247,12 +248,12 @@ def build_torch(verbose=False):
         "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
         "-Wno-unused-command-line-argument",
         f"-I{_INCLUDE}",
-        *[f"-I{p}" for p in ce.include_paths("cuda")],
+        *[f"-I{p}" for p in ce.include_paths("cuda")], f"-I{sysconfig.get_paths()['include']}",
         *[os.path.join(_CSRC, s) for s in TORCH_SOURCES],
         "-x", "none",
         *[f"-L{p}" for p in ce.library_paths("cuda") if os.path.isdir(p)],
         f"-L{os.path.dirname(hip_lib)}",
-        "-lmacko_hip", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-lamdhip64",
+        "-lmacko_hip", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-lamdhip64",
         "-Wl,-rpath,$ORIGIN",
         "-o", out,
     ]

@@ -9,9 +9,16 @@
 // the *MasqueradingAsCUDA guard and stream accessors.  There is deliberately no CPU kernel
 // for multiply: without a GPU the operator raises.
 
+#include <Python.h>  // first, as its headers ask for
+
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/record_function.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/library.h>
 
 #include <chrono>
@@ -59,7 +66,7 @@ at::Tensor multiply_hip(const at::Tensor &M_values, const at::Tensor &M_deltas, 
     TORCH_CHECK(V.numel() >= M_cols || M_values.numel() == 0, "V must hold at least M_cols elements");
 
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(M_values.device());
-    at::Tensor C = at::empty({M_rows}, M_values.options());
+    at::Tensor C = at::detail::empty_cuda({M_rows}, at::kHalf, M_values.device(), std::nullopt);
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
     const int rc = macko_spmv_f16(M_values.data_ptr(), M_deltas.data_ptr(), M_row_indices.data_ptr<int>(),
                                   V.data_ptr(), C.data_ptr(), (int32_t)M_rows, (int32_t)M_cols,
@@ -104,7 +111,7 @@ at::Tensor multiply_planned_hip(const at::Tensor &M_values, const at::Tensor &M_
     check_plan(plan, M_values);
     TORCH_CHECK(V.numel() >= M_cols || M_values.numel() == 0, "V must hold at least M_cols elements");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(M_values.device());
-    at::Tensor C = at::empty({M_rows}, M_values.options());
+    at::Tensor C = at::detail::empty_cuda({M_rows}, at::kHalf, M_values.device(), std::nullopt);
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
     const int rc = macko_spmv_f16_planned(M_values.data_ptr(), M_deltas.data_ptr(), M_row_indices.data_ptr<int>(),
                                           plan.numel() ? plan.data_ptr<int>() : nullptr, (int32_t)plan.numel(),
@@ -141,7 +148,7 @@ at::Tensor multiply_batched_hip(const at::Tensor &M_values, const at::Tensor &M_
     check_half_gpu(X, "X");
     TORCH_CHECK(X.dim() == 2 && X.size(1) >= M_cols, "X must be [batch, >= M_cols]");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(M_values.device());
-    at::Tensor Y = at::empty({X.size(0), M_rows}, M_values.options());
+    at::Tensor Y = at::detail::empty_cuda({X.size(0), M_rows}, at::kHalf, M_values.device(), std::nullopt);
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
     TORCH_CHECK(X.size(0) < (1ll << 31), "batch too large");
     int64_t scratch_bytes = 0;
@@ -291,7 +298,7 @@ at::Tensor multiply_int8_hip(const at::Tensor &M_values, const at::Tensor &M_del
     check_int8_operands(M_values, M_deltas, M_row_indices, M_rows, M_cols, V);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(M_values.device());
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
-    at::Tensor C = at::empty({M_rows}, V.options());
+    at::Tensor C = at::detail::empty_cuda({M_rows}, at::kHalf, V.device(), std::nullopt);
     check_rc(macko_spmv_i8f16(M_values.data_ptr(), M_deltas.data_ptr(), M_row_indices.data_ptr<int>(),
                               V.data_ptr(), C.data_ptr(), (int32_t)M_rows, (int32_t)M_cols, M_values.numel(),
                               (void *)stream),
@@ -417,7 +424,7 @@ at::Tensor multiply_rmsnorm_hip(const at::Tensor &M_values, const at::Tensor &M_
     check_half_gpu(norm_weight, "norm_weight");
     TORCH_CHECK(V.numel() == M_cols && norm_weight.numel() == M_cols, "V and norm_weight must hold M_cols elements");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(M_values.device());
-    at::Tensor C = at::empty({M_rows}, M_values.options());
+    at::Tensor C = at::detail::empty_cuda({M_rows}, at::kHalf, M_values.device(), std::nullopt);
     check_rc(macko_spmv_f16_rmsnorm(M_values.data_ptr(), M_deltas.data_ptr(), M_row_indices.data_ptr<int>(),
                                     V.data_ptr(), norm_weight.data_ptr(), (float)eps, C.data_ptr(), (int32_t)M_rows,
                                     (int32_t)M_cols, M_values.numel(),
@@ -697,7 +704,282 @@ at::Tensor prefill_attention_hip(const at::Tensor &q, const at::Tensor &k_cache,
     return packed;
 }
 
+// ---- eager calls from Python --------------------------------------------------------------------
+//
+// What torch.ops.macko_spmv.<name>.default(...) does on its way from Python to the functions above (the arguments through
+// the operator's schema onto a stack of values, the dispatcher, the stack again) takes longer than the rest of the call:
+// 777 x 3333 at density 0.25, 5.8 us a call of `multiply`, of which the launch is 2.2 and the kernel, meanwhile, 4.0.  The
+// functions below take the arguments from Python themselves, for calls that nothing but the CUDA kernel would see: plain
+// tensors on one GPU, through which no gradient has to flow, and no mode, transform, recording or profiler that is
+// between Python and the kernel.  Anything else is answered with NotImplemented, and the caller goes through the
+// operator.
+
+// Nothing in this thread looks at operators: modes of Python, torch.func, tracing and whatever else adds dispatch keys
+// of its own; __torch_function__ modes; the profiler.
+bool unobserved()
+{
+    const c10::impl::LocalDispatchKeySet tls = c10::impl::tls_local_dispatch_key_set();
+    return (tls.included_ | c10::default_included_set) == c10::default_included_set && !at::impl::torch_function_mode_enabled() && !at::hasCallbacks();
+}
+
+// A tensor whose operators only the CUDA kernel is registered for.
+bool plain(const at::Tensor &t)
+{
+    constexpr c10::DispatchKeySet usual =
+        c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutocastCUDA});
+    return t.defined() && t.is_cuda() && (t.key_set() | usual) == usual && !(t.requires_grad() && at::GradMode::is_enabled()) &&
+           !t._fw_grad(0).defined();
+}
+
+struct EagerCall {
+    int device = -1;
+    bool tensor(PyObject *o, const at::Tensor *&out)
+    {
+        if (!THPVariable_CheckExact(o)) return false;
+        out = &THPVariable_Unpack(o);
+        if (!plain(*out)) return false;
+        const int index = out->get_device();
+        if (device < 0) device = index;
+        return index == device;
+    }
+    static bool integer(PyObject *o, int64_t &out)
+    {
+        if (!PyLong_CheckExact(o)) return false;
+        int overflow = 0;
+        out = PyLong_AsLongLongAndOverflow(o, &overflow);
+        return overflow == 0;
+    }
+    static bool number(PyObject *o, double &out)
+    {
+        if (!PyFloat_CheckExact(o)) return false;
+        out = PyFloat_AS_DOUBLE(o);
+        return true;
+    }
+};
+
+// An argument of one of the functions above: what is kept of it while the call runs, and how it is handed over.
+template <typename T> struct EagerArg;
+template <> struct EagerArg<const at::Tensor &> {
+    const at::Tensor *kept = nullptr;
+    bool take(EagerCall &call, PyObject *o) { return call.tensor(o, kept); }
+    const at::Tensor &give() const { return *kept; }
+};
+template <> struct EagerArg<at::Tensor> : EagerArg<const at::Tensor &> {};
+template <> struct EagerArg<const std::optional<at::Tensor> &> {
+    std::optional<at::Tensor> kept;
+    bool take(EagerCall &call, PyObject *o)
+    {
+        if (o == Py_None) return true;
+        const at::Tensor *t = nullptr;
+        if (!call.tensor(o, t)) return false;
+        kept = *t;
+        return true;
+    }
+    const std::optional<at::Tensor> &give() const { return kept; }
+};
+template <> struct EagerArg<int64_t> {
+    int64_t kept = 0;
+    bool take(EagerCall &, PyObject *o) { return EagerCall::integer(o, kept); }
+    int64_t give() const { return kept; }
+};
+template <> struct EagerArg<double> {
+    double kept = 0.0;
+    bool take(EagerCall &, PyObject *o) { return EagerCall::number(o, kept); }
+    double give() const { return kept; }
+};
+template <> struct EagerArg<at::TensorList> {
+    std::vector<at::Tensor> kept;
+    bool take(EagerCall &call, PyObject *o)
+    {
+        if (!PyList_CheckExact(o)) return false;
+        for (Py_ssize_t i = 0; i < PyList_GET_SIZE(o); ++i) {
+            const at::Tensor *t = nullptr;
+            if (!call.tensor(PyList_GET_ITEM(o, i), t)) return false;
+            kept.push_back(*t);
+        }
+        return true;
+    }
+    at::TensorList give() const { return kept; }
+};
+template <> struct EagerArg<at::IntArrayRef> {
+    std::vector<int64_t> kept;
+    bool take(EagerCall &, PyObject *o)
+    {
+        if (!PyList_CheckExact(o)) return false;
+        for (Py_ssize_t i = 0; i < PyList_GET_SIZE(o); ++i) {
+            int64_t v = 0;
+            if (!EagerCall::integer(PyList_GET_ITEM(o, i), v)) return false;
+            kept.push_back(v);
+        }
+        return true;
+    }
+    at::IntArrayRef give() const { return kept; }
+};
+
+PyObject *to_python(at::Tensor &&t) { return THPVariable_Wrap(std::move(t)); }
+PyObject *to_python(std::vector<at::Tensor> &&all)
+{
+    PyObject *list = PyList_New((Py_ssize_t)all.size());
+    if (list == nullptr) return nullptr;
+    for (size_t i = 0; i < all.size(); ++i) PyList_SET_ITEM(list, (Py_ssize_t)i, THPVariable_Wrap(std::move(all[i])));
+    return list;
+}
+
+PyObject *not_implemented()
+{
+    Py_INCREF(Py_NotImplemented);
+    return Py_NotImplemented;
+}
+
+struct WithoutGil {  // as around an operator's call: a launch may wait for room in the stream's queue
+    PyThreadState *state = PyEval_SaveThread();
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+template <auto FUNCTION, typename R, typename... A, size_t... I>
+PyObject *eager_call(R (*)(A...), std::index_sequence<I...>, PyObject *const *args, Py_ssize_t n)
+{
+    if (n != (Py_ssize_t)sizeof...(A) || !unobserved()) return not_implemented();
+    EagerCall call;
+    std::tuple<EagerArg<A>...> kept;
+    if (!(std::get<I>(kept).take(call, args[I]) && ...)) return not_implemented();
+    if constexpr (std::is_void_v<R>) {
+        {
+            WithoutGil released;
+            FUNCTION(std::get<I>(kept).give()...);
+        }
+        Py_RETURN_NONE;
+    } else {
+        std::optional<R> out;
+        {
+            WithoutGil released;
+            out.emplace(FUNCTION(std::get<I>(kept).give()...));
+        }
+        return to_python(std::move(*out));
+    }
+}
+
+template <typename R, typename... A> constexpr size_t arity(R (*)(A...)) { return sizeof...(A); }
+
+// The operator's own arguments, one by one.
+template <auto FUNCTION> PyObject *eager(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    return eager_call<FUNCTION>(FUNCTION, std::make_index_sequence<arity(FUNCTION)>{}, args, n);
+    END_HANDLE_TH_ERRORS
+}
+
+// (compressed, V) and (compressed, V, C, alpha, beta) of a matrix that may carry its cuts as an attribute of row_indices
+// (macko_spmv_amd/__init__.py).
+PyObject *plan_attribute = nullptr;  // its name
+
+struct Compressed {
+    const at::Tensor *values = nullptr, *deltas = nullptr, *row_indices = nullptr, *plan = nullptr;
+    at::Tensor plan_kept;
+    int64_t rows = 0, cols = 0;
+    bool take(EagerCall &call, PyObject *o)
+    {
+        PyObject *const *item;
+        if (PyTuple_CheckExact(o) && PyTuple_GET_SIZE(o) >= 5)
+            item = &PyTuple_GET_ITEM(o, 0);
+        else
+            return false;
+        if (!call.tensor(item[0], values) || !call.tensor(item[1], deltas) || !call.tensor(item[2], row_indices) ||
+            !EagerCall::integer(item[3], rows) || !EagerCall::integer(item[4], cols))
+            return false;
+        PyObject *found = nullptr;
+        if (_PyObject_LookupAttr(item[2], plan_attribute, &found) < 0) {
+            PyErr_Clear();
+            return false;
+        }
+        if (found == nullptr) return true;
+        bool fits = found == Py_None;
+        if (!fits) {
+            const at::Tensor *t = nullptr;
+            fits = call.tensor(found, t);   // a plan of another device is the general path's to leave out
+            if (fits) {
+                plan_kept = *t;
+                plan = &plan_kept;
+            }
+        }
+        Py_DECREF(found);
+        return fits;
+    }
+};
+
+PyObject *eager_multiply(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    EagerCall call;
+    Compressed m;
+    const at::Tensor *v = nullptr;
+    if (n != 2 || !unobserved() || !m.take(call, args[0]) || !call.tensor(args[1], v) || !v->is_contiguous()) return not_implemented();
+    at::Tensor out;
+    {
+        WithoutGil released;
+        out = m.plan != nullptr ? multiply_planned_hip(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *m.plan)
+                                : multiply_hip(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v);
+    }
+    return to_python(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+PyObject *eager_multiply_axpby(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    EagerCall call;
+    Compressed m;
+    const at::Tensor *v = nullptr, *c = nullptr;
+    double alpha = 0.0, beta = 0.0;
+    if (n != 5 || !unobserved() || !m.take(call, args[0]) || !call.tensor(args[1], v) || !call.tensor(args[2], c) ||
+        !EagerCall::number(args[3], alpha) || !EagerCall::number(args[4], beta) || !v->is_contiguous() || !c->is_contiguous())
+        return not_implemented();
+    {
+        WithoutGil released;
+        if (m.plan != nullptr)
+            multiply_axpby_planned_hip(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *c, alpha, beta, *m.plan);
+        else
+            multiply_axpby_hip(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *c, alpha, beta);
+    }
+    Py_INCREF(args[2]);
+    return args[2];
+    END_HANDLE_TH_ERRORS
+}
+
+#define MACKO_EAGER(NAME, ...) {#NAME, (PyCFunction)(void (*)(void))&__VA_ARGS__, METH_FASTCALL, nullptr}
+PyMethodDef eager_functions[] = {
+    MACKO_EAGER(multiply, eager_multiply),
+    MACKO_EAGER(multiply_axpby, eager_multiply_axpby),
+    MACKO_EAGER(multiply_batched, eager<&multiply_batched_hip>),
+    MACKO_EAGER(multiply_int8, eager<&multiply_int8_hip>),
+    MACKO_EAGER(multiply_int8_axpby, eager<&multiply_int8_axpby_hip>),
+    MACKO_EAGER(multiply_rmsnorm, eager<&multiply_rmsnorm_hip>),
+    MACKO_EAGER(multiply_silu_mul_axpby, eager<&multiply_silu_mul_axpby_hip>),
+    MACKO_EAGER(multiply_attention_axpby, eager<&multiply_attention_axpby_hip>),
+    MACKO_EAGER(decode_rmsnorm, eager<&decode_rmsnorm_hip>),
+    MACKO_EAGER(decode_rope_append, eager<&decode_rope_append_hip>),
+    MACKO_EAGER(decode_attention, eager<&decode_attention_hip>),
+    MACKO_EAGER(decode_silu_mul, eager<&decode_silu_mul_hip>),
+    MACKO_EAGER(decode_rope_attention, eager<&decode_rope_attention_hip>),
+    MACKO_EAGER(decode_rope_attention_parts, eager<&decode_rope_attention_parts_hip>),
+    MACKO_EAGER(pack_rmsnorm, eager<&pack_rmsnorm_hip>),
+    MACKO_EAGER(rmsnorm_rows, eager<&rmsnorm_rows_hip>),
+    MACKO_EAGER(pack_silu_mul, eager<&pack_silu_mul_hip>),
+    MACKO_EAGER(multiply_packed, eager<&multiply_packed_hip>),
+    MACKO_EAGER(multiply_packed_several, eager<&multiply_packed_several_hip>),
+    MACKO_EAGER(prefill_rope_append, eager<&prefill_rope_append_hip>),
+    MACKO_EAGER(prefill_attention, eager<&prefill_attention_hip>),
+    {nullptr, nullptr, 0, nullptr}};
+#undef MACKO_EAGER
+PyModuleDef eager_module = {PyModuleDef_HEAD_INIT, "libmacko_torch", nullptr, -1, eager_functions, nullptr, nullptr, nullptr, nullptr};
+
 }  // namespace
+
+PyMODINIT_FUNC PyInit_libmacko_torch()
+{
+    plan_attribute = PyUnicode_InternFromString("_macko_spmv_plan");
+    return plan_attribute == nullptr ? nullptr : PyModule_Create(&eager_module);
+}
 
 TORCH_LIBRARY(macko_spmv, m)
 {

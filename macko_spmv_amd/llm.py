@@ -167,7 +167,7 @@ class RMSNorm(nn.Module):
         if not torch.jit.is_scripting():
             if (_inference_half(x, self.weight) and x.is_contiguous() and self.weight.shape == x.shape[-1:] and x.numel() > 0
                     and x.shape[-1] % 8 == 0 and self.weight.is_contiguous()):
-                return torch.ops.macko_spmv.rmsnorm_rows(x, self.weight, self.eps)
+                return macko_spmv.ops.rmsnorm_rows(x, self.weight, self.eps)
         v = x.float()
         v = v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + self.eps)
         return (v * self.weight.float()).to(x.dtype)
@@ -273,7 +273,7 @@ class Block(nn.Module):
         """The layer for several tokens with one kernel for each part between the projections; what a
         projection consumes is written in its operand order, and the residuals are added where the
         o and down projections round their results."""
-        ops, att, mlp = torch.ops.macko_spmv, self.self_attn, self.mlp
+        ops, att, mlp = macko_spmv.ops, self.self_attn, self.mlp
         t = x.shape[1]
         rows = x.reshape(t, -1).contiguous()
         positions = positions.contiguous()
@@ -463,7 +463,7 @@ class DecodeEngine:
     has no such hook, and keep their separate norm and gate kernels."""
 
     def __init__(self, model, fuse=True):
-        ops = torch.ops.macko_spmv
+        ops = macko_spmv.ops
         self.ops = ops
         self.fuse = fuse
         body = model.model
