@@ -298,7 +298,7 @@ __device__ __forceinline__ void wave_lds_fence()
 // A half without entries stores to a spare place (it would share its place with the half behind it).
 // Nibbles: 256-entry table by the lane's entry mask, packed; one or two OR operations on words that are
 // zero beforehand.
-// What bounds it is memory: 11008 x 4096 fp16 at density 0.5 reads 90 MB and writes 56 in 34.4 us (4.3 TB/s).
+// What bounds it is memory: 11008 x 4096 fp16 at density 0.5 reads 90 MB and writes 56 in 33.2 us (4.4 TB/s).
 // With a 4-byte LDS store per column behind a select, and the groups packed from those words again, it took
 // 39.7, half of them vector instructions.  Waiting for a row's loads all at once, so that no tile's wait
 // for its load is also one for the stores of the tile before, with 8 tiles in flight: 36.4.
@@ -416,8 +416,13 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
             const int b = hi - 8 * g < 8 ? hi - 8 * g : 8;
             const int out = (base >> 3) + g;
             if (a == 0 && b == 8) {
-                value_groups[out] = v;
-                delta_words[out] = word;
+                if (STREAM) {
+                    value_groups[out] = v;
+                    delta_words[out] = word;
+                } else {
+                    __builtin_nontemporal_store(v, value_groups + out);
+                    __builtin_nontemporal_store(word, delta_words + out);
+                }
             } else {
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
@@ -572,8 +577,11 @@ namespace macko {
 namespace {
 
 // The fill pass reads the matrix again after the count pass: up to about half the last-level
-// cache (256 MB) both leave it there (measured: 5 % faster at 90 MB), beyond that they read it
-// with the non-temporal hint (2 % faster at 470 MB and more).
+// cache (256 MB) both leave it there (measured: 5 % faster at 90 MB), and the results are stored with
+// the non-temporal hint, so that they do not take its place there (whole call, 11008 x 4096 at density 0.5:
+// 73.4 -> 65.9 us, at 0.9 78.7 -> 75.3, 4096 x 11008 73.5 -> 63.7); beyond that the matrix is read
+// with that hint (2 % faster at 470 MB and more) and the results are not stored with it (28672 x 8192 at 0.3: 243 us,
+// with it 269).
 template <typename Elem>
 bool streams_past_cache(int32_t rows, int32_t cols)
 {
