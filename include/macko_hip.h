@@ -130,6 +130,10 @@ MACKO_API int macko_compress_f16_count_total(const void *dense, int32_t rows, in
 MACKO_API int macko_compress_f16_fill(const void *dense, int32_t rows, int32_t cols,
                             const int32_t *row_ptr, void *values, void *deltas,
                             int64_t padded_entries, void *stream);
+/* The same, and the product's prepared cuts beside it (macko_spmv_plan_build's plan, in the same launch). */
+MACKO_API int macko_compress_f16_fill_plan(const void *dense, int32_t rows, int32_t cols, const int32_t *row_ptr,
+                                 void *values, void *deltas, int64_t padded_entries, int32_t *plan,
+                                 int32_t plan_entries, void *stream);
 
 /*
  * Y[b, :] = M X[b, :] for b < batch.  X is [batch, ldx] and Y [batch, ldy], row-major fp16 with

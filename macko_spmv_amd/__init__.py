@@ -276,6 +276,11 @@ def compress(M):
     through the current GPU).
     """
     assert M.is_contiguous()
+    if not _is_compiling():
+        made = _eager.compress(M)
+        if made is not NotImplemented:
+            setattr(made[2], _PLAN_ATTRIBUTE, made[5])
+            return made[:5]
     if M.device.type in ("cuda", "cpu"):
         return attach_plan(tuple(torch.ops.macko_spmv.compress.default(M)))
     raise NotImplementedError()

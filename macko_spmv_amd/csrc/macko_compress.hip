@@ -18,6 +18,7 @@
 // columns and learn the previous non-zero's column from a DPP running maximum.
 
 #include "macko_packed.h"
+#include "macko_spmv_detail.h"
 
 namespace macko {
 namespace {
@@ -315,8 +316,16 @@ template <typename F, bool STREAM>
 __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Elem *__restrict__ dense, int rows,
                                                            int cols, const int *__restrict__ row_ptr,
                                                            typename F::Elem *__restrict__ values,
-                                                           u32 *__restrict__ delta_words, int padded)
+                                                           u32 *__restrict__ delta_words, int padded,
+                                                           const spmv_detail::PlanArgs cuts, int cut_blocks)
 {
+    // The first workgroups make the product's cuts, a thread each (macko_spmv_plan_build): beside the rows they cost
+    // nothing, behind them a launch (11008 x 4096: 5 us).
+    if ((int)blockIdx.x < cut_blocks) {
+        const u32 k = blockIdx.x * kBlock + threadIdx.x;
+        if (k <= cuts.n_waves) spmv_detail::write_cut(cuts, k);
+        return;
+    }
     typedef typename F::Elem Elem;
     typedef typename F::Chunk Chunk;
     // the carried part of a group, a tile's entries, and what the last half stores behind its own
@@ -332,7 +341,7 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
     static_assert(kBlock == 256, "one table entry per thread");
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = uniform(threadIdx.x >> 6);
-    const int row = blockIdx.x * kRowsPerBlock + wave;
+    const int row = ((int)blockIdx.x - cut_blocks) * kRowsPerBlock + wave;
     const Elem *src = dense + (size_t)row * (size_t)cols;
 
     // kAhead tiles of the row in flight
@@ -617,7 +626,7 @@ int compress_count(const void *dense, int32_t rows, int32_t cols, int32_t *row_p
 
 template <typename F>
 int compress_fill(const void *dense, int32_t rows, int32_t cols, const int32_t *row_ptr, void *values,
-                  void *deltas, int64_t padded_entries, void *stream)
+                  void *deltas, int64_t padded_entries, const spmv_detail::PlanArgs &cuts, void *stream)
 {
     typedef typename F::Elem Elem;
     if (rows < 0 || cols < 0 || padded_entries < 0 || padded_entries % kChunk != 0)
@@ -632,13 +641,14 @@ int compress_fill(const void *dense, int32_t rows, int32_t cols, const int32_t *
         return MACKO_E_INVALID_ARGUMENT;
     hipStream_t s = as_stream(stream);
     if (rows == 0) return MACKO_E_INVALID_ARGUMENT;  // entries without rows
-    const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock);
+    const int cut_blocks = cuts.n_waves > 0 ? (int)(cuts.n_waves + kBlock) / kBlock : 0;
+    const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock + cut_blocks);
     if (streams_past_cache<Elem>(rows, cols))
         hipLaunchKernelGGL((fill_rows_kernel<F, true>), grid, dim3(kBlock), 0, s, (const Elem *)dense, rows, cols,
-                           row_ptr, (Elem *)values, (u32 *)deltas, (int)padded_entries);
+                           row_ptr, (Elem *)values, (u32 *)deltas, (int)padded_entries, cuts, cut_blocks);
     else
         hipLaunchKernelGGL((fill_rows_kernel<F, false>), grid, dim3(kBlock), 0, s, (const Elem *)dense, rows, cols,
-                           row_ptr, (Elem *)values, (u32 *)deltas, (int)padded_entries);
+                           row_ptr, (Elem *)values, (u32 *)deltas, (int)padded_entries, cuts, cut_blocks);
     return (int)hipGetLastError();
 }
 
@@ -654,8 +664,18 @@ extern "C" int macko_compress_f16_count(const void *dense, int32_t rows, int32_t
 extern "C" int macko_compress_f16_fill(const void *dense, int32_t rows, int32_t cols, const int32_t *row_ptr,
                                        void *values, void *deltas, int64_t padded_entries, void *stream)
 {
-    return macko::compress_fill<macko::Fp16Format>(dense, rows, cols, row_ptr, values, deltas, padded_entries,
-                                                   stream);
+    return macko::compress_fill<macko::Fp16Format>(dense, rows, cols, row_ptr, values, deltas, padded_entries, {}, stream);
+}
+
+extern "C" int macko_compress_f16_fill_plan(const void *dense, int32_t rows, int32_t cols, const int32_t *row_ptr,
+                                            void *values, void *deltas, int64_t padded_entries, int32_t *plan,
+                                            int32_t plan_entries, void *stream)
+{
+    using namespace macko;
+    spmv_detail::PlanArgs cuts;
+    const int rc = spmv_plan_args(row_ptr, rows, cols, padded_entries, plan, plan_entries, &cuts);
+    if (rc != 0) return rc;
+    return compress_fill<Fp16Format>(dense, rows, cols, row_ptr, values, deltas, padded_entries, cuts, stream);
 }
 
 extern "C" int macko_compress_f16_count_total(const void *dense, int32_t rows, int32_t cols, int32_t *row_ptr,
@@ -679,8 +699,7 @@ extern "C" int macko_compress_i8_count(const void *dense, int32_t rows, int32_t 
 extern "C" int macko_compress_i8_fill(const void *dense, int32_t rows, int32_t cols, const int32_t *row_ptr,
                                       void *values, void *deltas, int64_t padded_entries, void *stream)
 {
-    return macko::compress_fill<macko::Int8Format>(dense, rows, cols, row_ptr, values, deltas, padded_entries,
-                                                   stream);
+    return macko::compress_fill<macko::Int8Format>(dense, rows, cols, row_ptr, values, deltas, padded_entries, {}, stream);
 }
 
 extern "C" int macko_decompress_f16(const void *values, const void *deltas, const int32_t *row_ptr, int32_t rows,

@@ -1021,38 +1021,11 @@ int spmv_dispatch(const SpmvArgs &args, hipStream_t stream)
     return launch_stream<1024, 1, true, AXPBY, VB>(a, (int)grid, lds_x, stream);
 }
 
-// One thread per cut: cut k is where wave k of the launch starts (cut n_waves: the end), by the
-// rule the kernel itself applies when it has no plan: the first row r with
-// row_ptr[r] + row_cost * r >= target k, or the row before if that is nearer; even shares of the
-// rows when there are no more rows than waves.  plan[2k] = row, plan[2k + 1] = row_ptr[row].
-__global__ void plan_kernel(const SpmvArgs a, u32 n_waves, int *__restrict__ plan)
+// One thread per cut.
+__global__ void plan_kernel(const PlanArgs a)
 {
     const u32 k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k > n_waves) return;
-    int cut;
-    if (k == 0) {
-        cut = 0;
-    } else if (k == n_waves) {
-        cut = a.rows;
-    } else if (a.row_even) {
-        cut = (int)(k * a.rows_q + __umulhi(k, a.rows_frac));
-    } else {
-        const long long target = (long long)even_split(k, a.entries_q, a.entries_rem);
-        const long long row_cost = (long long)a.row_cost;
-        int lo = 0, hi = a.rows;  // cost(rows) = the whole sum >= any target
-        while (lo < hi) {
-            const int mid = lo + ((hi - lo) >> 1);
-            if ((long long)a.row_ptr[mid] + row_cost * mid >= target) hi = mid; else lo = mid + 1;
-        }
-        cut = lo;
-        if (cut > 0) {
-            const long long after = (long long)a.row_ptr[cut] + row_cost * cut;
-            const long long before = (long long)a.row_ptr[cut - 1] + row_cost * (cut - 1);
-            if (target - before < after - target) cut -= 1;
-        }
-    }
-    plan[2 * k] = cut;
-    plan[2 * k + 1] = a.row_ptr[cut];
+    if (k <= a.n_waves) write_cut(a, k);
 }
 
 // Waves of the launch a plan describes, 0 if this shape takes none (no stored entries, rows split
@@ -1143,15 +1116,13 @@ extern "C" int macko_spmv_plan_entries(int32_t rows, int32_t cols, int64_t padde
     return rc;
 }
 
-extern "C" int macko_spmv_plan_build(const int32_t *row_ptr, int32_t rows, int32_t cols, int64_t padded_entries,
-                                     int32_t *plan, int32_t plan_entries, void *stream)
+namespace macko {
+int spmv_plan_args(const int *row_ptr, int rows, int cols, long long padded, int *plan, int plan_entries, PlanArgs *out)
 {
-    using namespace macko;
-    if (rows < 0 || cols < 0 || padded_entries < 0 || padded_entries % kChunk != 0 ||
-        padded_entries >= (1ll << 31) - 8192)
-        return MACKO_E_INVALID_ARGUMENT;
+    *out = PlanArgs{};
+    if (rows < 0 || cols < 0 || padded < 0 || padded % kChunk != 0 || padded >= (1ll << 31) - 8192) return MACKO_E_INVALID_ARGUMENT;
     long long n_waves = 0;
-    const int rc = plan_waves(rows, cols, padded_entries, &n_waves);
+    const int rc = plan_waves(rows, cols, padded, &n_waves);
     if (rc != 0) return rc;
     if ((long long)plan_entries != (n_waves > 0 ? 2 * (n_waves + 1) : 0)) return MACKO_E_INVALID_ARGUMENT;
     if (n_waves == 0) return 0;
@@ -1159,18 +1130,27 @@ extern "C" int macko_spmv_plan_build(const int32_t *row_ptr, int32_t rows, int32
         (reinterpret_cast<uintptr_t>(plan) & 15))
         return MACKO_E_INVALID_ARGUMENT;
     SpmvArgs a{};
-    a.row_ptr = row_ptr;
     a.rows = rows;
-    a.cols = cols;
-    a.padded = padded_entries;
+    a.padded = padded;
     a.row_cost = kRowCost;
 #ifdef MACKO_DEV_HOOKS
     if (g_tuning.row_cost >= 0) a.row_cost = (u32)g_tuning.row_cost;
 #endif
     set_cut_fields(a, (u32)n_waves);
+    *out = PlanArgs{row_ptr, plan, rows, (u32)n_waves, a.row_cost, a.entries_q, a.entries_rem, a.rows_q, a.rows_frac, a.row_even};
+    return 0;
+}
+}  // namespace macko
+
+extern "C" int macko_spmv_plan_build(const int32_t *row_ptr, int32_t rows, int32_t cols, int64_t padded_entries,
+                                     int32_t *plan, int32_t plan_entries, void *stream)
+{
+    using namespace macko;
+    PlanArgs a;
+    const int rc = spmv_plan_args(row_ptr, rows, cols, padded_entries, plan, plan_entries, &a);
+    if (rc != 0 || a.n_waves == 0) return rc;
     const int threads = 256;
-    hipLaunchKernelGGL(plan_kernel, dim3((unsigned)((n_waves + 1 + threads - 1) / threads)), dim3(threads), 0,
-                       as_stream(stream), a, (u32)n_waves, plan);
+    hipLaunchKernelGGL(plan_kernel, dim3((a.n_waves + 1 + threads - 1) / threads), dim3(threads), 0, as_stream(stream), a);
     return (int)hipGetLastError();
 }
 

@@ -78,8 +78,48 @@ struct SpmvArgs {
 #define MACKO_STAMP(slot) do { } while (0)
 #endif
 
+// What a plan is made from (macko_spmv_plan_build): how the rows are dealt to n_waves waves, as in SpmvArgs.
+struct PlanArgs {
+    const int *row_ptr;
+    int *plan;
+    int rows;
+    u32 n_waves;
+    u32 row_cost, entries_q, entries_rem, rows_q, rows_frac, row_even;
+};
+
 // First item of part k when n items are dealt to the parts as evenly as possible.
 __device__ __forceinline__ u32 even_split(u32 k, u32 q, u32 rem) { return k * q + (k < rem ? k : rem); }
+
+// Cut k is where wave k of the launch starts (cut n_waves: the end), by the rule the kernel itself applies when it has
+// no plan: the first row r with row_ptr[r] + row_cost * r >= target k, or the row before if that is nearer; even
+// shares of the rows when there are no more rows than waves.  plan[2k] = row, plan[2k + 1] = row_ptr[row].
+__device__ __forceinline__ void write_cut(const PlanArgs &a, u32 k)
+{
+    int cut;
+    if (k == 0) {
+        cut = 0;
+    } else if (k == a.n_waves) {
+        cut = a.rows;
+    } else if (a.row_even) {
+        cut = (int)(k * a.rows_q + __umulhi(k, a.rows_frac));
+    } else {
+        const long long target = (long long)even_split(k, a.entries_q, a.entries_rem);
+        const long long row_cost = (long long)a.row_cost;
+        int lo = 0, hi = a.rows;  // cost(rows) = the whole sum >= any target
+        while (lo < hi) {
+            const int mid = lo + ((hi - lo) >> 1);
+            if ((long long)a.row_ptr[mid] + row_cost * mid >= target) hi = mid; else lo = mid + 1;
+        }
+        cut = lo;
+        if (cut > 0) {
+            const long long after = (long long)a.row_ptr[cut] + row_cost * cut;
+            const long long before = (long long)a.row_ptr[cut - 1] + row_cost * (cut - 1);
+            if (target - before < after - target) cut -= 1;
+        }
+    }
+    a.plan[2 * k] = cut;
+    a.plan[2 * k + 1] = a.row_ptr[cut];
+}
 
 __device__ __forceinline__ float half_bits_to_float(uint16_t h)
 {
@@ -313,6 +353,9 @@ __device__ __forceinline__ float pick_lane(const float (&c)[8], int idx, int L)
 // lds_x = bytes of LDS that x takes (0 when x is gathered from memory).  Returns an ABI error code.
 int spmv_split_launch(const spmv_detail::SpmvArgs &a, bool axpby, int value_bytes, int n_vectors, int fused,
                       bool x_in_lds, int grid, size_t lds_x, hipStream_t stream);
+
+// Checks a plan's size for this shape (macko_spmv_plan_build) and says what it is made from; out->n_waves 0: none to make.
+int spmv_plan_args(const int *row_ptr, int rows, int cols, long long padded, int *plan, int plan_entries, spmv_detail::PlanArgs *out);
 
 // How spmv_tile_kernel cuts a product up for a launch.
 struct TileShape {

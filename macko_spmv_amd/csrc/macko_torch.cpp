@@ -184,7 +184,7 @@ void multiply_axpby_hip(const at::Tensor &M_values, const at::Tensor &M_deltas, 
     check_rc(rc, "multiply_axpby");
 }
 
-std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t> compress_on_device(const at::Tensor &M)
+std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t> compress_on_device(const at::Tensor &M, at::Tensor *plan = nullptr)
 {
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(M.device());
     const int64_t rows = M.size(0), cols = M.size(1);
@@ -228,6 +228,16 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t> compress_on_dev
     const int64_t padded = (n + 7) / 8 * 8;
     at::Tensor values = at::empty({padded}, M.options());
     at::Tensor deltas = at::empty({padded / 2}, M.options().dtype(at::kByte));
+    if (plan != nullptr) {  // the product's cuts with it (fp16)
+        int32_t entries = 0;
+        check_rc(macko_spmv_plan_entries((int32_t)rows, (int32_t)cols, padded, &entries), "compress (plan)");
+        *plan = at::empty({entries}, row_ptr.options());
+        check_rc(macko_compress_f16_fill_plan(M.data_ptr(), (int32_t)rows, (int32_t)cols, row_ptr.data_ptr<int>(), values.data_ptr(),
+                                              deltas.data_ptr(), padded, entries > 0 ? plan->data_ptr<int>() : nullptr, entries,
+                                              (void *)stream),
+                 "compress (fill)");
+        return std::make_tuple(values, deltas, row_ptr, rows, cols);
+    }
     check_rc((int8 ? macko_compress_i8_fill : macko_compress_f16_fill)(
                  M.data_ptr(), (int32_t)rows, (int32_t)cols, row_ptr.data_ptr<int>(), values.data_ptr(),
                  deltas.data_ptr(), padded, (void *)stream),
@@ -946,8 +956,33 @@ PyObject *eager_multiply_axpby(PyObject *, PyObject *const *args, Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// compress(M): the five of the operator and the plan (None: products of this shape take none).
+PyObject *eager_compress(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    EagerCall call;
+    const at::Tensor *M = nullptr;
+    if (n != 1 || !unobserved() || !call.tensor(args[0], M) || M->dtype() != at::kHalf || M->dim() != 2 || !M->is_contiguous())
+        return not_implemented();
+    at::Tensor plan;
+    std::optional<std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t>> out;
+    {
+        WithoutGil released;
+        out.emplace(compress_on_device(*M, &plan));
+    }
+    PyObject *found = Py_None;
+    if (plan.numel() > 0)
+        found = THPVariable_Wrap(std::move(plan));
+    else
+        Py_INCREF(found);
+    return Py_BuildValue("NNNLLN", THPVariable_Wrap(std::get<0>(*out)), THPVariable_Wrap(std::get<1>(*out)),
+                         THPVariable_Wrap(std::get<2>(*out)), (long long)std::get<3>(*out), (long long)std::get<4>(*out), found);
+    END_HANDLE_TH_ERRORS
+}
+
 #define MACKO_EAGER(NAME, ...) {#NAME, (PyCFunction)(void (*)(void))&__VA_ARGS__, METH_FASTCALL, nullptr}
 PyMethodDef eager_functions[] = {
+    MACKO_EAGER(compress, eager_compress),
     MACKO_EAGER(multiply, eager_multiply),
     MACKO_EAGER(multiply_axpby, eager_multiply_axpby),
     MACKO_EAGER(multiply_batched, eager<&multiply_batched_hip>),

@@ -124,3 +124,21 @@ def test_refused_calls_stay_refused(case):
         with pytest.raises(error):
             call()
     assert np.isfinite(mk.multiply(c, x).float().cpu().numpy()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,density", [(1, 8, 1.0), (3, 100, 0.0), (64, 130, 0.3), (4097, 64, 0.4), (5000, 700, 0.2), (20000, 50, 0.2),
+                                               (12289, 257, 0.1), (300, 9000, 0.5), (9000, 9000, 0.02)])
+def test_cuts_made_beside_the_rows_are_those_of_the_operator(rows, cols, density):
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    keep = torch.rand(rows, cols, device="cuda", generator=g) < density * 2 * torch.rand(rows, 1, device="cuda", generator=g)
+    m = (torch.randn(rows, cols, device="cuda", generator=g) * keep).half()
+    c, general = mk.compress(m), torch.ops.macko_spmv.compress(m)
+    assert type(c) is tuple and len(c) == 5 and all(torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b for a, b in zip(c, general))
+    plan = torch.ops.macko_spmv.plan(c[2], rows, cols, c[0].numel())
+    made = getattr(c[2], mk._PLAN_ATTRIBUTE)
+    assert made is None if plan.numel() == 0 else torch.equal(made, plan)
+    with pytest.raises(AssertionError):
+        mk.compress(m.t()) if rows > 1 else mk.compress(m[:, ::2])
+    with pytest.raises(RuntimeError):
+        mk.compress(m.float())
