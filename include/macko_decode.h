@@ -70,6 +70,13 @@ MACKO_API int macko_decode_rope_attention_parts_f16(const void *q, const void *k
                                           float *parts, int32_t n_heads, int32_t head_dim,
                                           int32_t max_len, float scale, void *stream);
 
+/*
+ * y [rows] = W rmsnorm(x) for a dense fp16 W [rows, cols], the normed vector rounded to fp16 in between (the output
+ * layer of a decode step).  cols % 8 == 0, cols <= 4096; w, x and norm_weight 16-byte aligned.
+ */
+MACKO_API int macko_decode_norm_matvec_f16(const void *w, const void *x, const void *norm_weight, void *y,
+                                 int32_t rows, int32_t cols, float eps, void *stream);
+
 /* out[i] = silu(gate[i]) * up[i], i < n. */
 MACKO_API int macko_decode_silu_mul_f16(const void *gate, const void *up, void *out, int32_t n,
                               void *stream);

@@ -71,7 +71,7 @@ def _operator(name):
 # the operators that the package calls itself, as such functions
 ops = types.SimpleNamespace(**{name: _operator(name) for name in (
     "multiply_batched", "multiply_int8", "multiply_int8_axpby", "multiply_rmsnorm", "multiply_silu_mul_axpby",
-    "multiply_attention_axpby", "decode_rmsnorm", "decode_rope_append", "decode_attention", "decode_silu_mul",
+    "multiply_attention_axpby", "decode_rmsnorm", "decode_norm_matvec", "decode_rope_append", "decode_attention", "decode_silu_mul",
     "decode_rope_attention", "decode_rope_attention_parts", "pack_rmsnorm", "rmsnorm_rows", "pack_silu_mul", "multiply_packed",
     "multiply_packed_several", "prefill_rope_append", "prefill_attention")})
 
@@ -174,6 +174,11 @@ def _prefill_attention_fake(q, k_cache, v_cache, positions, scale):
 @torch.library.register_fake("macko_spmv::decode_rmsnorm")
 def _decode_rmsnorm_fake(x, weight, eps):
     return torch.empty_like(x)
+
+
+@torch.library.register_fake("macko_spmv::decode_norm_matvec")
+def _decode_norm_matvec_fake(W, x, norm_weight, eps):
+    return x.new_empty((W.shape[0],))
 
 
 @torch.library.register_fake("macko_spmv::decode_rope_append")

@@ -424,6 +424,24 @@ at::Tensor decode_silu_mul_hip(const at::Tensor &gate, const at::Tensor &up)
     return out;
 }
 
+// W @ rmsnorm(x) for a dense W.
+at::Tensor decode_norm_matvec_hip(const at::Tensor &W, const at::Tensor &x, const at::Tensor &norm_weight, double eps)
+{
+    check_half_gpu(W, "W");
+    check_half_gpu(x, "x");
+    check_half_gpu(norm_weight, "norm_weight");
+    TORCH_CHECK(W.dim() == 2 && x.numel() == W.size(1) && norm_weight.numel() == W.size(1) && W.size(0) < (1ll << 31) && W.size(1) < (1ll << 31),
+                "W must be [rows, cols], x and norm_weight hold cols elements");
+    TORCH_CHECK(x.device() == W.device() && norm_weight.device() == W.device(), "all operands must live on one GPU");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(W.device());
+    at::Tensor y = at::empty({W.size(0)}, W.options());
+    check_rc(macko_decode_norm_matvec_f16(W.data_ptr(), x.data_ptr(), norm_weight.data_ptr(), y.data_ptr(), (int32_t)W.size(0),
+                                          (int32_t)W.size(1), (float)eps,
+                                          (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()),
+             "decode_norm_matvec");
+    return y;
+}
+
 // M @ rmsnorm(V): the norm is applied while V is staged for the product.
 at::Tensor multiply_rmsnorm_hip(const at::Tensor &M_values, const at::Tensor &M_deltas,
                                 const at::Tensor &M_row_indices, int64_t M_rows, int64_t M_cols, const at::Tensor &V,
@@ -992,6 +1010,7 @@ PyMethodDef eager_functions[] = {
     MACKO_EAGER(multiply_silu_mul_axpby, eager<&multiply_silu_mul_axpby_hip>),
     MACKO_EAGER(multiply_attention_axpby, eager<&multiply_attention_axpby_hip>),
     MACKO_EAGER(decode_rmsnorm, eager<&decode_rmsnorm_hip>),
+    MACKO_EAGER(decode_norm_matvec, eager<&decode_norm_matvec_hip>),
     MACKO_EAGER(decode_rope_append, eager<&decode_rope_append_hip>),
     MACKO_EAGER(decode_attention, eager<&decode_attention_hip>),
     MACKO_EAGER(decode_silu_mul, eager<&decode_silu_mul_hip>),
@@ -1036,6 +1055,7 @@ TORCH_LIBRARY(macko_spmv, m)
     m.def("multiply_int8_axpby(Tensor M_values, Tensor M_deltas, Tensor M_row_indices, int M_rows, int M_cols, "
           "Tensor V, Tensor(a!) C, float alpha, float beta) -> ()");
     m.def("decode_rmsnorm(Tensor x, Tensor weight, float eps) -> Tensor");
+    m.def("decode_norm_matvec(Tensor W, Tensor x, Tensor norm_weight, float eps) -> Tensor");
     m.def("decode_rope_append(Tensor q, Tensor k, Tensor v, Tensor cos_table, Tensor sin_table, Tensor position, "
           "Tensor(a!) k_cache, Tensor(b!) v_cache) -> Tensor");
     m.def("decode_attention(Tensor q, Tensor k_cache, Tensor v_cache, Tensor position, float scale) -> Tensor");
@@ -1076,6 +1096,7 @@ TORCH_LIBRARY_IMPL(macko_spmv, CUDA, m)
     m.impl("multiply_int8", &multiply_int8_hip);
     m.impl("multiply_int8_axpby", &multiply_int8_axpby_hip);
     m.impl("decode_rmsnorm", &decode_rmsnorm_hip);
+    m.impl("decode_norm_matvec", &decode_norm_matvec_hip);
     m.impl("decode_rope_append", &decode_rope_append_hip);
     m.impl("decode_attention", &decode_attention_hip);
     m.impl("decode_silu_mul", &decode_silu_mul_hip);

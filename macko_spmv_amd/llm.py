@@ -561,7 +561,11 @@ class DecodeEngine:
             else:
                 gu = self._matvec(L["gate_up"], ops.decode_rmsnorm(x, L["norm2"], self.eps))
                 self._matvec_add(L["down"], ops.decode_silu_mul(gu[:I], gu[I:]), x)
-        return torch.mv(self.lm_head, ops.decode_rmsnorm(x, self.final_norm, self.eps))
+        head = self.lm_head
+        if (type(head) is torch.Tensor and head.dtype == torch.float16 and head.is_contiguous() and H % 8 == 0 and H <= 4096
+                and head.shape[1] == H and head.data_ptr() % 16 == self.final_norm.data_ptr() % 16 == 0):
+            return ops.decode_norm_matvec(head, x, self.final_norm, self.eps)  # norm and product in one launch
+        return torch.mv(head, ops.decode_rmsnorm(x, self.final_norm, self.eps))
 
 
 def engine_decode(engine, prompt, new_tokens, use_graph=True):

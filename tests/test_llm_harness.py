@@ -336,3 +336,25 @@ def test_engine_with_a_dense_o_projection_among_compressed_ones(head_dim):
             want = dense(tokens[:, i:i + 1], torch.tensor([i], device="cuda"))[0, 0].float()
             # as the engine's other tests: fp16 activations rounded in other places
             assert torch.allclose(got, want, rtol=2e-2, atol=2e-2), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(1, 8), (7, 504), (8, 512), (4096, 520), (4097, 1024), (5000, 1032), (32000, 2048), (1003, 2056), (9000, 4088), (32000, 4096)])
+def test_norm_and_dense_product_in_one_launch(rows, cols):
+    ops = torch.ops.macko_spmv
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    W = torch.randn(rows, cols, device="cuda", generator=g).mul_(0.02).half()
+    x = torch.randn(cols, device="cuda", generator=g).half()
+    w = (1 + 0.1 * torch.randn(cols, device="cuda", generator=g)).half()
+    y = ops.decode_norm_matvec(W, x, w, 1e-5)
+    staged = ops.decode_rmsnorm(x, w, 1e-5).double()
+    want = (W.double() * staged).sum(1)
+    # one rounding of an fp32 sum; and what a rounding of the normed vector in the other direction makes (the sum of squares in
+    # another order: at most 2^-10 of one element each)
+    bound = 2.0 ** -11 * want.abs() + 2.0 ** -24 + cols * 2.0 ** -24 * (W.double() * staged).abs().sum(1) + 2.0 ** -9 * (W.double() * staged).abs().max(1).values
+    assert ((y.double() - want).abs() <= bound).all()
+    torch.library.opcheck(ops.decode_norm_matvec, (W, x, w, 1e-5))
+    with pytest.raises(RuntimeError):
+        ops.decode_norm_matvec(W, x[1:], w, 1e-5)
+    with pytest.raises(RuntimeError):
+        ops.decode_norm_matvec(torch.zeros(2, 4104, device="cuda").half(), torch.zeros(4104, device="cuda").half(), torch.zeros(4104, device="cuda").half(), 1e-5)
