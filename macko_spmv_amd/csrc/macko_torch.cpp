@@ -743,11 +743,12 @@ at::Tensor prefill_attention_hip(const at::Tensor &q, const at::Tensor &k_cache,
 // operator.
 
 // Nothing in this thread looks at operators: modes of Python, torch.func, tracing and whatever else adds dispatch keys
-// of its own; __torch_function__ modes; the profiler.
+// of its own, autocasting (a program may have registered a rule); __torch_function__ modes; the profiler.
 bool unobserved()
 {
     const c10::impl::LocalDispatchKeySet tls = c10::impl::tls_local_dispatch_key_set();
-    return (tls.included_ | c10::default_included_set) == c10::default_included_set && !at::impl::torch_function_mode_enabled() && !at::hasCallbacks();
+    return (tls.included_ | c10::default_included_set) == c10::default_included_set &&
+           tls.excluded_.has(c10::DispatchKey::AutocastCUDA) && !at::impl::torch_function_mode_enabled() && !at::hasCallbacks();
 }
 
 // A tensor whose operators only the CUDA kernel is registered for.

@@ -110,6 +110,9 @@ def test_what_looks_at_operators_still_sees_them(case):
         assert mk._eager.multiply(c, leaf) is not NotImplemented
     with torch.inference_mode():
         assert torch.equal(mk.multiply(c, x), want)
+    with torch.autocast("cuda"):
+        assert mk._eager.multiply(c, x) is NotImplemented and torch.equal(mk.multiply(c, x), want)
+    assert mk._eager.multiply(c, x) is not NotImplemented
 
 
 @pytest.mark.gpu
