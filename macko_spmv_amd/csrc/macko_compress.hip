@@ -14,8 +14,8 @@
 // int8 elements, except that the padding entries after a row's last non-zero ARE stored.
 //
 // Pass 1 (count_rows_kernel + scan_rows_kernel) produces row_ptr; pass 2 (fill_rows_kernel)
-// writes values and nibbles.  One wave owns one row in both passes; lanes take 8 consecutive
-// columns and learn the previous non-zero's column from a DPP running maximum.
+// writes values and nibbles.  One wave owns one row in both passes (a few long rows: eight waves a row, each a piece
+// of whole tiles); lanes take 8 consecutive columns and learn the previous non-zero's column from a DPP running maximum.
 
 #include "macko_packed.h"
 #include "macko_spmv_detail.h"
@@ -173,46 +173,103 @@ __device__ __forceinline__ int wave_sum_int(int x)
     return __builtin_amdgcn_readlane(wave_scan_inclusive(x), kWave - 1);
 }
 
-template <typename F, bool STREAM>
-__global__ void __launch_bounds__(kBlock) count_rows_kernel(const typename F::Elem *__restrict__ dense, int rows,
-                                                            int cols, int *__restrict__ counts)
+// Columns [begin, end) of a row, whole tiles but for the row's end: the first and the last non-zero (kNoColumn where
+// there is none), and the entries up to the last one, taken as if a non-zero stood in front of `begin`.
+struct Piece {
+    int first, last, entries;
+};
+
+// The wave's piece of a row that PIECES waves share.
+template <int PIECES>
+__device__ __forceinline__ void piece_columns(int piece, int cols, int &begin, int &end)
 {
-    typedef typename F::Elem Elem;
+    begin = 0;
+    end = cols;
+    if (PIECES > 1) {
+        const int per = ((cols + kTile - 1) / kTile + PIECES - 1) / PIECES * kTile;
+        begin = piece * per < cols ? piece * per : cols;
+        end = begin + per < cols ? begin + per : cols;
+    }
+}
+
+template <typename F, bool STREAM>
+__device__ __forceinline__ Piece count_piece(const typename F::Elem *__restrict__ src, int begin, int end, int cols, int lane)
+{
     typedef typename F::Chunk Chunk;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int row = blockIdx.x * kRowsPerBlock + uniform(threadIdx.x >> 6);
-    if (row >= rows) return;
-    const Elem *src = dense + (size_t)row * (size_t)cols;
-    int carry = -1;  // column of the last non-zero seen in earlier passes
+    int carry = begin - 1;  // column of the last non-zero seen in earlier passes
     int mine = 0;
-    // kAhead tiles of the row are in flight at any time: a wave walks its row alone, so what hides
+    int least = kNoColumn;  // -1 - the lane's first non-zero
+    // kAhead tiles of the row are in flight at any time: a wave walks its columns alone, so what hides
     // the memory latency is the depth of its own queue
     Chunk ahead[kAhead];
 #pragma unroll
     for (int k = 0; k < kAhead; ++k) {
-        const int col = k * kTile + lane * kChunk;
-        ahead[k] = load8<F, STREAM>(src, col, cols);
+        const int col = begin + k * kTile + lane * kChunk;
+        ahead[k] = begin + k * kTile < end ? load8<F, STREAM>(src, col, cols) : Chunk{};
     }
-    for (int c0 = 0; c0 < cols; c0 += kAhead * kTile) {
+    for (int c0 = begin; c0 < end; c0 += kAhead * kTile) {
 #pragma unroll
         for (int k = 0; k < kAhead; ++k) {
             const int col = c0 + k * kTile + lane * kChunk;
-            if (c0 + k * kTile >= cols) break;  // wave-uniform
+            if (c0 + k * kTile >= end) break;  // wave-uniform
             const Chunk v = cut8<F>(ahead[k], c0 + k * kTile, col, cols);
             const int ncol = col + kAhead * kTile;
-            if (c0 + (k + kAhead) * kTile < cols) ahead[k] = load8<F, STREAM>(src, ncol, cols);
+            if (c0 + (k + kAhead) * kTile < end) ahead[k] = load8<F, STREAM>(src, ncol, cols);
             const u32 nz = F::nonzero_bits(v);
             const int own_last = nz ? col + 31 - __builtin_clz(nz) : kNoColumn;
             int pass_last;
             const int p = previous_nonzero(own_last, carry, pass_last);
             // every non-zero is an entry; padding entries can only stand in front of the first
             // non-zero of my 8 columns (the others follow their predecessor within 8 columns)
-            if (nz) mine += __builtin_popcount(nz) + ((col + __builtin_ctz(nz) - p - 1) >> 4);
+            if (nz) {
+                const int first = col + __builtin_ctz(nz);
+                mine += __builtin_popcount(nz) + ((first - p - 1) >> 4);
+                if (least == kNoColumn) least = -1 - first;
+            }
             carry = pass_last > carry ? pass_last : carry;
         }
     }
-    int total = wave_sum_int(mine);
-    if (F::kKeepTrailing) total += (cols - 1 - carry) >> 4;  // padding entries at carry+16, carry+32, ... < cols
+    const int most = __builtin_amdgcn_readlane(wave_scan_max_inclusive(least), kWave - 1);
+    return {most == kNoColumn ? kNoColumn : -1 - most, carry >= begin ? carry : kNoColumn, wave_sum_int(mine)};
+}
+
+// Puts a piece behind the pieces before it: `entries` counts up to the last non-zero so far, `last`.
+__device__ __forceinline__ void append_piece(const Piece &piece, int begin, int &entries, int &last)
+{
+    if (piece.first == kNoColumn) return;
+    entries += piece.entries - ((piece.first - begin) >> 4) + ((piece.first - last - 1) >> 4);
+    last = piece.last;
+}
+
+// PIECES waves work one row, PIECES = 1: kRowsPerBlock rows of a wave each.
+template <int PIECES>
+constexpr int kBlockOf = PIECES > 1 ? PIECES * kWave : kBlock;
+
+template <typename F, bool STREAM, int PIECES>
+__global__ void __launch_bounds__(kBlockOf<PIECES>) count_rows_kernel(const typename F::Elem *__restrict__ dense, int rows,
+                                                                      int cols, int *__restrict__ counts)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = uniform(threadIdx.x >> 6);
+    const int row = PIECES > 1 ? (int)blockIdx.x : (int)blockIdx.x * kRowsPerBlock + wave;
+    if (row >= rows) return;
+    int begin, end;
+    piece_columns<PIECES>(wave, cols, begin, end);
+    const Piece piece = count_piece<F, STREAM>(dense + (size_t)row * (size_t)cols, begin, end, cols, lane);
+    int total = 0, last = -1;
+    if (PIECES > 1) {
+        __shared__ Piece pieces[PIECES];
+        if (lane == 0) pieces[wave] = piece;
+        __syncthreads();
+        if (threadIdx.x != 0) return;
+        for (int w = 0; w < PIECES; ++w) {
+            piece_columns<PIECES>(w, cols, begin, end);
+            append_piece(pieces[w], begin, total, last);
+        }
+    } else {
+        append_piece(piece, 0, total, last);
+    }
+    if (F::kKeepTrailing) total += (cols - 1 - last) >> 4;  // padding entries at last+16, last+32, ... < cols
     if (lane == 0) counts[row] = total;
 }
 
@@ -312,17 +369,22 @@ __device__ __forceinline__ void wave_lds_fence()
 // of its first non-zero, or 15 for a padding entry); the later row's wave leaves the byte alone.
 // So every byte of `deltas` and every element of `values` has exactly one writer, and neither
 // array needs to be cleared beforehand.
-template <typename F, bool STREAM>
-__global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Elem *__restrict__ dense, int rows,
-                                                           int cols, const int *__restrict__ row_ptr,
-                                                           typename F::Elem *__restrict__ values,
-                                                           u32 *__restrict__ delta_words, int padded,
-                                                           const spmv_detail::PlanArgs cuts, int cut_blocks)
+//
+// PIECES > 1: the waves of a workgroup share a row, where a wave per row leaves most of the chip idle and walks its row
+// tile after tile (300 x 49152: 110 us for both passes, 39 with eight waves).  What a piece needs of those before it,
+// its first entry's place and the last non-zero, the waves find by counting their pieces (the read that follows comes from the
+// cache) and exchanging three numbers through LDS.  Pieces meet in a group as rows do.
+template <typename F, bool STREAM, int PIECES>
+__global__ void __launch_bounds__(kBlockOf<PIECES>) fill_rows_kernel(const typename F::Elem *__restrict__ dense, int rows,
+                                                                     int cols, const int *__restrict__ row_ptr,
+                                                                     typename F::Elem *__restrict__ values,
+                                                                     u32 *__restrict__ delta_words, int padded,
+                                                                     const spmv_detail::PlanArgs cuts, int cut_blocks)
 {
     // The first workgroups make the product's cuts, a thread each (macko_spmv_plan_build): beside the rows they cost
     // nothing, behind them a launch (11008 x 4096: 5 us).
     if ((int)blockIdx.x < cut_blocks) {
-        const u32 k = blockIdx.x * kBlock + threadIdx.x;
+        const u32 k = blockIdx.x * kBlockOf<PIECES> + threadIdx.x;
         if (k <= cuts.n_waves) spmv_detail::write_cut(cuts, k);
         return;
     }
@@ -330,29 +392,36 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
     typedef typename F::Chunk Chunk;
     // the carried part of a group, a tile's entries, and what the last half stores behind its own
     constexpr int kStage = 8 + kTile + 8;
+    constexpr int kWaves = kBlockOf<PIECES> / kWave;
     constexpr int kNibbleWords = kTile / 8 + 2;
-    __shared__ __attribute__((aligned(16))) Elem stage_all[kRowsPerBlock][kStage + 4 * kWave];  // + 4 spare places per lane
-    __shared__ u32 nibbles_all[kRowsPerBlock][kNibbleWords];
+    __shared__ __attribute__((aligned(16))) Elem stage_all[kWaves][kStage + 4 * kWave];  // + 4 spare places per lane
+    __shared__ u32 nibbles_all[kWaves][kNibbleWords];
     // gap_table[m]: the nibbles of a lane whose entries are the set bits of m, packed, lowest first: the
     // distance to the previous set bit less one, and 0 for the first, whose distance reaches back into
     // earlier lanes and is put in by the lane itself
     __shared__ u32 gap_table[256];
     __shared__ __attribute__((aligned(8))) u32 pack_table[16][F::kHalfWords];
-    static_assert(kBlock == 256, "one table entry per thread");
+    __shared__ Piece pieces[PIECES];
+    static_assert(kBlockOf<PIECES> >= 256, "one table entry per thread");
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = uniform(threadIdx.x >> 6);
-    const int row = ((int)blockIdx.x - cut_blocks) * kRowsPerBlock + wave;
+    const int row = PIECES > 1 ? (int)blockIdx.x - cut_blocks : ((int)blockIdx.x - cut_blocks) * kRowsPerBlock + wave;
     const Elem *src = dense + (size_t)row * (size_t)cols;
+    int begin, end;
+    piece_columns<PIECES>(wave, cols, begin, end);
+    if (PIECES > 1) {
+        const Piece piece = count_piece<F, false>(src, begin, end, cols, lane);
+        if (lane == 0) pieces[wave] = piece;
+    }
 
     // kAhead tiles of the row in flight
     Chunk ahead[kAhead];
 #pragma unroll
     for (int k = 0; k < kAhead; ++k) {
-        const int col = k * kTile + lane * kChunk;
-        ahead[k] = row < rows && k * kTile < cols ? load8<F, STREAM>(src, col, cols) : Chunk{};
+        const int col = begin + k * kTile + lane * kChunk;
+        ahead[k] = row < rows && begin + k * kTile < end ? load8<F, STREAM>(src, col, cols) : Chunk{};
     }
-    {
-        const u32 m = threadIdx.x;
+    if (const u32 m = threadIdx.x; m < 256) {
         u32 word = 0;
         int previous = -1, n = 0;
 #pragma unroll
@@ -369,28 +438,57 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
     if (row >= rows) return;
     const int e0 = row_ptr[row];
     const int e1 = row_ptr[row + 1];
+    // the wave's entries, and the last non-zero in front of its columns
+    int start = e0, stop = e1, carry = -1;
+    int inner_nibble = 0;  // the first nibble of the next piece's entries, where there are some
+    if (PIECES > 1) {
+        int entries = 0, other_begin, other_end;
+        for (int w = 0; w < wave; ++w) {
+            piece_columns<PIECES>(w, cols, other_begin, other_end);
+            append_piece(pieces[w], other_begin, entries, carry);
+        }
+        // up to column c a row holds its entries up to its last non-zero in front of c, and the padding entries behind it
+        // (but none behind the row's last entry)
+        start = e0 + entries + ((begin - 1 - carry) >> 4);
+        start = start < e1 ? start : e1;
+        int last = carry;
+        append_piece(pieces[wave], begin, entries, last);
+        if (end < cols) {
+            stop = e0 + entries + ((end - 1 - last) >> 4);
+            stop = stop < e1 ? stop : e1;
+        }
+        int next = kNoColumn;
+        for (int w = PIECES - 1; w > wave; --w) next = pieces[w].first != kNoColumn ? pieces[w].first : next;
+        const int pad = last + ((end - last + 15) >> 4 << 4);  // the first padding entry from `end` on, unless a non-zero comes before
+        inner_nibble = next != kNoColumn && next < pad ? next - last - 1 & 15 : 15;
+        start = uniform(start);
+        stop = uniform(stop);
+        carry = uniform(carry);
+        inner_nibble = uniform(inner_nibble);
+    }
     Elem *stage = stage_all[wave];
     u32 *nibbles = nibbles_all[wave];
     Chunk *value_groups = reinterpret_cast<Chunk *>(values);
     unsigned char *delta_bytes = reinterpret_cast<unsigned char *>(delta_words);
 
-    if (row == rows - 1) {  // the unused tail of the last 8-entry group (an odd e1's byte has its owner)
+    if (row == rows - 1 && (PIECES == 1 || wave == 0)) {  // the unused tail of the last 8-entry group (an odd e1's byte has its owner)
         for (int i = e1 + lane; i < padded; i += kWave) values[i] = 0;
         for (int i = ((e1 + 1) >> 1) + lane; i < (padded >> 1); i += kWave) delta_bytes[i] = 0;
     }
-    if (e0 == e1) return;
+    if (start == stop) return;
 
     // The first nibble behind my row, wanted if my last entry is the low half of a byte: asked for
     // now, on the guess that the next row is not empty, and looked at when my row is done.
-    const bool shares_last_byte = (e1 & 1) != 0;
+    const bool shares_last_byte = (stop & 1) != 0;
     const bool probe_lane = lane < 16 && lane < cols;
     int next_end = e1;
     u32 next_probe = 0;
-    if (shares_last_byte && row + 1 < rows) {
+    if (shares_last_byte && stop == e1 && row + 1 < rows) {
         next_end = row_ptr[row + 2];
         if (probe_lane) next_probe = dense[(size_t)(row + 1) * (size_t)cols + lane];
     }
     auto first_nibble_behind = [&]() -> u32 {
+        if (PIECES > 1 && stop != e1) return (u32)inner_nibble;
         int r2 = row + 1;
         if (r2 >= rows) return 0u;  // my row holds the last entry: the rest of the byte is padding
         if (next_end == e1) {       // empty rows behind mine: walk on to the next one that is not
@@ -407,10 +505,9 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
 
     // entry base + i is stage[i] and nibble i of `nibbles`; [lo, hi) is staged and not yet written out;
     // nibbles that are not staged are zero
-    int base = e0 & ~7;
-    int lo = e0 - base;
+    int base = start & ~7;
+    int lo = start - base;
     int hi = lo;
-    int carry = -1;
     nibbles[lane] = 0;
     if (lane < kNibbleWords - kWave) nibbles[kWave + lane] = 0;
     wave_lds_fence();
@@ -451,14 +548,14 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
     };
 
     bool row_done = false;
-    for (int c0 = 0; c0 < cols && !row_done; c0 += kAhead * kTile) {
+    for (int c0 = begin; c0 < end && !row_done; c0 += kAhead * kTile) {
 #pragma unroll
         for (int k = 0; k < kAhead; ++k) {
-            if (row_done || c0 + k * kTile >= cols) break;  // wave-uniform
+            if (row_done || c0 + k * kTile >= end) break;  // wave-uniform
             const int col = c0 + k * kTile + lane * kChunk;
             Chunk v = cut8<F>(ahead[k], c0 + k * kTile, col, cols);
             const int ncol = col + kAhead * kTile;
-            if (c0 + (k + kAhead) * kTile < cols) ahead[k] = load8<F, STREAM>(src, ncol, cols);
+            if (c0 + (k + kAhead) * kTile < end) ahead[k] = load8<F, STREAM>(src, ncol, cols);
             const u32 nz = F::nonzero_bits(v);
             const int own_last = nz ? col + 31 - __builtin_clz(nz) : kNoColumn;
             int pass_last;
@@ -476,8 +573,8 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
             const int mine = __builtin_popcount(entry_bits);
             const int incl = wave_scan_inclusive(mine);
             const int produced = __builtin_amdgcn_readlane(incl, kWave - 1);
-            // entries past e1 are padding entries behind the row's last non-zero: not stored
-            const int room = e1 - (base + hi);
+            // entries past the row's end are padding entries behind its last non-zero: not stored
+            const int room = stop - (base + hi);
             const int n_new = produced < room ? produced : room;
             // Those dropped entries are whole lanes: behind the row's last non-zero a lane holds at
             // most its one padding entry, and the lane of the last non-zero has its padding entry
@@ -517,7 +614,7 @@ __global__ void __launch_bounds__(kBlock) fill_rows_kernel(const typename F::Ele
             }
             hi += n_new;
             wave_lds_fence();
-            row_done = base + hi == e1;
+            row_done = base + hi == stop;
             const int n_groups = row_done ? (hi + 7) >> 3 : hi >> 3;
             flush(n_groups, row_done && shares_last_byte ? first_nibble_behind() : 0u);
             if (row_done) break;
@@ -597,6 +694,18 @@ bool streams_past_cache(int32_t rows, int32_t cols)
     return (size_t)rows * (size_t)cols * sizeof(Elem) > ((size_t)128 << 20);
 }
 
+// Which matrices have a row worked by kPieces waves instead of one (both passes; fp16, from a graph, us, 1 / 8 waves):
+// 64 x 2048 12.0 / 10.6, 64 x 8192 24.5 / 12.7, 64 x 49152 108 / 28, 300 x 49152 110 / 39, 500 x 8192 25.1 / 16.3;
+// 800 x 4096 16.7 / 17.1, 800 x 8192 26.1 / 22.2; 1200 x 4096 19.0 / 19.1, 1200 x 8192 28.4 / 25.1, 1200 x 32768 86 / 60;
+// 1800 x 12288 39.3 / 40.3, 1800 x 32768 89 / 83; 2600 x 8192 34.5 / 40.9; 5000 x 8192 50 / 66 (density 0.5; at 0.05 the
+// same within 4 %; int8 512 x 2048 11.6 / 11.5, 500 x 49152 98 / 35, 1280 x 8192 25.4 / 23.0).  Four waves are up to 10 % faster than eight around 1000 x 4096 and up to 30 % slower at few rows,
+// sixteen gain up to 10 % more below 200 rows of 32768 columns and lose up to 40 % elsewhere.
+constexpr int kPieces = 8;
+bool rows_in_pieces(int32_t rows, int32_t cols)
+{
+    return rows <= 512 ? cols >= 2048 : rows <= 1280 && cols >= 8192;
+}
+
 template <typename F>
 int compress_count(const void *dense, int32_t rows, int32_t cols, int32_t *row_ptr, int32_t *total, void *stream)
 {
@@ -610,13 +719,15 @@ int compress_count(const void *dense, int32_t rows, int32_t cols, int32_t *row_p
     hipStream_t s = as_stream(stream);
     if (rows > 0) {
         const bool stream_reads = streams_past_cache<Elem>(rows, cols);
-        const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock);
-        if (stream_reads)
-            hipLaunchKernelGGL((count_rows_kernel<F, true>), grid, dim3(kBlock), 0, s, (const Elem *)dense, rows, cols,
-                               row_ptr + 1);
+        auto launch = [&](auto kernel, int blocks, int threads) {
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, s, (const Elem *)dense, rows, cols, row_ptr + 1);
+        };
+        if (rows_in_pieces(rows, cols))
+            stream_reads ? launch(count_rows_kernel<F, true, kPieces>, rows, kBlockOf<kPieces>)
+                         : launch(count_rows_kernel<F, false, kPieces>, rows, kBlockOf<kPieces>);
         else
-            hipLaunchKernelGGL((count_rows_kernel<F, false>), grid, dim3(kBlock), 0, s, (const Elem *)dense, rows, cols,
-                               row_ptr + 1);
+            stream_reads ? launch(count_rows_kernel<F, true, 1>, (rows + kRowsPerBlock - 1) / kRowsPerBlock, kBlock)
+                         : launch(count_rows_kernel<F, false, 1>, (rows + kRowsPerBlock - 1) / kRowsPerBlock, kBlock);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }
@@ -641,14 +752,18 @@ int compress_fill(const void *dense, int32_t rows, int32_t cols, const int32_t *
         return MACKO_E_INVALID_ARGUMENT;
     hipStream_t s = as_stream(stream);
     if (rows == 0) return MACKO_E_INVALID_ARGUMENT;  // entries without rows
-    const int cut_blocks = cuts.n_waves > 0 ? (int)(cuts.n_waves + kBlock) / kBlock : 0;
-    const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock + cut_blocks);
-    if (streams_past_cache<Elem>(rows, cols))
-        hipLaunchKernelGGL((fill_rows_kernel<F, true>), grid, dim3(kBlock), 0, s, (const Elem *)dense, rows, cols,
-                           row_ptr, (Elem *)values, (u32 *)deltas, (int)padded_entries, cuts, cut_blocks);
+    const bool stream_reads = streams_past_cache<Elem>(rows, cols);
+    auto launch = [&](auto kernel, int blocks, int threads) {
+        const int cut_blocks = cuts.n_waves > 0 ? (int)(cuts.n_waves + threads) / threads : 0;
+        hipLaunchKernelGGL(kernel, dim3(blocks + cut_blocks), dim3(threads), 0, s, (const Elem *)dense, rows, cols, row_ptr,
+                           (Elem *)values, (u32 *)deltas, (int)padded_entries, cuts, cut_blocks);
+    };
+    if (rows_in_pieces(rows, cols))
+        stream_reads ? launch(fill_rows_kernel<F, true, kPieces>, rows, kBlockOf<kPieces>)
+                     : launch(fill_rows_kernel<F, false, kPieces>, rows, kBlockOf<kPieces>);
     else
-        hipLaunchKernelGGL((fill_rows_kernel<F, false>), grid, dim3(kBlock), 0, s, (const Elem *)dense, rows, cols,
-                           row_ptr, (Elem *)values, (u32 *)deltas, (int)padded_entries, cuts, cut_blocks);
+        stream_reads ? launch(fill_rows_kernel<F, true, 1>, (rows + kRowsPerBlock - 1) / kRowsPerBlock, kBlock)
+                     : launch(fill_rows_kernel<F, false, 1>, (rows + kRowsPerBlock - 1) / kRowsPerBlock, kBlock);
     return (int)hipGetLastError();
 }
 

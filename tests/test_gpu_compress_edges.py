@@ -34,3 +34,28 @@ def test_compress_at_edges(int8, density, offset):
         assert np.array_equal(v if int8 else v.view(np.uint16), values), (cols, rows)
         assert np.array_equal(got[1].cpu().numpy(), deltas), (cols, rows)
         assert np.array_equal(got[2].cpu().numpy(), row_ptr), (cols, rows)
+
+
+@pytest.mark.parametrize("int8", (False, True))
+@pytest.mark.parametrize("density", (0.0, 0.0004, 0.05, 0.97))
+def test_rows_of_several_waves(int8, density):
+    # few long rows: pieces that end with the row, before it or after it, pieces without entries, rows without
+    rng = np.random.default_rng(int(density * 10000))
+    for rows, cols, offset in ((1, 8192, 0), (3, 8193, 1), (2, 9215, 0), (5, 12288, 0), (64, 16385, 1), (7, 49152, 0)):
+        flat = rng.standard_normal(rows * cols + offset)
+        flat = np.clip(np.rint(flat * 60), -128, 127).astype(np.int8) if int8 else flat.astype(np.float16)
+        flat[rng.random(flat.size) >= density] = 0
+        dense = flat[offset:].reshape(rows, cols)
+        if rows > 2:
+            dense[1] = 0
+            dense[2, 1024:cols - 1024] = 0
+            dense[0, cols // 2:] = 0
+        if not int8:
+            dense[rows - 1, cols // 2] = np.nan
+        M = torch.from_numpy(flat).cuda()[offset:].view(rows, cols)
+        got = (mk.compress_int8 if int8 else mk.compress)(M)
+        values, deltas, row_ptr, n = (mo.compress_int8 if int8 else mo.compress)(dense)
+        v = got[0].cpu().numpy()
+        assert np.array_equal(v if int8 else v.view(np.uint16), values), (cols, rows)
+        assert np.array_equal(got[1].cpu().numpy(), deltas), (cols, rows)
+        assert np.array_equal(got[2].cpu().numpy(), row_ptr), (cols, rows)
