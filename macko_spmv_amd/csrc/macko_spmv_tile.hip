@@ -601,8 +601,8 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
                 tile_d[S][0] = __builtin_amdgcn_raw_buffer_load_b32(rs_deltas, (int)dof, 0, 0);
             }
 #pragma unroll
-            for (int w = 0; w < W; ++w)
-                tile_v[S][w] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_values, (int)vo, 16 * w, 0));
+            for (int w = 0; w < W; ++w)  // the whole offset is the lane's: what a scalar one adds need not be part of the range check
+                tile_v[S][w] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_values, (int)(vo + 16 * w), 0, 0));
         };
         u32 base = 0, buffer = 0, shift = 0;
         // Where my entries of set S go in this chunk, and which of the row's lanes belong to later ones: pos and

@@ -1,0 +1,63 @@
+"""Products of vectors in operand order that test_gpu_packed_products.py runs, and the kernel each of them takes
+(test_packed_routes_host.py)."""
+import dataclasses
+
+import numpy as np
+
+from tests import helpers
+
+
+@dataclasses.dataclass(frozen=True)
+class Product:
+    batch: int
+    rows: tuple        # of each matrix
+    cols: int
+    density: float
+    kernel: str        # with 256 compute units
+    empty: int = -1    # the matrix without entries
+
+    def __str__(self):
+        return f"{self.kernel[5:9]}{self.kernel[16:]}-{self.batch}x{self.cols}"
+
+
+PRODUCTS = [
+    # lanes of 16 entries: a matrix without entries among others, in front of and behind them
+    Product(17, (12288, 512, 4096), 257, 0.4, "spmv_pipe_kernel<1,16,true>", empty=1),
+    Product(129, (2048, 2048, 2049), 300, 0.4, "spmv_pipe_kernel<4,16,true>", empty=0),
+    # ... and arrays that end in the middle of a lane's entries
+    Product(17, (9001,), 257, 0.3, "spmv_pipe_kernel<1,16,false>"),
+    Product(129, (6143,), 257, 0.45, "spmv_pipe_kernel<4,16,false>"),
+]
+
+
+def matrices(product):
+    """The product's matrices: rows without entries, full rows, rows of one entry behind padding entries and gaps wider than
+    a lane's columns; the stored arrays end 8 entries behind a multiple of 16."""
+    rng = np.random.default_rng(sum(product.rows) + product.cols + product.batch)
+    out = []
+    for k, rows in enumerate(product.rows):
+        if k == product.empty:
+            out.append(np.zeros((rows, product.cols), dtype=np.float16))
+            continue
+        m = helpers.random_sparse(rng, rows, product.cols, product.density, scale=0.05)
+        m[::13, product.cols // 5:product.cols // 5 * 4] = 0
+        m[5::97] = 0
+        full = np.arange(3, rows, 211)
+        m[full] = rng.standard_normal((full.size, product.cols)).astype(np.float16)   # more entries in a chunk than a pass holds
+        m[7] = 0
+        m[7, -1] = 1.0
+        m[0] = 0
+        m[0, :(8 - stored_entries(m)) % 16] = 0.5
+        out.append(m)
+    return out
+
+
+def stored_entries(m):
+    """Entries of a compressed fp16 matrix: its non-zeros, and one for every 16 columns of the distance to the non-zero before."""
+    padded = np.zeros((m.shape[0], m.shape[1] + 1), dtype=bool)
+    padded[:, 0] = True   # a non-zero in front of the row
+    padded[:, 1:] = m != 0
+    at = np.flatnonzero(padded)
+    gap = np.diff(at)
+    first = at[1:] % (m.shape[1] + 1) == 0
+    return int((((gap - 1) >> 4) + 1)[~first].sum())

@@ -1,0 +1,75 @@
+"""Products of vectors in operand order, of one and of several matrices, by every kernel that takes them, against float64.
+
+Bound: the sum in fp32 of n terms in any order (n * 2^-24 of the sum of the terms' magnitudes) and one rounding to fp16 (2^-11
+of the value, 2^-25 where it is subnormal)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import macko_spmv_amd as mk
+from tests import packed_products
+
+pytestmark = pytest.mark.gpu
+ops = torch.ops.macko_spmv
+vp, i32, i64 = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64
+
+
+def _pack(lib, x):
+    batch, cols = x.shape
+    size = i64(-1)
+    assert lib.macko_packed_bytes(cols, batch, ctypes.byref(size)) == 0
+    packed = torch.empty(size.value // 2, dtype=torch.float16, device="cuda")
+    lib.macko_pack_f16.argtypes = [vp, i32, i32, i64, vp, vp]
+    assert lib.macko_pack_f16(x.data_ptr(), cols, batch, cols, packed.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    return packed
+
+
+def _check(y, x, dense, residual=None):
+    """x: finite but for column 1 of one vector, which a padding entry never stands for."""
+    y = y.cpu().double().numpy()
+    x64, d64 = np.where(np.isfinite(x), x, 0).astype(np.float64), dense.astype(np.float64)
+    spoiled = (~np.isfinite(x)).any(axis=1)[:, None] & (dense[:, 1] != 0)[None, :]
+    assert not np.isfinite(y[spoiled]).any() and np.isfinite(y[~spoiled]).all()
+    want = x64 @ d64.T
+    size = np.abs(x64) @ np.abs(d64).T
+    if residual is not None:
+        want, size = want + residual.astype(np.float64), size + np.abs(residual).astype(np.float64)
+    bound = 2.0 ** -11 * np.abs(want) + 2.0 ** -25 + (dense.shape[1] + 3) * 2.0 ** -24 * size
+    assert (np.abs(y - want) <= bound)[~spoiled].all()
+
+
+@pytest.mark.parametrize("product", packed_products.PRODUCTS, ids=str)
+def test_products_of_packed_vectors(product):
+    dense = packed_products.matrices(product)
+    c = [mk.compress(torch.from_numpy(m).cuda()) for m in dense]
+    rng = np.random.default_rng(product.cols)
+    x = rng.standard_normal((product.batch, product.cols)).astype(np.float16)
+    x[product.batch // 2, 1] = np.inf
+    lib = ctypes.CDLL(mk.HIP_LIBRARY_PATH)
+    packed = _pack(lib, torch.from_numpy(x).cuda())
+    if len(c) > 1:
+        args = ([m[0] for m in c], [m[1] for m in c], [m[2] for m in c], list(product.rows), product.cols, packed, product.batch)
+        got = ops.multiply_packed_several(*args)
+        for y, m in zip(got, dense):
+            _check(y, x, m)
+        for y, again in zip(got, ops.multiply_packed_several(*args)):
+            assert torch.equal(y.view(torch.int16), again.view(torch.int16))
+        return
+    (rows,), one = product.rows, c[0]
+    y = ops.multiply_packed(*one, packed, product.batch, None)
+    _check(y, x, dense[0])
+    assert torch.equal(y.view(torch.int16), ops.multiply_packed(*one, packed, product.batch, None).view(torch.int16))
+    # a residual; results of an odd row length that start at an odd element
+    r = rng.standard_normal((product.batch, rows)).astype(np.float16)
+    _check(ops.multiply_packed(*one, packed, product.batch, torch.from_numpy(r).cuda()), x, dense[0], r)
+    lib.macko_spmv_f16_packed.argtypes = [vp, vp, vp, vp, vp, vp, i32, i32, i64, i32, i64, vp]
+    ldy = rows + 2 + (rows + 1) % 2
+    flat = torch.full((product.batch * ldy + 1,), 7.0, dtype=torch.float16, device="cuda")
+    into = flat[1:].view(product.batch, ldy)
+    into[:, :rows] = torch.from_numpy(r).cuda()
+    assert lib.macko_spmv_f16_packed(one[0].data_ptr(), one[1].data_ptr(), one[2].data_ptr(), packed.data_ptr(), into.data_ptr(), into.data_ptr(),
+                                     rows, product.cols, one[0].numel(), product.batch, ldy, torch.cuda.current_stream().cuda_stream) == 0
+    _check(into[:, :rows], x, dense[0], r)
+    assert (into[:, rows:] == 7.0).all() and flat[0] == 7.0
