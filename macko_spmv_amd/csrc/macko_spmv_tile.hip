@@ -637,7 +637,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
             larger(__builtin_amdgcn_update_dpp(0, key, 0x141, 0xF, 0xF, true));   // row_half_mirror
             larger(__builtin_amdgcn_update_dpp(0, key, 0x140, 0xF, 0xF, true));   // row_mirror
             const int done = key & 0xff;   // lanes
-            pos += done * E;
+            pos += left > 0 ? done * E : 0;   // a lane behind the row's end stays there: the rest of the columns is no number of entries
             at_column += (u32)key >> 8;
             front = done ? ~0u : front;
             return __ballot(done == L && pos < end) != 0;

@@ -29,6 +29,9 @@ PRODUCTS = [
     Product(129, (6143,), 257, 0.45, "spmv_pipe_kernel<4,16,false>"),
 ]
 
+# an array that ends as near to 2^31 entries as is taken, and a row there that leaves more columns than that free
+LONG_ARRAY = dict(entries=2 ** 31 - 8200, rows=524288, cols=16384, batch=17, kernel="spmv_pipe_kernel<1,16,false>")
+
 
 def matrices(product):
     """The product's matrices: rows without entries, full rows, rows of one entry behind padding entries and gaps wider than

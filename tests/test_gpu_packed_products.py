@@ -73,3 +73,22 @@ def test_products_of_packed_vectors(product):
                                      rows, product.cols, one[0].numel(), product.batch, ldy, torch.cuda.current_stream().cuda_stream) == 0
     _check(into[:, :rows], x, dense[0], r)
     assert (into[:, rows:] == 7.0).all() and flat[0] == 7.0
+
+
+def test_rows_at_the_end_of_the_longest_array():
+    # 32 entries, in the first columns, for each of the last two rows; what the array holds elsewhere is no row's
+    entries, rows, cols, batch = (packed_products.LONG_ARRAY[k] for k in ("entries", "rows", "cols", "batch"))
+    values = torch.zeros(entries, dtype=torch.float16, device="cuda")
+    values[:1 << 20] = 100.0
+    values[-64:] = 1.0
+    deltas = torch.zeros(entries // 2, dtype=torch.uint8, device="cuda")
+    row_ptr = torch.full((rows + 1,), entries - 64, dtype=torch.int32, device="cuda")
+    row_ptr[-2:] = torch.tensor([entries - 32, entries], dtype=torch.int32)
+    x = np.random.default_rng(1).standard_normal((batch, cols)).astype(np.float16)
+    packed = _pack(ctypes.CDLL(mk.HIP_LIBRARY_PATH), torch.from_numpy(x).cuda())
+    y = ops.multiply_packed(values, deltas, row_ptr, rows, cols, packed, batch, None)
+    assert not y[:, :-2].any()
+    want = x[:, :32].astype(np.float64).sum(axis=1)
+    bound = 2.0 ** -11 * np.abs(want) + 33 * 2.0 ** -24 * np.abs(x[:, :32].astype(np.float64)).sum(axis=1)
+    for row in (-2, -1):
+        assert (np.abs(y[:, row].cpu().double().numpy() - want) <= bound).all()

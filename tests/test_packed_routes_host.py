@@ -2,7 +2,6 @@
 import os
 import subprocess
 
-import numpy as np
 import pytest
 
 from macko_spmv_amd import _build
@@ -40,3 +39,9 @@ def test_the_products_take_the_kernels_they_are_meant_for(routes, product):
     assert routes(product.cols, product.batch, sizes)[0] == product.kernel
     if len(sizes) == 1:
         assert routes(product.cols, product.batch, sizes, residual=True)[0] == product.kernel
+
+
+def test_the_longest_array_takes_the_kernel_it_is_meant_for(routes):
+    long = packed_products.LONG_ARRAY
+    assert routes(long["cols"], long["batch"], [(long["rows"], long["entries"])])[0] == long["kernel"]
+    assert routes(long["cols"], long["batch"], [(long["rows"], long["entries"] + 8)])[0] == "refused"
