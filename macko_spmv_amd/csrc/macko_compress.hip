@@ -131,9 +131,10 @@ struct Int8Format {
 // at most one cache line more per wave; element by element, as this was where rows are not 16-byte aligned,
 // it took eight loads).  The row's last elements come from a load that ends with the row and are moved to
 // their place when they are used (cut8), so that no lane has a path of its own.  STREAM: the dense matrix
-// will not be read again soon (non-temporal hint).
+// will not be read again soon (non-temporal hint).  Columns are unsigned: those of the last tile and of the tiles asked
+// for ahead may lie beyond 2^31.
 template <typename F, bool STREAM>
-__device__ __forceinline__ typename F::Chunk load8(const typename F::Elem *__restrict__ row, int col, int cols)
+__device__ __forceinline__ typename F::Chunk load8(const typename F::Elem *__restrict__ row, u32 col, u32 cols)
 {
     typename F::Chunk v = {};
     if (cols >= 8) {
@@ -141,17 +142,17 @@ __device__ __forceinline__ typename F::Chunk load8(const typename F::Elem *__res
         v = STREAM ? __builtin_nontemporal_load(p) : *p;
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) F::put(v, i, col + i < cols ? (u32)row[col + i] : 0u);
+        for (u32 i = 0; i < 8; ++i) F::put(v, (int)i, col + i < cols ? (u32)row[col + i] : 0u);
     }
     return v;
 }
 
 // what load8 gave for columns [col, col + 8) of the tile that starts at `first`: zero beyond `cols`
 template <typename F>
-__device__ __forceinline__ typename F::Chunk cut8(typename F::Chunk v, int first, int col, int cols)
+__device__ __forceinline__ typename F::Chunk cut8(typename F::Chunk v, u32 first, u32 col, u32 cols)
 {
     if (first + kTile > cols && cols >= 8) {  // wave-uniform
-        const int by = col - (cols - 8);
+        const int by = (int)(col - (cols - 8));
         v = F::shift(v, by > 0 ? by : 0);
     }
     return v;
@@ -186,9 +187,10 @@ __device__ __forceinline__ void piece_columns(int piece, int cols, int &begin, i
     begin = 0;
     end = cols;
     if (PIECES > 1) {
-        const int per = ((cols + kTile - 1) / kTile + PIECES - 1) / PIECES * kTile;
-        begin = piece * per < cols ? piece * per : cols;
-        end = begin + per < cols ? begin + per : cols;
+        const u32 per = (((u32)cols + kTile - 1) / kTile + PIECES - 1) / PIECES * kTile;
+        const u32 from = (u32)piece * per;   // both may lie beyond 2^31
+        begin = from < (u32)cols ? (int)from : cols;
+        end = from + per < (u32)cols ? (int)(from + per) : cols;
     }
 }
 
@@ -203,20 +205,20 @@ __device__ __forceinline__ Piece count_piece(const typename F::Elem *__restrict_
     // the memory latency is the depth of its own queue
     Chunk ahead[kAhead];
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-        const int col = begin + k * kTile + lane * kChunk;
-        ahead[k] = begin + k * kTile < end ? load8<F, STREAM>(src, col, cols) : Chunk{};
+    for (u32 k = 0; k < kAhead; ++k) {
+        const u32 col = (u32)begin + k * kTile + (u32)lane * kChunk;
+        ahead[k] = (u32)begin + k * kTile < (u32)end ? load8<F, STREAM>(src, col, cols) : Chunk{};
     }
-    for (int c0 = begin; c0 < end; c0 += kAhead * kTile) {
+    for (u32 c0 = begin; c0 < (u32)end; c0 += kAhead * kTile) {
 #pragma unroll
-        for (int k = 0; k < kAhead; ++k) {
-            const int col = c0 + k * kTile + lane * kChunk;
-            if (c0 + k * kTile >= end) break;  // wave-uniform
-            const Chunk v = cut8<F>(ahead[k], c0 + k * kTile, col, cols);
-            const int ncol = col + kAhead * kTile;
-            if (c0 + (k + kAhead) * kTile < end) ahead[k] = load8<F, STREAM>(src, ncol, cols);
+        for (u32 k = 0; k < kAhead; ++k) {
+            const u32 at = c0 + k * kTile + (u32)lane * kChunk;
+            const int col = (int)at;   // of a lane that holds elements
+            if (c0 + k * kTile >= (u32)end) break;  // wave-uniform
+            const Chunk v = cut8<F>(ahead[k], c0 + k * kTile, at, cols);
+            if (c0 + (k + kAhead) * kTile < (u32)end) ahead[k] = load8<F, STREAM>(src, at + kAhead * kTile, cols);
             const u32 nz = F::nonzero_bits(v);
-            const int own_last = nz ? col + 31 - __builtin_clz(nz) : kNoColumn;
+            const int own_last = nz ? col + (31 - __builtin_clz(nz)) : kNoColumn;
             int pass_last;
             const int p = previous_nonzero(own_last, carry, pass_last);
             // every non-zero is an entry; padding entries can only stand in front of the first
@@ -417,9 +419,9 @@ __global__ void __launch_bounds__(kBlockOf<PIECES>) fill_rows_kernel(const typen
     // kAhead tiles of the row in flight
     Chunk ahead[kAhead];
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-        const int col = begin + k * kTile + lane * kChunk;
-        ahead[k] = row < rows && begin + k * kTile < end ? load8<F, STREAM>(src, col, cols) : Chunk{};
+    for (u32 k = 0; k < kAhead; ++k) {
+        const u32 col = (u32)begin + k * kTile + (u32)lane * kChunk;
+        ahead[k] = row < rows && (u32)begin + k * kTile < (u32)end ? load8<F, STREAM>(src, col, cols) : Chunk{};
     }
     if (const u32 m = threadIdx.x; m < 256) {
         u32 word = 0;
@@ -548,28 +550,28 @@ __global__ void __launch_bounds__(kBlockOf<PIECES>) fill_rows_kernel(const typen
     };
 
     bool row_done = false;
-    for (int c0 = begin; c0 < end && !row_done; c0 += kAhead * kTile) {
+    for (u32 c0 = begin; c0 < (u32)end && !row_done; c0 += kAhead * kTile) {
 #pragma unroll
-        for (int k = 0; k < kAhead; ++k) {
-            if (row_done || c0 + k * kTile >= end) break;  // wave-uniform
-            const int col = c0 + k * kTile + lane * kChunk;
-            Chunk v = cut8<F>(ahead[k], c0 + k * kTile, col, cols);
-            const int ncol = col + kAhead * kTile;
-            if (c0 + (k + kAhead) * kTile < end) ahead[k] = load8<F, STREAM>(src, ncol, cols);
+        for (u32 k = 0; k < kAhead; ++k) {
+            if (row_done || c0 + k * kTile >= (u32)end) break;  // wave-uniform
+            const u32 at = c0 + k * kTile + (u32)lane * kChunk;
+            const int col = (int)at;   // of a lane that holds elements
+            Chunk v = cut8<F>(ahead[k], c0 + k * kTile, at, cols);
+            if (c0 + (k + kAhead) * kTile < (u32)end) ahead[k] = load8<F, STREAM>(src, at + kAhead * kTile, cols);
             const u32 nz = F::nonzero_bits(v);
-            const int own_last = nz ? col + 31 - __builtin_clz(nz) : kNoColumn;
+            const int own_last = nz ? col + (31 - __builtin_clz(nz)) : kNoColumn;
             int pass_last;
             const int p = previous_nonzero(own_last, carry, pass_last);
             carry = pass_last > carry ? pass_last : carry;
             // Non-zeros are entries.  A padding entry stands at p + 16, p + 32, ...: among my 8
             // columns at most one, and only in front of my first non-zero (behind it the previous
             // non-zero is less than 8 columns away).
-            const int pad_at = p + (((col - p + 15) >> 4) << 4) - col;  // >= 0, my column index of it
-            const int first_nz = nz ? __builtin_ctz(nz) : 8;
-            const bool has_pad = pad_at < first_nz && col + pad_at < cols;
+            const u32 pad_at = (u32)p + (((at - (u32)p + 15) >> 4) << 4) - at;  // my column index of it
+            const u32 first_nz = nz ? (u32)__builtin_ctz(nz) : 8;
+            const bool has_pad = pad_at < first_nz && at + pad_at < (u32)cols;
             const u32 entry_bits = nz | (has_pad ? 1u << pad_at : 0u);
             // a padding entry is 16 columns or a multiple of that behind p: 15, too
-            const u32 first = has_pad ? 15u : (u32)(col + first_nz - p - 1) & 15u;
+            const u32 first = has_pad ? 15u : (at + first_nz - (u32)p - 1) & 15u;
             const int mine = __builtin_popcount(entry_bits);
             const int incl = wave_scan_inclusive(mine);
             const int produced = __builtin_amdgcn_readlane(incl, kWave - 1);

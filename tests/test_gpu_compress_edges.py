@@ -59,3 +59,23 @@ def test_rows_of_several_waves(int8, density):
         assert np.array_equal(v if int8 else v.view(np.uint16), values), (cols, rows)
         assert np.array_equal(got[1].cpu().numpy(), deltas), (cols, rows)
         assert np.array_equal(got[2].cpu().numpy(), row_ptr), (cols, rows)
+
+
+@pytest.mark.parametrize("int8", (False, True))
+def test_the_longest_row(int8):
+    # 2^31 - 1 columns; non-zeros in the first, a middle and the last piece, one of them the last column
+    cols = 2 ** 31 - 1
+    at = torch.tensor([5, 4096, 2 ** 30 + 3, 2 ** 31 - 4099, 2 ** 31 - 520, 2 ** 31 - 2], device="cuda")
+    M = torch.zeros(1, cols, dtype=torch.int8 if int8 else torch.float16, device="cuda")
+    M[0, at] = torch.arange(1, 7, device="cuda", dtype=M.dtype)
+    values, deltas, row_ptr = (mk.compress_int8 if int8 else mk.compress)(M)[:3]
+    gap = torch.diff(at, prepend=torch.tensor([-1], device="cuda")) - 1
+    place = torch.cumsum((gap >> 4) + 1, 0) - 1   # an entry for every 16 columns of a gap, and the non-zero's
+    entries = int(place[-1]) + 1
+    assert row_ptr.tolist() == [0, entries] and values.numel() == (entries + 7) // 8 * 8
+    assert torch.equal(values.nonzero()[:, 0], place) and values[place].tolist() == [1, 2, 3, 4, 5, 6]
+    nibbles = torch.stack((deltas & 15, deltas >> 4), 1).view(-1)
+    assert torch.equal(nibbles[place], (gap & 15).to(torch.uint8)) and not nibbles[entries:].any()
+    others = nibbles[:entries] != 15
+    others[place] = False
+    assert not others.any()
