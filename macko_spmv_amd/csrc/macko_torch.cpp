@@ -424,7 +424,8 @@ at::Tensor decode_silu_mul_hip(const at::Tensor &gate, const at::Tensor &up)
     return out;
 }
 
-// W @ rmsnorm(x) for a dense W.
+// W @ rmsnorm(x) for a dense W.  Operands that do not start at a 16-byte address go through the norm and the library's
+// product; asked here, where a graph of the step does not see it.
 at::Tensor decode_norm_matvec_hip(const at::Tensor &W, const at::Tensor &x, const at::Tensor &norm_weight, double eps)
 {
     check_half_gpu(W, "W");
@@ -434,6 +435,8 @@ at::Tensor decode_norm_matvec_hip(const at::Tensor &W, const at::Tensor &x, cons
                 "W must be [rows, cols], x and norm_weight hold cols elements");
     TORCH_CHECK(x.device() == W.device() && norm_weight.device() == W.device(), "all operands must live on one GPU");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(W.device());
+    if ((reinterpret_cast<uintptr_t>(W.data_ptr()) | reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(norm_weight.data_ptr())) & 15)
+        return at::mv(W, decode_rmsnorm_hip(x, norm_weight, eps).view({-1}));
     at::Tensor y = at::empty({W.size(0)}, W.options());
     check_rc(macko_decode_norm_matvec_f16(W.data_ptr(), x.data_ptr(), norm_weight.data_ptr(), y.data_ptr(), (int32_t)W.size(0),
                                           (int32_t)W.size(1), (float)eps,

@@ -460,7 +460,8 @@ class DecodeEngine:
     attention share one kernel, and, for MACKO projections, the two RMS norms and the SiLU gate are
     applied by the product that consumes them while it stages its input (multiply_rmsnorm,
     multiply_silu_mul_axpby).  Dense projections go through the BLAS matrix-vector product, which
-    has no such hook, and keep their separate norm and gate kernels."""
+    has no such hook, and keep their separate norm and gate kernels.  The output layer is dense and, up to 4096 columns,
+    one launch with the norm in front of it, whatever `fuse` is."""
 
     def __init__(self, model, fuse=True):
         ops = macko_spmv.ops
@@ -563,7 +564,7 @@ class DecodeEngine:
                 self._matvec_add(L["down"], ops.decode_silu_mul(gu[:I], gu[I:]), x)
         head = self.lm_head
         if (type(head) is torch.Tensor and head.dtype == torch.float16 and head.is_contiguous() and H % 8 == 0 and H <= 4096
-                and head.shape[1] == H and head.data_ptr() % 16 == self.final_norm.data_ptr() % 16 == 0):
+                and head.shape[1] == H):
             return ops.decode_norm_matvec(head, x, self.final_norm, self.eps)  # norm and product in one launch
         return torch.mv(head, ops.decode_rmsnorm(x, self.final_norm, self.eps))
 

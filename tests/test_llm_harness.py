@@ -358,3 +358,25 @@ def test_norm_and_dense_product_in_one_launch(rows, cols):
         ops.decode_norm_matvec(W, x[1:], w, 1e-5)
     with pytest.raises(RuntimeError):
         ops.decode_norm_matvec(torch.zeros(2, 4104, device="cuda").half(), torch.zeros(4104, device="cuda").half(), torch.zeros(4104, device="cuda").half(), 1e-5)
+
+
+@pytest.mark.gpu
+def test_decode_step_as_one_graph_and_with_a_head_that_starts_anywhere():
+    model, _ = llm.build_model(0.5, 2, 128, 256, 2, 500, 32, seed=3)
+    engine = llm.DecodeEngine(model.requires_grad_(False))
+    token, position = torch.tensor([7], device="cuda"), torch.tensor([0], device="cuda")
+    want = engine.step(token, position)
+    torch._dynamo.reset()
+    compiled = torch.compile(engine.step, fullgraph=True, backend="eager")
+    assert torch.equal(compiled(token, position), want)
+
+    def moved(t, by):
+        flat = torch.empty(t.numel() + by, dtype=t.dtype, device="cuda")
+        flat[by:] = t.reshape(-1)
+        return flat[by:].view(t.shape)
+
+    head, norm = engine.lm_head, engine.final_norm
+    for engine.lm_head, engine.final_norm in ((moved(head, 1), norm), (head, moved(norm, 3)), (moved(head, 4), moved(norm, 4))):
+        for step in (engine.step, torch.compile(engine.step, fullgraph=True, backend="eager")):
+            # the same sums in another order: fp16 results of about 1
+            assert torch.allclose(step(token, position).float(), want.float(), rtol=2.0 ** -9, atol=2.0 ** -9)

@@ -80,6 +80,25 @@ def test_one_graph_takes_prompts_of_any_length():
     assert len(graphs) == 1
 
 
+@pytest.mark.parametrize("fuse", [True, False])
+def test_decode_step_compiles_as_one_graph(fuse, monkeypatch):
+    def stacked(parts):   # of tensors that hold nothing: the sizes
+        return (torch.cat([p[0] for p in parts]), torch.cat([p[1] for p in parts]),
+                torch.empty(sum(p[3] for p in parts) + 1, dtype=torch.int32, device="cuda"), sum(p[3] for p in parts), parts[0][4])
+
+    monkeypatch.setattr(llm, "concat_compressed", stacked)
+    mode = FakeTensorMode(allow_non_fake_inputs=True)
+    model = _fake_model(mode)
+    with mode, torch.no_grad(), torch.device("cuda"):
+        engine = llm.DecodeEngine(model, fuse=fuse)
+        found = _operators(engine.step, torch.empty((1,), dtype=torch.long), torch.empty((1,), dtype=torch.long))
+    per_layer = ["multiply_rmsnorm", "decode_rope_attention_parts", "multiply_attention_axpby", "multiply_rmsnorm", "multiply_silu_mul_axpby"]
+    if not fuse:
+        per_layer = ["decode_rmsnorm", "multiply", "decode_rope_append", "decode_attention", "multiply_axpby",
+                     "decode_rmsnorm", "multiply", "decode_silu_mul", "multiply_axpby"]
+    assert found == 2 * per_layer + ["decode_norm_matvec"]
+
+
 def _dense_model():
     torch.manual_seed(0)
     model = llm.LlamaDecoder(100, 64, 128, 2, 2, 32).requires_grad_(False)
