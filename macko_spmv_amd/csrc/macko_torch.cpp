@@ -13,6 +13,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -184,7 +185,10 @@ void multiply_axpby_hip(const at::Tensor &M_values, const at::Tensor &M_deltas, 
     check_rc(rc, "multiply_axpby");
 }
 
-std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t> compress_on_device(const at::Tensor &M, at::Tensor *plan = nullptr)
+// plan: where the product's cuts go if they are wanted (fp16).  go_on: asked while the count pass runs; if it says no, that
+// pass is all that is done, and undefined tensors are returned.
+std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t> compress_on_device(const at::Tensor &M, at::Tensor *plan = nullptr,
+                                                                                    bool (*go_on)() noexcept = nullptr)
 {
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(M.device());
     const int64_t rows = M.size(0), cols = M.size(1);
@@ -216,6 +220,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t> compress_on_dev
                  M.data_ptr(), (int32_t)rows, (int32_t)cols, row_ptr.data_ptr<int>(), total_word->data_ptr<int>(),
                  (void *)stream),
              "compress (count)");
+    const bool whole = go_on == nullptr || go_on();
     const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
     while (__atomic_load_n(total, __ATOMIC_ACQUIRE) < 0 && std::chrono::steady_clock::now() < give_up) {
     }
@@ -225,10 +230,11 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t> compress_on_dev
     }
     const int64_t n = __atomic_load_n(total, __ATOMIC_ACQUIRE);
     TORCH_CHECK(n >= 0, "macko_spmv: compress: the count pass did not deliver the entry count");
+    if (!whole) return {};
     const int64_t padded = (n + 7) / 8 * 8;
     at::Tensor values = at::empty({padded}, M.options());
     at::Tensor deltas = at::empty({padded / 2}, M.options().dtype(at::kByte));
-    if (plan != nullptr) {  // the product's cuts with it (fp16)
+    if (plan != nullptr) {
         int32_t entries = 0;
         check_rc(macko_spmv_plan_entries((int32_t)rows, (int32_t)cols, padded, &entries), "compress (plan)");
         *plan = at::empty({entries}, row_ptr.options());
@@ -741,9 +747,9 @@ at::Tensor prefill_attention_hip(const at::Tensor &q, const at::Tensor &k_cache,
 // the operator's schema onto a stack of values, the dispatcher, the stack again) takes longer than the rest of the call:
 // 777 x 3333 at density 0.25, 5.8 us a call of `multiply`, of which the launch is 2.2 and the kernel, meanwhile, 4.0.  The
 // functions below take the arguments from Python themselves, for calls that nothing but the CUDA kernel would see: plain
-// tensors on one GPU, through which no gradient has to flow, and no mode, transform, recording or profiler that is
-// between Python and the kernel.  Anything else is answered with NotImplemented, and the caller goes through the
-// operator.
+// tensors on one GPU, through which no gradient has to flow, and no mode, transform, recording, profiler or kernel of the
+// program's own that is between Python and the kernel.  Anything else is answered with NotImplemented, and the caller goes
+// through the operator.
 
 // Nothing in this thread looks at operators: modes of Python, torch.func, tracing and whatever else adds dispatch keys
 // of its own, autocasting (a program may have registered a rule); __torch_function__ modes; the profiler.
@@ -762,6 +768,52 @@ bool plain(const at::Tensor &t)
     return t.defined() && t.is_cuda() && (t.key_set() | usual) == usual && !(t.requires_grad() && at::GradMode::is_enabled()) &&
            !t._fw_grad(0).defined();
 }
+
+// An operator and its kernel for the GPU.
+template <typename F> class Operator;
+template <typename R, typename... A> class Operator<R(A...)> {
+    c10::OperatorHandle handle_;
+    c10::TypedOperatorHandle<R(A...)> typed_;
+    std::string registered_;
+
+    std::string kernel_in_place() const { return handle_.getComputedKernelForDispatchKey(c10::DispatchKey::CUDA).debug(); }
+
+public:
+    explicit Operator(const char *name)
+        : handle_(c10::Dispatcher::singleton().findSchemaOrThrow(name, "")), typed_(handle_.typed<R(A...)>()), registered_(kernel_in_place())
+    {
+    }
+    // A program may have registered a kernel for what comes in front of the GPU's.
+    bool first() const
+    {
+        for (const c10::DispatchKey key : {c10::DispatchKey::Autograd, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::ADInplaceOrView,
+                                           c10::DispatchKey::BackendSelect})
+            if (handle_.hasKernelForDispatchKey(key)) return false;
+        return true;
+    }
+    // ... or one in its place (asked only where the kernel is not called as the operator's)
+    bool replaced() const { return kernel_in_place() != registered_; }
+    R operator()(A... args) const { return typed_.redispatch(c10::DispatchKeySet(c10::DispatchKey::CUDA), std::forward<A>(args)...); }
+};
+
+#define MACKO_OPERATORS(X) \
+    X(multiply) X(multiply_planned) X(multiply_axpby) X(multiply_axpby_planned) X(compress) X(plan)            \
+    X(multiply_batched) X(multiply_int8) X(multiply_int8_axpby) X(multiply_rmsnorm) X(multiply_silu_mul_axpby) \
+    X(multiply_attention_axpby) X(decode_rmsnorm) X(decode_norm_matvec) X(decode_rope_append)                  \
+    X(decode_attention) X(decode_silu_mul) X(decode_rope_attention) X(decode_rope_attention_parts)             \
+    X(pack_rmsnorm) X(rmsnorm_rows) X(pack_silu_mul) X(multiply_packed) X(multiply_packed_several)             \
+    X(prefill_rope_append) X(prefill_attention)                                                               
+#define MACKO_OPERATOR(NAME)                                                                  \
+    struct NAME##_operator {                                                                   \
+        typedef Operator<std::remove_pointer_t<decltype(&NAME##_hip)>> Type;                   \
+        static const Type &get()                                                               \
+        {                                                                                      \
+            static const Type op("macko_spmv::" #NAME);                                        \
+            return op;                                                                         \
+        }                                                                                      \
+    };
+MACKO_OPERATORS(MACKO_OPERATOR)
+#undef MACKO_OPERATOR
 
 struct EagerCall {
     int device = -1;
@@ -868,36 +920,40 @@ struct WithoutGil {  // as around an operator's call: a launch may wait for room
     ~WithoutGil() { PyEval_RestoreThread(state); }
 };
 
-template <auto FUNCTION, typename R, typename... A, size_t... I>
-PyObject *eager_call(R (*)(A...), std::index_sequence<I...>, PyObject *const *args, Py_ssize_t n)
+template <typename R, typename... A, size_t... I>
+PyObject *eager_call(const Operator<R(A...)> &op, std::index_sequence<I...>, PyObject *const *args, Py_ssize_t n)
 {
-    if (n != (Py_ssize_t)sizeof...(A) || !unobserved()) return not_implemented();
+    if (n != (Py_ssize_t)sizeof...(A) || !unobserved() || !op.first()) return not_implemented();
     EagerCall call;
     std::tuple<EagerArg<A>...> kept;
     if (!(std::get<I>(kept).take(call, args[I]) && ...)) return not_implemented();
     if constexpr (std::is_void_v<R>) {
         {
             WithoutGil released;
-            FUNCTION(std::get<I>(kept).give()...);
+            op(std::get<I>(kept).give()...);
         }
         Py_RETURN_NONE;
     } else {
         std::optional<R> out;
         {
             WithoutGil released;
-            out.emplace(FUNCTION(std::get<I>(kept).give()...));
+            out.emplace(op(std::get<I>(kept).give()...));
         }
         return to_python(std::move(*out));
     }
 }
 
-template <typename R, typename... A> constexpr size_t arity(R (*)(A...)) { return sizeof...(A); }
+template <typename R, typename... A>
+PyObject *eager_call(const Operator<R(A...)> &op, PyObject *const *args, Py_ssize_t n)
+{
+    return eager_call(op, std::index_sequence_for<A...>{}, args, n);
+}
 
 // The operator's own arguments, one by one.
-template <auto FUNCTION> PyObject *eager(PyObject *, PyObject *const *args, Py_ssize_t n)
+template <typename OPERATOR> PyObject *eager(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    return eager_call<FUNCTION>(FUNCTION, std::make_index_sequence<arity(FUNCTION)>{}, args, n);
+    return eager_call(OPERATOR::get(), args, n);
     END_HANDLE_TH_ERRORS
 }
 
@@ -946,11 +1002,14 @@ PyObject *eager_multiply(PyObject *, PyObject *const *args, Py_ssize_t n)
     Compressed m;
     const at::Tensor *v = nullptr;
     if (n != 2 || !unobserved() || !m.take(call, args[0]) || !call.tensor(args[1], v) || !v->is_contiguous()) return not_implemented();
+    const auto &planned = multiply_planned_operator::get();
+    const auto &bare = multiply_operator::get();
+    if (!(m.plan != nullptr ? planned.first() : bare.first())) return not_implemented();
     at::Tensor out;
     {
         WithoutGil released;
-        out = m.plan != nullptr ? multiply_planned_hip(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *m.plan)
-                                : multiply_hip(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v);
+        out = m.plan != nullptr ? planned(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *m.plan)
+                                : bare(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v);
     }
     return to_python(std::move(out));
     END_HANDLE_TH_ERRORS
@@ -966,19 +1025,37 @@ PyObject *eager_multiply_axpby(PyObject *, PyObject *const *args, Py_ssize_t n)
     if (n != 5 || !unobserved() || !m.take(call, args[0]) || !call.tensor(args[1], v) || !call.tensor(args[2], c) ||
         !EagerCall::number(args[3], alpha) || !EagerCall::number(args[4], beta) || !v->is_contiguous() || !c->is_contiguous())
         return not_implemented();
+    const auto &planned = multiply_axpby_planned_operator::get();
+    const auto &bare = multiply_axpby_operator::get();
+    if (!(m.plan != nullptr ? planned.first() : bare.first())) return not_implemented();
     {
         WithoutGil released;
         if (m.plan != nullptr)
-            multiply_axpby_planned_hip(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *c, alpha, beta, *m.plan);
+            planned(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *c, alpha, beta, *m.plan);
         else
-            multiply_axpby_hip(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *c, alpha, beta);
+            bare(*m.values, *m.deltas, *m.row_indices, m.rows, m.cols, *v, *c, alpha, beta);
     }
     Py_INCREF(args[2]);
     return args[2];
     END_HANDLE_TH_ERRORS
 }
 
-// compress(M): the five of the operator and the plan (None: products of this shape take none).
+// Whether compress and plan still have their own kernels.  The dispatcher answers with copies of strings, so it is asked while
+// the count pass is running anyway.
+bool compress_not_replaced() noexcept
+{
+    const PyGILState_STATE state = PyGILState_Ensure();  // kernels are registered with the lock held
+    bool replaced = true;
+    try {
+        replaced = compress_operator::get().replaced() || plan_operator::get().replaced();
+    } catch (...) {
+    }
+    PyGILState_Release(state);
+    return !replaced;
+}
+
+// compress(M): the five of the operator and the plan (None: products of this shape take none), which the operator `plan` makes
+// otherwise.
 PyObject *eager_compress(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
@@ -986,12 +1063,14 @@ PyObject *eager_compress(PyObject *, PyObject *const *args, Py_ssize_t n)
     const at::Tensor *M = nullptr;
     if (n != 1 || !unobserved() || !call.tensor(args[0], M) || M->dtype() != at::kHalf || M->dim() != 2 || !M->is_contiguous())
         return not_implemented();
+    if (!compress_operator::get().first() || !plan_operator::get().first()) return not_implemented();
     at::Tensor plan;
     std::optional<std::tuple<at::Tensor, at::Tensor, at::Tensor, int64_t, int64_t>> out;
     {
         WithoutGil released;
-        out.emplace(compress_on_device(*M, &plan));
+        out.emplace(compress_on_device(*M, &plan, &compress_not_replaced));
     }
+    if (!std::get<0>(*out).defined()) return not_implemented();
     PyObject *found = Py_None;
     if (plan.numel() > 0)
         found = THPVariable_Wrap(std::move(plan));
@@ -1007,26 +1086,26 @@ PyMethodDef eager_functions[] = {
     MACKO_EAGER(compress, eager_compress),
     MACKO_EAGER(multiply, eager_multiply),
     MACKO_EAGER(multiply_axpby, eager_multiply_axpby),
-    MACKO_EAGER(multiply_batched, eager<&multiply_batched_hip>),
-    MACKO_EAGER(multiply_int8, eager<&multiply_int8_hip>),
-    MACKO_EAGER(multiply_int8_axpby, eager<&multiply_int8_axpby_hip>),
-    MACKO_EAGER(multiply_rmsnorm, eager<&multiply_rmsnorm_hip>),
-    MACKO_EAGER(multiply_silu_mul_axpby, eager<&multiply_silu_mul_axpby_hip>),
-    MACKO_EAGER(multiply_attention_axpby, eager<&multiply_attention_axpby_hip>),
-    MACKO_EAGER(decode_rmsnorm, eager<&decode_rmsnorm_hip>),
-    MACKO_EAGER(decode_norm_matvec, eager<&decode_norm_matvec_hip>),
-    MACKO_EAGER(decode_rope_append, eager<&decode_rope_append_hip>),
-    MACKO_EAGER(decode_attention, eager<&decode_attention_hip>),
-    MACKO_EAGER(decode_silu_mul, eager<&decode_silu_mul_hip>),
-    MACKO_EAGER(decode_rope_attention, eager<&decode_rope_attention_hip>),
-    MACKO_EAGER(decode_rope_attention_parts, eager<&decode_rope_attention_parts_hip>),
-    MACKO_EAGER(pack_rmsnorm, eager<&pack_rmsnorm_hip>),
-    MACKO_EAGER(rmsnorm_rows, eager<&rmsnorm_rows_hip>),
-    MACKO_EAGER(pack_silu_mul, eager<&pack_silu_mul_hip>),
-    MACKO_EAGER(multiply_packed, eager<&multiply_packed_hip>),
-    MACKO_EAGER(multiply_packed_several, eager<&multiply_packed_several_hip>),
-    MACKO_EAGER(prefill_rope_append, eager<&prefill_rope_append_hip>),
-    MACKO_EAGER(prefill_attention, eager<&prefill_attention_hip>),
+    MACKO_EAGER(multiply_batched, eager<multiply_batched_operator>),
+    MACKO_EAGER(multiply_int8, eager<multiply_int8_operator>),
+    MACKO_EAGER(multiply_int8_axpby, eager<multiply_int8_axpby_operator>),
+    MACKO_EAGER(multiply_rmsnorm, eager<multiply_rmsnorm_operator>),
+    MACKO_EAGER(multiply_silu_mul_axpby, eager<multiply_silu_mul_axpby_operator>),
+    MACKO_EAGER(multiply_attention_axpby, eager<multiply_attention_axpby_operator>),
+    MACKO_EAGER(decode_rmsnorm, eager<decode_rmsnorm_operator>),
+    MACKO_EAGER(decode_norm_matvec, eager<decode_norm_matvec_operator>),
+    MACKO_EAGER(decode_rope_append, eager<decode_rope_append_operator>),
+    MACKO_EAGER(decode_attention, eager<decode_attention_operator>),
+    MACKO_EAGER(decode_silu_mul, eager<decode_silu_mul_operator>),
+    MACKO_EAGER(decode_rope_attention, eager<decode_rope_attention_operator>),
+    MACKO_EAGER(decode_rope_attention_parts, eager<decode_rope_attention_parts_operator>),
+    MACKO_EAGER(pack_rmsnorm, eager<pack_rmsnorm_operator>),
+    MACKO_EAGER(rmsnorm_rows, eager<rmsnorm_rows_operator>),
+    MACKO_EAGER(pack_silu_mul, eager<pack_silu_mul_operator>),
+    MACKO_EAGER(multiply_packed, eager<multiply_packed_operator>),
+    MACKO_EAGER(multiply_packed_several, eager<multiply_packed_several_operator>),
+    MACKO_EAGER(prefill_rope_append, eager<prefill_rope_append_operator>),
+    MACKO_EAGER(prefill_attention, eager<prefill_attention_operator>),
     {nullptr, nullptr, 0, nullptr}};
 #undef MACKO_EAGER
 PyModuleDef eager_module = {PyModuleDef_HEAD_INIT, "libmacko_torch", nullptr, -1, eager_functions, nullptr, nullptr, nullptr, nullptr};
@@ -1035,8 +1114,13 @@ PyModuleDef eager_module = {PyModuleDef_HEAD_INIT, "libmacko_torch", nullptr, -1
 
 PyMODINIT_FUNC PyInit_libmacko_torch()
 {
+    HANDLE_TH_ERRORS
+#define MACKO_OPERATOR(NAME) NAME##_operator::get();
+    MACKO_OPERATORS(MACKO_OPERATOR)   // with the kernels that are registered now
+#undef MACKO_OPERATOR
     plan_attribute = PyUnicode_InternFromString("_macko_spmv_plan");
     return plan_attribute == nullptr ? nullptr : PyModule_Create(&eager_module);
+    END_HANDLE_TH_ERRORS
 }
 
 TORCH_LIBRARY(macko_spmv, m)

@@ -146,3 +146,44 @@ def test_cuts_made_beside_the_rows_are_those_of_the_operator(rows, cols, density
         mk.compress(m.t()) if rows > 1 else mk.compress(m[:, ::2])
     with pytest.raises(RuntimeError):
         mk.compress(m.float())
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:.*overrid")
+@pytest.mark.parametrize("key", ["Autograd", "AutogradCUDA", "ADInplaceOrView", "BackendSelect", "CUDA"])
+def test_kernels_that_a_program_registers_see_the_calls(case, key):
+    c, x, w = case
+    X, y = torch.stack([x, -x]), torch.ones(333, device="cuda").half()
+    seen = []
+
+    def kernel(name, result):
+        def f(*args):
+            seen.append(name)
+            return result
+        return f
+
+    made = torch.ops.macko_spmv.compress(w)
+    cuts = torch.ops.macko_spmv.plan(made[2], 333, 200, made[0].numel())
+    bare = tuple(t.clone() if isinstance(t, torch.Tensor) else t for t in c)
+    calls = {"multiply_planned": (x, lambda: mk.multiply(c, x)), "multiply": (x, lambda: mk.multiply(bare, x)),
+             "multiply_batched": (X, lambda: mk.multiply_batched(c, X)),
+             "multiply_axpby_planned": (None, lambda: mk.multiply_axpby(c, x, y, 2.0, 0.25)), "multiply_axpby": (None, lambda: mk.multiply_axpby(bare, x, y, 2.0, 0.25)),
+             "compress": (made, lambda: mk.compress(w)), "plan": (cuts, lambda: mk.compress(w))}
+    before = y.clone()
+    for name, (result, call) in calls.items():
+        library = torch.library.Library("macko_spmv", "IMPL")
+        seen.clear()
+        try:
+            library.impl(name, kernel(name, result), key, allow_override=True)
+            got = call()
+            assert seen == [name], key
+            if name.startswith("multiply_axpby"):
+                assert got is y and torch.equal(y, before)
+            elif name.startswith("multiply"):
+                assert got is result or torch.equal(got, result)
+        finally:
+            library._destroy()
+        call()
+        assert seen == [name]   # taken back
+        y.copy_(before)
+    assert torch.equal(mk.multiply(c, x), mk.multiply(bare, x)) and mk._eager.multiply(c, x) is not NotImplemented
