@@ -36,9 +36,10 @@ def _load_native():
     try:
         hip = ctypes.CDLL(hip_path, mode=ctypes.RTLD_GLOBAL)
         torch.ops.load_library(torch_path)
-        # the same library as a module: the operators' functions for eager calls
+        # the operators' functions for eager calls, a Python module
+        eager_path = _build.eager_lib_path()
         spec = importlib.util.spec_from_file_location(
-            "libmacko_torch", torch_path, loader=importlib.machinery.ExtensionFileLoader("libmacko_torch", torch_path))
+            "libmacko_eager", eager_path, loader=importlib.machinery.ExtensionFileLoader("libmacko_eager", eager_path))
         eager = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(eager)
     except (OSError, ImportError) as exc:  # no silent fallback: the HIP path is the only path
@@ -53,8 +54,8 @@ _hip_lib, HIP_LIBRARY_PATH, TORCH_LIBRARY_PATH, _eager = _load_native()
 
 
 def _operator(name):
-    """An operator as a function: for plain tensors that nothing else looks at, straight to its kernel (csrc/macko_torch.cpp,
-    "eager calls": 2 us of a call's 6 less), else torch.ops.macko_spmv.<name>."""
+    """An operator as a function: for plain tensors that nothing else looks at, straight to its kernel (csrc/macko_eager.cpp:
+    2 us of a call's 6 less), else torch.ops.macko_spmv.<name>."""
     eager, general = getattr(_eager, name), getattr(torch.ops.macko_spmv, name).default
 
     def call(*args):

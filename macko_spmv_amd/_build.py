@@ -1,10 +1,11 @@
-"""Build recipes for the two native libraries of this package.
+"""Build recipes for the native libraries of this package.
 
   libmacko_hip.so    torch-free HIP kernels behind the C ABI of include/macko_hip.h (gfx950)
   libmacko_torch.so  PyTorch-ROCm operator library that forwards to the C ABI
+  libmacko_eager.so  Python module of the same operators for eager calls, past the dispatcher's stack
   libmacko_bench.so  the benchmark's own kernels (streaming-read yardstick, counter calibration)
 
-Both are built in-tree (next to this file) unless MACKO_SPMV_BUILD_DIRECTORY names another
+All are built in-tree (next to this file) unless MACKO_SPMV_BUILD_DIRECTORY names another
 directory -- the same variable the upstream package reads for its JIT cache
 (src/macko_spmv/__init__.py:12).  hipcc cross-compiles for gfx950 without a GPU present.
 
@@ -25,12 +26,14 @@ _INCLUDE = os.path.join(_ROOT, "include")
 
 HIP_LIB = "libmacko_hip.so"
 TORCH_LIB = "libmacko_torch.so"
+EAGER_LIB = "libmacko_eager.so"
 BENCH_LIB = "libmacko_bench.so"  # kernels of bench.py only; the package never loads it
 ARCH = "gfx950"
 
 HIP_SOURCES = ["macko_spmv.hip", "macko_spmv_split.hip", "macko_spmv_tile.hip", "macko_compress.hip", "macko_runtime.hip", "macko_decode.hip",
                "macko_prefill.hip"]
 TORCH_SOURCES = ["macko_torch.cpp"]
+EAGER_SOURCES = ["macko_eager.cpp"]
 BENCH_SOURCES = ["macko_bench_kernels.hip"]
 
 
@@ -45,6 +48,10 @@ def build_directory():
 def lib_paths():
     d = build_directory()
     return os.path.join(d, HIP_LIB), os.path.join(d, TORCH_LIB)
+
+
+def eager_lib_path():
+    return os.path.join(build_directory(), EAGER_LIB)
 
 
 def _hipcc():
@@ -207,7 +214,7 @@ STAMP = "macko_build.stamp"
 
 
 def source_digest():
-    """Hash of everything the two libraries are built from (csrc/, include/, this recipe)."""
+    """Hash of everything the libraries are built from (csrc/, include/, this recipe)."""
     import hashlib
 
     h = hashlib.sha256()
@@ -227,38 +234,47 @@ def stamp_path():
 
 
 def is_current():
-    """True when both libraries exist and were built from the sources as they are now."""
+    """True when the libraries exist and were built from the sources as they are now."""
     hip_lib, torch_lib = lib_paths()
-    if not all(os.path.exists(f) for f in (hip_lib, torch_lib, bench_lib_path(), stamp_path())):
+    if not all(os.path.exists(f) for f in (hip_lib, torch_lib, eager_lib_path(), bench_lib_path(), stamp_path())):
         return False
     with open(stamp_path()) as f:
         return f.read().strip() == source_digest()
 
 
-def build_torch(verbose=False):
+def _build_with_torch(out, sources, include, libraries, verbose):
     import torch
     from torch.utils import cpp_extension as ce
 
-    hip_lib, out = lib_paths()
-    if not os.path.exists(hip_lib):
-        build_hip(verbose)
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
-    cmd = [
+    _run([
         _hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared",
         "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
         "-Wno-unused-command-line-argument",
         f"-I{_INCLUDE}",
-        *[f"-I{p}" for p in ce.include_paths("cuda")], f"-I{sysconfig.get_paths()['include']}",
-        *[os.path.join(_CSRC, s) for s in TORCH_SOURCES],
+        *[f"-I{p}" for p in ce.include_paths("cuda")], *[f"-I{p}" for p in include],
+        *[os.path.join(_CSRC, s) for s in sources],
         "-x", "none",
         *[f"-L{p}" for p in ce.library_paths("cuda") if os.path.isdir(p)],
-        f"-L{os.path.dirname(hip_lib)}",
-        "-lmacko_hip", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-lamdhip64",
+        f"-L{os.path.dirname(out)}", *libraries,
         "-Wl,-rpath,$ORIGIN",
         "-o", out,
-    ]
-    _run(cmd, verbose)
+    ], verbose)
     return out
+
+
+def build_torch(verbose=False):
+    hip_lib, out = lib_paths()
+    if not os.path.exists(hip_lib):
+        build_hip(verbose)
+    # nothing of Python: a C++ program loads it as it loads any library of operators
+    return _build_with_torch(out, TORCH_SOURCES, [],
+                             ["-lmacko_hip", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-lamdhip64"], verbose)
+
+
+def build_eager(verbose=False):
+    return _build_with_torch(eager_lib_path(), EAGER_SOURCES, [sysconfig.get_paths()["include"]],
+                             ["-lmacko_torch", "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"], verbose)
 
 
 def bench_lib_path():
@@ -291,6 +307,7 @@ def build_all(verbose=False):
     if os.path.exists(stamp_path()):
         os.remove(stamp_path())
     built = build_hip(verbose), build_torch(verbose)
+    build_eager(verbose)
     build_bench(verbose)
     with open(stamp_path(), "w") as f:
         f.write(source_digest() + "\n")

@@ -191,7 +191,7 @@ def test_build_directory_variable_redirects_every_artefact(tmp_path, monkeypatch
     in_tree = os.path.dirname(_build.lib_paths()[0])
     target = tmp_path / "elsewhere"
     monkeypatch.setenv("MACKO_SPMV_BUILD_DIRECTORY", str(target))
-    paths = [*_build.lib_paths(), _build.bench_lib_path(), _build.stamp_path()]
+    paths = [*_build.lib_paths(), _build.eager_lib_path(), _build.bench_lib_path(), _build.stamp_path()]
     assert target.is_dir()
     assert all(os.path.dirname(p) == str(target) for p in paths)
     assert not _build.is_current()
@@ -212,3 +212,35 @@ def test_kernel_resource_check_refuses_scratch_and_stacks():
     for bad in (remarks(scratch=16), remarks(spilled=3), remarks(stack="True"), ""):
         with pytest.raises(RuntimeError):
             _build.check_kernel_resources(bad)
+
+
+def test_operator_library_loads_without_python(tmp_path):
+    """A program without Python has the operators by loading libmacko_torch.so; what needs Python is libmacko_eager.so."""
+    import subprocess
+
+    import torch
+
+    source, program = tmp_path / "load.c", str(tmp_path / "load")
+    source.write_text(r"""
+        #include <dlfcn.h>
+        #include <stdio.h>
+        #include <string.h>
+        #include <unistd.h>
+        int main(int n, char **v)
+        {
+            char line[4096];
+            if (!dlopen(v[1], RTLD_NOW | RTLD_GLOBAL)) { puts(dlerror()); return 1; }
+            FILE *maps = fopen("/proc/self/maps", "r");
+            while (fgets(line, sizeof line, maps))
+                if (strstr(line, "libpython") || strstr(line, "libtorch_python")) { puts(line); return 2; }
+            puts("loaded");
+            fflush(stdout);
+            _exit(0);
+        }""")
+    subprocess.run(["gcc", str(source), "-o", program, "-ldl"], check=True)
+    from macko_spmv_amd import _build
+
+    assert os.path.basename(macko_spmv_amd.TORCH_LIBRARY_PATH) == _build.TORCH_LIB
+    env = dict(os.environ, LD_LIBRARY_PATH=os.path.join(os.path.dirname(torch.__file__), "lib"))
+    out = subprocess.run([program, macko_spmv_amd.TORCH_LIBRARY_PATH], env=env, stdout=subprocess.PIPE, text=True)
+    assert out.returncode == 0 and out.stdout.strip() == "loaded", out.stdout
