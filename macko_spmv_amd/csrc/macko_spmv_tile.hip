@@ -55,21 +55,33 @@ constexpr int kTileFront = 16;   // the same in front of the first row
 constexpr long long kPackFrom = 100000;
 constexpr long long kPackUnalignedFrom = 12000;
 
-// One of the matrices of a launch.  Several with the same columns and vectors stand below each other; their rows
-// are numbered on, and where there is more than one, every one but the last ends on a whole unit of four rows.
+// One of the matrices of a launch.
 struct TileSource {
+    uint16_t *y;
+    u32 ldy;
+    u32 padded;
     const u32 *values;
     const u32 *deltas;
     const int *row_ptr;
-    uint16_t *y;
-    int first;   // its first row; behind the last matrix: no row
-    u32 padded;
-    u32 ldy;
 };
 constexpr int kMaxSources = MACKO_PACKED_MATRICES;
 
-// What a launch of one matrix and one of several have in common, and the launch's arguments: with one matrix a wave
-// fetches no more of them than it needs (4096 x 4096, 8 vectors: 0.15 us a launch).
+// Several with the same columns and vectors stand below each other; their rows are numbered on, and every one but the
+// last ends on a whole unit of four rows.  first: a matrix's first row; behind the last matrix: no row.
+template <int SOURCES>
+struct TileSources {
+    TileSource source[SOURCES];
+    int first[SOURCES];
+};
+template <>
+struct TileSources<1> {
+    TileSource source[1];
+};
+
+// What a launch of one matrix and one of several have in common.  A launch's arguments are its matrices, then these; with
+// one matrix a wave fetches no more of them than it needs (4096 x 4096, 8 vectors: 0.15 us a launch).  They end, and the grid's
+// size behind them stands, within 128 bytes, and what the loop needs is fetched at once, in front of row_ptr: 8.53 us,
+// 8.57 with a third line of 64 bytes to wait for and x fetched behind row_ptr.
 struct TileCommon {
     const uint16_t *x;
     int rows, cols, batch;   // rows of all matrices
@@ -86,9 +98,9 @@ struct TileCommon {
     const uint16_t *residual;  // added to Y before it is rounded (laid out like Y, may be Y), or null
 };
 template <int SOURCES>
-struct TileArgs : TileCommon {
-    TileSource source[SOURCES];
+struct TileArgs : TileSources<SOURCES>, TileCommon {
 };
+static_assert(sizeof(TileArgs<1>) == 120, "one matrix: two lines of 64 bytes with the grid's size");
 
 __device__ __forceinline__ void lds_barrier()
 {
@@ -133,14 +145,21 @@ __device__ __forceinline__ float exact_row_times_vector(const u32 *values, const
     return wave_sum(acc);
 }
 
-// The matrix a row of the launch belongs to.
+// The matrix a row of the launch belongs to, and its row_ptr from that row on.
 template <bool SEVERAL, int SOURCES>
 __device__ __forceinline__ int source_of(const TileArgs<SOURCES> &a, int row)
 {
     int m = 0;
     if constexpr (SEVERAL)
-        for (int k = 1; k < SOURCES; ++k) m += row >= a.source[k].first ? 1 : 0;
+        for (int k = 1; k < SOURCES; ++k) m += row >= a.first[k] ? 1 : 0;
     return m;
+}
+
+template <int SOURCES>
+__device__ __forceinline__ const int *row_ptr_at(const TileArgs<SOURCES> &a, int matrix, int row)
+{
+    if constexpr (SOURCES > 1) row -= a.first[matrix];
+    return a.source[matrix].row_ptr + row;
 }
 
 // The end of a launch: the partial sums of every tile of 16 rows and 16 vectors lie in LDS at `red`
@@ -168,8 +187,9 @@ __device__ __forceinline__ void finish_tiles(const TileArgs<SOURCES> &a, u32 red
                 bad &= bad - 1;
                 const int bad_row = __builtin_amdgcn_readlane(row, L) + i;
                 const int bad_n = __builtin_amdgcn_readlane(n, L);
-                const TileSource &m = a.source[source_of<SEVERAL>(a, bad_row)];
-                const int *row_ptr = m.row_ptr + (SEVERAL ? bad_row - m.first : bad_row);
+                const int matrix = source_of<SEVERAL>(a, bad_row);
+                const TileSource &m = a.source[matrix];
+                const int *row_ptr = row_ptr_at(a, matrix, bad_row);
                 u32 e0 = (u32)uniform(row_ptr[0]), e1 = (u32)uniform(row_ptr[1]);
                 e0 = e0 < m.padded ? e0 : m.padded;
                 e1 = e1 < m.padded ? e1 : m.padded;
@@ -192,10 +212,10 @@ __device__ __forceinline__ void finish_tiles(const TileArgs<SOURCES> &a, u32 red
             if constexpr (SEVERAL) {  // my four rows are of one matrix
 #pragma unroll
                 for (int k = 1; k < kMaxSources; ++k)
-                    if (row >= a.source[k].first) {
+                    if (row >= a.first[k]) {
                         y = a.source[k].y;
                         ldy = a.source[k].ldy;
-                        at = row - a.source[k].first;
+                        at = row - a.first[k];
                     }
             }
             uint16_t *dst = y + (size_t)n * ldy + at;
@@ -295,11 +315,12 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs<
     static_for<RT>([&](auto slot) {
         constexpr int J = decltype(slot)::value;
         const int row = row0 + wave + 16 * J;
-        const TileSource &m = a.source[source_of<SEVERAL>(a, row)];
+        const int matrix = source_of<SEVERAL>(a, row);
+        const TileSource &m = a.source[matrix];
         if constexpr (SEVERAL) describe(J, m);
         u32 e0 = 0, e1 = 0;
         if (row < row1) {
-            const int *row_ptr = m.row_ptr + (SEVERAL ? row - m.first : row);
+            const int *row_ptr = row_ptr_at(a, matrix, row);
             e0 = (u32)uniform(row_ptr[0]);
             e1 = (u32)uniform(row_ptr[1]);
             e0 = e0 < m.padded ? e0 : m.padded;
@@ -564,7 +585,8 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
     if (wave < kPipeProducers) {
         const int l = lane & (L - 1), h = lane / L;   // lane of a row, row of the unit
         const int unit_row = row0 + wave * kRowUnit, row = unit_row + h;
-        const TileSource &m = a.source[source_of<SEVERAL>(a, unit_row)];
+        const int matrix = source_of<SEVERAL>(a, unit_row);
+        const TileSource &m = a.source[matrix];
         const __amdgpu_buffer_rsrc_t rs_values = __builtin_amdgcn_make_buffer_rsrc((void *)m.values, 0, (int)(m.padded * 2), 0x00020000);
         const __amdgpu_buffer_rsrc_t rs_deltas = __builtin_amdgcn_make_buffer_rsrc((void *)m.deltas, 0, (int)(m.padded / 2), 0x00020000);
         u32x4 tile_v[2][W];
@@ -577,7 +599,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
         {
             u32 e0 = 0, e1 = 0;
             if (row < row1) {
-                const int *row_ptr = m.row_ptr + (SEVERAL ? row - m.first : row);
+                const int *row_ptr = row_ptr_at(a, matrix, row);
                 e0 = (u32)row_ptr[0];
                 e1 = (u32)row_ptr[1];
             }
@@ -768,7 +790,10 @@ int launch_with(const TileArgs<kMaxSources> &all, unsigned grid, size_t lds_byte
 {
     TileArgs<SEVERAL ? kMaxSources : 1> a;
     static_cast<TileCommon &>(a) = all;
-    for (int k = 0; k < (SEVERAL ? kMaxSources : 1); ++k) a.source[k] = all.source[k];
+    if constexpr (SEVERAL)
+        static_cast<TileSources<kMaxSources> &>(a) = all;
+    else
+        a.source[0] = all.source[0];
     if (lds_bytes > 64 * 1024) {
         // one-time opt-in to more than 64 KiB of dynamic LDS, per device and kernel
         static std::atomic<bool> done[64];
@@ -795,7 +820,7 @@ int launch_tile(const TileArgs<kMaxSources> &a, unsigned grid, size_t lds_bytes,
 TileArgs<kMaxSources> no_matrices()
 {
     TileArgs<kMaxSources> a{};
-    for (TileSource &m : a.source) m.first = 0x7fffffff;
+    for (int &row : a.first) row = 0x7fffffff;
     return a;
 }
 
@@ -831,10 +856,10 @@ int launch_tile_shape(TileArgs<kMaxSources> a, const TileShape &s, int max_lds, 
     a.group_shift = s.group_shift;
     const int vectors = 16 * s.wave_tiles * groups;
     a.vector_blocks = (a.batch + vectors - 1) / vectors;
-    const bool several = a.source[1].first < a.rows;
+    const bool several = a.first[1] < a.rows;
     a.vector_store = 1;
-    for (const TileSource &m : a.source)
-        if (m.first < a.rows && (m.ldy % 4 != 0 || (reinterpret_cast<uintptr_t>(m.y) & 7) != 0)) a.vector_store = 0;
+    for (int k = 0; k < kMaxSources; ++k)
+        if (a.first[k] < a.rows && (a.source[k].ldy % 4 != 0 || (reinterpret_cast<uintptr_t>(a.source[k].y) & 7) != 0)) a.vector_store = 0;
     const long long grid = s.row_blocks * a.vector_blocks;
     if (grid >= (1ll << 31)) return MACKO_E_INVALID_ARGUMENT;
     a.packed_tiles = packed_tiles(a.batch);
@@ -1021,7 +1046,8 @@ size_t spmv_tile_workspace(int cols, int batch, const void *x, long long ldx)
 int spmv_tile_launch(const SpmvArgs &args, int batch, const TileShape &shape, void *workspace, const DeviceInfo &info, hipStream_t stream)
 {
     TileArgs<kMaxSources> a = no_matrices();
-    a.source[0] = TileSource{args.values, args.deltas, args.row_ptr, args.y, 0, (u32)args.padded, (u32)args.ldy};
+    a.source[0] = TileSource{args.y, (u32)args.ldy, (u32)args.padded, args.values, args.deltas, args.row_ptr};
+    a.first[0] = 0;
     a.x = args.x;
     a.rows = args.rows;
     a.cols = args.cols;
@@ -1068,8 +1094,8 @@ int packed_product(const macko_packed_matrix *matrices, int n, const void *packe
             (reinterpret_cast<uintptr_t>(residual) & 1) || (reinterpret_cast<uintptr_t>(m.y) & 1))
             return MACKO_E_INVALID_ARGUMENT;
         if (rows % kRowUnit != 0) return MACKO_E_INVALID_ARGUMENT;  // the matrix in front does not end on a whole unit
-        a.source[used++] = TileSource{(const u32 *)m.values, (const u32 *)m.deltas, m.row_ptr, (uint16_t *)m.y, (int)rows,
-                                      (u32)m.padded_entries, (u32)m.ldy};
+        a.first[used] = (int)rows;
+        a.source[used++] = TileSource{(uint16_t *)m.y, (u32)m.ldy, (u32)m.padded_entries, (const u32 *)m.values, (const u32 *)m.deltas, m.row_ptr};
         rows += m.rows;
         padded += m.padded_entries;
         if (used > 1 && rows >= (1ll << 31) - kRowUnit) return MACKO_E_INVALID_ARGUMENT;
