@@ -171,7 +171,8 @@ MACKO_API int macko_spmv_f16_batched(const void *values, const void *deltas, con
  *   macko_spmv_f16_packed Y[b, :] = M X[b, :] (+ residual[b, :], laid out like Y, NULL: none; may be Y)
  *                         with one rounding to fp16.
  *   macko_spmv_f16_packed_several  the same (without a residual) for up to MACKO_PACKED_MATRICES matrices of
- *                         the same columns in one launch; in front of another matrix, rows % 4 == 0
+ *                         the same columns in one launch, or in one each where their densities are so
+ *                         unequal that it takes less time; in front of another matrix, rows % 4 == 0
  */
 #define MACKO_PACKED_MATRICES 3
 typedef struct macko_packed_matrix {

@@ -959,10 +959,20 @@ bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, in
     return found;
 }
 
-// The shape of a launch of spmv_pipe_kernel and its estimated time in us.  The terms were fitted to 27000 products of
-// packed vectors (1500 to 28000 rows, 256 to 11000 columns, densities 0.05 to 0.9, 17 to 256 vectors; 7 % off in the
-// median, 16 % for one in ten): per launch, per round of workgroups, per chunk (a pass of 16 entries a lane costs
-// more than one of 8), and per column and vector.
+// The estimated time in us of a launch of spmv_pipe_kernel.  The terms were fitted to 27000 products of packed vectors (1500
+// to 28000 rows, 256 to 11000 columns, densities 0.05 to 0.9, 17 to 256 vectors; 7 % off in the median, 16 % for one in
+// ten): per launch, per round of workgroups, per chunk and pass (of 16 entries a lane it costs more than one of 8), and per
+// column and vector.
+double pipe_us(const TileShape &s, int cols, int batch, const DeviceInfo &info, double passes)
+{
+    const int vectors = 16 * kPipeGroups * s.wave_tiles;
+    const long long blocks = (batch + vectors - 1) / vectors;
+    const double full = (double)((s.row_blocks * blocks + info.compute_units - 1) / info.compute_units);
+    const int n_chunks = (cols + s.chunk - 1) / s.chunk;
+    return 0.93 + full * (3.25 + n_chunks * ((s.lane_entries == 8 ? 0.31 : 0.56) * passes + s.chunk / 512.0 * (0.31 + 0.26 * s.wave_tiles)));
+}
+
+// The shape of a launch of spmv_pipe_kernel and its estimated time.
 bool choose_pipe_shape(TileShape *shape, int rows, int cols, long long padded, int batch, const DeviceInfo &info, double *us)
 {
     if (batch <= 16 || rows < 1 || padded < 1) return false;
@@ -994,13 +1004,14 @@ bool choose_pipe_shape(TileShape *shape, int rows, int cols, long long padded, i
         const int n_chunks = (cols + chunk - 1) / chunk;
         s.chunk = ((cols + n_chunks - 1) / n_chunks + kPipeChunkStep - 1) / kPipeChunkStep * kPipeChunkStep;
         if (pipe_lds_bytes(s) > (size_t)info.max_lds_bytes) continue;
-        const double full = (double)((s.row_blocks * blocks + info.compute_units - 1) / info.compute_units);
-        *us = 0.93 + full * (3.25 + n_chunks * ((e == 8 ? 0.31 : 0.56) + s.chunk / 512.0 * (0.31 + 0.26 * s.wave_tiles)));
+        *us = pipe_us(s, cols, batch, info, 1.0);
         *shape = s;
         return true;
     }
     return false;
 }
+
+constexpr double kTileUsPerCycle = 1.06 / 2400.0;
 
 // The kernel and the shape of a launch, and its estimated time in us (without packing; at 2.4 GHz).  Right to about 10 %
 // where it decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1:
@@ -1010,7 +1021,7 @@ bool choose_shape(TileShape *shape, int rows, int cols, long long padded, int ba
 {
     double cycles = 0.0, pipe_us = 0.0;
     if (!choose_tile_shape(shape, rows, cols, padded, batch, packed, info, &cycles)) return false;
-    *us = cycles * (1.06 / 2400.0);
+    *us = cycles * kTileUsPerCycle;
     TileShape pipe;
     if (packed && choose_pipe_shape(&pipe, rows, cols, padded, batch, info, &pipe_us) && pipe_us < 0.97 * *us) {
         *shape = pipe;
@@ -1074,6 +1085,42 @@ int spmv_tile_pack(const uint16_t *x, int cols, int batch, long long ldx, void *
 namespace macko {
 namespace {
 
+// Whether several matrices of one launch are better launched one by one.  A launch has one shape, which suits the mean density, and
+// XCDs have consecutive rows: with a much denser matrix among them, its rows take more passes a chunk and the XCDs that have
+// it work on when the others are done.  What its rows take is what the launch takes; the estimate for that is up to 20 %
+// low with the tile kernel, so launches apart are given 10 %.  4096 columns, us, one launch / one by one: 2 x 11008 rows
+// at densities 0.9 and 0.1, 16 vectors 46.4 / 35.2, 128 51.1 / 46.2; 3 x 4096 at 0.9, 0.1 and 0.1, 16 vectors 24.9 / 22.8, but
+// 128 23.5 / 41.7; at 0.5 each, 16 vectors 17.3 / 25.4, 128 22.9 / 43.5, which is not asked: up to a tenth above the mean a
+// matrix's rows fit the launch's passes.
+bool better_apart(const TileArgs<kMaxSources> &a, int used, const TileShape &shape, const DeviceInfo &info)
+{
+    double entries = 0.0, densest = 0.0;
+    for (int k = 0; k < used; ++k) {
+        const int rows = (k + 1 < used ? a.first[k + 1] : a.rows) - a.first[k];
+        const double density = (double)a.source[k].padded / ((double)rows * (double)a.cols);
+        entries += a.source[k].padded;
+        densest = density > densest ? density : densest;
+    }
+    if (densest * (double)a.rows * (double)a.cols <= 1.1 * entries) return false;
+    double apart = 0.0, together = 0.0;
+    for (int k = 0; k < used; ++k) {
+        const int rows = (k + 1 < used ? a.first[k + 1] : a.rows) - a.first[k];
+        TileShape own;
+        double us = 0.0;
+        if (!choose_shape(&own, rows, a.cols, a.source[k].padded, a.batch, true, info, &us)) return false;
+        apart += us;
+    }
+    if (shape.lane_entries > 0) {
+        const double held = kPipeLanes * shape.lane_entries;
+        together = pipe_us(shape, a.cols, a.batch, info, std::ceil((densest * shape.chunk + shape.lane_entries + 8) / held));
+    } else {
+        const long long units = ((long long)a.rows + kRowUnit - 1) / kRowUnit;
+        const double whole = std::ceil(densest * shape.chunk / 504.0) * 504.0 / shape.chunk;   // passes
+        together = tile_cost(shape, units, a.cols, whole, a.batch, true, info.compute_units) * kTileUsPerCycle;
+    }
+    return together > 0.9 * apart;
+}
+
 int packed_product(const macko_packed_matrix *matrices, int n, const void *packed, const void *residual, int cols, int batch, void *stream)
 {
     if (matrices == nullptr || n < 1 || n > kMaxSources || cols < 64 || batch < 1 || (n > 1 && residual != nullptr)) return MACKO_E_INVALID_ARGUMENT;
@@ -1112,6 +1159,13 @@ int packed_product(const macko_packed_matrix *matrices, int n, const void *packe
     TileShape shape;
     double us = 0.0;
     if (!choose_shape(&shape, a.rows, cols, padded, batch, true, info, &us)) return MACKO_E_INVALID_ARGUMENT;
+    if (used > 1 && better_apart(a, used, shape, info)) {
+        for (int k = 0; k < n; ++k) {
+            const int e = packed_product(matrices + k, 1, packed, nullptr, cols, batch, stream);
+            if (e != 0) return e;
+        }
+        return 0;
+    }
     return launch_tile_shape(a, shape, info.max_lds_bytes, as_stream(stream));
 }
 

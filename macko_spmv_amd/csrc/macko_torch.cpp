@@ -650,7 +650,7 @@ at::Tensor multiply_packed_hip(const at::Tensor &M_values, const at::Tensor &M_d
     return Y;
 }
 
-// The same for several matrices of M_cols columns in one launch -> one [batch, rows] per matrix.  All but the last
+// The same for several matrices of M_cols columns at once -> one [batch, rows] per matrix.  All but the last
 // have a multiple of four rows.
 std::vector<at::Tensor> multiply_packed_several_hip(at::TensorList M_values, at::TensorList M_deltas, at::TensorList M_row_indices,
                                                     at::IntArrayRef M_rows, int64_t M_cols, const at::Tensor &packed, int64_t batch)

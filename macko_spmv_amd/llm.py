@@ -282,8 +282,9 @@ class Block(nn.Module):
             return ops.multiply_packed(linear.c_0, linear.c_1, linear.c_2, linear.c_3, linear.c_4, packed, t, residual)
 
         def products(packed, *linears):
-            # one launch for all of them: what a launch costs besides its rows is 5 us (128 tokens, dim 4096: q, k and v
-            # 47 us one by one, 29 together).  A compiled graph keeps an operator for each projection.
+            # one launch for all of them, unless their densities differ too much for that: what a launch costs besides its
+            # rows is 5 us (128 tokens, dim 4096: q, k and v 47 us one by one, 29 together).  A compiled graph keeps an
+            # operator for each projection.
             if torch.compiler.is_compiling() or any(linear.c_3 % 4 != 0 for linear in linears):
                 return [product(linear, packed) for linear in linears]
             return ops.multiply_packed_several([linear.c_0 for linear in linears], [linear.c_1 for linear in linears],

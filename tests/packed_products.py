@@ -32,6 +32,9 @@ PRODUCTS = [
 # an array that ends as near to 2^31 entries as is taken, and a row there that leaves more columns than that free
 LONG_ARRAY = dict(entries=2 ** 31 - 8200, rows=524288, cols=16384, batch=17, kernel="spmv_pipe_kernel<1,16,false>")
 
+# matrices of so unequal densities that each has a launch of its own: batch, rows of each, cols, their densities
+UNEQUAL = dict(batch=16, rows=(11008, 11006), cols=1300, densities=(0.95, 0.03))
+
 
 def matrices(product):
     """The product's matrices: rows without entries, full rows, rows of one entry behind padding entries and gaps wider than

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import macko_spmv_amd as mk
-from tests import packed_products
+from tests import helpers, packed_products
 
 pytestmark = pytest.mark.gpu
 ops = torch.ops.macko_spmv
@@ -73,6 +73,19 @@ def test_products_of_packed_vectors(product):
                                      rows, product.cols, one[0].numel(), product.batch, ldy, torch.cuda.current_stream().cuda_stream) == 0
     _check(into[:, :rows], x, dense[0], r)
     assert (into[:, rows:] == 7.0).all() and flat[0] == 7.0
+
+
+def test_matrices_of_unequal_densities():
+    batch, rows, cols, densities = (packed_products.UNEQUAL[k] for k in ("batch", "rows", "cols", "densities"))
+    rng = np.random.default_rng(cols)
+    dense = [helpers.random_sparse(rng, r, cols, d, scale=0.05) for r, d in zip(rows, densities)]
+    c = [mk.compress(torch.from_numpy(m).cuda()) for m in dense]
+    x = rng.standard_normal((batch, cols)).astype(np.float16)
+    packed = _pack(ctypes.CDLL(mk.HIP_LIBRARY_PATH), torch.from_numpy(x).cuda())
+    got = ops.multiply_packed_several([m[0] for m in c], [m[1] for m in c], [m[2] for m in c], list(rows), cols, packed, batch)
+    for y, m, one in zip(got, dense, c):
+        _check(y, x, m)
+        assert torch.equal(y, ops.multiply_packed(*one, packed, batch, None))
 
 
 def test_rows_at_the_end_of_the_longest_array():

@@ -23,7 +23,7 @@ def routes(tmp_path_factory):
 
     def ask(cols, batch, matrices, residual=False):
         line = " ".join(str(v) for v in (cols, batch, int(residual), len(matrices), *(v for m in matrices for v in m)))
-        return subprocess.run([program], input=line + "\n", stdout=subprocess.PIPE, text=True, check=True).stdout.split()
+        return subprocess.run([program], input=line + "\n", stdout=subprocess.PIPE, text=True, check=True).stdout.split()  # an answer for each launch
 
     return ask
 
@@ -36,12 +36,31 @@ def test_the_products_take_the_kernels_they_are_meant_for(routes, product):
         assert n == packed_products.stored_entries(m)
         assert k == product.empty or values.size % 16 == 8
         sizes.append((m.shape[0], values.size))
-    assert routes(product.cols, product.batch, sizes)[0] == product.kernel
+    launches = routes(product.cols, product.batch, sizes)
+    assert [name.split(":")[0] for name in launches] == [product.kernel]
     if len(sizes) == 1:
-        assert routes(product.cols, product.batch, sizes, residual=True)[0] == product.kernel
+        assert routes(product.cols, product.batch, sizes, residual=True) == launches
 
 
 def test_the_longest_array_takes_the_kernel_it_is_meant_for(routes):
     long = packed_products.LONG_ARRAY
-    assert routes(long["cols"], long["batch"], [(long["rows"], long["entries"])])[0] == long["kernel"]
+    assert routes(long["cols"], long["batch"], [(long["rows"], long["entries"])])[0].split(":")[0] == long["kernel"]
     assert routes(long["cols"], long["batch"], [(long["rows"], long["entries"] + 8)])[0] == "refused"
+
+
+@pytest.mark.parametrize("rows,densities,batch,launches", [
+    (11008, (0.5, 0.5), 16, 1), (11008, (0.9, 0.1), 16, 2), (11008, (0.1, 0.9), 128, 2), (11008, (0.7, 0.2), 2, 2), (11008, (0.5, 0.48), 128, 1),
+    (4096, (0.5, 0.5, 0.5), 128, 1), (4096, (0.9, 0.1, 0.1), 16, 3), (4096, (0.9, 0.1, 0.1), 128, 1), (4096, (0.1, 0.9, 0.9), 2, 3),
+    (512, (0.9, 0.1, 0.1), 16, 1), (4096, (0.3, 0.0, 0.3), 64, 1), (4096, (0.0, 0.0, 0.0), 64, 1)])
+def test_matrices_of_unequal_densities_share_a_launch_where_it_takes_less_time(routes, rows, densities, batch, launches):
+    sizes = [(rows, int(rows * 4096 * d) // 8 * 8) for d in densities]
+    got = routes(4096, batch, sizes)
+    assert len(got) == launches and got[0] != "refused"
+    if launches > 1:   # each as it is launched on its own
+        assert got == [routes(4096, batch, [size])[0] for size in sizes]
+
+
+def test_the_unequal_matrices_are_launched_apart(routes):
+    unequal = packed_products.UNEQUAL
+    sizes = [(rows, int(rows * unequal["cols"] * max(d, 1 / 16)) // 8 * 8) for rows, d in zip(unequal["rows"], unequal["densities"])]
+    assert len(routes(unequal["cols"], unequal["batch"], sizes)) == 2

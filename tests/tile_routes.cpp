@@ -1,8 +1,8 @@
 // Which kernel a product of packed vectors launches, on the host: the host code of csrc/macko_spmv_tile.hip and, in the place of
 // the HIP runtime, functions that write down what would be launched.
 //
-// Reads lines "cols batch residual n rows_1 entries_1 ... rows_n entries_n", prints "<kernel> <workgroups> <bytes of LDS>" or
-// "refused <code>" for each.
+// Reads lines "cols batch residual n rows_1 entries_1 ... rows_n entries_n", prints "<kernel>:<workgroups>:<bytes of LDS>" of each
+// launch, or "refused <code>".
 #include <cxxabi.h>
 
 #include <cstdio>
@@ -18,7 +18,7 @@ static std::map<const void *, std::string> &kernels()
     static std::map<const void *, std::string> all;
     return all;
 }
-static std::string launched;
+static std::string launched, configuration;
 
 extern "C" {
 void **__hipRegisterFatBinary(const void *) { return nullptr; }
@@ -33,17 +33,16 @@ void __hipRegisterFunction(void **, const void *function, char *, const char *na
 }
 hipError_t __hipPushCallConfiguration(dim3 grid, dim3, size_t lds, hipStream_t)
 {
-    launched = " " + std::to_string(grid.x) + " " + std::to_string(lds);
+    configuration = ":" + std::to_string(grid.x) + ":" + std::to_string(lds);
     return hipSuccess;
 }
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
 hipError_t hipLaunchKernel(const void *function, dim3, dim3, void **, size_t, hipStream_t)
 {
-    std::string name = kernels()[function];
-    std::string packed;
-    for (char c : name)
-        if (c != ' ') packed += c;
-    launched = packed + launched;
+    if (!launched.empty()) launched += " ";
+    for (char c : kernels()[function])
+        if (c != ' ') launched += c;
+    launched += configuration;
     return hipSuccess;
 }
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
