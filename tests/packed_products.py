@@ -27,6 +27,18 @@ PRODUCTS = [
     # ... and arrays that end in the middle of a lane's entries
     Product(17, (9001,), 257, 0.3, "spmv_pipe_kernel<1,16,false>"),
     Product(129, (6143,), 257, 0.45, "spmv_pipe_kernel<4,16,false>"),
+    # columns in several chunks: every width of vectors and of lanes, one and several matrices, the last one of any rows
+    Product(17, (9003,), 1300, 0.1, "spmv_pipe_kernel<1,8,false>"),
+    Product(32, (6140, 512, 2049), 1411, 0.12, "spmv_pipe_kernel<1,8,true>"),
+    Product(31, (4096, 4096, 1025), 1300, 0.3, "spmv_pipe_kernel<1,16,true>"),
+    Product(33, (12291,), 1281, 0.08, "spmv_pipe_kernel<2,8,false>"),
+    Product(64, (8000, 2048, 2050), 1300, 0.1, "spmv_pipe_kernel<2,8,true>"),
+    Product(63, (12285,), 1301, 0.4, "spmv_pipe_kernel<2,16,false>"),
+    Product(40, (4096, 4096, 4095), 1300, 0.35, "spmv_pipe_kernel<2,16,true>"),
+    Product(65, (12289,), 1281, 0.1, "spmv_pipe_kernel<4,8,false>"),
+    Product(127, (4096, 4100, 4099), 1300, 0.08, "spmv_pipe_kernel<4,8,true>"),
+    Product(128, (12287,), 1337, 0.5, "spmv_pipe_kernel<4,16,false>"),
+    Product(128, (4096, 4096, 4094), 1300, 0.45, "spmv_pipe_kernel<4,16,true>"),
 ]
 
 # an array that ends as near to 2^31 entries as is taken, and a row there that leaves more columns than that free
