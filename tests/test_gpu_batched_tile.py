@@ -51,8 +51,9 @@ def test_edges_of_tiles_and_chunks(rows, cols, density, batch):
     assert torch.equal(Y, macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda()))
 
 
-# many rows and more than 16 vectors: the kernel whose waves scatter or multiply (48 rows, units of 4; lanes of 8 or 16
-# entries, 16 lanes a row; chunks of a multiple of 128 columns; 32, 64 or 128 vectors)
+# many rows and more than 16 vectors through the entry point, which packs X from 100000 elements on (12000 where a row is not
+# 16-byte aligned) and has the kernel whose waves scatter or multiply for 65 and more of them here; every shape of that
+# kernel: test_gpu_packed_products.py
 @pytest.mark.parametrize("rows,cols,density,batch", [
     (12288, 300, 0.05, 17), (12285, 512, 0.1, 32), (12289, 513, 0.3, 33), (24575, 128, 0.5, 64), (12001, 1281, 0.2, 65), (11009, 767, 0.45, 128),
     (11500, 1025, 0.08, 128), (24001, 250, 0.3, 129), (49000, 70, 0.4, 40), (12288, 2000, 0.03, 100)])
@@ -68,12 +69,11 @@ def test_many_rows(rows, cols, density, batch):
     X[batch // 2, 1] = np.inf
     c = macko_spmv.compress(torch.from_numpy(dense).cuda())
     Y = macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda())
-    got, finite = Y.cpu().numpy(), np.ones((batch, rows), dtype=bool)
-    finite[batch // 2] = dense[:, 1] == 0       # and a padding entry multiplies it too (zero times inf)
+    got, finite = Y.cpu().numpy(), dense[:, 1] == 0   # a padding entry stands on column 15 at the first, never on column 1
     exact = np.where(np.isfinite(X), X, 0).astype(np.float16)
-    keep = np.isfinite(got[batch // 2])
-    assert not keep[~finite[batch // 2]].any()
-    got[batch // 2] = np.where(keep, got[batch // 2], (exact[batch // 2].astype(np.float64) @ dense.astype(np.float64).T).astype(np.float16))
+    spoiled = got[batch // 2]
+    assert np.isfinite(spoiled[finite]).all() and not np.isfinite(spoiled[~finite]).any()
+    spoiled[~finite] = (exact[batch // 2].astype(np.float64) @ dense.astype(np.float64).T).astype(np.float16)[~finite]
     _check(got, dense, exact, f"{rows}x{cols} d={density} b={batch}")
     assert torch.equal(Y.view(torch.int16), macko_spmv.multiply_batched(c, torch.from_numpy(X).cuda()).view(torch.int16))
 
