@@ -874,7 +874,8 @@ constexpr u32 kRowsPassMin = 3;
 constexpr int kRowsPassBelow = 192;
 // ... and rows per wave from which on: the pass costs three round trips to LDS, which a wave with
 // a handful of rows in its only tile cannot hide (20000 x 300 at density 0.02, 32 rows per wave:
-// 15.0 -> 8.0 us; 5000 x 64 at 0.5, 8 rows: 10.0 -> 7.6 us; 1000 x 1000 at 0.05, 3 rows: 6.0 -> 6.4 us).
+// 15.0 -> 8.0 us; 1000 x 1000 at 0.05 with 3 rows per wave, when it had fewer waves than rows: 6.0 -> 6.4 us).  By
+// launch_shape a wave has six rows only from 12289 rows on (256 compute units).
 constexpr long long kRowsPassRowsPerWave = 6;
 
 #ifdef MACKO_DEV_HOOKS

@@ -1,7 +1,7 @@
 """GPU parity tests for matrices of short rows (a few to a few dozen stored entries a row, many rows
 per wave): the product then works all the rows of a 512-entry tile in one pass instead of row by row.
-The shapes below are chosen so that this variant is the one launched (mean row length below 192
-entries and at least six rows per wave of the launch); what they exercise is named per case.
+It is launched for a mean row length below 192 entries and at least six rows per wave of the launch, so with 256 compute units
+from 12289 rows on; smaller matrices have a wave per row, up to three of them.  What the shapes exercise is named per case.
 
 Bars: compressed arrays bit-exact with the oracle's; products within |err| <= 1e-3 + 1e-2 * |want|
 of the dense float64 product of the same fp16 data, and within rtol 1e-2 / atol 1e-3 of the oracle's
@@ -34,13 +34,15 @@ def _check(dense, x, label, oracle=True):
 @pytest.mark.parametrize("rows,cols,density", [
     (20000, 300, 0.02),    # 6 entries a row: more than 64 rows end in a tile, the row window slides inside it
     (20000, 300, 0.05),
-    (5000, 64, 0.5),       # half a tile per wave
+    (5000, 64, 0.5),       # too few rows for the variant: one or two rows per wave
+    (13001, 64, 0.5),      # half a tile per wave
     (30000, 40, 0.3),
     (50000, 16, 0.2),      # 3 entries a row, every fifth row or so empty
     (100000, 8, 0.05),     # mostly empty rows
     (65536, 512, 0.2),     # 100 entries a row, several tiles per wave
     (40000, 1, 1.0),       # one entry a row
-    (12000, 2000, 0.05),   # 100 entries a row with long gaps (padding entries)
+    (12000, 2000, 0.05),   # as 5000 x 64, three rows per wave: 175 entries a row with long gaps (padding entries)
+    (30000, 2000, 0.03),   # 155 entries a row with long gaps, seven rows per wave
 ])
 def test_short_rows(rows, cols, density):
     rng = np.random.default_rng(rows + 7 * cols)
@@ -132,7 +134,7 @@ def test_short_rows_keep_inf_and_nan_to_the_rows_that_read_them():
     (1, 8, 1.0), (16, 3, 0.5), (17, 200, 0.1), (63, 128, 0.3), (64, 128, 0.05), (1030, 100, 0.02),   # a wave per row, with one to 65 workgroups
     (4095, 70, 0.2), (4097, 70, 0.2),         # one row per wave of a full chip of 256 compute units, and the first wave with two
     (12288, 90, 0.1), (12289, 90, 0.1),       # the last shape with three rows per wave; the next has waves by tiles
-    (13000, 64, 0.5), (13000, 2000, 0.05),    # ... half a tile per wave; long gaps
+    (13000, 64, 0.5), (13000, 2000, 0.05),    # ... half a tile per wave; a full chip with three rows per wave, long gaps
 ])
 @pytest.mark.parametrize("int8", [False, True])
 def test_a_wave_per_row(rows, cols, density, int8):
