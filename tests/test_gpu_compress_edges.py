@@ -61,6 +61,25 @@ def test_rows_of_several_waves(int8, density):
         assert np.array_equal(got[2].cpu().numpy(), row_ptr), (cols, rows)
 
 
+# the last shapes whose rows are shared and the first whose are not; matrices of more than 128 MB, which are read past the cache
+@pytest.mark.parametrize("rows,cols,int8", [
+    (512, 2048, False), (512, 2047, False), (513, 2048, False), (1280, 8192, False), (1280, 8191, False), (1281, 8192, False),
+    (512, 2048, True), (1280, 8192, True), (1280, 53001, False), (40, 1700001, False), (1280, 104999, True)])
+def test_which_rows_several_waves_share(rows, cols, int8):
+    rng = np.random.default_rng(rows + cols)
+    dense = np.zeros((rows, cols), dtype=np.int8 if int8 else np.float16)
+    for r in range(rows):
+        at = np.flatnonzero(rng.random(cols, dtype=np.float32) < (0.0, 0.001, 0.05, 0.5)[r % 4])
+        dense[r, at] = rng.integers(1, 100, size=at.size)
+    dense[3::8, cols // 3:] = 0
+    got = (mk.compress_int8 if int8 else mk.compress)(torch.from_numpy(dense).cuda())
+    values, deltas, row_ptr, n = (mo.compress_int8 if int8 else mo.compress)(dense)
+    v = got[0].cpu().numpy()
+    assert np.array_equal(got[2].cpu().numpy(), row_ptr)
+    assert np.array_equal(v if int8 else v.view(np.uint16), values)
+    assert np.array_equal(got[1].cpu().numpy(), deltas)
+
+
 @pytest.mark.parametrize("int8", (False, True))
 def test_the_longest_row(int8):
     # 2^31 - 1 columns; non-zeros in the first, a middle and the last piece, one of them the last column
