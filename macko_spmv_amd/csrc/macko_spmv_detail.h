@@ -362,7 +362,7 @@ struct TileShape {
     int row_tiles;     // RT: a workgroup's rows / 16, rounded up
     int wave_tiles;    // NTW: vector tiles (16 vectors) per wave
     int steps;         // SC: 64-column steps of X a wave keeps in registers per chunk
-    int group_shift;   // log2 of the vector groups of a workgroup
+    int group_shift;   // log2 of the vector groups of a workgroup (spmv_pipe_kernel: of spmv_tile_kernel, whose parts of a sum it has)
     long long row_blocks;
     int chunk;         // columns per chunk
     int lane_entries;  // spmv_pipe_kernel: entries a lane takes at once; 0: spmv_tile_kernel

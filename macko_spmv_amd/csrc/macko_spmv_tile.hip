@@ -20,7 +20,7 @@
 // of X per row block; the gather kernels read LDS once per entry for a few vectors and stream the
 // matrix again for the next few.  Measured on 11008 x 4096 at density 0.5, 128 vectors: 341 us through the
 // gather kernels in groups of eight (17 TFLOP/s), 27.4 here (211 TFLOP/s of stored entries, twice that
-// on the matrix cores; 25.2 by spmv_pipe_kernel below, which takes such products now).  What bounds it: no unit alone.  Of the 54500 cycles a wave of that launch lives
+// on the matrix cores; spmv_pipe_kernel below takes such products now, 25.3 with packing, 27.9 here).  What bounds it: no unit alone.  Of the 54500 cycles a wave of that launch lives
 // the vector units are busy 25000 (decoding), LDS 28300 (12400 of them bank conflicts) and the matrix cores
 // 12300, by the counters; waves wait for 40 % of their cycles, for one another and for X out of L2.
 //
@@ -90,7 +90,10 @@ struct TileCommon {
     int n_chunks;
     u32 units_q, units_rem;  // 4-row units per row block (even_split)
     int vector_blocks;
-    int group_shift;      // log2 of the number of vector groups of a workgroup (1, 2, 4)
+    union {
+        int group_shift;  // spmv_tile_kernel: log2 of the number of vector groups of a workgroup (1, 2, 4)
+        int block_chunks; // spmv_pipe_kernel: chunks whose products are one sum
+    };
     int vector_store;     // 8-byte stores of Y are aligned
     const u32x4 *packed;  // X in operand order (pack_vectors_kernel), null: read X itself
     int packed_tiles;     // vector tiles in it
@@ -542,10 +545,10 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs<
 //     front of the stores of this one.
 // The multiplying waves run at a higher priority: a matrix instruction and a v_dot8 of another wave on the same SIMD
 // exclude each other (measured: a v_dot8 takes 18 cycles beside a stream of matrix instructions, a plain addition 10).
-// 11008 x 4096, vectors in operand order, three matrices in turn: 128 vectors at density 0.5 28.7 -> 25.2 us, 0.15
-// 28.5 -> 18.8, 0.05 27.3 -> 18.0; 64 vectors at 0.2 19.4 -> 16.9; 28672 x 1024, 64 vectors, 0.1: 23.7 -> 15.7.  What bounds it: 2.2 us
-// in front of the first product and 1.5 behind the last one (row_ptr, the first entries, the sums); between them X out of
-// L2 (128 vectors: 1 MB per compute unit, 7 us at 64 bytes a cycle) and vector and matrix instructions in turn.  Tried
+// 11008 x 4096, vectors in operand order, three matrices in turn, spmv_tile_kernel and this one: 128 vectors at density 0.5
+// 25.7 and 22.9 us, 0.15 25.1 and 17.7, 0.05 24.8 and 17.0; 64 vectors at 0.2 18.1 and 16.4; 28672 x 1024, 64 vectors, 0.1: 22.8
+// and 17.0.  What bounds it: 2.2 us in front of the first product and 1.5 behind the last one (row_ptr, the first entries, the
+// sums); between them X out of L2 (128 vectors: 1 MB per compute unit, 7 us at 64 bytes a cycle) and vector and matrix instructions in turn.  Tried
 // and slower: 8 + 8 waves, both roles at one priority, a chunk's places worked out behind the stores of the one
 // before, the next unit's A requested between products, lines touched some chunks ahead.
 constexpr int kPipeProducers = 12;
@@ -555,6 +558,14 @@ constexpr int kPipeGroups = 2;
 constexpr int kPipeDepth = 2;          // units of 32 columns of X a wave has in flight
 constexpr int kPipeLanes = 16;         // lanes per row of a pass
 constexpr int kPipeChunkStep = 32 * kPipeParts * kPipeDepth;  // chunks are multiples of this
+// Column parts of a result: two waves', of each of them two where there are registers for it (sets), and blocks of chunks,
+// whose sums the scattering waves keep and add up: as many as spmv_tile_kernel has for the same product (4 or 8), so that a
+// sum in fp32 is as exact.  Results of 10^5 that are not the exact one rounded to fp16, with the two waves' parts alone, by
+// spmv_tile_kernel, and here (4096 columns): 11008 rows at 0.5, 128 vectors 190, 159, 158; 3 x 4096 rows 188, 128, 127; 11008 rows at
+// 0.3, 64 vectors 183, 126, 123.  A block's end is a barrier and 48 KB through LDS: 11008 x 4096 at 0.5, 128 vectors 22.5 us
+// without and 22.9 with two blocks, 28672 x 1024 at 0.1, 64 vectors 15.0 and 17.0.  One chunk (up to about 700 columns) has no
+// blocks: at most 11 matrix instructions a sum, where one of 4096 columns in eight parts has 16 (600 columns: 49, 44).
+constexpr int pipe_sets(int wave_tiles) { return wave_tiles > 2 ? 1 : 2; }
 constexpr int pipe_pad(int entries) { return entries * 16 + 8; }  // columns between rows; 16-byte aligned, rows on other banks
 
 template <int NTW, int E, bool SEVERAL>
@@ -581,6 +592,9 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
     const u32 red = (u32)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
     const u32 lds0 = red + pipe_pad(E) * 2;
     const int last = a.n_chunks - 1;
+    const int parts = last >= a.block_chunks ? 2 * kPipeParts : kPipeParts;   // of the sums that meet in LDS in the end
+    // a block's sums lie where the first entries of a wave's rows may go in front of the next rows
+    const bool overlap = kRowUnit * stride - pipe_pad(E) * 2 < 1024 * NTW;
 
     if (wave < kPipeProducers) {
         const int l = lane & (L - 1), h = lane / L;   // lane of a row, row of the unit
@@ -625,6 +639,20 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
 #pragma unroll
             for (int w = 0; w < W; ++w)  // the whole offset is the lane's: what a scalar one adds need not be part of the range check
                 tile_v[S][w] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_values, (int)(vo + 16 * w), 0, 0));
+        };
+        float4v kept[NTW];   // the sums of the blocks behind: tile row, group and part by my number, as the multiplying waves hand them over
+#pragma unroll
+        for (int t = 0; t < NTW; ++t) kept[t] = float4v{0.f, 0.f, 0.f, 0.f};
+        int block_left = a.block_chunks + 2;
+        auto keep = [&](u32 from) __attribute__((always_inline)) {
+            float4v sum[NTW];
+            lds_barrier();
+#pragma unroll
+            for (int t = 0; t < NTW; ++t) sum[t] = __builtin_bit_cast(float4v, *(lds_w32x4)(uintptr_t)(from + 1024 * t));
+            if (overlap) lds_barrier();
+#pragma unroll
+            for (int t = 0; t < NTW; ++t) kept[t] += sum[t];
+            block_left = a.block_chunks;
         };
         u32 base = 0, buffer = 0, shift = 0;
         // Where my entries of set S go in this chunk, and which of the row's lanes belong to later ones: pos and
@@ -694,6 +722,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
             bool more = place(set);
             request(other);
             __builtin_amdgcn_sched_barrier(0);
+            if (--block_left == 0) keep(buffer + my_rows);  // the chunk two before was the last one of a block, and its buffer holds the block's sums
             u32 z = buffer + my_rows;   // my four rows and what is between them, zero
             int left = (int)stride * kRowUnit - 1024;
             for (; left >= 0; left -= 1024) {
@@ -715,16 +744,31 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
             scatter(index_constant<1>{}, c + 1);
             if (c + 1 >= last) break;
         }
+        if (--block_left == 0) keep(lds0 + (last & 1 ? 0u : buffer_bytes) + my_rows);
         lds_barrier();
+        if (parts > kPipeParts)
+#pragma unroll
+            for (int t = 0; t < NTW; ++t) {
+                const u32 slot = (u32)((wave >> 1) * NTW + t) * (u32)parts + (u32)(kPipeParts + (wave & 1));
+                *(lds_w32x4)(uintptr_t)(red + slot * 1024 + (u32)lane * 16) = __builtin_bit_cast(u32x4, kept[t]);
+            }
     } else {
         __builtin_amdgcn_s_setprio(1);
         const int sub = lane & 15, quarter = lane >> 4;
         const int group = wave & 1, part = (wave >> 1) & 1;
-        float4v acc[RT][NTW];
+        constexpr int SETS = pipe_sets(NTW);
+        float4v acc[SETS][RT][NTW];
+        auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
+            for (int s = 0; s < SETS; ++s)
 #pragma unroll
-            for (int t = 0; t < NTW; ++t) acc[r][t] = float4v{0.f, 0.f, 0.f, 0.f};
+                for (int r = 0; r < RT; ++r)
+#pragma unroll
+                    for (int t = 0; t < NTW; ++t) acc[s][r][t] = float4v{0.f, 0.f, 0.f, 0.f};
+        };
+        auto summed = [&](int r, int t) __attribute__((always_inline)) {
+            return __builtin_bit_cast(u32x4, SETS > 1 ? acc[0][r][t] + acc[SETS - 1][r][t] : acc[0][r][t]);
+        };
         // A unit is 32 columns: half (u & 1) of the 64-column block u >> 1 of the operand order.  Mine are every
         // other one: the same half of every block.  Beyond the last block it is requested again, for columns
         // that hold zeros.
@@ -751,38 +795,53 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
         static_for<kPipeDepth>([&](auto slot) { request(slot); });
         lds_barrier();
         const u32 mine = lds0 + (u32)sub * stride + (u32)quarter * 32 + (u32)part * 16;
-        for (int c = 0; c <= last; ++c) {
-            u32 at = mine + (c & 1 ? buffer_bytes : 0u);
-            for (int u = 0; u < a.chunk; u += kPipeChunkStep) {
-                static_for<kPipeDepth>([&](auto slot) {
-                    constexpr int J = decltype(slot)::value;
-                    u32x4 av[RT];
+        // (loops that end at their bottom: with one that may not run at all, the compiler keeps the sums and zeros side by side)
+        for (int c = 0;;) {
+            clear();
+            const int behind = c + a.block_chunks <= last ? c + a.block_chunks : last + 1;
+            do {
+                u32 at = mine + (c & 1 ? buffer_bytes : 0u);
+                int left = a.chunk;
+                do {
+                    static_for<kPipeDepth>([&](auto slot) {
+                        constexpr int J = decltype(slot)::value;
+                        u32x4 av[RT];
 #pragma unroll
-                    for (int r = 0; r < RT; ++r) av[r] = *(lds_w32x4)(uintptr_t)(at + (u32)(16 * r) * stride);
-                    at += 128;
-                    __builtin_amdgcn_sched_barrier(0);
+                        for (int r = 0; r < RT; ++r) av[r] = *(lds_w32x4)(uintptr_t)(at + (u32)(16 * r) * stride);
+                        at += 128;
+                        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int r = 0; r < RT; ++r)
+                        for (int r = 0; r < RT; ++r)
 #pragma unroll
-                        for (int t = 0; t < NTW; ++t)
-                            acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, av[r]),
-                                                                               __builtin_bit_cast(half8, b[J][t]), acc[r][t], 0, 0, 0);
-                    request(slot);
-                });
-            }
+                            for (int t = 0; t < NTW; ++t)
+                                acc[J % SETS][r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                    __builtin_bit_cast(half8, av[r]), __builtin_bit_cast(half8, b[J][t]), acc[J % SETS][r][t], 0, 0, 0);
+                        request(slot);
+                    });
+                } while ((left -= kPipeChunkStep) > 0);
+                lds_barrier();
+            } while (++c < behind);
+            if (c > last) break;
+            // into the buffer that has just been read, each to the rows of the wave that keeps it
+            const u32 to = lds0 + (c & 1 ? 0u : buffer_bytes) + (u32)(group * kPipeParts + part) * (kRowUnit * stride) + (u32)lane * 16;
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+#pragma unroll
+                for (int t = 0; t < NTW; ++t) *(lds_w32x4)(uintptr_t)(to + (u32)(r * 4) * (kRowUnit * stride) + 1024 * t) = summed(r, t);
             lds_barrier();
+            if (overlap) lds_barrier();
         }
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
             for (int t = 0; t < NTW; ++t) {
-                const u32 slot = (u32)((r * kPipeGroups + group) * NTW + t) * (u32)kPipeParts + (u32)part;
-                *(lds_w32x4)(uintptr_t)(red + slot * 1024 + (u32)lane * 16) = __builtin_bit_cast(u32x4, acc[r][t]);
+                const u32 slot = (u32)((r * kPipeGroups + group) * NTW + t) * (u32)parts + (u32)part;
+                *(lds_w32x4)(uintptr_t)(red + slot * 1024 + (u32)lane * 16) = summed(r, t);
             }
         __builtin_amdgcn_s_setprio(0);
     }
     lds_barrier();
-    finish_tiles<true, SEVERAL>(a, red, RT * kPipeGroups * NTW, kPipeGroups * NTW, kPipeParts, vector0, row0, row1);
+    finish_tiles<true, SEVERAL>(a, red, RT * kPipeGroups * NTW, kPipeGroups * NTW, parts, vector0, row0, row1);
 }
 
 template <bool SEVERAL, auto KERNEL>
@@ -824,11 +883,20 @@ TileArgs<kMaxSources> no_matrices()
     return a;
 }
 
+// Chunks of a block.
+int pipe_block_chunks(const TileShape &s, int n_chunks)
+{
+    const int have = kPipeParts * pipe_sets(s.wave_tiles), parts = kTileWaves >> s.group_shift, blocks = parts > have ? parts / have : 1;
+    // what a wave keeps is handed over in its four rows
+    if (kRowUnit * 2 * (s.chunk + pipe_pad(s.lane_entries)) < 1024 * s.wave_tiles) return n_chunks;
+    return (n_chunks + blocks - 1) / blocks;
+}
+
 size_t pipe_lds_bytes(const TileShape &s)
 {
     const size_t pad = 2 * (size_t)pipe_pad(s.lane_entries);
     const size_t dense = pad + 2 * (size_t)(16 * kPipeRowTiles) * (2 * (size_t)s.chunk + pad);
-    const size_t sums = (size_t)kPipeRowTiles * s.wave_tiles * kPipeGroups * kPipeParts * 1024;
+    const size_t sums = (size_t)kPipeRowTiles * s.wave_tiles * kPipeGroups * 2 * kPipeParts * 1024;
     return dense > sums ? dense : sums;
 }
 
@@ -853,7 +921,10 @@ int launch_tile_shape(TileArgs<kMaxSources> a, const TileShape &s, int max_lds, 
     a.n_chunks = (a.cols + s.chunk - 1) / s.chunk;
     a.units_q = (u32)(units / s.row_blocks);
     a.units_rem = (u32)(units % s.row_blocks);
-    a.group_shift = s.group_shift;
+    if (pipe)
+        a.block_chunks = pipe_block_chunks(s, a.n_chunks);
+    else
+        a.group_shift = s.group_shift;
     const int vectors = 16 * s.wave_tiles * groups;
     a.vector_blocks = (a.batch + vectors - 1) / vectors;
     const bool several = a.first[1] < a.rows;
@@ -912,14 +983,15 @@ double tile_cost(const TileShape &s, long long units, int cols, double density, 
 // where there are few rows per compute unit (4096 x 4096, density 0.5, 128 vectors: 18.3 us against
 // 20.4; 11008 x 4096: 39.4 against 28.4).
 bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info,
-                       double *cycles)
+                       double *cycles, int most_shift = 2)
 {
     const long long units = ((long long)rows + kRowUnit - 1) / kRowUnit;
     const double density = (double)padded / ((double)rows * (double)cols);
     const int tiles = (batch + 15) / 16;
     double least = 0.0;
     bool found = false;
-    for (int shift = tiles <= 1 ? 0 : (tiles <= 4 ? 1 : 2); shift >= (tiles > 4 ? 1 : (tiles <= 1 ? 0 : 1)); --shift) {
+    const int first_shift = tiles <= 1 ? 0 : (tiles <= 4 ? 1 : 2);
+    for (int shift = first_shift < most_shift ? first_shift : most_shift; shift >= (tiles > 4 ? 1 : (tiles <= 1 ? 0 : 1)); --shift) {
         TileShape s{};
         s.group_shift = shift;
         s.wave_tiles = tiles > 2 ? 2 : 1;
@@ -961,22 +1033,24 @@ bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, in
 
 // The estimated time in us of a launch of spmv_pipe_kernel.  The terms were fitted to 27000 products of packed vectors (1500
 // to 28000 rows, 256 to 11000 columns, densities 0.05 to 0.9, 17 to 256 vectors; 7 % off in the median, 16 % for one in
-// ten): per launch, per round of workgroups, per chunk and pass (of 16 entries a lane it costs more than one of 8), and per
-// column and vector.
+// ten): per launch, per round of workgroups, per chunk and pass (of 16 entries a lane it costs more than one of 8), per
+// column and vector, and per block's end.
 double pipe_us(const TileShape &s, int cols, int batch, const DeviceInfo &info, double passes)
 {
     const int vectors = 16 * kPipeGroups * s.wave_tiles;
     const long long blocks = (batch + vectors - 1) / vectors;
     const double full = (double)((s.row_blocks * blocks + info.compute_units - 1) / info.compute_units);
     const int n_chunks = (cols + s.chunk - 1) / s.chunk;
-    return 0.93 + full * (3.25 + n_chunks * ((s.lane_entries == 8 ? 0.31 : 0.56) * passes + s.chunk / 512.0 * (0.31 + 0.26 * s.wave_tiles)));
+    const double ends = (n_chunks - 1) / pipe_block_chunks(s, n_chunks);
+    return 0.93 + full * (3.25 + 0.35 * ends + n_chunks * ((s.lane_entries == 8 ? 0.31 : 0.56) * passes + s.chunk / 512.0 * (0.31 + 0.26 * s.wave_tiles)));
 }
 
-// The shape of a launch of spmv_pipe_kernel and its estimated time.
-bool choose_pipe_shape(TileShape *shape, int rows, int cols, long long padded, int batch, const DeviceInfo &info, double *us)
+// The shape of a launch of spmv_pipe_kernel and its estimated time.  group_shift: spmv_tile_kernel's, whose parts of a sum it has.
+bool choose_pipe_shape(TileShape *shape, int rows, int cols, long long padded, int batch, int group_shift, const DeviceInfo &info, double *us)
 {
     if (batch <= 16 || rows < 1 || padded < 1) return false;
     TileShape s{};
+    s.group_shift = group_shift;
     s.wave_tiles = batch > 64 ? 4 : batch > 32 ? 2 : 1;
     const int vectors = 16 * kPipeGroups * s.wave_tiles;
     const long long blocks = (batch + vectors - 1) / vectors;
@@ -1015,15 +1089,16 @@ constexpr double kTileUsPerCycle = 1.06 / 2400.0;
 
 // The kernel and the shape of a launch, and its estimated time in us (without packing; at 2.4 GHz).  Right to about 10 %
 // where it decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1:
-// 24.4, 21).  Of the 27000 products above, the pipe kernel is taken for half, which are 22 % faster in the mean (up to
-// twice; 7 in 10000 are more than 3 % slower).
-bool choose_shape(TileShape *shape, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, double *us)
+// 24.4, 21).  Of the 27000 products above, timed when a result had two parts only, the pipe kernel was taken for half, which
+// were 22 % faster in the mean (up to twice; 7 in 10000 more than 3 % slower).
+bool choose_shape(TileShape *shape, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, double *us,
+                  int most_shift = 2)
 {
     double cycles = 0.0, pipe_us = 0.0;
-    if (!choose_tile_shape(shape, rows, cols, padded, batch, packed, info, &cycles)) return false;
+    if (!choose_tile_shape(shape, rows, cols, padded, batch, packed, info, &cycles, most_shift)) return false;
     *us = cycles * kTileUsPerCycle;
     TileShape pipe;
-    if (packed && choose_pipe_shape(&pipe, rows, cols, padded, batch, info, &pipe_us) && pipe_us < 0.97 * *us) {
+    if (packed && choose_pipe_shape(&pipe, rows, cols, padded, batch, shape->group_shift, info, &pipe_us) && pipe_us < 0.97 * *us) {
         *shape = pipe;
         *us = pipe_us;
     }
@@ -1158,7 +1233,14 @@ int packed_product(const macko_packed_matrix *matrices, int n, const void *packe
     a.residual = (const uint16_t *)residual;
     TileShape shape;
     double us = 0.0;
-    if (!choose_shape(&shape, a.rows, cols, padded, batch, true, info, &us)) return MACKO_E_INVALID_ARGUMENT;
+    int most_shift = 2;
+    if (used > 1) {  // a launch has no fewer parts of a sum than the smallest of its matrices has on its own
+        int least = 0;
+        auto rows_of = [&](int k) { return (k + 1 < used ? a.first[k + 1] : a.rows) - a.first[k]; };
+        for (int k = 1; k < used; ++k) least = rows_of(k) < rows_of(least) ? k : least;
+        if (choose_tile_shape(&shape, rows_of(least), cols, a.source[least].padded, batch, true, info, &us)) most_shift = shape.group_shift;
+    }
+    if (!choose_shape(&shape, a.rows, cols, padded, batch, true, info, &us, most_shift)) return MACKO_E_INVALID_ARGUMENT;
     if (used > 1 && better_apart(a, used, shape, info)) {
         for (int k = 0; k < n; ++k) {
             const int e = packed_product(matrices + k, 1, packed, nullptr, cols, batch, stream);

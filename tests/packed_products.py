@@ -30,8 +30,8 @@ PRODUCTS = [
     # columns in several chunks: every width of vectors and of lanes, one and several matrices, the last one of any rows
     Product(17, (9003,), 1300, 0.1, "spmv_pipe_kernel<1,8,false>"),
     Product(32, (6140, 512, 2049), 1411, 0.12, "spmv_pipe_kernel<1,8,true>"),
-    Product(31, (4096, 4096, 1025), 1300, 0.3, "spmv_pipe_kernel<1,16,true>"),
-    Product(33, (12291,), 1281, 0.08, "spmv_pipe_kernel<2,8,false>"),
+    Product(31, (4096, 4096, 4093), 1300, 0.3, "spmv_pipe_kernel<1,16,true>"),
+    Product(33, (12285,), 1281, 0.08, "spmv_pipe_kernel<2,8,false>"),
     Product(64, (8000, 2048, 2050), 1300, 0.1, "spmv_pipe_kernel<2,8,true>"),
     Product(63, (12285,), 1301, 0.4, "spmv_pipe_kernel<2,16,false>"),
     Product(40, (4096, 4096, 4095), 1300, 0.35, "spmv_pipe_kernel<2,16,true>"),
@@ -46,6 +46,12 @@ LONG_ARRAY = dict(entries=2 ** 31 - 8200, rows=524288, cols=16384, batch=17, ker
 
 # matrices of so unequal densities that each has a launch of its own: batch, rows of each, cols, their densities
 UNEQUAL = dict(batch=16, rows=(11008, 11006), cols=1300, densities=(0.95, 0.03))
+
+
+# sums that are long enough to show in the rounded results: batch, rows of each of several matrices (the kernel of two roles), cols,
+# density; the matrices one by one go through the other kernel
+SUMS = [(128, (4096, 4096, 4096), 4096, 0.5), (40, (4096, 4096, 4096), 4096, 0.3), (20, (4096, 4096, 4096), 4096, 0.4),
+        (100, (4096, 4096, 4096), 2048, 0.1)]
 
 
 def matrices(product):

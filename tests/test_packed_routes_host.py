@@ -64,3 +64,11 @@ def test_the_unequal_matrices_are_launched_apart(routes):
     unequal = packed_products.UNEQUAL
     sizes = [(rows, int(rows * unequal["cols"] * max(d, 1 / 16)) // 8 * 8) for rows, d in zip(unequal["rows"], unequal["densities"])]
     assert len(routes(unequal["cols"], unequal["batch"], sizes)) == 2
+
+
+@pytest.mark.parametrize("batch,rows,cols,density", packed_products.SUMS)
+def test_long_sums_of_both_kernels(routes, batch, rows, cols, density):
+    sizes = [(r, int(r * cols * density) // 8 * 8) for r in rows]
+    together = routes(cols, batch, sizes)
+    assert len(together) == 1 and together[0].startswith("spmv_pipe_kernel")
+    assert all(routes(cols, batch, [size])[0].startswith("spmv_tile_kernel") for size in sizes)
