@@ -541,31 +541,43 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs<
 //     sum has four steps instead of six, and what a pass costs besides its entries is shared by four rows);
 //   - no column is clamped: rows stand 16 * E columns apart in LDS, which is as far as the entries of a lane that reaches
 //     beyond its chunk can go on either side;
-//   - entries are requested into one of two register sets as soon as it is known where the next chunk starts, in
-//     front of the stores of this one.
+//   - entries are requested into one of two register sets as soon as this chunk's stores are on their way.  The requests of all
+//     waves queue behind those for X for 200 to 1100 cycles (stamps of a launch), which the stores, in front of them, need
+//     not wait for; they are there well before the next chunk (128 vectors at 0.5: 21.85 us with the requests in front, 20.98);
+//   - only the columns of a chunk are cleared, not what lies between rows, where only entries of other chunks go (three stores
+//     a wave and chunk at 0.5 instead of six), in front of the first look at the entries.
 // The multiplying waves run at a higher priority: a matrix instruction and a v_dot8 of another wave on the same SIMD
 // exclude each other (measured: a v_dot8 takes 18 cycles beside a stream of matrix instructions, a plain addition 10).
 // 11008 x 4096, vectors in operand order, three matrices in turn, spmv_tile_kernel and this one: 128 vectors at density 0.5
-// 25.7 and 22.9 us, 0.15 25.1 and 17.7, 0.05 24.8 and 17.0; 64 vectors at 0.2 18.1 and 16.4; 28672 x 1024, 64 vectors, 0.1: 22.8
-// and 17.0.  What bounds it: 2.2 us in front of the first product and 1.5 behind the last one (row_ptr, the first entries, the
-// sums); between them X out of L2 (128 vectors: 1 MB per compute unit, 7 us at 64 bytes a cycle) and vector and matrix instructions in turn.  Tried
-// and slower: 8 + 8 waves, both roles at one priority, a chunk's places worked out behind the stores of the one
-// before, the next unit's A requested between products, lines touched some chunks ahead.
+// 25.4 and 20.6 us, 0.3 25.0 and 19.4, 0.15 25.0 and 17.5, 0.05 24.6 and 16.0; 64 vectors at 0.2 18.1 and 14.6; 28672 x 1024, 64
+// vectors, 0.1: 23.0 and 15.2; 12288 x 4096, 32 vectors at 0.5 18.2 and 16.3.  What bounds it: 2.2 us in front of the first product and
+// 1.5 behind the last one (row_ptr, the first entries, the sums).  Between them a chunk of 384 columns takes 3600 cycles, in which LDS
+// is busy for 2400 (each of the 16 stores of a pass for 7: 32 lanes at random places meet in a bank three or four times), the
+// path from L2 for 2000 (X: 1 MB per compute unit at 64 bytes a cycle), vector and matrix instructions, which exclude each
+// other, for 2600: 21.2 us with the entries always in L2 and 18.6 with X in L1 as well.  Tried and not faster: 8 + 8 waves, both
+// roles at one priority (22.7), a chunk's places worked out behind the stores of the one before, by all or by some of the waves (21.5 to
+// 22.0), the next unit's A requested between products, lines touched some chunks ahead; chunks that end anywhere in the
+// ring of units: the compiler then waits for all loads or spills.
 constexpr int kPipeProducers = 12;
 constexpr int kPipeRowTiles = 3;
 constexpr int kPipeParts = 2;          // of the columns, per group of vectors
 constexpr int kPipeGroups = 2;
-constexpr int kPipeDepth = 2;          // units of 32 columns of X a wave has in flight
 constexpr int kPipeLanes = 16;         // lanes per row of a pass
-constexpr int kPipeChunkStep = 32 * kPipeParts * kPipeDepth;  // chunks are multiples of this
+// Units of 32 columns of X a wave has in flight; chunks are whole rounds of them.  A unit of X is asked for behind the entries of
+// the next chunk, and loads return in order: with two units on the way the products waited for them more than half of their time
+// (11008 x 4096, 128 vectors at 0.5: 20.98 us, with three 20.56; 64 vectors at 0.1 12.9, with four 12.1).  64 and more
+// sums a lane leave room for three; where 8 entries a lane do, chunks of 640 columns in whole rounds of two are worth more
+// (0.15: 17.4, 18.7 with three).
+constexpr int pipe_depth(int wave_tiles, int entries) { return entries == 16 ? 3 : wave_tiles > 2 ? 2 : 4; }
+constexpr int pipe_chunk_step(int wave_tiles, int entries) { return 32 * kPipeParts * pipe_depth(wave_tiles, entries); }
 // Column parts of a result: two waves', of each of them two where there are registers for it (sets), and blocks of chunks,
 // whose sums the scattering waves keep and add up: as many as spmv_tile_kernel has for the same product (4 or 8), so that a
 // sum in fp32 is as exact.  Results of 10^5 that are not the exact one rounded to fp16, with the two waves' parts alone, by
 // spmv_tile_kernel, and here (4096 columns): 11008 rows at 0.5, 128 vectors 190, 159, 158; 3 x 4096 rows 188, 128, 127; 11008 rows at
 // 0.3, 64 vectors 183, 126, 123.  A block's end is a barrier and 48 KB through LDS: 11008 x 4096 at 0.5, 128 vectors 22.5 us
-// without and 22.9 with two blocks, 28672 x 1024 at 0.1, 64 vectors 15.0 and 17.0.  One chunk (up to about 700 columns) has no
+// without and 22.9 with two blocks when that was measured.  One chunk (up to about 700 columns) has no
 // blocks: at most 11 matrix instructions a sum, where one of 4096 columns in eight parts has 16 (600 columns: 49, 44).
-constexpr int pipe_sets(int wave_tiles) { return wave_tiles > 2 ? 1 : 2; }
+constexpr int pipe_sets(int wave_tiles, int entries) { return wave_tiles > 2 ? 1 : entries == 16 ? 3 : 2; }  // a divisor of the depth
 constexpr int pipe_pad(int entries) { return entries * 16 + 8; }  // columns between rows; 16-byte aligned, rows on other banks
 
 template <int NTW, int E, bool SEVERAL>
@@ -575,6 +587,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
     typedef __attribute__((address_space(3))) u32x4 *lds_w32x4;
     typedef __attribute__((address_space(3))) uint16_t *lds_w16;
     constexpr int RT = kPipeRowTiles, L = kPipeLanes, W = E / 8;  // W: words of nibbles a lane has
+    constexpr int DEPTH = pipe_depth(NTW, E);
     static_assert(E == 8 || E == 16, "entries per lane");
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = uniform(threadIdx.x >> 6);
@@ -719,18 +732,15 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
             constexpr index_constant<1 - S> other{};
             buffer = lds0 + (S ? buffer_bytes : 0u);
             shift = buffer - (u32)(c * a.chunk) * 2;
-            bool more = place(set);
-            request(other);
-            __builtin_amdgcn_sched_barrier(0);
             if (--block_left == 0) keep(buffer + my_rows);  // the chunk two before was the last one of a block, and its buffer holds the block's sums
-            u32 z = buffer + my_rows;   // my four rows and what is between them, zero
-            int left = (int)stride * kRowUnit - 1024;
-            for (; left >= 0; left -= 1024) {
-                *(lds_w32x4)(uintptr_t)z = u32x4{0u, 0u, 0u, 0u};
-                z += 1024;
-            }
-            if (lane * 16 < left + 1024) *(lds_w32x4)(uintptr_t)z = u32x4{0u, 0u, 0u, 0u};
+            u32 z = buffer + my_row + (u32)l * 16;   // my row's columns, zero; what is between rows is never read
+            for (int left = a.chunk; left > 0; left -= 8 * L, z += 16 * L) *(lds_w32x4)(uintptr_t)z = u32x4{0u, 0u, 0u, 0u};
+            __builtin_amdgcn_sched_barrier(0);
+            bool more = place(set);
+            __builtin_amdgcn_sched_barrier(0);
             write(set);
+            __builtin_amdgcn_sched_barrier(0);
+            request(other);
             while (__builtin_expect(more, 0)) {
                 more = place(other);
                 write(other);
@@ -756,7 +766,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
         __builtin_amdgcn_s_setprio(1);
         const int sub = lane & 15, quarter = lane >> 4;
         const int group = wave & 1, part = (wave >> 1) & 1;
-        constexpr int SETS = pipe_sets(NTW);
+        constexpr int SETS = pipe_sets(NTW, E);
         float4v acc[SETS][RT][NTW];
         auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -767,12 +777,15 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
                     for (int t = 0; t < NTW; ++t) acc[s][r][t] = float4v{0.f, 0.f, 0.f, 0.f};
         };
         auto summed = [&](int r, int t) __attribute__((always_inline)) {
-            return __builtin_bit_cast(u32x4, SETS > 1 ? acc[0][r][t] + acc[SETS - 1][r][t] : acc[0][r][t]);
+            float4v sum = acc[0][r][t];
+#pragma unroll
+            for (int s = 1; s < SETS; ++s) sum += acc[s][r][t];
+            return __builtin_bit_cast(u32x4, sum);
         };
         // A unit is 32 columns: half (u & 1) of the 64-column block u >> 1 of the operand order.  Mine are every
         // other one: the same half of every block.  Beyond the last block it is requested again, for columns
         // that hold zeros.
-        u32x4 b[kPipeDepth][NTW];
+        u32x4 b[DEPTH][NTW];
         const __amdgpu_buffer_rsrc_t rs_x =
             __builtin_amdgcn_make_buffer_rsrc((void *)a.packed, 0, (int)((u32)(a.packed_tiles * a.packed_steps) * (kBlockPieces * 16)), 0x00020000);
         int x_of[NTW];
@@ -792,7 +805,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
             x_at = x_at < x_last ? x_at + x_step : x_last;
             __builtin_amdgcn_sched_barrier(0);  // the waits count on this order
         };
-        static_for<kPipeDepth>([&](auto slot) { request(slot); });
+        static_for<DEPTH>([&](auto slot) { request(slot); });
         lds_barrier();
         const u32 mine = lds0 + (u32)sub * stride + (u32)quarter * 32 + (u32)part * 16;
         // (loops that end at their bottom: with one that may not run at all, the compiler keeps the sums and zeros side by side)
@@ -801,9 +814,10 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
             const int behind = c + a.block_chunks <= last ? c + a.block_chunks : last + 1;
             do {
                 u32 at = mine + (c & 1 ? buffer_bytes : 0u);
-                int left = a.chunk;
+                const int rest = a.cols - c * a.chunk;
+                int left = rest < a.chunk ? rest : a.chunk;
                 do {
-                    static_for<kPipeDepth>([&](auto slot) {
+                    static_for<DEPTH>([&](auto slot) {
                         constexpr int J = decltype(slot)::value;
                         u32x4 av[RT];
 #pragma unroll
@@ -818,7 +832,7 @@ __global__ void __launch_bounds__(kTileThreads) spmv_pipe_kernel(const TileArgs<
                                     __builtin_bit_cast(half8, av[r]), __builtin_bit_cast(half8, b[J][t]), acc[J % SETS][r][t], 0, 0, 0);
                         request(slot);
                     });
-                } while ((left -= kPipeChunkStep) > 0);
+                } while ((left -= pipe_chunk_step(NTW, E)) > 0);
                 lds_barrier();
             } while (++c < behind);
             if (c > last) break;
@@ -886,7 +900,7 @@ TileArgs<kMaxSources> no_matrices()
 // Chunks of a block.
 int pipe_block_chunks(const TileShape &s, int n_chunks)
 {
-    const int have = kPipeParts * pipe_sets(s.wave_tiles), parts = kTileWaves >> s.group_shift, blocks = parts > have ? parts / have : 1;
+    const int have = kPipeParts * pipe_sets(s.wave_tiles, s.lane_entries), parts = kTileWaves >> s.group_shift, blocks = (parts + have - 1) / have;
     // what a wave keeps is handed over in its four rows
     if (kRowUnit * 2 * (s.chunk + pipe_pad(s.lane_entries)) < 1024 * s.wave_tiles) return n_chunks;
     return (n_chunks + blocks - 1) / blocks;
@@ -914,7 +928,7 @@ int launch_tile_shape(TileArgs<kMaxSources> a, const TileShape &s, int max_lds, 
     const size_t lds = pipe ? pipe_lds_bytes(s) : tile_lds_bytes(s);
     const long long units = (a.rows + kRowUnit - 1) / kRowUnit;
     if (lds > (size_t)max_lds || s.chunk <= 0 || s.row_blocks < 1 ||
-        (pipe ? s.chunk % kPipeChunkStep != 0 || a.packed == nullptr : s.chunk % 64 != 0 || s.chunk > 64 * parts * s.steps) ||
+        (pipe ? s.chunk % pipe_chunk_step(s.wave_tiles, s.lane_entries) != 0 || a.packed == nullptr : s.chunk % 64 != 0 || s.chunk > 64 * parts * s.steps) ||
         (units + s.row_blocks - 1) / s.row_blocks > 4 * (pipe ? kPipeRowTiles : s.row_tiles))
         return MACKO_E_INVALID_ARGUMENT;
     a.chunk = s.chunk;
@@ -1031,10 +1045,10 @@ bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, in
     return found;
 }
 
-// The estimated time in us of a launch of spmv_pipe_kernel.  The terms were fitted to 27000 products of packed vectors (1500
-// to 28000 rows, 256 to 11000 columns, densities 0.05 to 0.9, 17 to 256 vectors; 7 % off in the median, 16 % for one in
-// ten): per launch, per round of workgroups, per chunk and pass (of 16 entries a lane it costs more than one of 8), per
-// column and vector, and per block's end.
+// The estimated time in us of a launch of spmv_pipe_kernel.  The terms were fitted to 839 products of packed vectors (1500
+// to 28000 rows, 256 to 11000 columns, densities 0.05 to 0.6, 17 to 256 vectors; 6 % off in the median, 17 % for one in
+// ten): per round of workgroups, per block's end, per chunk and pass (of 16 entries a lane it costs more than one of 8) and
+// per column and vector.
 double pipe_us(const TileShape &s, int cols, int batch, const DeviceInfo &info, double passes)
 {
     const int vectors = 16 * kPipeGroups * s.wave_tiles;
@@ -1042,7 +1056,8 @@ double pipe_us(const TileShape &s, int cols, int batch, const DeviceInfo &info, 
     const double full = (double)((s.row_blocks * blocks + info.compute_units - 1) / info.compute_units);
     const int n_chunks = (cols + s.chunk - 1) / s.chunk;
     const double ends = (n_chunks - 1) / pipe_block_chunks(s, n_chunks);
-    return 0.93 + full * (3.25 + 0.35 * ends + n_chunks * ((s.lane_entries == 8 ? 0.31 : 0.56) * passes + s.chunk / 512.0 * (0.31 + 0.26 * s.wave_tiles)));
+    const double products = s.wave_tiles == 4 ? 1.31 : s.wave_tiles == 2 ? 0.59 : 0.43;   // 512 columns
+    return full * (3.6 + 0.13 * ends + n_chunks * (s.lane_entries == 8 ? 0.315 : 0.47) * passes + cols / 512.0 * products);
 }
 
 // The shape of a launch of spmv_pipe_kernel and its estimated time.  group_shift: spmv_tile_kernel's, whose parts of a sum it has.
@@ -1061,22 +1076,22 @@ bool choose_pipe_shape(TileShape *shape, int rows, int cols, long long padded, i
     if (s.row_blocks * most < units) s.row_blocks = (units + most - 1) / most;
     if (s.row_blocks > units) return false;
     const double density = (double)padded / ((double)rows * (double)cols);
-    const int whole = (cols + kPipeChunkStep - 1) / kPipeChunkStep * kPipeChunkStep;
     for (int e = 8; e <= 16; e += 8) {
         s.lane_entries = e;
+        const int step = pipe_chunk_step(s.wave_tiles, e), whole = (cols + step - 1) / step * step;
         // columns per chunk: what LDS holds twice, and what a pass holds of a row's entries (with a margin for the spread
         // between rows, for the lane that is not done and for what stands in front of the first entry)
         const int pad = pipe_pad(e);
-        int chunk = ((info.max_lds_bytes - 2 * pad) / (2 * 16 * kPipeRowTiles) - 2 * pad) / 2 / kPipeChunkStep * kPipeChunkStep;
+        int chunk = ((info.max_lds_bytes - 2 * pad) / (2 * 16 * kPipeRowTiles) - 2 * pad) / 2 / step * step;
         chunk = chunk < whole ? chunk : whole;
         auto fits = [&](int c) {
             const double mean = c * density;
             return mean + 3.0 * std::sqrt(mean * (density < 1.0 ? 1.0 - density : 0.0)) + e + 8 <= kPipeLanes * e;
         };
-        while (chunk > 0 && !fits(chunk)) chunk -= kPipeChunkStep;
+        while (chunk > 0 && !fits(chunk)) chunk -= step;
         if (chunk < (e == 8 ? 512 : 384) && chunk < whole) continue;
         const int n_chunks = (cols + chunk - 1) / chunk;
-        s.chunk = ((cols + n_chunks - 1) / n_chunks + kPipeChunkStep - 1) / kPipeChunkStep * kPipeChunkStep;
+        s.chunk = ((cols + n_chunks - 1) / n_chunks + step - 1) / step * step;
         if (pipe_lds_bytes(s) > (size_t)info.max_lds_bytes) continue;
         *us = pipe_us(s, cols, batch, info, 1.0);
         *shape = s;
@@ -1089,8 +1104,8 @@ constexpr double kTileUsPerCycle = 1.06 / 2400.0;
 
 // The kernel and the shape of a launch, and its estimated time in us (without packing; at 2.4 GHz).  Right to about 10 %
 // where it decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1:
-// 24.4, 21).  Of the 27000 products above, timed when a result had two parts only, the pipe kernel was taken for half, which
-// were 22 % faster in the mean (up to twice; 7 in 10000 more than 3 % slower).
+// 24.4, 21).  Of the 839 products above the pipe kernel is taken for 69 %; what is taken is 0.3 % behind the
+// better of the two in the mean, more than 3 % for 4 % of them (15 % at most).
 bool choose_shape(TileShape *shape, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, double *us,
                   int most_shift = 2)
 {
