@@ -122,6 +122,14 @@ MACKO_API int macko_compress_f16_count_total(const void *dense, int32_t rows, in
                                              int32_t *row_ptr, int32_t *total, void *stream);
 
 /*
+ * As macko_compress_f16_count_total, but *total is stored as soon as it is known, before row_ptr is
+ * complete: a host thread that waits for it has the outputs allocated and step 2 launched meanwhile.
+ * What reads row_ptr has to be ordered behind this call on the stream, as step 2 is.
+ */
+MACKO_API int macko_compress_f16_count_early(const void *dense, int32_t rows, int32_t cols,
+                                             int32_t *row_ptr, int32_t *total, void *stream);
+
+/*
  * Compressor, step 2 of 2.  Fills values [P] (16-byte aligned) and deltas [P/2] (4-byte
  * aligned) from `dense` and the row_ptr produced by step 1; both arrays are fully written,
  * tail zero-filled, whatever they held before.  P must be ceil(row_ptr[rows]/8)*8.
@@ -234,6 +242,9 @@ MACKO_API int macko_compress_i8_count(const void *dense, int32_t rows, int32_t c
                             int32_t *row_ptr, void *stream);
 /* int8 twin of macko_compress_f16_count_total. */
 MACKO_API int macko_compress_i8_count_total(const void *dense, int32_t rows, int32_t cols,
+                                            int32_t *row_ptr, int32_t *total, void *stream);
+/* int8 twin of macko_compress_f16_count_early. */
+MACKO_API int macko_compress_i8_count_early(const void *dense, int32_t rows, int32_t cols,
                                             int32_t *row_ptr, int32_t *total, void *stream);
 MACKO_API int macko_compress_i8_fill(const void *dense, int32_t rows, int32_t cols,
                            const int32_t *row_ptr, void *values, void *deltas,

@@ -207,7 +207,7 @@ Compressed compress_on_device(const at::Tensor &M, at::Tensor *plan, bool (*go_o
         new at::Tensor(at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true)));
     volatile int *total = total_word->data_ptr<int>();
     *total = -1;
-    check_rc((int8 ? macko_compress_i8_count_total : macko_compress_f16_count_total)(
+    check_rc((int8 ? macko_compress_i8_count_early : macko_compress_f16_count_early)(
                  M.data_ptr(), (int32_t)rows, (int32_t)cols, row_ptr.data_ptr<int>(), total_word->data_ptr<int>(),
                  (void *)stream),
              "compress (count)");

@@ -98,3 +98,16 @@ def test_the_longest_row(int8):
     others = nibbles[:entries] != 15
     others[place] = False
     assert not others.any()
+
+
+# the scan over the rows: 8 rows a thread, 8192 a slice, 24576 a round of the total, each one short of it, whole and one over
+@pytest.mark.parametrize("rows", (1, 7, 8, 9, 8191, 8192, 8193, 16383, 16385, 24575, 24576, 24577, 49161))
+def test_scan_of_the_rows(rows):
+    rng = np.random.default_rng(rows)
+    dense = rng.standard_normal((rows, 5)).astype(np.float16)
+    dense[rng.random((rows, 5)) >= 0.4] = 0
+    got = mk.compress(torch.from_numpy(dense).cuda())
+    values, deltas, row_ptr, n = mo.compress(dense)
+    assert np.array_equal(got[2].cpu().numpy(), row_ptr)
+    assert np.array_equal(got[0].cpu().numpy().view(np.uint16), values)
+    assert np.array_equal(got[1].cpu().numpy(), deltas)
