@@ -181,6 +181,11 @@ MACKO_API int macko_spmv_f16_batched(const void *values, const void *deltas, con
  *   macko_spmv_f16_packed_several  the same (without a residual) for up to MACKO_PACKED_MATRICES matrices of
  *                         the same columns in one launch, or in one each where their densities are so
  *                         unequal that it takes less time; in front of another matrix, rows % 4 == 0
+ *   macko_packed_together whether that is one launch (y and ldy are not looked at)
+ *   macko_spmv_f16_packed_silu  silu(G X) * (U X) of two matrices of as many rows (>= 64, a multiple of 8), each product
+ *                         rounded to fp16, in operand order (`out`: macko_packed_bytes of `rows` elements,
+ *                         16-byte aligned, not `packed`), in one launch; y and ldy are not looked at.  The bits are those of
+ *                         the products in one launch and macko_prefill_pack_silu_mul_f16 behind them
  */
 #define MACKO_PACKED_MATRICES 3
 typedef struct macko_packed_matrix {
@@ -201,6 +206,10 @@ MACKO_API int macko_spmv_f16_packed(const void *values, const void *deltas, cons
                           void *stream);
 MACKO_API int macko_spmv_f16_packed_several(const macko_packed_matrix *matrices, int32_t n_matrices,
                           const void *packed, int32_t cols, int32_t batch, void *stream);
+MACKO_API int macko_packed_together(const macko_packed_matrix *matrices, int32_t n_matrices,
+                          const void *packed, int32_t cols, int32_t batch, int32_t *together);
+MACKO_API int macko_spmv_f16_packed_silu(const macko_packed_matrix *gate, const macko_packed_matrix *up,
+                          const void *packed, void *out, int32_t cols, int32_t batch, void *stream);
 
 /*
  * Products whose input vector is produced on the fly while it is staged for the product, so a

@@ -74,7 +74,7 @@ ops = types.SimpleNamespace(**{name: _operator(name) for name in (
     "multiply_batched", "multiply_int8", "multiply_int8_axpby", "multiply_rmsnorm", "multiply_silu_mul_axpby",
     "multiply_attention_axpby", "decode_rmsnorm", "decode_norm_matvec", "decode_rope_append", "decode_attention", "decode_silu_mul",
     "decode_rope_attention", "decode_rope_attention_parts", "pack_rmsnorm", "rmsnorm_rows", "pack_silu_mul", "multiply_packed",
-    "multiply_packed_several", "prefill_rope_append", "prefill_attention")})
+    "multiply_packed_several", "multiply_packed_silu", "prefill_rope_append", "prefill_attention")})
 
 
 @torch.library.register_fake("macko_spmv::multiply")
@@ -160,6 +160,11 @@ def _multiply_packed_fake(M_values, M_deltas, M_row_indices, M_rows, M_cols, pac
 @torch.library.register_fake("macko_spmv::multiply_packed_several")
 def _multiply_packed_several_fake(M_values, M_deltas, M_row_indices, M_rows, M_cols, packed, batch):
     return [torch.empty((batch, rows), device=values.device, dtype=values.dtype) for values, rows in zip(M_values, M_rows)]
+
+
+@torch.library.register_fake("macko_spmv::multiply_packed_silu")
+def _multiply_packed_silu_fake(M_values, M_deltas, M_row_indices, M_rows, M_cols, packed, batch):
+    return _packed_like(packed, M_rows, batch)
 
 
 @torch.library.register_fake("macko_spmv::prefill_rope_append")

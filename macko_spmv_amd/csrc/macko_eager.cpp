@@ -75,7 +75,7 @@ public:
     X(multiply_attention_axpby) X(decode_rmsnorm) X(decode_norm_matvec) X(decode_rope_append)                  \
     X(decode_attention) X(decode_silu_mul) X(decode_rope_attention) X(decode_rope_attention_parts)             \
     X(pack_rmsnorm) X(rmsnorm_rows) X(pack_silu_mul) X(multiply_packed) X(multiply_packed_several)             \
-    X(prefill_rope_append) X(prefill_attention)
+    X(multiply_packed_silu) X(prefill_rope_append) X(prefill_attention)
 #define MACKO_OPERATOR(NAME)                                                                  \
     struct NAME##_operator {                                                                   \
         typedef Operator<std::remove_pointer_t<decltype(&NAME##_hip)>> Type;                   \
@@ -377,6 +377,7 @@ PyMethodDef eager_functions[] = {
     MACKO_EAGER(pack_silu_mul, eager<pack_silu_mul_operator>),
     MACKO_EAGER(multiply_packed, eager<multiply_packed_operator>),
     MACKO_EAGER(multiply_packed_several, eager<multiply_packed_several_operator>),
+    MACKO_EAGER(multiply_packed_silu, eager<multiply_packed_silu_operator>),
     MACKO_EAGER(prefill_rope_append, eager<prefill_rope_append_operator>),
     MACKO_EAGER(prefill_attention, eager<prefill_attention_operator>),
     {nullptr, nullptr, 0, nullptr}};

@@ -21,6 +21,9 @@ __device__ __forceinline__ size_t packed_piece(int p, int n, int tiles)
     return ((size_t)(p >> 3) * (size_t)tiles + (size_t)(n >> 4)) * kBlockPieces + (size_t)((p & 1) * 64 + ((p >> 1) & 3) * 16 + (n & 15));
 }
 
+// The gate of a Llama layer.
+__device__ __forceinline__ float silu_mul(float gate, float up) { return gate / (1.0f + __expf(-gate)) * up; }
+
 // The halves of a 16-byte piece from element `by` on, zeros behind them (by >= 8: all zero).
 __device__ __forceinline__ u32x4 shift_down(u32x4 v, int by)
 {

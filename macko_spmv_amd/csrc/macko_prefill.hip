@@ -93,9 +93,8 @@ __global__ void __launch_bounds__(256) pack_silu_mul_kernel(const u32x4 *__restr
         u32x4 o = {0, 0, 0, 0};
         if (n < batch && p < pieces) {
             const u32x4 g = gate[(size_t)n * pieces + p], u = up[(size_t)n * pieces + p];
-            auto gated = [](float gv, float uv) { return gv / (1.0f + __expf(-gv)) * uv; };
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = pack2(gated(lo(g[e]), lo(u[e])), gated(hi(g[e]), hi(u[e])));
+            for (int e = 0; e < 4; ++e) o[e] = pack2(silu_mul(lo(g[e]), lo(u[e])), silu_mul(hi(g[e]), hi(u[e])));
         }
         packed[packed_piece(p, n, tiles)] = o;
     }

@@ -681,6 +681,40 @@ std::vector<at::Tensor> multiply_packed_several_hip(at::TensorList M_values, at:
     return Y;
 }
 
+// silu(G X) * (U X) for `batch` vectors in operand order, in operand order: matrices G and U of M_rows rows.  One
+// launch, or the products and the gate on their own where the matrices are better launched one by one.
+at::Tensor multiply_packed_silu_hip(at::TensorList M_values, at::TensorList M_deltas, at::TensorList M_row_indices, int64_t M_rows,
+                                    int64_t M_cols, const at::Tensor &packed, int64_t batch)
+{
+    TORCH_CHECK(M_values.size() == 2 && M_deltas.size() == 2 && M_row_indices.size() == 2, "two matrices, gate and up");
+    TORCH_CHECK(M_rows >= 64 && M_rows % 8 == 0, "M_rows must be a multiple of 8, 64 or more");
+    check_half_gpu(packed, "packed");
+    int64_t bytes = 0;
+    TORCH_CHECK(batch >= 1 && batch < (1ll << 31), "bad batch");
+    check_rc(macko_packed_bytes((int32_t)M_cols, (int32_t)batch, &bytes), "multiply_packed_silu");
+    TORCH_CHECK(packed.numel() * 2 == bytes, "packed must hold `batch` vectors of M_cols elements");
+    macko_packed_matrix matrices[2];
+    for (size_t i = 0; i < 2; ++i) {
+        check_macko_operands(M_values[i], M_deltas[i], M_row_indices[i], M_rows, M_cols);
+        TORCH_CHECK(M_values[i].device() == packed.device(), "the matrices and the vectors must live on one GPU");
+        matrices[i] = {M_values[i].data_ptr(), M_deltas[i].data_ptr(), M_row_indices[i].data_ptr<int>(), nullptr, (int32_t)M_rows,
+                       M_values[i].numel(), 0};
+    }
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(packed.device());
+    int32_t together = 0;
+    check_rc(macko_packed_together(matrices, 2, packed.data_ptr(), (int32_t)M_cols, (int32_t)batch, &together), "multiply_packed_silu");
+    if (!together) {
+        const int64_t rows[2] = {M_rows, M_rows};
+        const auto products = multiply_packed_several_hip(M_values, M_deltas, M_row_indices, rows, M_cols, packed, batch);
+        return pack_silu_mul_hip(products[0], products[1]);
+    }
+    at::Tensor out = packed_like(packed, M_rows, batch);
+    check_rc(macko_spmv_f16_packed_silu(&matrices[0], &matrices[1], packed.data_ptr(), out.data_ptr(), (int32_t)M_cols, (int32_t)batch,
+                                        current_stream()),
+             "multiply_packed_silu");
+    return out;
+}
+
 void check_caches(const at::Tensor &k_cache, const at::Tensor &v_cache, const at::Tensor &positions, int64_t batch, int64_t width)
 {
     check_half_gpu(k_cache, "k_cache");
@@ -778,6 +812,8 @@ TORCH_LIBRARY(macko_spmv, m)
           "Tensor packed, SymInt batch, Tensor? residual) -> Tensor");
     m.def("multiply_packed_several(Tensor[] M_values, Tensor[] M_deltas, Tensor[] M_row_indices, int[] M_rows, int M_cols, "
           "Tensor packed, SymInt batch) -> Tensor[]");
+    m.def("multiply_packed_silu(Tensor[] M_values, Tensor[] M_deltas, Tensor[] M_row_indices, int M_rows, int M_cols, "
+          "Tensor packed, int batch) -> Tensor");
     m.def("prefill_rope_append(Tensor(a!) q, Tensor k, Tensor v, Tensor cos_rows, Tensor sin_rows, Tensor positions, "
           "Tensor(b!) k_cache, Tensor(c!) v_cache) -> ()");
     m.def("prefill_attention(Tensor q, Tensor k_cache, Tensor v_cache, Tensor positions, float scale) -> Tensor");
@@ -811,6 +847,7 @@ TORCH_LIBRARY_IMPL(macko_spmv, CUDA, m)
     m.impl("pack_silu_mul", &pack_silu_mul_hip);
     m.impl("multiply_packed", &multiply_packed_hip);
     m.impl("multiply_packed_several", &multiply_packed_several_hip);
+    m.impl("multiply_packed_silu", &multiply_packed_silu_hip);
     m.impl("prefill_rope_append", &prefill_rope_append_hip);
     m.impl("prefill_attention", &prefill_attention_hip);
     m.impl("decompress", &decompress_hip);

@@ -70,6 +70,8 @@ at::Tensor multiply_packed_hip(const at::Tensor &M_values, const at::Tensor &M_d
 std::vector<at::Tensor> multiply_packed_several_hip(at::TensorList M_values, at::TensorList M_deltas,
                                                     at::TensorList M_row_indices, at::IntArrayRef M_rows,
                                                     int64_t M_cols, const at::Tensor &packed, int64_t batch);
+at::Tensor multiply_packed_silu_hip(at::TensorList M_values, at::TensorList M_deltas, at::TensorList M_row_indices, int64_t M_rows,
+                                    int64_t M_cols, const at::Tensor &packed, int64_t batch);
 void prefill_rope_append_hip(at::Tensor q, const at::Tensor &k, const at::Tensor &v, const at::Tensor &cos_rows,
                              const at::Tensor &sin_rows, const at::Tensor &positions, at::Tensor k_cache,
                              at::Tensor v_cache);

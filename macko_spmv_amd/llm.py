@@ -298,7 +298,11 @@ class Block(nn.Module):
         attended = ops.prefill_attention(q, k_cache, v_cache, positions, 1.0 / math.sqrt(att.head_dim))
         rows = product(att.o_proj, attended, rows)
         normed = ops.pack_rmsnorm(rows, self.post_attention_layernorm.weight, self.post_attention_layernorm.eps)
-        gated = ops.pack_silu_mul(*products(normed, mlp.gate_proj, mlp.up_proj))
+        gate, up = mlp.gate_proj, mlp.up_proj
+        if torch.compiler.is_compiling():
+            gated = ops.pack_silu_mul(product(gate, normed), product(up, normed))
+        else:
+            gated = ops.multiply_packed_silu([gate.c_0, up.c_0], [gate.c_1, up.c_1], [gate.c_2, up.c_2], gate.c_3, gate.c_4, normed, t)
         return product(mlp.down_proj, gated, rows).view(1, t, -1)
 
     def forward(self, x, cos, sin, positions, mask):

@@ -128,3 +128,34 @@ def test_long_sums_are_as_exact_as_the_other_kernel_s(batch, rows, cols, density
         wrong[1] += int((ops.multiply_packed(*one, packed, batch, None) != exact).sum())
     print("not the rounded result:", wrong, "of", batch * sum(rows), flush=True)
     assert wrong[1] > 100 and wrong[0] <= 1.25 * wrong[1]
+
+
+# the gate's product: pairs of units of four rows over row blocks of every kernel, columns that fill up no block of 64, vectors that
+# fill up no block of 16, one chunk and several, matrices of one density and of two that are launched one by one
+@pytest.mark.parametrize("rows,cols,batch,densities", [
+    (64, 64, 2, (0.5, 0.5)), (72, 100, 16, (0.3, 0.3)), (1376, 512, 17, (0.5, 0.5)), (1376, 512, 128, (0.1, 0.1)),
+    (2752, 1024, 33, (0.9, 0.85)), (5504, 2048, 100, (0.5, 0.5)), (11008, 4096, 128, (0.5, 0.5)), (11000, 1000, 130, (0.2, 0.2)),
+    (11016, 640, 250, (0.4, 0.4)), (11008, 1024, 128, (0.9, 0.05)), (4096, 4096, 5, (0.05, 0.05)), (28672, 512, 64, (0.1, 0.12)),
+    (1376, 512, 40, (0.0, 0.0))])
+@pytest.mark.parametrize("special", (False, True))
+def test_product_of_gate_and_up(rows, cols, batch, densities, special):
+    generator = torch.Generator(device="cuda")
+    generator.manual_seed(rows + cols + batch)
+    c = []
+    for density in densities:
+        w = torch.randn((rows, cols), device="cuda", generator=generator, dtype=torch.float16).mul_(0.1)
+        w.mul_(torch.rand((rows, cols), device="cuda", generator=generator) < density)
+        w[rows // 2] = 0
+        c.append(mk.compress(w))
+    x = torch.randn((batch, cols), device="cuda", generator=generator, dtype=torch.float16)
+    if special:
+        x[batch // 2, cols // 3] = float("inf")
+        x[0, cols - 1] = float("nan")
+    packed = _pack(ctypes.CDLL(mk.HIP_LIBRARY_PATH), x)
+    args = ([m[0] for m in c], [m[1] for m in c], [m[2] for m in c])
+    got = ops.multiply_packed_silu(*args, rows, cols, packed, batch)
+    for again in (ops.multiply_packed_silu(*args, rows, cols, packed, batch), mk.ops.multiply_packed_silu(*args, rows, cols, packed, batch)):
+        assert torch.equal(again.view(torch.int16), got.view(torch.int16))
+    want = ops.pack_silu_mul(*ops.multiply_packed_several(*args, [rows, rows], cols, packed, batch))
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(), want.nan_to_num())
