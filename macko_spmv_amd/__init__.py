@@ -75,6 +75,8 @@ ops = types.SimpleNamespace(**{name: _operator(name) for name in (
     "multiply_attention_axpby", "decode_rmsnorm", "decode_norm_matvec", "decode_rope_append", "decode_attention", "decode_silu_mul",
     "decode_rope_attention", "decode_rope_attention_parts", "pack_rmsnorm", "rmsnorm_rows", "pack_silu_mul", "multiply_packed",
     "multiply_packed_several", "multiply_packed_silu", "prefill_rope_append", "prefill_attention")})
+# a prompt's layer, or NotImplemented (Block.forward_fused in llm.py, which goes through `ops` then)
+eager_prefill_layer = _eager.prefill_layer
 
 
 @torch.library.register_fake("macko_spmv::multiply")

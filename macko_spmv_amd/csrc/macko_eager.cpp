@@ -354,6 +354,71 @@ PyObject *eager_compress(PyObject *, PyObject *const *args, Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// What Block.forward_fused (llm.py) does with the layer of a prompt, operator by operator, in one call: (x, cos, sin,
+// positions, k_cache, v_cache, scale, norm weight, eps, norm weight, eps, then the five of q, k, v, o, gate, up and down each).
+// A layer's nine launches take less time than Python takes between them where the layer is small: a prompt of 16 tokens,
+// 4 layers of dim 512 391 -> 347 us, 100 tokens, 3 layers of dim 1024 323 -> 285; 128 tokens at dim 4096 the same (699).
+PyObject *eager_prefill_layer(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    struct Linear {
+        const at::Tensor *values, *deltas, *row_indices;
+        int64_t rows, cols;
+    };
+    constexpr int kLinears = 7, kOthers = 11;
+    enum { Q, K, V, O, GATE, UP, DOWN };
+    EagerCall call;
+    const at::Tensor *x, *cos, *sin, *positions, *k_cache, *v_cache, *norm[2];
+    double scale, eps[2];
+    Linear m[kLinears];
+    if (n != kOthers + 5 * kLinears || !unobserved() || !call.tensor(args[0], x) || !call.tensor(args[1], cos) || !call.tensor(args[2], sin) ||
+        !call.tensor(args[3], positions) || !call.tensor(args[4], k_cache) || !call.tensor(args[5], v_cache) ||
+        !EagerCall::number(args[6], scale) || !call.tensor(args[7], norm[0]) || !EagerCall::number(args[8], eps[0]) ||
+        !call.tensor(args[9], norm[1]) || !EagerCall::number(args[10], eps[1]))
+        return not_implemented();
+    for (int i = 0; i < kLinears; ++i) {
+        PyObject *const *five = args + kOthers + 5 * i;
+        if (!call.tensor(five[0], m[i].values) || !call.tensor(five[1], m[i].deltas) || !call.tensor(five[2], m[i].row_indices) ||
+            !EagerCall::integer(five[3], m[i].rows) || !EagerCall::integer(five[4], m[i].cols))
+            return not_implemented();
+    }
+    const auto &normed = pack_rmsnorm_operator::get();
+    const auto &several = multiply_packed_several_operator::get();
+    const auto &rope = prefill_rope_append_operator::get();
+    const auto &attention = prefill_attention_operator::get();
+    const auto &product = multiply_packed_operator::get();
+    const auto &gate = multiply_packed_silu_operator::get();
+    if (x->dim() != 3 || x->size(0) != 1 || k_cache->dim() != 4 || v_cache->dim() != 4 || !normed.first() || !several.first() ||
+        !rope.first() || !attention.first() || !product.first() || !gate.first())
+        return not_implemented();
+    at::Tensor out;
+    {
+        WithoutGil released;
+        const int64_t tokens = x->size(1);
+        const at::Tensor rows = x->reshape({tokens, -1}).contiguous(), at = positions->contiguous();
+        const at::Tensor keys = k_cache->select(0, 0), values = v_cache->select(0, 0);
+        at::Tensor packed = normed(rows, *norm[0], eps[0]);
+        {
+            const at::Tensor v[3] = {*m[Q].values, *m[K].values, *m[V].values}, d[3] = {*m[Q].deltas, *m[K].deltas, *m[V].deltas},
+                             r[3] = {*m[Q].row_indices, *m[K].row_indices, *m[V].row_indices};
+            const int64_t n_rows[3] = {m[Q].rows, m[K].rows, m[V].rows};
+            const auto qkv = several(v, d, r, n_rows, m[Q].cols, packed, tokens);
+            rope(qkv[0], qkv[1], qkv[2], cos->reshape({tokens, -1}), sin->reshape({tokens, -1}), at, keys, values);
+            packed = attention(qkv[0], keys, values, at, scale);
+        }
+        const at::Tensor after = product(*m[O].values, *m[O].deltas, *m[O].row_indices, m[O].rows, m[O].cols, packed, tokens, rows);
+        packed = normed(after, *norm[1], eps[1]);
+        {
+            const at::Tensor v[2] = {*m[GATE].values, *m[UP].values}, d[2] = {*m[GATE].deltas, *m[UP].deltas},
+                             r[2] = {*m[GATE].row_indices, *m[UP].row_indices};
+            packed = gate(v, d, r, m[GATE].rows, m[GATE].cols, packed, tokens);
+        }
+        out = product(*m[DOWN].values, *m[DOWN].deltas, *m[DOWN].row_indices, m[DOWN].rows, m[DOWN].cols, packed, tokens, after).view({1, tokens, -1});
+    }
+    return to_python(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
 #define MACKO_EAGER(NAME, ...) {#NAME, (PyCFunction)(void (*)(void))&__VA_ARGS__, METH_FASTCALL, nullptr}
 PyMethodDef eager_functions[] = {
     MACKO_EAGER(compress, eager_compress),
@@ -380,6 +445,7 @@ PyMethodDef eager_functions[] = {
     MACKO_EAGER(multiply_packed_silu, eager<multiply_packed_silu_operator>),
     MACKO_EAGER(prefill_rope_append, eager<prefill_rope_append_operator>),
     MACKO_EAGER(prefill_attention, eager<prefill_attention_operator>),
+    MACKO_EAGER(prefill_layer, eager_prefill_layer),
     {nullptr, nullptr, 0, nullptr}};
 #undef MACKO_EAGER
 PyModuleDef eager_module = {PyModuleDef_HEAD_INIT, "libmacko_eager", nullptr, -1, eager_functions, nullptr, nullptr, nullptr, nullptr};

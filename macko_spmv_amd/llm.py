@@ -274,6 +274,15 @@ class Block(nn.Module):
         projection consumes is written in its operand order, and the residuals are added where the
         o and down projections round their results."""
         ops, att, mlp = macko_spmv.ops, self.self_attn, self.mlp
+        first, second, scale = self.input_layernorm, self.post_attention_layernorm, 1.0 / math.sqrt(att.head_dim)
+        if not torch.compiler.is_compiling():
+            # all of what follows in one call, for plain tensors that nothing else looks at
+            five = [part for linear in (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj)
+                    for part in (linear.c_0, linear.c_1, linear.c_2, linear.c_3, linear.c_4)]
+            out = macko_spmv.eager_prefill_layer(x, cos, sin, positions, att.k_cache, att.v_cache, scale, first.weight, first.eps,
+                                                 second.weight, second.eps, *five)
+            if out is not NotImplemented:
+                return out
         t = x.shape[1]
         rows = x.reshape(t, -1).contiguous()
         positions = positions.contiguous()
@@ -291,13 +300,13 @@ class Block(nn.Module):
                                                [linear.c_2 for linear in linears], [linear.c_3 for linear in linears],
                                                linears[0].c_4, packed, t)
 
-        normed = ops.pack_rmsnorm(rows, self.input_layernorm.weight, self.input_layernorm.eps)
+        normed = ops.pack_rmsnorm(rows, first.weight, first.eps)
         q, k, v = products(normed, att.q_proj, att.k_proj, att.v_proj)
         k_cache, v_cache = att.k_cache[0], att.v_cache[0]
         ops.prefill_rope_append(q, k, v, cos.reshape(t, -1), sin.reshape(t, -1), positions, k_cache, v_cache)
-        attended = ops.prefill_attention(q, k_cache, v_cache, positions, 1.0 / math.sqrt(att.head_dim))
+        attended = ops.prefill_attention(q, k_cache, v_cache, positions, scale)
         rows = product(att.o_proj, attended, rows)
-        normed = ops.pack_rmsnorm(rows, self.post_attention_layernorm.weight, self.post_attention_layernorm.eps)
+        normed = ops.pack_rmsnorm(rows, second.weight, second.eps)
         gate, up = mlp.gate_proj, mlp.up_proj
         if torch.compiler.is_compiling():
             gated = ops.pack_silu_mul(product(gate, normed), product(up, normed))

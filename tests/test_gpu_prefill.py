@@ -6,6 +6,7 @@ import ctypes
 import numpy as np
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import macko_spmv_amd as mk
 from macko_spmv_amd import llm
@@ -321,3 +322,85 @@ def test_norm_goes_the_general_way_where_the_kernel_cannot():
     y, tangent = torch.func.jvp(norm, (x,), (x,))
     # the norm does not change with its input's length, up to eps and the rounding of x times the weight
     assert torch.equal(y, norm(unaligned)) and tangent.abs().max() < 1e-2
+
+
+class _Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(func.__name__)
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.filterwarnings("ignore:.*overrid")
+@pytest.mark.parametrize("t,max_len,start", [(2, 80, 0), (19, 80, 40), (64, 80, 16)])
+@torch.no_grad()
+def test_layer_in_one_call(monkeypatch, t, max_len, start):
+    # the same operators one by one and in one call; what looks at operators, and a kernel that a program registers, sees them
+    model, _ = llm.build_model(0.4, sparse=True, n_layers=2, dim=256, hidden=712, n_heads=4, vocab=1000, max_len=max_len)
+    layers = model.model.layers
+    prompt = torch.randint(0, 1000, (1, t), device="cuda")
+    pos = torch.arange(start, start + t, device="cuda").repeat_interleave(2)[::2]   # not contiguous
+
+    def outputs():
+        for layer in layers:
+            layer.self_attn.k_cache.fill_(0.25)
+            layer.self_attn.v_cache.fill_(0.5)
+        logits = model(prompt, pos)
+        return [logits] + [c.clone() for layer in layers for c in (layer.self_attn.k_cache, layer.self_attn.v_cache)]
+
+    taken = []
+    one_call = mk.eager_prefill_layer
+
+    def watched(*args):
+        out = one_call(*args)
+        taken.append(out is not NotImplemented)
+        return out
+
+    monkeypatch.setattr(mk, "eager_prefill_layer", watched)
+    got = outputs()
+    assert taken == [True, True]
+    with _Seen() as seen:
+        observed = outputs()
+    assert taken == [True, True, False, False]
+    monkeypatch.setattr(mk, "eager_prefill_layer", lambda *args: NotImplemented)
+    want = outputs()
+    for a, b, c in zip(got, want, observed):
+        assert torch.equal(a, b) and torch.equal(a, c)
+    assert sum(name.startswith("multiply_packed_silu") for name in seen.names) == 2
+    monkeypatch.setattr(mk, "eager_prefill_layer", watched)
+    for key in ("Autograd", "CUDA"):
+        library, calls = torch.library.Library("macko_spmv", "IMPL"), []
+        try:
+            library.impl("prefill_attention", lambda q, *rest: (calls.append(1), mk._packed_like(q, q.shape[1], q.shape[0]).zero_())[1], key,
+                         allow_override=True)
+            model(prompt, pos)
+        finally:
+            library._destroy()
+        assert len(calls) == 2, key
+
+
+def test_layer_in_one_call_refuses_what_the_operators_refuse():
+    model, _ = llm.build_model(0.4, sparse=True, n_layers=1, dim=256, hidden=704, n_heads=2, vocab=1000, max_len=48)
+    layer = model.model.layers[0]
+    x, pos = torch.zeros(1, 5, 256, device="cuda").half(), torch.arange(5, device="cuda")
+    table = torch.ones(1, 1, 5, 128, device="cuda").half()
+    with torch.no_grad():
+        assert torch.isfinite(layer.forward_fused(x, table, table, pos)).all()
+        for args in ((x, table, table, pos[:4]), (x, table[..., :64], table, pos), (x.float(), table, table, pos), (x, table, table, pos.int())):
+            with pytest.raises(RuntimeError):
+                layer.forward_fused(*args)
+    assert mk.eager_prefill_layer(x.cpu(), table, table, pos) is NotImplemented
+
+
+def test_product_of_gate_and_up_is_an_operator():
+    w = torch.randn(72, 64, device="cuda").half()
+    c, x = mk.compress(w), torch.randn(5, 64, device="cuda").half()
+    ops = torch.ops.macko_spmv
+    packed = ops.pack_rmsnorm(x, torch.ones(64, device="cuda").half(), 1e-5)
+    torch.library.opcheck(ops.multiply_packed_silu, ([c[0]] * 2, [c[1]] * 2, [c[2]] * 2, 72, 64, packed, 5))
+    for rows, batch, n in ((72, 17, 2), (56, 5, 2), (72, 5, 1), (76, 5, 2)):
+        with pytest.raises(RuntimeError):
+            ops.multiply_packed_silu([c[0]] * n, [c[1]] * n, [c[2]] * n, rows, 64, packed, batch)
