@@ -20,7 +20,7 @@
 // of X per row block; the gather kernels read LDS once per entry for a few vectors and stream the
 // matrix again for the next few.  Measured on 11008 x 4096 at density 0.5, 128 vectors: 341 us through the
 // gather kernels in groups of eight (17 TFLOP/s), 27.4 here (211 TFLOP/s of stored entries, twice that
-// on the matrix cores; spmv_pipe_kernel below takes such products now, 25.3 with packing, 27.9 here).  What bounds it: no unit alone.  Of the 54500 cycles a wave of that launch lives
+// on the matrix cores; spmv_pipe_kernel below takes such products now, 23.6 with packing, 27.9 here).  What bounds it: no unit alone.  Of the 54500 cycles a wave of that launch lives
 // the vector units are busy 25000 (decoding), LDS 28300 (12400 of them bank conflicts) and the matrix cores
 // 12300, by the counters; waves wait for 40 % of their cycles, for one another and for X out of L2.
 //
@@ -191,8 +191,23 @@ __device__ __forceinline__ void finish_tiles(const TileArgs<SOURCES> &a, u32 red
     const int lane = threadIdx.x & (kWave - 1), wave = uniform(threadIdx.x >> 6), sub = lane & 15, quarter = lane >> 4;
     for (int tile = wave; tile < n_tiles; tile += kTileWaves) {
         float4v sum = float4v{0.f, 0.f, 0.f, 0.f};
-        for (int p = 0; p < parts; ++p)
-            sum += __builtin_bit_cast(float4v, *(lds_w32x4)(uintptr_t)(red + (u32)(tile * parts + p) * 1024 + (u32)lane * 16));
+        u32 at = red + (u32)(tile * parts) * 1024 + (u32)lane * 16;
+        // Up to eight parts are read together, and added one after the other as before: a read behind each addition was what a
+        // launch of few vectors ended with (4096 x 4096, 8 vectors at 0.5: 8.76 us, four together 8.48, eight 8.43; 5 at 0.2
+        // 6.05, 5.72, 5.65; 777 x 3333, 8 at 0.25 7.44, 7.13, 7.07; 11008 x 4096, 8 at 0.5 16.16, 15.89, 15.82).
+        auto add = [&](auto count) __attribute__((always_inline)) {
+            constexpr int N = decltype(count)::value;
+            float4v some[N];
+#pragma unroll
+            for (int p = 0; p < N; ++p) some[p] = __builtin_bit_cast(float4v, *(lds_w32x4)(uintptr_t)(at + 1024 * p));
+#pragma unroll
+            for (int p = 0; p < N; ++p) sum += some[p];
+            at += 1024 * N;
+        };
+        int left = parts;  // 2, 4, 8 or 16
+        for (; left >= 8; left -= 8) add(index_constant<8>{});
+        if (left & 4) add(index_constant<4>{});
+        if (left & 2) add(index_constant<2>{});
         const int r = tile / vector_tiles;
         const int n = vector0 + (tile - r * vector_tiles) * 16 + sub;
         const int row = row0 + r * 16 + quarter * 4;
