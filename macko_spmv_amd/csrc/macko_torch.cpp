@@ -813,7 +813,7 @@ TORCH_LIBRARY(macko_spmv, m)
     m.def("multiply_packed_several(Tensor[] M_values, Tensor[] M_deltas, Tensor[] M_row_indices, int[] M_rows, int M_cols, "
           "Tensor packed, SymInt batch) -> Tensor[]");
     m.def("multiply_packed_silu(Tensor[] M_values, Tensor[] M_deltas, Tensor[] M_row_indices, int M_rows, int M_cols, "
-          "Tensor packed, int batch) -> Tensor");
+          "Tensor packed, SymInt batch) -> Tensor");
     m.def("prefill_rope_append(Tensor(a!) q, Tensor k, Tensor v, Tensor cos_rows, Tensor sin_rows, Tensor positions, "
           "Tensor(b!) k_cache, Tensor(c!) v_cache) -> ()");
     m.def("prefill_attention(Tensor q, Tensor k_cache, Tensor v_cache, Tensor positions, float scale) -> Tensor");

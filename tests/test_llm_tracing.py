@@ -2,7 +2,9 @@
 Python may not break a graph, and a traced graph computes what the modules compute."""
 import pytest
 import torch
+from torch._dynamo.source import ConstantSource
 from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.symbolic_shapes import DimDynamic, ShapeEnv
 
 from macko_spmv_amd import llm
 
@@ -38,6 +40,21 @@ def _operators(function, *args):
     torch.compile(function, fullgraph=True, backend=backend)(*args)
     assert len(graphs) == 1
     return [str(n.target).split(".")[1] for n in graphs[0].graph.nodes if str(n.target).startswith("macko_spmv.")]
+
+
+def test_a_symbolic_number_of_tokens_stays_symbolic():
+    # fake tensors alone, nothing compiled or recorded: the operators that an eager prompt goes through
+    shapes = ShapeEnv()
+    mode = FakeTensorMode(allow_non_fake_inputs=True, shape_env=shapes)
+    layer = _fake_model(mode).model.layers[0]
+    with mode, torch.no_grad(), torch.device("cuda"):
+        # 19 is one number of tokens, which nothing may hold on to
+        tokens = shapes.create_symintnode(shapes.create_symbol(19, source=ConstantSource("tokens"), dynamic_dim=DimDynamic.DYNAMIC), hint=19)
+        x = torch.empty((1, tokens, 256), dtype=torch.float16)
+        table, positions = torch.empty((1, 1, tokens, 128), dtype=torch.float16), torch.empty((tokens,), dtype=torch.long)
+        assert layer.takes_fused(x)
+        out = layer.forward_fused(x, table, table, positions)
+    assert isinstance(out.shape[1], torch.SymInt) and not shapes.replacements
 
 
 def test_decoder_compiles_as_one_graph():
