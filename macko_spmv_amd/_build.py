@@ -165,12 +165,14 @@ def verify_fixed_registers(verbose=False, extra_flags=()):
 RESOURCE_REMARKS = "-Rpass-analysis=kernel-resource-usage"
 # keeps a row of k and eight pieces of v per thread in flight and spills 31 registers of them; measured as it is
 KNOWN_TO_SPILL = ("attention_kernelILb1ELi128E",)
+# kernels of which two workgroups of 16 waves share a compute unit: part of the name -> most vector registers a wave
+VGPR_LIMITS = {"spmv_pipe_kernelILi1E": 64}
 
 
 def check_kernel_resources(remarks):
     """`remarks`: what the compiler prints with RESOURCE_REMARKS.  Returns the number of kernels; raises if
-    one of them uses scratch memory, spills vector registers or has a dynamic stack (scalar registers spill to
-    lanes of a vector register)."""
+    one of them uses scratch memory, spills vector registers, has a dynamic stack (scalar registers spill to
+    lanes of a vector register) or uses more vector registers than VGPR_LIMITS has for it."""
     kernel, checked = None, 0
     for line in remarks.splitlines():
         m = re.search(r"remark:\s+([\w ]+?)(?: \[[^\]]*\])?: (\S+)", line)
@@ -184,6 +186,8 @@ def check_kernel_resources(remarks):
             if any(known in kernel for known in KNOWN_TO_SPILL):
                 continue
             raise RuntimeError(f"{name}: {value} in {kernel}")
+        elif name == "VGPRs" and any(part in kernel and int(value) > most for part, most in VGPR_LIMITS.items()):
+            raise RuntimeError(f"{name}: {value} in {kernel}, which leaves room for one workgroup")
     if checked == 0:
         raise RuntimeError("the compiler names no kernels; the resource check is stale")
     return checked

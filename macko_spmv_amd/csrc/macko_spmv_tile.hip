@@ -626,8 +626,11 @@ constexpr int kPipeLanes = 16;         // lanes per row of a pass
 // the next chunk, and loads return in order: with two units on the way the products waited for them more than half of their time
 // (11008 x 4096, 128 vectors at 0.5: 20.98 us, with three 20.56; 64 vectors at 0.1 12.9, with four 12.1).  64 and more
 // sums a lane leave room for three; where 8 entries a lane do, chunks of 640 columns in whole rounds of two are worth more
-// (0.15: 17.4, 18.7 with three).
-constexpr int pipe_depth(int wave_tiles, int entries) { return entries == 16 ? 3 : wave_tiles > 2 ? 2 : 4; }
+// (0.15: 17.4, 18.7 with three).  Up to 32 vectors it is two: with those (and two sets of sums) a wave needs 64 registers at
+// most, so that two workgroups of short chunks share a compute unit (VGPR_LIMITS, _build.py).  1226 products of 17 to 32 vectors, three or
+// four units and one workgroup, two and two: above 12288 rows 19 % slower in the mean up to 250 columns (28379 x 244, 21 vectors
+// at 0.17 8.43 and 7.27 us), 3 to 4 % from 250 to 4000 columns.
+constexpr int pipe_depth(int wave_tiles, int entries) { return wave_tiles == 1 ? 2 : entries == 16 ? 3 : wave_tiles > 2 ? 2 : 4; }
 constexpr int pipe_chunk_step(int wave_tiles, int entries) { return 32 * kPipeParts * pipe_depth(wave_tiles, entries); }
 // Column parts of a result: two waves', of each of them two where there are registers for it (sets), and blocks of chunks,
 // whose sums the scattering waves keep and add up: as many as spmv_tile_kernel has for the same product (4 or 8), so that a
@@ -636,7 +639,7 @@ constexpr int pipe_chunk_step(int wave_tiles, int entries) { return 32 * kPipePa
 // 0.3, 64 vectors 183, 126, 123.  A block's end is a barrier and 48 KB through LDS: 11008 x 4096 at 0.5, 128 vectors 22.5 us
 // without and 22.9 with two blocks when that was measured.  One chunk (up to about 700 columns) has no
 // blocks: at most 11 matrix instructions a sum, where one of 4096 columns in eight parts has 16 (600 columns: 49, 44).
-constexpr int pipe_sets(int wave_tiles, int entries) { return wave_tiles > 2 ? 1 : entries == 16 ? 3 : 2; }  // a divisor of the depth
+constexpr int pipe_sets(int wave_tiles, int entries) { return wave_tiles > 2 ? 1 : wave_tiles == 2 && entries == 16 ? 3 : 2; }  // a divisor of the depth
 constexpr int pipe_pad(int entries) { return entries * 16 + 8; }  // columns between rows; 16-byte aligned, rows on other banks
 
 template <int NTW, int E, bool SEVERAL>

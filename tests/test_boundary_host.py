@@ -214,6 +214,45 @@ def test_kernel_resource_check_refuses_scratch_and_stacks():
             _build.check_kernel_resources(bad)
 
 
+def test_kernels_of_which_two_workgroups_share_a_compute_unit(tmp_path):
+    import struct
+    import subprocess
+
+    from macko_spmv_amd import _build
+
+    def remarks(name, registers):
+        lines = [f"Function Name: {name}", f"VGPRs: {registers}", "ScratchSize [bytes/lane]: 0"]
+        return "\n".join(f"k.hip:84:1: remark:     {line} [-Rpass-analysis=kernel-resource-usage]" for line in lines)
+
+    name = "_ZN5macko16spmv_pipe_kernelILi1ELi8ELb0EEEvv"
+    assert _build.check_kernel_resources(remarks(name, 64) + "\n" + remarks(name.replace("ILi1E", "ILi2E"), 100)) == 2
+    with pytest.raises(RuntimeError):
+        _build.check_kernel_resources(remarks(name, 65))
+
+    # what the library holds: the code objects of its bundles say how many registers a kernel has
+    with open(_build.lib_paths()[0], "rb") as f:
+        library = f.read()
+    magic, found, at = b"__CLANG_OFFLOAD_BUNDLE__", {}, 0
+    while (at := library.find(magic, at)) >= 0:
+        place = at + len(magic) + 8
+        for _ in range(struct.unpack_from("<Q", library, at + len(magic))[0]):
+            offset, size, length = struct.unpack_from("<QQQ", library, place)
+            target = library[place + 24:place + 24 + length].decode()
+            place += 24 + length
+            if "gfx950" not in target:
+                continue
+            (tmp_path / "code.o").write_bytes(library[at + offset:at + offset + size])
+            notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", str(tmp_path / "code.o")], stdout=subprocess.PIPE, text=True,
+                                   check=True).stdout
+            names, counts = re.findall(r"^ +\.name: +(_Z\S+)$", notes, re.M), re.findall(r"^ +\.vgpr_count: +(\d+)$", notes, re.M)
+            assert len(names) == len(counts)
+            found.update(zip(names, map(int, counts)))
+        at = place
+    for part, most in _build.VGPR_LIMITS.items():
+        these = {kernel: count for kernel, count in found.items() if part in kernel}
+        assert len(these) == 4 and max(these.values()) <= most, these
+
+
 def test_operator_library_loads_without_python(tmp_path):
     """A program without Python has the operators by loading libmacko_torch.so; what needs Python is libmacko_eager.so."""
     import subprocess
