@@ -623,14 +623,15 @@ constexpr int kPipeParts = 2;          // of the columns, per group of vectors
 constexpr int kPipeGroups = 2;
 constexpr int kPipeLanes = 16;         // lanes per row of a pass
 // Units of 32 columns of X a wave has in flight; chunks are whole rounds of them.  A unit of X is asked for behind the entries of
-// the next chunk, and loads return in order: with two units on the way the products waited for them more than half of their time
-// (11008 x 4096, 128 vectors at 0.5: 20.98 us, with three 20.56; 64 vectors at 0.1 12.9, with four 12.1).  64 and more
-// sums a lane leave room for three; where 8 entries a lane do, chunks of 640 columns in whole rounds of two are worth more
-// (0.15: 17.4, 18.7 with three).  Up to 32 vectors it is two: with those (and two sets of sums) a wave needs 64 registers at
+// the next chunk, and loads return in order: with two units on the way the products wait for them (11008 x 4096, 128 vectors at 0.5:
+// 20.98 us, with three 20.56; 33 to 64 vectors of 16 entries a lane and more than 4000 columns, 102 products of 6000 rows and more: 10 to 13 %
+// slower with two).  Two where a lane has 8 entries: chunks of up to 640 columns in whole rounds of 128 are worth more
+// (128 vectors at 0.15: 17.4 us, 18.7 with three; 33 to 64 vectors with four, in rounds of 256, 640 columns in two chunks 11 % slower, 128 columns 4 to 6 %,
+// from 641 columns on the same within 2 %).  Up to 32 vectors two as well: with those (and two sets of sums) a wave needs 64 registers at
 // most, so that two workgroups of short chunks share a compute unit (VGPR_LIMITS, _build.py).  1226 products of 17 to 32 vectors, three or
 // four units and one workgroup, two and two: above 12288 rows 19 % slower in the mean up to 250 columns (28379 x 244, 21 vectors
 // at 0.17 8.43 and 7.27 us), 3 to 4 % from 250 to 4000 columns.
-constexpr int pipe_depth(int wave_tiles, int entries) { return wave_tiles == 1 ? 2 : entries == 16 ? 3 : wave_tiles > 2 ? 2 : 4; }
+constexpr int pipe_depth(int wave_tiles, int entries) { return wave_tiles > 1 && entries == 16 ? 3 : 2; }
 constexpr int pipe_chunk_step(int wave_tiles, int entries) { return 32 * kPipeParts * pipe_depth(wave_tiles, entries); }
 // Column parts of a result: two waves', of each of them two where there are registers for it (sets), and blocks of chunks,
 // whose sums the scattering waves keep and add up: as many as spmv_tile_kernel has for the same product (4 or 8), so that a
