@@ -1148,8 +1148,9 @@ bool choose_pipe_shape(TileShape *shape, int rows, int cols, long long padded, i
         const int pad = pipe_pad(e);
         int chunk = ((info.max_lds_bytes - 2 * pad) / (2 * 16 * kPipeRowTiles) - 2 * pad) / 2 / step * step;
         chunk = chunk < whole ? chunk : whole;
+        const int held = (cols + 127) / 128 * 128;  // a chunk may end a round of units behind the last column, and a pass has no entries there
         auto fits = [&](int c) {
-            const double mean = c * density;
+            const double mean = (c < held ? c : held) * density;
             return mean + 3.0 * std::sqrt(mean * (density < 1.0 ? 1.0 - density : 0.0)) + e + 8 <= kPipeLanes * e;
         };
         while (chunk > 0 && !fits(chunk)) chunk -= step;

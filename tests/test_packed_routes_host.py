@@ -76,8 +76,10 @@ def test_long_sums_of_both_kernels(routes, batch, rows, cols, density):
 
 @pytest.mark.parametrize("rows,cols,batch,density,kernel,chunk", [
     (26268, 576, 41, 0.128, "spmv_pipe_kernel<2,8,false>", 640), (16546, 640, 39, 0.085, "spmv_pipe_kernel<2,8,false>", 640),
-    (28369, 110, 64, 0.2, "spmv_pipe_kernel<2,8,false>", 128), (28379, 244, 21, 0.17, "spmv_pipe_kernel<1,8,false>", 256)])
+    (28369, 110, 64, 0.2, "spmv_pipe_kernel<2,8,false>", 128), (28379, 244, 21, 0.17, "spmv_pipe_kernel<1,8,false>", 256),
+    # rows that fill a pass, whose last round of units they do not
+    (9831, 242, 64, 0.61, "spmv_pipe_kernel<2,16,false>", 384), (25680, 242, 138, 0.758, "spmv_pipe_kernel<4,16,false>", 384)])
 def test_columns_that_fit_into_one_chunk(routes, rows, cols, batch, density, kernel, chunk):
     name, _, lds = routes(cols, batch, [(rows, int(rows * cols * density) // 8 * 8)])[0].split(":")
-    pad = 2 * (16 * int(kernel[19]) + 8)   # bytes behind a row; 48 rows, twice, and one pad in front
+    pad = 2 * (16 * int(kernel.split(",")[1]) + 8)   # bytes behind a row; 48 rows, twice, and one pad in front
     assert name == kernel and int(lds) == pad + 96 * (2 * chunk + pad)
