@@ -1109,10 +1109,10 @@ bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, in
     return found;
 }
 
-// The estimated time in us of a launch of spmv_pipe_kernel.  The terms were fitted to 839 products of packed vectors (1500
-// to 28000 rows, 256 to 11000 columns, densities 0.05 to 0.6, 17 to 256 vectors; 6 % off in the median, 17 % for one in
-// ten): per round of workgroups, per block's end, per chunk and pass (of 16 entries a lane it costs more than one of 8) and
-// per column and vector.
+// The estimated time in us of a launch of spmv_pipe_kernel, for the choice between it and spmv_tile_kernel, whose estimate it
+// is compared with: per round of workgroups, per block's end, per chunk and pass (of 16 entries a lane it costs more than one of
+// 8) and per column and vector.  Fitted, to what decides rather than to the time itself (8 % off in the median), to 7000 products
+// of packed vectors that both kernels can do: 64 to 28672 rows and columns, densities 0.04 to 0.95, 17 to 256 vectors.
 double pipe_us(const TileShape &s, int cols, int batch, const DeviceInfo &info, double passes)
 {
     const int vectors = 16 * kPipeGroups * s.wave_tiles;
@@ -1120,8 +1120,11 @@ double pipe_us(const TileShape &s, int cols, int batch, const DeviceInfo &info, 
     const double full = (double)((s.row_blocks * blocks + info.compute_units - 1) / info.compute_units);
     const int n_chunks = (cols + s.chunk - 1) / s.chunk;
     const double ends = (n_chunks - 1) / pipe_block_chunks(s, n_chunks);
-    const double products = s.wave_tiles == 4 ? 1.31 : s.wave_tiles == 2 ? 0.59 : 0.43;   // 512 columns
-    return full * (3.6 + 0.13 * ends + n_chunks * (s.lane_entries == 8 ? 0.315 : 0.47) * passes + cols / 512.0 * products);
+    const double round = s.wave_tiles == 4 ? 4.15 : s.wave_tiles == 2 ? 3.9 : 3.8;
+    const double products = s.wave_tiles == 4 ? 1.28 : s.wave_tiles == 2 ? 0.75 : 0.6;   // 512 columns
+    // two units of X on the way wait longer where X leaves L2 (4962 x 20544 at 0.1, 38 vectors 53.9 us, by the other kernel 39.7)
+    const double columns = cols + (s.lane_entries == 8 && cols > 8192 ? 0.5 * (cols - 8192) : 0.0);
+    return full * (round + 0.17 * ends + n_chunks * (s.lane_entries == 8 ? 0.22 : 0.38) * passes + columns / 512.0 * products);
 }
 
 // The shape of a launch of spmv_pipe_kernel and its estimated time.  group_shift: spmv_tile_kernel's, whose parts of a sum it has.
@@ -1169,16 +1172,18 @@ constexpr double kTileUsPerCycle = 1.06 / 2400.0;
 
 // The kernel and the shape of a launch, and its estimated time in us (without packing; at 2.4 GHz).  Right to about 10 %
 // where it decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1:
-// 24.4, 21).  Of the 839 products above the pipe kernel is taken for 69 %; what is taken is 0.3 % behind the
-// better of the two in the mean, more than 3 % for 4 % of them (15 % at most).
+// 24.4, 21).  several: of more than one matrix, which spmv_tile_kernel looks up row by row; its estimate is that for one
+// (up to 64 vectors, 280 launches of two and three matrices of 512 to 4096 columns: what is taken is 0.1 % behind the better one, with the line
+// for one matrix 1 %).
 bool choose_shape(TileShape *shape, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, double *us,
-                  int most_shift = 2)
+                  int most_shift = 2, bool several = false)
 {
     double cycles = 0.0, pipe_us = 0.0;
     if (!choose_tile_shape(shape, rows, cols, padded, batch, packed, info, &cycles, most_shift)) return false;
     *us = cycles * kTileUsPerCycle;
     TileShape pipe;
-    if (packed && choose_pipe_shape(&pipe, rows, cols, padded, batch, shape->group_shift, info, &pipe_us) && pipe_us < 0.97 * *us) {
+    if (packed && choose_pipe_shape(&pipe, rows, cols, padded, batch, shape->group_shift, info, &pipe_us) &&
+        pipe_us < (several && pipe.wave_tiles <= 2 ? 1.03 : 0.97) * *us) {
         *shape = pipe;
         *us = pipe_us;
     }
@@ -1324,7 +1329,7 @@ int packed_product(const macko_packed_matrix *matrices, int n, const void *packe
         for (int k = 1; k < used; ++k) least = rows_of(k) < rows_of(least) ? k : least;
         if (choose_tile_shape(&shape, rows_of(least), cols, a.source[least].padded, batch, true, info, &us)) most_shift = shape.group_shift;
     }
-    if (!choose_shape(&shape, a.rows, cols, padded, batch, true, info, &us, most_shift)) return MACKO_E_INVALID_ARGUMENT;
+    if (!choose_shape(&shape, a.rows, cols, padded, batch, true, info, &us, most_shift, used > 1)) return MACKO_E_INVALID_ARGUMENT;
     const bool apart = used > 1 && gated_out == nullptr && better_apart(a, used, shape, info);
     if (together != nullptr) {
         *together = apart ? 0 : 1;

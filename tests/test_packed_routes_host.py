@@ -83,3 +83,22 @@ def test_columns_that_fit_into_one_chunk(routes, rows, cols, batch, density, ker
     name, _, lds = routes(cols, batch, [(rows, int(rows * cols * density) // 8 * 8)])[0].split(":")
     pad = 2 * (16 * int(kernel.split(",")[1]) + 8)   # bytes behind a row; 48 rows, twice, and one pad in front
     assert name == kernel and int(lds) == pad + 96 * (2 * chunk + pad)
+
+
+# Products between the two kernels: few rows in each workgroup, few columns, far more columns than rows.
+# us, by the kernel of two roles and by the other one: 652 x 79, 215 vectors 4.89 and 4.04, 2164 x 221, 125 5.30 and 4.17, 4962 x 20544, 38
+# 53.9 and 39.7, 5466 x 16693, 38 44.4 and 33.9.
+@pytest.mark.parametrize("rows,cols,batch,density,kernel", [
+    (652, 79, 215, 0.914, "spmv_tile_kernel"), (1071, 191, 37, 0.3, "spmv_tile_kernel"), (2164, 221, 125, 0.389, "spmv_tile_kernel"),
+    (2904, 293, 86, 0.448, "spmv_tile_kernel"), (4962, 20544, 38, 0.104, "spmv_tile_kernel"), (5466, 16693, 38, 0.113, "spmv_tile_kernel"),
+    (8061, 13857, 23, 0.216, "spmv_tile_kernel"),
+    (11008, 4096, 128, 0.5, "spmv_pipe_kernel"), (28672, 1024, 64, 0.1, "spmv_pipe_kernel"), (6149, 1024, 205, 0.507, "spmv_pipe_kernel"),
+    (11514, 64, 172, 0.082, "spmv_pipe_kernel"), (26429, 225, 36, 0.695, "spmv_pipe_kernel")])
+def test_the_choice_holds_for_products_of_any_size(routes, rows, cols, batch, density, kernel):
+    assert routes(cols, batch, [(rows, int(rows * cols * density) // 8 * 8)])[0].startswith(kernel)
+
+
+def test_several_matrices_leave_the_kernel_that_looks_them_up_row_by_row_sooner(routes):
+    # gate and up of dim 1024, 17 vectors at 0.1: 5.26 us by the kernel of two roles, 5.61
+    sizes = [(2752, 2752 * 1024 // 10 // 8 * 8)] * 2
+    assert routes(1024, 17, sizes)[0].startswith("spmv_pipe_kernel")
