@@ -633,13 +633,14 @@ constexpr int kPipeLanes = 16;         // lanes per row of a pass
 // at 0.17 8.43 and 7.27 us), 3 to 4 % from 250 to 4000 columns.
 constexpr int pipe_depth(int wave_tiles, int entries) { return wave_tiles > 1 && entries == 16 ? 3 : 2; }
 constexpr int pipe_chunk_step(int wave_tiles, int entries) { return 32 * kPipeParts * pipe_depth(wave_tiles, entries); }
-// Column parts of a result: two waves', of each of them two where there are registers for it (sets), and blocks of chunks,
-// whose sums the scattering waves keep and add up: as many as spmv_tile_kernel has for the same product (4 or 8), so that a
-// sum in fp32 is as exact.  Results of 10^5 that are not the exact one rounded to fp16, with the two waves' parts alone, by
-// spmv_tile_kernel, and here (4096 columns): 11008 rows at 0.5, 128 vectors 190, 159, 158; 3 x 4096 rows 188, 128, 127; 11008 rows at
-// 0.3, 64 vectors 183, 126, 123.  A block's end is a barrier and 48 KB through LDS: 11008 x 4096 at 0.5, 128 vectors 22.5 us
-// without and 22.9 with two blocks when that was measured.  One chunk (up to about 700 columns) has no
-// blocks: at most 11 matrix instructions a sum, where one of 4096 columns in eight parts has 16 (600 columns: 49, 44).
+// Column parts of a result: two waves', of each of them two or three where there are registers for it (sets), and blocks of chunks,
+// whose sums the scattering waves keep and add up: with several chunks at least as many as spmv_tile_kernel has for the same product
+// (4 or 8; 12 with three sets in two blocks), so that a sum in fp32 is as exact.  Results of 10^5 that are not the exact one rounded to fp16, with
+// the two waves' parts alone, by spmv_tile_kernel, and here (4096 columns): 11008 rows at 0.5, 128 vectors 190, 159, 158; 3 x 4096 rows
+// 188, 128, 127; 11008 rows at 0.3, 64 vectors 183, 126, 123.  A block's end is a barrier and 48 KB through LDS: 11008 x 4096 at
+// 0.5, 128 vectors 22.5 us without and 22.9 with two blocks when that was measured.  One chunk (up to 640 columns with 8 entries a
+// lane, 512 with 16) has no blocks: up to ten matrix instructions a part (pipe_us says what that is worth).  One chunk in two blocks, the first
+// one's sums through LDS behind the dense columns, was as exact as the other kernel and took 10 to 17 % longer.
 constexpr int pipe_sets(int wave_tiles, int entries) { return wave_tiles > 2 ? 1 : wave_tiles == 2 && entries == 16 ? 3 : 2; }  // a divisor of the depth
 constexpr int pipe_pad(int entries) { return entries * 16 + 8; }  // columns between rows; 16-byte aligned, rows on other banks
 
@@ -1109,10 +1110,21 @@ bool choose_tile_shape(TileShape *best, int rows, int cols, long long padded, in
     return found;
 }
 
+// Parts of a sum in a launch of spmv_pipe_kernel.
+int pipe_parts(const TileShape &s, int cols)
+{
+    const int n_chunks = (cols + s.chunk - 1) / s.chunk, block = pipe_block_chunks(s, n_chunks);
+    return kPipeParts * pipe_sets(s.wave_tiles, s.lane_entries) * ((n_chunks + block - 1) / block);
+}
+
 // The estimated time in us of a launch of spmv_pipe_kernel, for the choice between it and spmv_tile_kernel, whose estimate it
 // is compared with: per round of workgroups, per block's end, per chunk and pass (of 16 entries a lane it costs more than one of
 // 8) and per column and vector.  Fitted, to what decides rather than to the time itself (8 % off in the median), to 7000 products
 // of packed vectors that both kernels can do: 64 to 28672 rows and columns, densities 0.04 to 0.95, 17 to 256 vectors.
+// Where its sums have fewer parts than the other kernel's (one chunk; few chunks and more than 64 vectors) and a part is more than two
+// matrix instructions, 4 to 30 % more of its results are not the exact one rounded to fp16.  That has to be worth something: the
+// estimate is higher there (4963 x 570 at 0.18, 82 vectors, goes to the other kernel: 7.2 us, 5.9 here).  What it leaves here takes 23 % less
+// time than there, and over 7000 products 1.5 % more results are not the rounded ones than by the other kernel alone, 1.9 % without it.
 double pipe_us(const TileShape &s, int cols, int batch, const DeviceInfo &info, double passes)
 {
     const int vectors = 16 * kPipeGroups * s.wave_tiles;
@@ -1120,6 +1132,11 @@ double pipe_us(const TileShape &s, int cols, int batch, const DeviceInfo &info, 
     const double full = (double)((s.row_blocks * blocks + info.compute_units - 1) / info.compute_units);
     const int n_chunks = (cols + s.chunk - 1) / s.chunk;
     const double ends = (n_chunks - 1) / pipe_block_chunks(s, n_chunks);
+    const int parts = pipe_parts(s, cols);
+    if (parts < kTileWaves >> s.group_shift && cols > 64 * parts) {
+        const double columns = n_chunks > 1 ? n_chunks * s.chunk : (cols + 127) / 128 * 128;
+        return 0.93 + full * (3.25 + 0.35 * ends + n_chunks * (s.lane_entries == 8 ? 0.31 : 0.56) * passes + columns / 512.0 * (0.31 + 0.26 * s.wave_tiles));
+    }
     const double round = s.wave_tiles == 4 ? 4.15 : s.wave_tiles == 2 ? 3.9 : 3.8;
     const double products = s.wave_tiles == 4 ? 1.28 : s.wave_tiles == 2 ? 0.75 : 0.6;   // 512 columns
     // two units of X on the way wait longer where X leaves L2 (4962 x 20544 at 0.1, 38 vectors 53.9 us, by the other kernel 39.7)
@@ -1158,7 +1175,8 @@ bool choose_pipe_shape(TileShape *shape, int rows, int cols, long long padded, i
         };
         while (chunk > 0 && !fits(chunk)) chunk -= step;
         if (chunk < (e == 8 ? 512 : 384) && chunk < whole) continue;
-        const int n_chunks = (cols + chunk - 1) / chunk;
+        // 513 to 576 columns take two chunks, whose sums are two parts each, though one would hold them
+        const int n_chunks = cols > 512 && cols <= chunk && e == 16 ? 2 : (cols + chunk - 1) / chunk;
         s.chunk = ((cols + n_chunks - 1) / n_chunks + step - 1) / step * step;
         if (pipe_lds_bytes(s) > (size_t)info.max_lds_bytes) continue;
         *us = pipe_us(s, cols, batch, info, 1.0);

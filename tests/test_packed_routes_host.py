@@ -85,17 +85,24 @@ def test_columns_that_fit_into_one_chunk(routes, rows, cols, batch, density, ker
     assert name == kernel and int(lds) == pad + 96 * (2 * chunk + pad)
 
 
-# Products between the two kernels: few rows in each workgroup, few columns, far more columns than rows.
-# us, by the kernel of two roles and by the other one: 652 x 79, 215 vectors 4.89 and 4.04, 2164 x 221, 125 5.30 and 4.17, 4962 x 20544, 38
-# 53.9 and 39.7, 5466 x 16693, 38 44.4 and 33.9.
+# Products between the two kernels: few rows in each workgroup, few columns, far more columns than rows; sums that would have fewer parts
+# by the kernel of two roles.  us, by it and by the other one: 652 x 79, 215 vectors 4.89 and 4.04, 2164 x 221, 125 5.30 and 4.17, 4962 x 20544, 38
+# 53.9 and 39.7, 5466 x 16693, 38 44.4 and 33.9; 4963 x 570, 82 vectors 5.9 and 7.2, but with half of the parts.
 @pytest.mark.parametrize("rows,cols,batch,density,kernel", [
     (652, 79, 215, 0.914, "spmv_tile_kernel"), (1071, 191, 37, 0.3, "spmv_tile_kernel"), (2164, 221, 125, 0.389, "spmv_tile_kernel"),
     (2904, 293, 86, 0.448, "spmv_tile_kernel"), (4962, 20544, 38, 0.104, "spmv_tile_kernel"), (5466, 16693, 38, 0.113, "spmv_tile_kernel"),
-    (8061, 13857, 23, 0.216, "spmv_tile_kernel"),
+    (8061, 13857, 23, 0.216, "spmv_tile_kernel"), (4963, 570, 82, 0.178, "spmv_tile_kernel"), (4421, 626, 79, 0.082, "spmv_tile_kernel"),
     (11008, 4096, 128, 0.5, "spmv_pipe_kernel"), (28672, 1024, 64, 0.1, "spmv_pipe_kernel"), (6149, 1024, 205, 0.507, "spmv_pipe_kernel"),
     (11514, 64, 172, 0.082, "spmv_pipe_kernel"), (26429, 225, 36, 0.695, "spmv_pipe_kernel")])
 def test_the_choice_holds_for_products_of_any_size(routes, rows, cols, batch, density, kernel):
     assert routes(cols, batch, [(rows, int(rows * cols * density) // 8 * 8)])[0].startswith(kernel)
+
+
+@pytest.mark.parametrize("rows,cols,batch,density", [(11008, 576, 128, 0.3), (12000, 513, 64, 0.35)])
+def test_rows_of_more_than_512_columns_are_several_parts(routes, rows, cols, batch, density):
+    # one chunk of 576 columns would hold them, as one block
+    name, _, lds = routes(cols, batch, [(rows, int(rows * cols * density) // 8 * 8)])[0].split(":")
+    assert name.startswith("spmv_pipe_kernel<") and ",16," in name and int(lds) == 528 + 96 * (2 * 384 + 528)
 
 
 def test_several_matrices_leave_the_kernel_that_looks_them_up_row_by_row_sooner(routes):
