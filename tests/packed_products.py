@@ -54,6 +54,29 @@ SUMS = [(128, (4096, 4096, 4096), 4096, 0.5), (40, (4096, 4096, 4096), 4096, 0.3
         (100, (4096, 4096, 4096), 2048, 0.1)]
 
 
+
+# silu(gate) * up in one launch: rows of each of the two matrices, cols, vectors, density, and the kernel that is meant; every variant that
+# takes several matrices
+GATED = [
+    (11256, 137, 20, 0.25, "spmv_pipe_kernel<1,8,true>"), (7912, 435, 31, 0.35, "spmv_pipe_kernel<1,16,true>"),
+    (9016, 213, 53, 0.15, "spmv_pipe_kernel<2,8,true>"), (8952, 279, 37, 0.4, "spmv_pipe_kernel<2,16,true>"),
+    (11192, 119, 110, 0.3, "spmv_pipe_kernel<4,8,true>"), (7800, 339, 119, 0.35, "spmv_pipe_kernel<4,16,true>"),
+    (712, 619, 14, 0.4, "spmv_tile_kernel<1,1,1,true,true>"), (1576, 651, 23, 0.2, "spmv_tile_kernel<1,1,2,true,true>"),
+    (488, 463, 60, 0.4, "spmv_tile_kernel<1,2,1,true,true>"), (736, 1027, 76, 0.2, "spmv_tile_kernel<1,2,2,true,true>"),
+    (2728, 775, 12, 0.15, "spmv_tile_kernel<2,1,1,true,true>"), (2120, 1497, 22, 0.25, "spmv_tile_kernel<2,1,2,true,true>"),
+    (1064, 971, 109, 0.7, "spmv_tile_kernel<2,2,1,true,true>"), (1192, 1677, 98, 0.07, "spmv_tile_kernel<2,2,2,true,true>"),
+    (5736, 419, 11, 0.7, "spmv_tile_kernel<3,1,1,true,true>"), (4360, 1147, 28, 0.7, "spmv_tile_kernel<3,1,2,true,true>"),
+    (5136, 487, 45, 0.9, "spmv_tile_kernel<3,2,1,true,true>"), (2504, 1249, 107, 0.3, "spmv_tile_kernel<3,2,2,true,true>"),
+]
+
+
+def gate_and_up(rows, cols, density):
+    rng = np.random.default_rng(rows + cols)
+    both = [helpers.random_sparse(rng, rows, cols, density, scale=0.1) for _ in range(2)]
+    for m in both:
+        m[rows // 2] = 0
+    return both
+
 def matrices(product):
     """The product's matrices: rows without entries, full rows, rows of one entry behind padding entries and gaps wider than
     a lane's columns; the stored arrays end 8 entries behind a multiple of 16."""

@@ -1,5 +1,8 @@
 """The compressor at the edges of its lanes (8 columns), tiles (512) and rounds (2048), on rows that start at
 any element: bit for bit what the checker gives."""
+import ctypes
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -111,3 +114,35 @@ def test_scan_of_the_rows(rows):
     assert np.array_equal(got[2].cpu().numpy(), row_ptr)
     assert np.array_equal(got[0].cpu().numpy().view(np.uint16), values)
     assert np.array_equal(got[1].cpu().numpy(), deltas)
+
+
+# ... as the C interface has it: without a total, with one when row_ptr is complete, with one before it is
+@pytest.mark.parametrize("rows", (1, 8, 8191, 8193, 16385, 24576, 24577, 49161))
+@pytest.mark.parametrize("int8", (False, True))
+def test_scan_of_the_rows_by_every_entry_point(rows, int8):
+    rng = np.random.default_rng(rows)
+    dense = rng.integers(-3, 4, (rows, 5)).astype(np.int8 if int8 else np.float16)
+    row_ptr = (mo.compress_int8 if int8 else mo.compress)(dense)[2]
+    M = torch.from_numpy(dense).cuda()
+    lib, kind = ctypes.CDLL(mk.HIP_LIBRARY_PATH), "i8" if int8 else "f16"
+    stream, other = torch.cuda.current_stream(), torch.cuda.Stream()
+    pointer, i32 = ctypes.c_void_p, ctypes.c_int32
+    for ending in ("count", "count_total", "count_early"):
+        entry = getattr(lib, f"macko_compress_{kind}_{ending}")
+        entry.argtypes = [pointer, i32, i32, pointer] + ([pointer] if ending != "count" else []) + [pointer]
+        for with_total in (False, True) if ending != "count" else (False,):
+            got = torch.full((rows + 1,), -1, dtype=torch.int32, device="cuda")
+            total = torch.full((1,), -1, dtype=torch.int32).pin_memory()
+            at = total.data_ptr() if with_total else None
+            torch.cuda.synchronize()
+            assert entry(M.data_ptr(), rows, 5, got.data_ptr(), *(() if ending == "count" else (at,)), stream.cuda_stream) == 0
+            if ending == "count_total" and with_total:   # who sees the word finds row_ptr complete: read by a stream that waits for nothing
+                until = time.monotonic() + 5.0
+                while int(total) == -1 and time.monotonic() < until:
+                    pass
+                with torch.cuda.stream(other):
+                    seen = got.to("cpu", non_blocking=False)
+                assert np.array_equal(seen.numpy(), row_ptr)
+            torch.cuda.synchronize()
+            assert np.array_equal(got.cpu().numpy(), row_ptr)
+            assert int(total) == (row_ptr[-1] if with_total else -1)

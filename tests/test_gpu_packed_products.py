@@ -130,7 +130,19 @@ def test_long_sums_are_as_exact_as_the_other_kernel_s(batch, rows, cols, density
     assert wrong[1] > 100 and wrong[0] <= 1.25 * wrong[1]
 
 
-# the gate's product: pairs of units of four rows over row blocks of every kernel, columns that fill up no block of 64, vectors that
+def _check_gated(c, rows, cols, batch, x):
+    """Twice the same bits, and those of the products in one launch and the gate behind them."""
+    packed = _pack(ctypes.CDLL(mk.HIP_LIBRARY_PATH), x)
+    args = ([m[0] for m in c], [m[1] for m in c], [m[2] for m in c])
+    got = ops.multiply_packed_silu(*args, rows, cols, packed, batch)
+    for again in (ops.multiply_packed_silu(*args, rows, cols, packed, batch), mk.ops.multiply_packed_silu(*args, rows, cols, packed, batch)):
+        assert torch.equal(again.view(torch.int16), got.view(torch.int16))
+    want = ops.pack_silu_mul(*ops.multiply_packed_several(*args, [rows, rows], cols, packed, batch))
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+# the gate's product: pairs of units of four rows over row blocks, columns that fill up no block of 64, vectors that
 # fill up no block of 16, one chunk and several, matrices of one density and of two that are launched one by one
 @pytest.mark.parametrize("rows,cols,batch,densities", [
     (64, 64, 2, (0.5, 0.5)), (72, 100, 16, (0.3, 0.3)), (1376, 512, 17, (0.5, 0.5)), (1376, 512, 128, (0.1, 0.1)),
@@ -151,11 +163,12 @@ def test_product_of_gate_and_up(rows, cols, batch, densities, special):
     if special:
         x[batch // 2, cols // 3] = float("inf")
         x[0, cols - 1] = float("nan")
-    packed = _pack(ctypes.CDLL(mk.HIP_LIBRARY_PATH), x)
-    args = ([m[0] for m in c], [m[1] for m in c], [m[2] for m in c])
-    got = ops.multiply_packed_silu(*args, rows, cols, packed, batch)
-    for again in (ops.multiply_packed_silu(*args, rows, cols, packed, batch), mk.ops.multiply_packed_silu(*args, rows, cols, packed, batch)):
-        assert torch.equal(again.view(torch.int16), got.view(torch.int16))
-    want = ops.pack_silu_mul(*ops.multiply_packed_several(*args, [rows, rows], cols, packed, batch))
-    assert torch.equal(got.isnan(), want.isnan())
-    assert torch.equal(got.nan_to_num(), want.nan_to_num())
+    _check_gated(c, rows, cols, batch, x)
+
+
+# ... by every kernel that takes two matrices (test_packed_routes_host.py)
+@pytest.mark.parametrize("rows,cols,batch,density,kernel", packed_products.GATED)
+def test_product_of_gate_and_up_by_every_kernel(rows, cols, batch, density, kernel):
+    c = [mk.compress(torch.from_numpy(m).cuda()) for m in packed_products.gate_and_up(rows, cols, density)]
+    x = torch.from_numpy(np.random.default_rng(batch).standard_normal((batch, cols)).astype(np.float16)).cuda()
+    _check_gated(c, rows, cols, batch, x)

@@ -395,6 +395,43 @@ def test_layer_in_one_call_refuses_what_the_operators_refuse():
     assert mk.eager_prefill_layer(x.cpu(), table, table, pos) is NotImplemented
 
 
+class _Subclass(torch.Tensor):
+    pass
+
+
+def test_layer_in_one_call_looks_at_every_argument():
+    model, _ = llm.build_model(0.4, sparse=True, n_layers=1, dim=256, hidden=704, n_heads=2, vocab=1000, max_len=48)
+    layer = model.model.layers[0]
+    att, mlp = layer.self_attn, layer.mlp
+    first, second = layer.input_layernorm, layer.post_attention_layernorm
+    x, pos = torch.randn(1, 5, 256, device="cuda").half(), torch.arange(5, device="cuda")
+    table = torch.ones(1, 1, 5, 128, device="cuda").half()
+    args = [x, table, table.clone(), pos, att.k_cache, att.v_cache, att.head_dim ** -0.5, first.weight, first.eps, second.weight, second.eps]
+    for linear in (att.q_proj, att.k_proj, att.v_proj, att.o_proj, mlp.gate_proj, mlp.up_proj, mlp.down_proj):
+        args += [linear.c_0, linear.c_1, linear.c_2, linear.c_3, linear.c_4]
+    # what the layer hands over with gradients off, and on where none of them asks for one
+    for enabled in (False, True):
+        with torch.set_grad_enabled(enabled):
+            taken = mk.eager_prefill_layer(*[a.detach() if isinstance(a, torch.Tensor) else a for a in args])
+            assert torch.equal(taken.detach(), layer.forward_fused(x, table, table, pos))
+    refused = lambda place, value: mk.eager_prefill_layer(*args[:place], value, *args[place + 1:]) is NotImplemented  # noqa: E731
+    with torch.no_grad():
+        assert mk.eager_prefill_layer(*args) is not NotImplemented
+        for place, value in enumerate(args):
+            if isinstance(value, torch.Tensor):
+                assert refused(place, value.cpu()) and refused(place, value.detach().as_subclass(_Subclass)) and refused(place, None), place
+            elif isinstance(value, float):
+                assert refused(place, 1) and refused(place, torch.tensor(value)), place
+            else:
+                assert refused(place, float(value)) and refused(place, True), place
+        assert refused(0, x[0]) and refused(0, x.expand(2, 5, 256)) and refused(4, att.k_cache[0])
+        assert mk.eager_prefill_layer(*args[:-1]) is NotImplemented and mk.eager_prefill_layer(*args, 1) is NotImplemented
+    with torch.enable_grad():
+        assert refused(0, x.clone().requires_grad_())
+    with torch.autograd.forward_ad.dual_level(), torch.no_grad():
+        assert refused(0, torch.autograd.forward_ad.make_dual(x, x))
+
+
 def test_product_of_gate_and_up_is_an_operator():
     w = torch.randn(72, 64, device="cuda").half()
     c, x = mk.compress(w), torch.randn(5, 64, device="cuda").half()

@@ -21,8 +21,8 @@ def routes(tmp_path_factory):
                     "-c", os.path.join(HERE, "tile_routes.cpp"), "-o", obj], check=True)
     subprocess.run(["g++", "-pie", "-Wl,--defsym=__hip_fatbin=0", obj, "-o", program], check=True)
 
-    def ask(cols, batch, matrices, residual=False):
-        line = " ".join(str(v) for v in (cols, batch, int(residual), len(matrices), *(v for m in matrices for v in m)))
+    def ask(cols, batch, matrices, residual=False, gated=False):
+        line = " ".join(str(v) for v in (cols, batch, 2 if gated else int(residual), len(matrices), *(v for m in matrices for v in m)))
         return subprocess.run([program], input=line + "\n", stdout=subprocess.PIPE, text=True, check=True).stdout.split()  # an answer for each launch
 
     return ask
@@ -109,3 +109,11 @@ def test_several_matrices_leave_the_kernel_that_looks_them_up_row_by_row_sooner(
     # gate and up of dim 1024, 17 vectors at 0.1: 5.26 us by the kernel of two roles, 5.61
     sizes = [(2752, 2752 * 1024 // 10 // 8 * 8)] * 2
     assert routes(1024, 17, sizes)[0].startswith("spmv_pipe_kernel")
+
+
+@pytest.mark.parametrize("rows,cols,batch,density,kernel", packed_products.GATED)
+def test_gate_and_up_take_the_kernel_they_are_meant_for(routes, rows, cols, batch, density, kernel):
+    sizes = [(rows, -(-packed_products.stored_entries(m) // 8) * 8) for m in packed_products.gate_and_up(rows, cols, density)]
+    launches = routes(cols, batch, sizes, gated=True)
+    assert [name.split(":")[0] for name in launches] == [kernel]
+    assert launches == routes(cols, batch, sizes)   # row blocks are whole units of eight rows where they are gated, of four otherwise

@@ -1,8 +1,8 @@
 // Which kernel a product of packed vectors launches, on the host: the host code of csrc/macko_spmv_tile.hip and, in the place of
 // the HIP runtime, functions that write down what would be launched.
 //
-// Reads lines "cols batch residual n rows_1 entries_1 ... rows_n entries_n", prints "<kernel>:<workgroups>:<bytes of LDS>" of each
-// launch, or "refused <code>".
+// Reads lines "cols batch form n rows_1 entries_1 ... rows_n entries_n" (form 1: with a residual, 2: silu(gate) * up of two),
+// prints "<kernel>:<workgroups>:<bytes of LDS>" of each launch, or "refused <code>".
 #include <cxxabi.h>
 
 #include <cstdio>
@@ -65,8 +65,8 @@ int device_info(DeviceInfo *out)
 int main()
 {
     void *somewhere = reinterpret_cast<void *>(uintptr_t{1} << 20);  // never read here
-    int cols, batch, residual, n;
-    while (std::scanf("%d %d %d %d", &cols, &batch, &residual, &n) == 4) {
+    int cols, batch, form, n;
+    while (std::scanf("%d %d %d %d", &cols, &batch, &form, &n) == 4) {
         std::vector<macko_packed_matrix> all((size_t)n);
         for (macko_packed_matrix &m : all) {
             long long rows, entries;
@@ -75,8 +75,9 @@ int main()
         }
         launched.clear();
         const macko_packed_matrix &m = all[0];
-        const int rc = n > 1 ? macko_spmv_f16_packed_several(all.data(), n, somewhere, cols, batch, nullptr)
-                             : macko_spmv_f16_packed(m.values, m.deltas, m.row_ptr, somewhere, residual ? somewhere : nullptr, m.y, m.rows,
+        const int rc = form == 2 && n == 2 ? macko_spmv_f16_packed_silu(&all[0], &all[1], somewhere, somewhere, cols, batch, nullptr)
+                       : n > 1 ? macko_spmv_f16_packed_several(all.data(), n, somewhere, cols, batch, nullptr)
+                             : macko_spmv_f16_packed(m.values, m.deltas, m.row_ptr, somewhere, form ? somewhere : nullptr, m.y, m.rows,
                                                      cols, m.padded_entries, batch, m.ldy, nullptr);
         if (rc != 0)
             std::printf("refused %d\n", rc);
