@@ -1192,7 +1192,7 @@ constexpr double kTileUsPerCycle = 1.06 / 2400.0;
 // where it decides about the route (28672 x 4096, 8 vectors, density 0.05: 40.7 us, estimated 40; 5120 x 13824, 8, 0.1:
 // 24.4, 21).  several: of more than one matrix, which spmv_tile_kernel looks up row by row; its estimate is that for one
 // (up to 64 vectors, 280 launches of two and three matrices of 512 to 4096 columns: what is taken is 0.1 % behind the better one, with the line
-// for one matrix 1 %).
+// for one matrix 1 %).  Fewer columns were not among them and have the line for one matrix.
 bool choose_shape(TileShape *shape, int rows, int cols, long long padded, int batch, bool packed, const DeviceInfo &info, double *us,
                   int most_shift = 2, bool several = false)
 {
@@ -1201,7 +1201,7 @@ bool choose_shape(TileShape *shape, int rows, int cols, long long padded, int ba
     *us = cycles * kTileUsPerCycle;
     TileShape pipe;
     if (packed && choose_pipe_shape(&pipe, rows, cols, padded, batch, shape->group_shift, info, &pipe_us) &&
-        pipe_us < (several && pipe.wave_tiles <= 2 ? 1.03 : 0.97) * *us) {
+        pipe_us < (several && cols >= 512 && pipe.wave_tiles <= 2 ? 1.03 : 0.97) * *us) {
         *shape = pipe;
         *us = pipe_us;
     }

@@ -117,3 +117,11 @@ def test_gate_and_up_take_the_kernel_they_are_meant_for(routes, rows, cols, batc
     launches = routes(cols, batch, sizes, gated=True)
     assert [name.split(":")[0] for name in launches] == [kernel]
     assert launches == routes(cols, batch, sizes)   # row blocks are whole units of eight rows where they are gated, of four otherwise
+
+
+def test_several_matrices_of_few_columns_are_launched_as_each_of_them(routes):
+    # a compiled graph, which launches gate and up one by one, gives the bits of the eager layer (dim 256, hidden 704)
+    sizes = [(704, int(704 * 256 * 0.4) // 8 * 8)] * 2
+    for gated in (False, True):
+        assert routes(256, 19, sizes, gated=gated)[0].startswith("spmv_tile_kernel")
+    assert routes(256, 19, sizes[:1])[0].startswith("spmv_tile_kernel")
