@@ -608,12 +608,12 @@ __global__ void __launch_bounds__(kTileThreads) spmv_tile_kernel(const TileArgs<
 // The multiplying waves run at a higher priority: a matrix instruction and a v_dot8 of another wave on the same SIMD
 // exclude each other (measured: a v_dot8 takes 18 cycles beside a stream of matrix instructions, a plain addition 10).
 // 11008 x 4096, vectors in operand order, three matrices in turn, spmv_tile_kernel and this one: 128 vectors at density 0.5
-// 25.4 and 20.6 us, 0.3 25.0 and 19.4, 0.15 25.0 and 17.5, 0.05 24.6 and 16.0; 64 vectors at 0.2 18.1 and 14.6; 28672 x 1024, 64
-// vectors, 0.1: 23.0 and 15.2; 12288 x 4096, 32 vectors at 0.5 18.2 and 16.3.  What bounds it: 2.2 us in front of the first product and
-// 1.5 behind the last one (row_ptr, the first entries, the sums).  Between them a chunk of 384 columns takes 3600 cycles, in which LDS
-// is busy for 2400 (each of the 16 stores of a pass for 7: 32 lanes at random places meet in a bank three or four times), the
-// path from L2 for 2000 (X: 1 MB per compute unit at 64 bytes a cycle), vector and matrix instructions, which exclude each
-// other, for 2600: 21.2 us with the entries always in L2 and 18.6 with X in L1 as well.  Tried and not faster: 8 + 8 waves, both
+// 24.8 and 20.4 us, 0.3 24.7 and 18.6, 0.15 25.0 and 17.3, 0.05 24.6 and 15.9; 64 vectors at 0.2 18.0 and 14.7; 28672 x 1024, 64
+// vectors, 0.1: 22.4 and 15.1; 12288 x 4096, 32 vectors at 0.5 18.0 and 16.1.  What bounds it: 2.2 us in front of the first product and
+// 1.5 behind the last one (row_ptr, the first entries, the sums).  Between them a chunk of 384 columns takes 3100 cycles by the
+// counters (128 vectors at 0.5), in which LDS is busy for 2100 (each of the 16 stores of a pass for 7: 32 lanes at random places meet in a bank three or four
+// times), the path from L2 for 2000 (X: 1 MB per compute unit at 64 bytes a cycle), vector and matrix instructions, which exclude
+// each other, for 2500.  While it took 21.9 us: 21.2 with the entries always in L2 and 18.6 with X in L1 as well.  Tried and not faster: 8 + 8 waves, both
 // roles at one priority (22.7), a chunk's places worked out behind the stores of the one before, by all or by some of the waves (21.5 to
 // 22.0), the next unit's A requested between products, lines touched some chunks ahead; chunks that end anywhere in the
 // ring of units: the compiler then waits for all loads or spills.
